@@ -193,6 +193,90 @@ def run(state):
     return list(net.predict_batches(state["batches"]))
 
 
+def _conv64(x, w, bias, cd):
+    """A convolution of doubles, image by image, as one matrix product over the unfolded image."""
+    top, bottom, left, right = cd.pads
+    filters, _, r, s = w.shape
+    out = []
+    for image in torch.nn.functional.pad(x, (left, right, top, bottom)):
+        columns = torch.nn.functional.unfold(image[None], (r, s), stride=(cd.sr, cd.sc))[0]
+        out.append(w.reshape(filters, -1) @ columns + (bias[:, None] if cd.use_bias else 0.0))
+    rows = (x.shape[2] + top + bottom - r) // cd.sr + 1
+    return torch.stack(out).reshape(x.shape[0], filters, rows, -1)
+
+
+def _layer64(layer, ins, p):
+    x, kind = ins[0], layer.kind
+    if kind == "conv2d":
+        return _conv64(x, p["K"], p["bias"], layer.attrs["cd"])
+    if kind == "dense":
+        return x @ p["W"] + p["bias"]
+    if kind == "batchnorm":
+        m, v, g, b = (p[k][None, :, None, None] for k in ("mean", "variance", "bn_g", "bn_b"))
+        return (x - m) / torch.sqrt(v + layer.attrs["epsilon"]) * g + b
+    if kind == "relu":
+        return torch.relu(x)
+    if kind == "maxpool2d":
+        pd = layer.attrs["pd"]
+        top, bottom, left, right = pd.pad
+        return torch.nn.functional.max_pool2d(torch.nn.functional.pad(x, (left, right, top, bottom), value=-3.40282e38), pd.ksize, pd.stride)
+    if kind == "avgpool2d":  # (the networks pool whole planes)
+        return x.mean((2, 3), keepdim=True)
+    if kind == "resize":
+        fy, fx = layer.out_shape[2] // x.shape[2], layer.out_shape[3] // x.shape[3]
+        return x.repeat_interleave(fy, 2).repeat_interleave(fx, 3)
+    if kind == "concat":
+        return torch.cat(ins, layer.attrs["axis"])
+    if kind == "pad":
+        top, right, bottom, left = layer.attrs["pads"]
+        return torch.nn.functional.pad(x, (left, right, top, bottom), value=layer.attrs["constant"])
+    if kind == "reshape":
+        return x.reshape(x.shape[0], *layer.out_shape[1:])
+    if kind == "softmax":
+        return torch.softmax(x, layer.attrs["axis"])
+    if kind == "sigmoid":
+        return torch.sigmoid(x)
+    if kind in ("sum", "add_n"):
+        return sum(ins[1:], x)
+    raise ValueError("no 64-bit form of layer kind " + kind)
+
+
+def exact(case, seed):
+    """What ``run`` returns for the parameters and inputs of ``prepare``, computed with torch in 64 bits.  The coordinates that
+    the block's pool writes are choices, not computed numbers."""
+    state = prepare(case, seed)
+    net = state["net"]
+    heads = [l for l in net.layers for c in l.children if c.kind in ("reshape", "softmax")]
+    readers = {id(l): len(l.children) for l in net.layers}
+
+    def forward(x):
+        values, kept = {}, {}
+        left = dict(readers)
+        for layer in net.layers:
+            if layer.kind == "input":
+                y = x
+            else:
+                params = {k: _as_torch(t).double() for k, t in net.dparams.get(id(layer), {}).items()}
+                y = _layer64(layer, [values[id(q)] for q in layer.parents], params)
+                for q in layer.parents:
+                    left[id(q)] -= 1
+                    if left[id(q)] == 0:
+                        del values[id(q)]
+            values[id(layer)] = y
+            if layer in net.lout or layer in heads:
+                kept[id(layer)] = y.reshape(layer.out_shape)
+        return kept
+
+    if case["mode"] == "forward":
+        kept = forward(_as_torch(state["x"]).double())
+        return [kept[id(l)] for l in net.lout + heads] + [None] * (len(state["out"]) - len(net.lout + heads))
+    outs = []
+    for batch in state["batches"]:
+        kept = forward(torch.from_numpy(batch).cuda().double())
+        outs.append([kept[id(l)].cpu().numpy() for l in net.lout])
+    return outs[0] if case["mode"] == "predict" else outs
+
+
 def _work(case):
     """Flops of the convolutions and dense layers in the direct form; bytes: parameters, inputs and outputs of the network.
     A layer walk also hands every layer's output over in memory: written once and read once."""

@@ -2223,6 +2223,8 @@ __global__ __launch_bounds__(256) void wino_fused_reduce_kernel(const ConvParams
     for (int k = 0; k < 4; k++) wino_store_row(p, chan[k], m_first + k, img, ty, tx, plane, pair, y[k].x, y[k].y, y[k].z, y[k].w);
 }
 
+#include "conv_split.h"
+
 // ---------------------------------------------------------------- host side
 int g_algo = 0;
 // Measurement: while collecting, every launch of a convolution kernel (not the filter repack, not
@@ -2322,6 +2324,30 @@ constexpr int FUSED_TILE0 = 6;      // plan "tile" numbers 6 .. 6 + NUM_FUSED - 
 constexpr int FUSED_ROW_ALIGN = 8;  // the transformed filters are padded to whole K-steps of every variant
 constexpr int UP2X2_TILE = FUSED_TILE0 + NUM_FUSED;  // plan "tiles" of the upsampled-input form of a 2x2 convolution: conv_up2x2_kernel<3>, <2>
 constexpr int NUM_PLAN_TILES = UP2X2_TILE + 2;
+
+// The split form (conv_split.h): plan "tiles" from 16 on (10 .. 15 name nothing and stay refused in a plans file).
+// Tile shapes, measured at batch 64 (us; fp32 tiles before): 128x128 for many tiles of long K (256 channels 3x3 on 56x56, batch
+// 32: 826 -> 537, 220 TFLOP/s of fp32 work: the engine clock falls to 1.73 GHz under it and the matrix pipe is busy 69 % of
+// that), 128x64 for most 1x1 layers (1024 -> 256 on 14x14: 60 -> 42; 256 -> 1024: 60 -> 44; 64 -> 256 on 56x56: 73 -> 63, of
+// which 256 MB of traffic are 43), 64x128 where there are 64 filters (256 -> 64 on 56x56: 68 -> 54), 64x64 for few tiles.
+// A 128x64 tile gives every wavefront filters of its own and all the pixels: its filters then cross L1 once, not twice.
+#define SPLIT(WM, WN, TM, TN, WGS)                                                                                                           \
+    {                                                                                                                                        \
+        "conv_split_kernel<" #WM "," #WN "," #TM "," #TN "," #WGS ">", WM *TM * 32, WN *TN * 32, SPLIT_K, conv_split_kernel<WM, WN, TM, TN, WGS>, \
+            conv_reduce_kernel<WM, WN, TM, TN>, 0                                                                                            \
+    }
+const Variant ksplit[] = {SPLIT(2, 2, 2, 2, 2), SPLIT(4, 1, 1, 2, 3), SPLIT(2, 2, 1, 2, 3), SPLIT(2, 2, 1, 1, 4)};
+constexpr int NUM_SPLIT = (int)(sizeof(ksplit) / sizeof(ksplit[0]));
+constexpr int SPLIT_TILE0 = 16;
+bool is_split_tile(int tile) { return tile >= SPLIT_TILE0 && tile < SPLIT_TILE0 + NUM_SPLIT; }
+bool is_plan_tile(int tile) { return (tile >= -1 && tile < NUM_PLAN_TILES) || is_split_tile(tile); }
+int split_steps(int C, int RS) { return (C + SPLIT_K - 1) / SPLIT_K * RS; }
+size_t split_filter_bytes(int C, int RS, int Mp) { return (size_t)split_steps(C, RS) * 2 * (Mp / 32) * SPLIT_UNIT; }
+// Whether the split form can run a convolution: filters within a buffer descriptor, and channels in whole groups of eight also
+// where a folded Concat has two tensors for them.
+bool split_applies(int C, int Kf, int R, int S) {
+    return C % 16 == 0 && split_filter_bytes(C, R * S, (Kf + M_ALIGN - 1) / M_ALIGN * M_ALIGN) < ((size_t)1 << 31);
+}
 
 // K slices of the left-over tiles of a one-launch Winograd plan that asks for `slices` of them (T blocks in the launch):
 // the tiles beyond a whole number per CU are divided, as in forced_plan; 1 = nothing is divided
@@ -2426,7 +2452,7 @@ Plan forced_plan(const Variant *family, int tile, int slices, int Kf, int C, int
     const Variant &v = family[tile];
     Plan pl;
     pl.tile = tile;
-    pl.nsteps = v.cpb ? (C + v.cpb - 1) / v.cpb : (C * RS + 15) / 16;
+    pl.nsteps = v.cpb == SPLIT_K ? split_steps(C, RS) : (v.cpb ? (C + v.cpb - 1) / v.cpb : (C * RS + 15) / 16);
     pl.tiles = (long long)((Kf + v.bm - 1) / v.bm) * ((npix + v.bn - 1) / v.bn);
     pl.leftover = pl.tiles % num_cu;
     int want = slices < 1 ? 1 : (slices > pl.nsteps ? pl.nsteps : slices);
@@ -2451,6 +2477,7 @@ struct CachedFilters {
     int wino_rows;
     float *Wfused;  // 3x3 filters: the transformed filters of the one-launch Winograd form [fused_rows][16][Mp], made on first use
     int fused_rows;
+    void *Wsplit;  // the filters as three bf16 parts in the operand order of the split form (split_filter_kernel), made on first use
     float *Wup;  // 2x2 filters: the nine weight-sum rows per channel of the upsampled-input form [C][9][Mp] (up2x2_filter_kernel), made on first use
     bool stale;  // K was written through this library since the last repack
 };
@@ -2465,6 +2492,14 @@ int cache_rows(int C, int R, int S) {
         if (r > rows) rows = r;
     }
     return rows;
+}
+
+int launch_split_filters(int dev, const float *K, void *Ws, int Kf, int C, int RS, int Mp) {
+    const int mblocks = Mp / 32, k16s = split_steps(C, RS) * 2;
+    hipLaunchKernelGGL(split_filter_kernel, dim3((unsigned)(((size_t)k16s * mblocks * 64 + 255) / 256)), dim3(256), 0, state(dev).stream, K, (uintx4 *)Ws, Kf, C, RS,
+                       mblocks, k16s);
+    EH_CHECK_LAUNCH();
+    return 0;
 }
 
 int repack(int dev, CachedFilters &e) {
@@ -2486,6 +2521,7 @@ int repack(int dev, CachedFilters &e) {
         hipLaunchKernelGGL(up2x2_filter_kernel, dim3((unsigned)(((size_t)e.C * e.Mp + 255) / 256)), dim3(256), 0, state(dev).stream, e.K, e.Wup, e.Kf, e.C, e.Mp);
         EH_CHECK_LAUNCH();
     }
+    if (e.Wsplit != nullptr) EH_TRY(launch_split_filters(dev, e.K, e.Wsplit, e.Kf, e.C, e.R * e.S, e.Mp));
     e.stale = false;
     return 0;
 }
@@ -2530,6 +2566,7 @@ void conv_filters_released(int dev, const void *base, size_t bytes) {
             if (c[i].Wwino) (void)hipFree(c[i].Wwino);
             if (c[i].Wfused) (void)hipFree(c[i].Wfused);
             if (c[i].Wup) (void)hipFree(c[i].Wup);
+            if (c[i].Wsplit) (void)hipFree(c[i].Wsplit);
             c[i] = c.back();
             c.pop_back();
         } else {
@@ -2565,6 +2602,7 @@ int eddlhip_conv2d_cache_filters(int dev, const float *K, int Kf, int C, int R, 
     e.Wfused = nullptr;
     e.fused_rows = 0;
     e.Wup = nullptr;
+    e.Wsplit = nullptr;
     e.stale = true;
     EH_REQUIRE((size_t)e.rows * e.Mp * sizeof(float) < ((size_t)1 << 31),
                "conv2d_cache_filters: the repacked filter matrix (%d taps x %d channels) exceeds the 2 GiB a buffer descriptor covers", e.rows, e.Mp);
@@ -2592,6 +2630,7 @@ int eddlhip_conv2d_uncache_filters(int dev, const float *K) {
             if (c[i].Wwino) EH_TRY_HIP(hipFree(c[i].Wwino));
             if (c[i].Wfused) EH_TRY_HIP(hipFree(c[i].Wfused));
             if (c[i].Wup) EH_TRY_HIP(hipFree(c[i].Wup));
+            if (c[i].Wsplit) EH_TRY_HIP(hipFree(c[i].Wsplit));
             c[i] = c.back();
             c.pop_back();
         } else {
@@ -2602,9 +2641,10 @@ int eddlhip_conv2d_uncache_filters(int dev, const float *K) {
 }
 
 int eddlhip_conv2d_force_plan(int tile, int slices) {
-    EH_REQUIRE(tile >= -1 && tile < NUM_PLAN_TILES,
-               "conv2d_force_plan: tile is -1 (automatic), 0..3, 4 .. %d (the Winograd forms where they apply) or %d, %d (a 2x2 filter on an input upsampled twice)",
-               UP2X2_TILE - 1, UP2X2_TILE, UP2X2_TILE + 1);
+    EH_REQUIRE(is_plan_tile(tile),
+               "conv2d_force_plan: tile is -1 (automatic), 0..3, 4 .. %d (the Winograd forms where they apply), %d, %d (a 2x2 filter on an input upsampled twice) "
+               "or %d .. %d (the split form where it applies)",
+               UP2X2_TILE - 1, UP2X2_TILE, UP2X2_TILE + 1, SPLIT_TILE0, SPLIT_TILE0 + NUM_SPLIT - 1);
     g_force_tile = tile;
     g_force_slices = slices;
     return 0;
@@ -2651,7 +2691,7 @@ int eddlhip_conv2d_tuned_load(int dev, const char *host_path) {
         int *k = t.key;
         const int got = sscanf(line, "%d %d %d %d %d %d %d %d %d %d | %d %d", k, k + 1, k + 2, k + 3, k + 4, k + 5, k + 6, k + 7, k + 8, k + 9, &t.tile,
                                &t.slices);
-        if (got != 12 || t.tile < -1 || t.tile >= NUM_PLAN_TILES || t.slices < 1 || t.slices > 16) {  // (no search tries more than 16 slices)
+        if (got != 12 || !is_plan_tile(t.tile) || t.slices < 1 || t.slices > 16) {  // (no search tries more than 16 slices)
             bad = true;
             break;
         }
@@ -2759,6 +2799,8 @@ int conv2d_winograd_fused(int variant, int slices, int dev, const float *I, cons
 int conv2d_up2x2(int variant, int dev, const float *I, const float *K, const float *bias, float *O, int N, int C, int H, int W, int Kf, int P, int Q, const float *bn_g,
                  const float *bn_b, const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu);
 
+int conv2d_split(const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs);
+
 // Whether a convolution is the one conv_up2x2_kernel computes: a 2x2 stride-1 filter on ONE tensor upsampled twice in both
 // directions, no padding above or to the left (below and to the right the image is followed by zeros, as many as the
 // output size asks for), whole K-steps of 4 channels, and everything within 32-bit offsets.
@@ -2831,7 +2873,7 @@ size_t winograd_workspace(bool fold, int N, int C, int Kf, int fs, int P, int Q,
 // fewer K slices first.  Returns 0 with *out filled, 1 when these tensors cannot be searched on (the output overlaps an
 // input: repeating the call would change what it reads), or minus the error code of a runtime failure.
 int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, long long chunk_pix, bool wino_ok, bool fold_ok, bool fused_ok, bool up_ok,
-                TunedPlan *out) {
+                bool split_ok, TunedPlan *out) {
     {
         const size_t out_bytes = (size_t)c.N * c.Kf * c.P * c.Q * 4, in_bytes = (size_t)c.N * (c.I2 ? c.C / 2 : c.C) * c.H * c.W * 4;
         const char *o_lo = (const char *)c.O, *o_hi = o_lo + out_bytes;
@@ -2908,6 +2950,16 @@ int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, l
                 if (ns == last_slices) continue;  // the same plan as the one before
                 last_slices = ns;
                 time_plan(1 + (NUM_FUSED - 1 - fv), FUSED_TILE0 + fv, sl);
+            }
+        }
+    if (split_ok)  // the split form: its tile shapes, undivided and with the left-over tiles in K slices
+        for (int v = 0; v < NUM_SPLIT; v++) {
+            int last_slices = 0;
+            for (int sl : kSearchSlices) {
+                const Plan fp = forced_plan(ksplit, v, sl, c.Kf, c.C, c.R * c.S, chunk_pix, num_cu);
+                if (fp.nslices == last_slices) continue;
+                last_slices = fp.nslices;
+                time_plan(5 + v, SPLIT_TILE0 + v, sl);
             }
         }
     for (int tile = 0; tile < 4; tile++) {
@@ -3117,6 +3169,13 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     if ((wino_ok && (g_force_tile == 4 || (g_wino && g_force_tile < 0 && !g_tuning))) || (fold_ok && g_force_tile == 5))
         return conv2d_winograd(g_force_tile == 5, R, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top, pad_left, P, Q, bn_g, bn_b,
                                bn_mean, bn_var, bn_eps, residual, relu);
+    // the split form: any filter shape, as long as a chunk of the input is addressed like the direct kernels do; never from the
+    // fixed scratch array (its filters take half as much again as the repacked ones)
+    const bool split_ok = !gemm && !no_alloc && g_algo == 0 && split_applies(C, Kf, R, S);
+    if (split_ok && is_split_tile(g_force_tile)) {
+        const int tile = g_force_tile - SPLIT_TILE0;
+        return conv2d_split(ksplit[tile], forced_plan(ksplit, tile, g_force_slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p, chunk_imgs);
+    }
     const bool query = gemm != nullptr && gemm->need_out != nullptr;  // report the workspace need, launch nothing
     bool plan_open = false;                                         // a search could still pick any plan for this geometry
     if (g_autotune && g_force_tile < 0 && g_algo == 0 && g_split != 0) {
@@ -3134,7 +3193,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
             TunedPlan best;
             memcpy(best.key, key, sizeof(key));
             const size_t ws_before = state(dev).workspace_bytes;
-            const int src = search_plan(call, family, plan, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, &best);
+            const int src = search_plan(call, family, plan, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, split_ok, &best);
             if (src < 0) return -src;  // a runtime error inside the search
             // the candidates may have taken far more workspace than the plan that stays: let it grow back to what is needed
             // (not inside another convolution's call, whose buffers live there)
@@ -3152,6 +3211,10 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
         if (found != nullptr && found->tile >= FUSED_TILE0 && found->tile < FUSED_TILE0 + NUM_FUSED && fused_ok)
             return conv2d_winograd_fused(found->tile - FUSED_TILE0, found->slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top, pad_left, P, Q, bn_g,
                                          bn_b, bn_mean, bn_var, bn_eps, residual, relu);
+        if (found != nullptr && is_split_tile(found->tile) && split_ok) {
+            const int tile = found->tile - SPLIT_TILE0;
+            return conv2d_split(ksplit[tile], forced_plan(ksplit, tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p, chunk_imgs);
+        }
         if (found != nullptr && found->tile >= 0 && found->tile < 4)
             plan = forced_plan(family, found->tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu);
     }
@@ -3630,6 +3693,81 @@ int conv2d_winograd_fused(int variant, int slices, int dev, const float *I, cons
     const char *name = wide ? fv.name_wide : fv.name;
     if (leftover > 0) snprintf(g_last_kernel, sizeof(g_last_kernel), "winograd[%s +ksplit(%lld tiles x %d), %lld blocks]", name, leftover, nslices, (long long)N * per_img);
     else snprintf(g_last_kernel, sizeof(g_last_kernel), "winograd[%s, %lld blocks]", name, (long long)N * per_img);
+    return 0;
+}
+
+// The split form (conv_split.h) of the call that `call` describes, under a plan of split steps.
+// Workspace: [split filters unless kept][partial tiles].
+int conv2d_split(const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs) {
+    hipStream_t st = state(dev).stream;
+    const int RS = call.R * call.S, N = call.N;
+    EH_REQUIRE(plan.tiles <= 0x3fffffffLL, "conv2d: too many tiles");
+    const long long leftover = plan.nslices > 1 ? plan.leftover : 0;
+    const size_t w_bytes = split_filter_bytes(call.C, RS, call.Mp);
+    const size_t partial_bytes = (size_t)plan.nslices * leftover * v.bm * v.bn * sizeof(float);
+    const void *Ws = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(g_cache_mutex);
+        for (CachedFilters &e : g_cache[dev]) {
+            if (e.K == call.K && e.Kf == call.Kf && e.C == call.C && e.R == call.R && e.S == call.S) {
+                if (e.Wsplit == nullptr && !state(dev).capturing) {
+                    if (hipMalloc(&e.Wsplit, w_bytes) != hipSuccess) {
+                        e.Wsplit = nullptr;
+                        (void)hipGetLastError();
+                        break;  // no room to keep them: split per call
+                    }
+                    e.stale = true;
+                }
+                if (e.Wsplit != nullptr) {
+                    if (e.stale) EH_TRY(repack(dev, e));
+                    Ws = e.Wsplit;
+                }
+                break;
+            }
+        }
+    }
+    const size_t ws_filters = Ws ? 0 : ((w_bytes + 255) & ~(size_t)255);
+    void *ws = nullptr;
+    if (ws_filters + partial_bytes > 0) EH_TRY(get_workspace(dev, ws_filters + partial_bytes, &ws));
+    if (Ws == nullptr) {
+        EH_TRY(launch_split_filters(dev, call.K, ws, call.Kf, call.C, RS, call.Mp));
+        Ws = ws;
+    }
+    ConvParams q = call;
+    q.Wp = (const float *)Ws;
+    q.wp_bytes = (unsigned)w_bytes;
+    q.partial = (float *)((char *)ws + ws_filters);
+    q.nsteps = plan.nsteps;
+    q.gm = (call.Kf + v.bm - 1) / v.bm;
+    const size_t img_elems = (size_t)call.Cimg * call.H * call.W, out_elems = (size_t)call.Kf * call.PQ;
+    for (long long b0 = 0; b0 < N; b0 += chunk_imgs) {
+        const int nb = (int)((N - b0 < chunk_imgs) ? N - b0 : chunk_imgs);
+        q.N = nb;
+        q.I = call.I + b0 * img_elems;
+        q.I2 = call.I2 + b0 * img_elems;
+        q.O = call.O + b0 * out_elems;
+        q.residual = call.residual ? call.residual + b0 * out_elems : nullptr;
+        q.npix = (long long)nb * call.PQ;
+        q.in_bytes = (unsigned)(nb * img_elems * sizeof(float));
+        const long long gn = (q.npix + v.bn - 1) / v.bn, tiles = gn * q.gm;
+        q.gn = (int)gn;
+        const long long split_tiles = (nb == chunk_imgs) ? leftover : 0;  // a short last chunk runs undivided
+        q.main_tiles = (int)(tiles - split_tiles);
+        q.nslices = split_tiles > 0 ? plan.nslices : 1;
+        q.slice_steps = split_tiles > 0 ? plan.slice_steps : plan.nsteps;
+        const long long wgs = q.main_tiles + split_tiles * q.nslices;
+        q.trace = (g_trace != nullptr && wgs <= g_trace_wgs) ? g_trace : nullptr;
+        EH_TRY(prof_begin(st));
+        hipLaunchKernelGGL(v.kernel, dim3((unsigned)wgs), dim3(256), 0, st, q);
+        EH_CHECK_LAUNCH();
+        EH_TRY(prof_end(st));
+        if (split_tiles > 0) {
+            hipLaunchKernelGGL(v.reduce, dim3((unsigned)(split_tiles * (v.bm / 32) * (v.bn / 32))), dim3(256), 0, st, q);
+            EH_CHECK_LAUNCH();
+        }
+    }
+    if (leftover > 0) snprintf(g_last_kernel, sizeof(g_last_kernel), "%s +ksplit(%lld tiles x %d)", v.name, leftover, plan.nslices);
+    else snprintf(g_last_kernel, sizeof(g_last_kernel), "%s", v.name);
     return 0;
 }
 

@@ -253,6 +253,11 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * (same tolerance).  Because a convolution of the stored, enlarged tensor cannot take this form, such a call is a
  * geometry of its own in the plans table (kind 2 / 3 instead of 0 / 1): the same layer run after a stand-alone
  * UpSampling2D keeps its own plan, and the two agree to the convolution's tolerance, not bit for bit.
+ * The split form (force_plan(16 .. 19, .), or the search; any filter, channel counts that are multiples of 16): every fp32
+ * number as an exact sum of three bf16 numbers, the six largest of their nine products on the bf16 matrix instructions,
+ * fp32 sums.  Its error against exact sums is below the fp32 instruction's (fewer roundings per sum); infinities, NaN and
+ * overflow come out as the fp32 kernels bring them (a tile that is not finite is computed again by them).  Workspace: the
+ * split filters, 6 bytes a weight, unless registered; never taken by eddlhip_conv2d_fwd_noalloc.
  *
  * eddlhip_conv2d_last_kernel() names the kernel the calling thread's last eddlhip_conv2d_fwd
  * launched, followed by " +ksplit(T tiles x S)" when T tiles were divided into S slices; for the Winograd form
@@ -266,7 +271,7 @@ const char *eddlhip_conv2d_last_kernel(void);
  * shape x K slices and the Winograd forms, every launch timed by itself, the fastest of three to nine launches per plan,
  * on the call's own tensors) and remembers one; later calls with that geometry take it.  Which one: of all plans within
  * 3 % of the fastest, the first in a fixed order of preference (the planner's own plan, the one-launch Winograd form, the
- * direct tiles, the Winograd forms that keep a transformed input in memory - those are tried only below 512 MB of
+ * split form, the direct tiles, the Winograd forms that keep a transformed input in memory - those are tried only below 512 MB of
  * workspace; within a form fewer K slices first), so that two searches of one geometry agree unless two plans differ by
  * just that margin.  A caller that needs run-to-run identical bits loads a plans file instead of searching.  The call's
  * tensors must not alias: when the output overlaps an input or the residual, nothing is searched or recorded and the
@@ -296,7 +301,8 @@ int eddlhip_conv2d_tuned_load(int dev, const char *host_path);
  * (1 = none).  tile = 4: the Winograd form wherever it applies (its product launch is planned or searched as usual),
  * 5: its folded form wherever that applies, 6 / 7: its one-launch form on tiles of 32 / 64 filters x 32 blocks, `slices`
  * K slices for the left-over tiles as above; 8 / 9: the upsampled-input form of a 2x2 filter, built for three / two
- * workgroups per CU; the planner's choice wherever a form does not apply.  Acts on the calling thread only. */
+ * workgroups per CU; 16 .. 19: the split form on tiles of 128x128, 128x64, 64x128, 64x64 outputs; the planner's choice
+ * wherever a form does not apply.  Acts on the calling thread only. */
 int eddlhip_conv2d_force_plan(int tile, int slices);
 
 /* Filters that stay fixed between calls (inference).  Every eddlhip_conv2d_fwd first repacks its

@@ -82,6 +82,21 @@ def test_tuned_plan_table_round_trips_through_a_file(tmp_path):
     assert lib.eddlhip_conv2d_tuned_plans(0) == 0
 
 
+def test_plans_of_the_split_form_are_accepted(tmp_path):
+    """Plan numbers 16 .. 19 name the tiles of the split form; their neighbours name nothing."""
+    from eddl_amd import _lib
+    lib = _lib.load()
+    lib.eddlhip_conv2d_autotune(-1)
+    path = tmp_path / "plans.txt"
+    for tile in range(10, 24):
+        path.write_text("4 128 64 1 1 1 1 %d 28 1 | %d 2\n" % (tile, tile))
+        assert (lib.eddlhip_conv2d_tuned_load(0, str(path).encode()) == 0) == (16 <= tile <= 19), tile
+        assert (lib.eddlhip_conv2d_force_plan(tile, 1) == 0) == (16 <= tile <= 19), tile
+    lib.eddlhip_conv2d_force_plan(-1, 1)
+    assert lib.eddlhip_conv2d_tuned_plans(0) == 4
+    lib.eddlhip_conv2d_autotune(-1)
+
+
 def test_committed_plans_files_load():
     """The plans files the profiled commands name (profiles/plans_<workload>.txt) are in the loader's format, and what the
     loader keeps of each is what the file says, line for line."""

@@ -1158,3 +1158,129 @@ def test_conv2d_autotune_searches_once_per_geometry_and_stays_within_tolerance(h
     assert hip.conv_tuned_plans() == 0
     hip.conv2D(dx, dw, None, O, 1, 1, 1, 1)
     assert hip.conv_tuned_plans() == 0                        # switched off: no search
+
+
+# ------------------------------------------------------------------ the split form (three bf16 parts per fp32 number)
+# N C H W Kf R S strides pads(top, left): edges of the pixel tiles (64, 128), of the filter tiles (64, 128), half and partial
+# K-steps of 32 channels, taps outside the image on every side, strides, filters that are not square
+SPLIT_CASES = {
+    "1x1 one pixel": (1, 16, 1, 1, 1, 1, 1, (1, 1), (0, 0)),
+    "1x1 ragged": (3, 48, 9, 13, 70, 1, 1, (1, 1), (0, 0)),
+    "1x1 stride 2": (2, 96, 15, 17, 129, 1, 1, (2, 2), (0, 0)),
+    "3x3": (2, 32, 11, 13, 65, 3, 3, (1, 1), (1, 1)),
+    "3x3 stride 2": (5, 80, 14, 9, 64, 3, 3, (2, 2), (1, 1)),
+    "2x5": (2, 64, 8, 10, 33, 2, 5, (1, 2), (0, 2)),
+    "7x7": (1, 16, 20, 23, 31, 7, 7, (2, 1), (3, 3)),
+    "long K": (1, 512, 7, 9, 40, 3, 3, (1, 1), (1, 1)),
+}
+
+
+def _conv64(x, w, stride, pad, P, Q):
+    """The convolution of doubles, tap by tap."""
+    N, C, H, W = x.shape
+    Kf, _, R, S = w.shape
+    big = np.zeros((N, C, (P - 1) * stride[0] + R + H, (Q - 1) * stride[1] + S + W))
+    big[:, :, pad[0]:pad[0] + H, pad[1]:pad[1] + W] = x
+    out = np.zeros((N, Kf, P, Q))
+    for ky in range(R):
+        for kx in range(S):
+            win = big[:, :, ky:ky + (P - 1) * stride[0] + 1:stride[0], kx:kx + (Q - 1) * stride[1] + 1:stride[1]]
+            out += np.einsum("kc,ncpq->nkpq", w[:, :, ky, kx].astype(np.float64), win)
+    return out
+
+
+@pytest.mark.parametrize("plan", [(16, 1), (17, 1), (17, 3), (18, 1), (18, 2), (19, 1), (19, 16)])
+@pytest.mark.parametrize("case", sorted(SPLIT_CASES))
+def test_conv2d_split_form_is_no_further_from_64_bits_than_the_fp32_form(hip, case, plan):
+    N, C, H, W, Kf, R, S, stride, pad = SPLIT_CASES[case]
+    P, Q = (H + 2 * pad[0] - R) // stride[0] + 1, (W + 2 * pad[1] - S) // stride[1] + 1
+    rng = np.random.default_rng(1700 + sorted(SPLIT_CASES).index(case))
+    x = rng.standard_normal((N, C, H, W), dtype=np.float32)
+    w = (rng.standard_normal((Kf, C, R, S)) * np.sqrt(2.0 / (C * R * S))).astype(np.float32)
+    X, Wd, O = hip.array(x), hip.array(w), hip.full((N, Kf, P, Q), np.nan)
+    try:
+        # undivided: a sum's error grows with the roundings of its longest chain, and slices shorten the chain of either form
+        hip.force_conv_plan(2, 1)
+        hip.conv2D(X, Wd, None, O, *stride, *pad)
+        fp32 = O.numpy()
+        assert not hip.last_conv_kernel().startswith("conv_split")
+        hip.force_conv_plan(*plan)
+        hip.fill_(O, np.nan)
+        hip.conv2D(X, Wd, None, O, *stride, *pad)
+        assert hip.last_conv_kernel().startswith("conv_split")
+        got = O.numpy()
+        hip.cache_conv_filters(Wd)                      # from registered filters: the same bits
+        hip.fill_(O, np.nan)
+        hip.conv2D(X, Wd, None, O, *stride, *pad)
+        assert np.array_equal(got, O.numpy())
+        hip.uncache_conv_filters(Wd)
+    finally:
+        hip.force_conv_plan(-1, 1)
+    ref = _conv64(x, w, stride, pad, P, Q)
+    scale = np.linalg.norm(ref)
+    # the result's own rounding to fp32 (2^-24 of a value at most, both forms have it) beside the fp32 form's error
+    assert np.linalg.norm(got - ref) <= np.linalg.norm(fp32 - ref) + 2.0 ** -24 * scale
+    assert_conv_close(ref, got, case)
+
+
+@pytest.mark.parametrize("plan", [(16, 1), (17, 2), (18, 1), (19, 4)])
+def test_conv2d_split_form_reads_folded_inputs_and_applies_the_epilogue(hip, plan):
+    """A folded Concat and a folded UpSampling give the bits of the stored tensor; the epilogue those of the separate layers."""
+    rng = np.random.default_rng(1790)
+    N, C, H, W, Kf = 2, 48, 6, 10, 72
+    a, b = rng.standard_normal((2, N, C // 2, H, W), dtype=np.float32)
+    w = (rng.standard_normal((Kf, C, 3, 3)) * 0.06).astype(np.float32)
+    bias = rng.standard_normal(Kf).astype(np.float32)
+    g, bb, mean = rng.uniform(0.8, 1.2, Kf).astype(np.float32), *(rng.standard_normal((2, Kf)) * 0.1).astype(np.float32)
+    var = rng.uniform(0.5, 1.5, Kf).astype(np.float32)
+    A, B, AB, Wd = hip.array(a), hip.array(b), hip.array(np.concatenate([a, b], 1)), hip.array(w)
+    up = hip.array(np.repeat(np.repeat(np.concatenate([a, b], 1), 2, 2), 3, 3))
+    try:
+        hip.force_conv_plan(*plan)
+        O1, O2 = hip.empty((N, Kf, H, W)), hip.empty((N, Kf, H, W))
+        hip.conv2D(A, Wd, None, O1, 1, 1, 1, 1, second=B)
+        assert hip.last_conv_kernel().startswith("conv_split")
+        hip.conv2D(AB, Wd, None, O2, 1, 1, 1, 1)
+        assert np.array_equal(O1.numpy(), O2.numpy())
+        U1, U2 = hip.empty((N, Kf, 2 * H, 3 * W)), hip.empty((N, Kf, 2 * H, 3 * W))
+        hip.conv2D(AB, Wd, None, U1, 1, 1, 1, 1, upsample=(2, 3))
+        hip.conv2D(up, Wd, None, U2, 1, 1, 1, 1)
+        assert np.array_equal(U1.numpy(), U2.numpy())
+        res = rng.standard_normal((N, Kf, H, W), dtype=np.float32)
+        E = hip.empty((N, Kf, H, W))
+        hip.conv2D(AB, Wd, hip.array(bias), E, 1, 1, 1, 1, bn=tuple(hip.array(v) for v in (g, bb, mean, var)) + (1e-5,), residual=hip.array(res), relu=True)
+        col = lambda v: v[None, :, None, None]
+        t = O2.numpy() + col(bias)
+        t = (t - col(mean)) / col(np.sqrt(var + np.float32(1e-5))) * col(g) + col(bb) + res
+        assert np.array_equal(E.numpy(), np.maximum(t, np.float32(0)))
+    finally:
+        hip.force_conv_plan(-1, 1)
+
+
+@pytest.mark.parametrize("plan", [(16, 1), (17, 1), (18, 1), (19, 2)])
+def test_conv2d_split_form_keeps_infinities_nan_and_the_largest_numbers(hip, plan):
+    """Infinities, NaN and numbers that round up to infinity in 16 bits, in the image and in a filter: what the fp32 form gives."""
+    rng = np.random.default_rng(1795)
+    N, C, H, W, Kf = 2, 32, 12, 12, 64
+    x = rng.standard_normal((N, C, H, W), dtype=np.float32)
+    w = (rng.standard_normal((Kf, C, 3, 3)) * 0.05).astype(np.float32)
+    w[3, 4] = 1.0                                       # (short factors: their mid and lo parts are zero)
+    x[0, 3, 2, 2], x[0, 9, 8, 8], x[1, 0, 0, 0], x[1, 5, 6, 6] = np.inf, -np.inf, np.nan, 3.4e38
+    x[1, 7, 11, 11] = 1e-40
+    w[60, 2, 1, 1] = np.inf
+    O = hip.empty((N, Kf, H, W))
+    X, Wd = hip.array(x), hip.array(w)
+    hip.conv2D(X, Wd, None, O, 1, 1, 1, 1)
+    want = O.numpy()
+    assert np.isinf(want).any() and np.isnan(want).any() and np.isfinite(want).any()
+    try:
+        hip.force_conv_plan(*plan)
+        hip.conv2D(X, Wd, None, O, 1, 1, 1, 1)
+        assert hip.last_conv_kernel().startswith("conv_split")
+    finally:
+        hip.force_conv_plan(-1, 1)
+    got = O.numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    assert np.array_equal(np.isneginf(got), np.isneginf(want))
+    ok = np.isfinite(want)
+    assert np.allclose(got[ok], want[ok], rtol=1e-4, atol=1e-5)

@@ -5,9 +5,9 @@
 // product is bound by streaming B from HBM once.  One wavefront owns a 32-row x 128-column
 // output block over a slice of k: per pair of k it loads ONE float4 of B per lane (lane l of a
 // half wavefront covers columns 4l..4l+3: 512 contiguous bytes per k row) and one dword of the
-// transposed activations, and issues four v_mfma_f32_32x32x2_f32, one per column phase
-// (accumulator j holds columns 4l + j).  The activations are transposed first (At[k][32], a few
-// MB, L2-resident) so that their loads are coalesced too.  k is split over wavefronts so the
+// activations, and issues four v_mfma_f32_32x32x2_f32, one per column phase
+// (accumulator j holds columns 4l + j).  Except for one row or few short ones (reads_rows), the
+// activations are transposed first (At[k][32], a few MB, L2-resident) so that their loads are coalesced too.  k is split over wavefronts so the
 // whole device streams B; the per-slice partial blocks go to the private workspace and a second
 // kernel adds them in slice order (fixed summation order, no atomics).
 #include <algorithm>
@@ -45,7 +45,9 @@ __global__ __launch_bounds__(256) void dense_transpose_kernel(const float *__res
 // VEC: n is a multiple of 4 and B is 16-byte aligned, so a lane's four columns are one float4.
 // STREAM (with VEC): the weights are read with the streaming (non-temporal) hint - for matrices larger than
 // the device's caches, which no later kernel finds there anyway (25088 x 4096: 96 -> 88 us).
-template <bool VEC, bool STREAM, int MT>
+// DIRECT (one row tile): At is A[m][k] itself and a lane reads its row where it stands, so there is no transposed copy to make;
+// lanes of rows past m read the last row again (their results are not stored).  The same products and sums, bit for bit.
+template <bool VEC, bool STREAM, int MT, bool DIRECT = false>
 __global__ __launch_bounds__(64) void dense_partial_kernel(const float *__restrict__ At, const float *__restrict__ B,
                                                            float *__restrict__ part, int m, int k, int n, int kslice) {
     const int lane = threadIdx.x, half = lane >> 5, l = lane & 31;
@@ -58,7 +60,8 @@ __global__ __launch_bounds__(64) void dense_partial_kernel(const float *__restri
     // row tile mt0 + t of this group, or the last existing one again (its results are not stored)
     const float *ap[MT];
 #pragma unroll
-    for (int t = 0; t < MT; t++) ap[t] = At + (size_t)(mt0 + t < mtiles ? mt0 + t : mtiles - 1) * k * 32 + l;
+    for (int t = 0; t < MT; t++) ap[t] = DIRECT ? At + (size_t)(l < m ? l : m - 1) * k : At + (size_t)(mt0 + t < mtiles ? mt0 + t : mtiles - 1) * k * 32 + l;
+    constexpr size_t A_STEP = DIRECT ? 1 : 32;  // floats from one tap of a row to the next
     floatx16 acc[MT][4];
 #pragma unroll
     for (int t = 0; t < MT; t++)
@@ -99,7 +102,7 @@ __global__ __launch_bounds__(64) void dense_partial_kernel(const float *__restri
         for (int u = 0; u < U; u++) {
             const int ki = kk + 2 * u + half;
 #pragma unroll
-            for (int t = 0; t < MT; t++) a[u][t] = ap[t][(size_t)ki * 32];
+            for (int t = 0; t < MT; t++) a[u][t] = ap[t][(size_t)ki * A_STEP];
             const float *row = B + (size_t)ki * n;
             if (VEC) {
                 const floatx4 *src = reinterpret_cast<const floatx4 *>(row + col0);
@@ -115,7 +118,7 @@ __global__ __launch_bounds__(64) void dense_partial_kernel(const float *__restri
         const int ki = kk + half;
         float a[MT];
 #pragma unroll
-        for (int t = 0; t < MT; t++) a[t] = ki < kend ? ap[t][(size_t)ki * 32] : 0.0f;
+        for (int t = 0; t < MT; t++) a[t] = ki < kend ? ap[t][(size_t)ki * A_STEP] : 0.0f;
         multiply(a, load_b(ki));
     }
     // part[ks][row][col]: accumulator j, lane column l -> column col0 + j; rows 8*(v/4) + 4*half + v%4
@@ -166,6 +169,12 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(const float *__restri
 
 namespace {
 
+// Whether a product reads the activations where they are instead of from a transposed copy.  The copy is a launch of its own,
+// about 3 us: one row, 2048 x 1000 13.9 -> 10.9 us, 4096 x 4096 22.6 -> 19.6; 32 rows 16.4 -> 13.5, 26.0 -> 24.3.  Rows of
+// 25088 taps, read once per column tile from as many cache lines as there are rows, lose it again: 25088 x 4096 (413 MB, the
+// copy's 84 us are 4.9 TB/s) one row 83.9 -> 81.5 us, two 83.6 -> 86.6, 32 rows 91 -> 138.
+bool reads_rows(int m, int k) { return m == 1 || (m <= 32 && k <= 4096); }
+
 int dense_impl(int dev, const float *A, const float *B, float *C, int m, int k, int n, int incC, const float *bias, int relu,
                const char *what) {
     EH_REQUIRE(m >= 0 && k > 0 && n > 0, "%s: bad shape %dx%d * %dx%d", what, m, k, k, n);
@@ -188,21 +197,25 @@ int dense_impl(int dev, const float *A, const float *B, float *C, int m, int k, 
     int kslice = ((k + nslices - 1) / nslices + 1) & ~1;  // even, so MFMA tap pairs do not straddle slices
     nslices = (k + kslice - 1) / kslice;
     EH_REQUIRE(nslices <= 65535 && mgroups <= 65535, "%s: shape out of range", what);
-    const size_t at_bytes = ((size_t)mt * k * 32 * sizeof(float) + 255) & ~(size_t)255;
+    const bool direct = reads_rows(m, k);
+    const size_t at_bytes = direct ? 0 : ((size_t)mt * k * 32 * sizeof(float) + 255) & ~(size_t)255;
     void *ws = nullptr;
     EH_TRY(get_workspace(dev, at_bytes + (size_t)nslices * m * n * sizeof(float), &ws));
     float *At = (float *)ws, *part = (float *)((char *)ws + at_bytes);
-    hipLaunchKernelGGL(dense_transpose_kernel, dim3((k + 31) / 32, mt), dim3(256), 0, st, A, At, m, k);
-    EH_CHECK_LAUNCH();
+    if (!direct) {
+        hipLaunchKernelGGL(dense_transpose_kernel, dim3((k + 31) / 32, mt), dim3(256), 0, st, A, At, m, k);
+        EH_CHECK_LAUNCH();
+    }
     const bool vec = (n % 4 == 0) && (((uintptr_t)B & 15u) == 0);
     const bool stream = vec && (size_t)k * n * sizeof(float) > ((size_t)256 << 20);  // beyond the 256 MB last-level cache
     typedef void (*partial_fn)(const float *, const float *, float *, int, int, int, int);
-    static const partial_fn kernels[3][3] = {
+    static const partial_fn kernels[4][3] = {
         {dense_partial_kernel<false, false, 1>, dense_partial_kernel<true, false, 1>, dense_partial_kernel<true, true, 1>},
         {dense_partial_kernel<false, false, 2>, dense_partial_kernel<true, false, 2>, dense_partial_kernel<true, true, 2>},
-        {dense_partial_kernel<false, false, 4>, dense_partial_kernel<true, false, 4>, dense_partial_kernel<true, true, 4>}};
-    const partial_fn kern = kernels[MT == 1 ? 0 : MT == 2 ? 1 : 2][!vec ? 0 : (stream ? 2 : 1)];
-    hipLaunchKernelGGL(kern, dim3(nt, nslices, mgroups), dim3(64), 0, st, At, B, part, m, k, n, kslice);
+        {dense_partial_kernel<false, false, 4>, dense_partial_kernel<true, false, 4>, dense_partial_kernel<true, true, 4>},
+        {dense_partial_kernel<false, false, 1, true>, dense_partial_kernel<true, false, 1, true>, dense_partial_kernel<true, true, 1, true>}};
+    const partial_fn kern = kernels[direct ? 3 : MT == 1 ? 0 : MT == 2 ? 1 : 2][!vec ? 0 : (stream ? 2 : 1)];
+    hipLaunchKernelGGL(kern, dim3(nt, nslices, mgroups), dim3(64), 0, st, direct ? A : (const float *)At, B, part, m, k, n, kslice);
     EH_CHECK_LAUNCH();
     size_t mn = (size_t)m * n;
     hipLaunchKernelGGL(dense_reduce_kernel, dim3(eh_blocks(mn, 256, 65536)), dim3(256), 0, st, (const float *)part, C, mn, nslices, incC,

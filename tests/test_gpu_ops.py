@@ -944,6 +944,24 @@ def test_upsample_concat_pad_bit_exact(hip, oracle):
         assert np.array_equal(B.numpy(), ref), (shape, pads)
 
 
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (1, 4099, 131), (2, 4096, 4), (3, 4097, 100), (5, 18, 132), (31, 37, 130), (32, 4096, 64), (32, 15, 3)])
+def test_dense_rows_read_in_place_equal_the_transposed_ones(hip, m, k, n):
+    """A few rows give the bits that they give among 33 (always transposed, K slices alike), and no row touches another."""
+    rng = np.random.default_rng(409)
+    a = rng.standard_normal((33, k), dtype=np.float32)
+    a[m - 1, 0], a[m:] = np.nan, np.inf
+    W = hip.array((rng.standard_normal((k, n)) * np.sqrt(2.0 / k)).astype(np.float32))
+    C, D = hip.full((m, n), 7.0), hip.empty((33, n))
+    hip.mult2D(hip.array(a[:m]), W, C)
+    hip.mult2D(hip.array(a), W, D)
+    got = C.numpy()
+    assert np.isnan(got[m - 1]).all() and np.isfinite(got[:m - 1]).all()
+    assert np.array_equal(got[:m - 1], D.numpy()[:m - 1])
+    hip.mult2D(hip.array(np.nan_to_num(a[:m])), W, C)
+    hip.mult2D(hip.array(np.nan_to_num(a, posinf=1.0)), W, D)
+    assert np.array_equal(C.numpy(), D.numpy()[:m])
+
+
 def test_dense_sigmoid_softmax_within_tolerance(hip, oracle):
     rng = np.random.default_rng(405)
     for m, k, n in [(32, 512, 1000), (5, 37, 300), (64, 2048, 10), (33, 100, 65), (70, 1001, 131), (32, 3136, 4096), (1, 2, 1),

@@ -1,16 +1,21 @@
 // Convolution in fp32 accuracy on the bf16 matrix instructions (included by conv.hip only).
 //
-// Every fp32 number is the sum of three bf16 numbers: hi = bf16(x), mid = bf16(x - hi), lo = x - hi - mid.  A bf16 holds 8
-// significant bits with the exponent range of an fp32, both differences are exact, and 3 x 8 bits hold the 24 of the fp32,
-// so nothing of x is lost.  Of the nine products of two such sums the six largest are multiplied -
+// Every fp32 number x, enlarged 2^24 times, is the sum of three bf16 numbers (Henry, Tang and Heinecke, "Leveraging the bfloat16
+// artificial intelligence datatype for higher-precision computations", 2019): hi = bf16(y), mid = bf16(y - hi),
+// lo = y - hi - mid with y = 2^24 x.  A bf16 holds 8 significant bits with the exponent range of an fp32, both differences are
+// exact, and 3 x 8 bits hold the 24 of the fp32.  The factor keeps the last bit of the smallest number in range: y is a
+// multiple of 2^-125, so every part is zero or a normal bf16 and nothing of x is lost, subnormal numbers included (without it
+// numbers below 2^-110 lost bits of lo, below 2^-118 of mid).  The finished sums, 2^48 times too large, are scaled back.
+// Of the nine products of two such sums the six largest are multiplied -
 //   hi hi + (hi mid + mid hi) + (hi lo + mid mid + lo hi)
-// - and the three left out are below 2^-25 of the product, less than the rounding of one fp32 product.  The products are
-// exact in the instruction and the sums stay in fp32 accumulators.  v_mfma_f32_32x32x16_bf16 does 16 times the work of
-// v_mfma_f32_32x32x2_f32 in the same cycles per flop of K, so six of them per 16 taps cost 6/16 of the fp32 instruction's.
+// - and the three left out are together below 2^-24 of the product (each of mid lo and lo mid can reach 2^-25), the rounding of
+// one fp32 product.  The products are exact in the instruction and the sums stay in fp32 accumulators.
+// v_mfma_f32_32x32x16_bf16 does 16 times the work of v_mfma_f32_32x32x2_f32 in the same cycles per flop of K, so six of them
+// per 16 taps cost 6/16 of the fp32 instruction's.
 //
-// Not for infinities: inf - inf is NaN, and inf times the zero mid of a short factor is too.  A wavefront whose finished
-// accumulators are not all finite takes its tile again with the fp32 instruction, from the original filters
-// (split_tile_again), so infinities and NaN come out as the fp32 kernels bring them.
+// Not for infinities: inf - inf is NaN, and inf times the zero mid of a short factor is too; numbers from 2^104 and sums from
+// 2^80 on are infinite here as well.  A wavefront whose finished accumulators are not all finite takes its tile again with the
+// fp32 instruction, from the original filters (split_tile_again), so infinities and NaN come out as the fp32 kernels bring them.
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -30,6 +35,9 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned &hi, unsig
     lo = split_round(ra - __builtin_bit_cast(float, mid << 16), rb - __builtin_bit_cast(float, mid & 0xffff0000u));
 }
 
+constexpr float SPLIT_UP = 16777216.0f;                    // 2^24, of pixels and filters
+constexpr float SPLIT_DOWN = 1.0f / SPLIT_UP / SPLIT_UP;   // of their products
+
 // K[Kf][C][RS] -> Ws[k16][Mp / 32][part][lane][8]: the operand of lane l of the matrix instruction is filter l % 32 of the
 // block, channels 8 (l / 32) .. + 7 of the 16.  k16 = 2 (cb RS + tap) + g covers channels 32 cb + 16 g .. + 15 under one tap;
 // channels past C and filters past Kf are zeros.  Bound by the write (6 bytes a weight); once per registered filter tensor.
@@ -44,8 +52,8 @@ __global__ __launch_bounds__(256) void split_filter_kernel(const float *__restri
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int c = c0 + 2 * j;
-        const float a = m < Kf && c < C ? K[((size_t)m * C + c) * RS + tap] : 0.0f;
-        const float b = m < Kf && c + 1 < C ? K[((size_t)m * C + c + 1) * RS + tap] : 0.0f;
+        const float a = m < Kf && c < C ? SPLIT_UP * K[((size_t)m * C + c) * RS + tap] : 0.0f;
+        const float b = m < Kf && c + 1 < C ? SPLIT_UP * K[((size_t)m * C + c + 1) * RS + tap] : 0.0f;
         unsigned h, md, l;
         split_pair(a, b, h, md, l);
         hi[j] = h;
@@ -77,7 +85,9 @@ __device__ __forceinline__ int split_pixel(const ConvParams &p, unsigned magic_h
 }
 
 // The K-steps [step_lo, step_hi) of a wavefront's blocks once more with the fp32 instruction, two channels at a time in the
-// order of the split filters; reads the image and the original filters where they are.  Only infinities and NaN come here.
+// order of the split filters; reads the image and the original filters where they are.  Only infinities, NaN and numbers near
+// the end of the fp32 range come here.  (The fp32 kernels take the channels slowest: a sum that overflows in one of the two
+// orders and not in the other can differ.)
 template <int TM, int TN>
 __device__ __forceinline__ void split_tile_again(const ConvParams &p, floatx16 (&acc)[TM][TN], __amdgpu_buffer_rsrc_t in1, __amdgpu_buffer_rsrc_t in2, int m_first,
                                                  int n_first, int step_lo, int step_hi, int lane) {
@@ -206,7 +216,7 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             unsigned h, m, l;
-            split_pair(raw[chunk][2 * j], raw[chunk][2 * j + 1], h, m, l);
+            split_pair(SPLIT_UP * raw[chunk][2 * j], SPLIT_UP * raw[chunk][2 * j + 1], h, m, l);
             hi[j] = h;
             mid[j] = m;
             lo[j] = l;
@@ -291,7 +301,7 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
 #pragma unroll
             for (int i = 0; i < 6 * TM * TN; i++) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, TM * TN == 4 ? 3 : (TM * TN == 2 ? 5 : 9), 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, TM * TN == 4 ? 3 : (TM * TN == 2 ? 6 : 10), 0);
             }
             __builtin_amdgcn_sched_group_barrier(0x200, 3, 0);
             __builtin_amdgcn_sched_group_barrier(0x020, 8, 0);
@@ -305,7 +315,7 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
 #pragma unroll
         for (int tn = 0; tn < TN; tn++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[tm][tn][v] = __fadd_rn(acc[tm][tn][v], small[tm][tn][v]);
+            for (int v = 0; v < 16; v++) acc[tm][tn][v] = SPLIT_DOWN * __fadd_rn(acc[tm][tn][v], small[tm][tn][v]);
 
     float finite = 0.0f;
 #pragma unroll

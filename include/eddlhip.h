@@ -254,9 +254,12 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * geometry of its own in the plans table (kind 2 / 3 instead of 0 / 1): the same layer run after a stand-alone
  * UpSampling2D keeps its own plan, and the two agree to the convolution's tolerance, not bit for bit.
  * The split form (force_plan(16 .. 19, .), or the search; any filter, channel counts that are multiples of 16): every fp32
- * number as an exact sum of three bf16 numbers, the six largest of their nine products on the bf16 matrix instructions,
- * fp32 sums.  Its error against exact sums is below the fp32 instruction's (fewer roundings per sum); infinities, NaN and
- * overflow come out as the fp32 kernels bring them (a tile that is not finite is computed again by them).  Workspace: the
+ * number as an exact sum of three bf16 numbers (scaled by 2^24, so that subnormal numbers keep their bits too), the six
+ * largest of their nine products on the bf16 matrix instructions, fp32 sums.  Its error against exact sums is below the fp32
+ * instruction's (fewer roundings per sum) over the whole range of the inputs; infinities and NaN come out as the fp32 kernels
+ * bring them (a tile whose scaled sums are not finite - numbers from 2^104 or sums from 2^80 on, too - is computed with
+ * the fp32 instruction, 32 channels of a tap at a time: a sum that overflows in only one order of its terms can differ
+ * from those kernels').  Workspace: the
  * split filters, 6 bytes a weight, unless registered; never taken by eddlhip_conv2d_fwd_noalloc.
  *
  * eddlhip_conv2d_last_kernel() names the kernel the calling thread's last eddlhip_conv2d_fwd

@@ -1302,3 +1302,31 @@ def test_conv2d_split_form_keeps_infinities_nan_and_the_largest_numbers(hip, pla
     assert np.array_equal(np.isneginf(got), np.isneginf(want))
     ok = np.isfinite(want)
     assert np.allclose(got[ok], want[ok], rtol=1e-4, atol=1e-5)
+
+
+def _small_or_large(rng, shape, e):
+    """Normal random numbers times 2^e, as fp32 holds them (below 2^-126 with the bits that are left there)."""
+    return np.ldexp(rng.standard_normal(shape, dtype=np.float32).astype(np.float64), e).astype(np.float32)
+
+
+@pytest.mark.parametrize("plan", [(16, 1), (17, 1), (18, 2), (19, 1)])
+@pytest.mark.parametrize("e_pixels,e_filters", [(-112, 90), (90, -112), (-118, 90), (90, -118), (-126, 100), (100, -126), (-140, 100), (100, -140), (-60, -60),
+                                                (110, -60), (-60, 110), (40, 45), (60, 60)])
+def test_conv2d_split_form_keeps_24_bits_of_small_and_large_numbers(hip, plan, e_pixels, e_filters):
+    """Pixels or filters anywhere in the fp32 range, subnormal numbers too, with sums in the normal range: the relative error is
+    that of numbers around one.  Bound: the products left out are 2^-24 of a product each, an fp32 sum of 64 / 16 products of the
+    high parts rounds four times and the sum of all parts twice more, 2^-24 each: 7 x 2^-24 < 2^-21 of sums of like terms.  Beyond
+    the scaled range (110, 60 + 60) the fp32 instruction rounds 32 times, at random: about sqrt(32) x 2^-25."""
+    rng = np.random.default_rng(1797)
+    N, C, H, W, Kf = 1, 64, 9, 11, 70
+    x, w = _small_or_large(rng, (N, C, H, W), e_pixels), _small_or_large(rng, (Kf, C, 1, 1), e_filters)
+    O = hip.full((N, Kf, H, W), np.nan)
+    try:
+        hip.force_conv_plan(*plan)
+        hip.conv2D(hip.array(x), hip.array(w), None, O, 1, 1, 0, 0)
+        assert hip.last_conv_kernel().startswith("conv_split")
+    finally:
+        hip.force_conv_plan(-1, 1)
+    ref = np.einsum("kc,nchw->nkhw", w[:, :, 0, 0].astype(np.float64), x.astype(np.float64))
+    err = np.linalg.norm(O.numpy() - ref) / np.linalg.norm(ref)
+    assert err <= 2.0 ** -21, err

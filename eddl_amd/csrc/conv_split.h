@@ -14,8 +14,9 @@
 // per 16 taps cost 6/16 of the fp32 instruction's.
 //
 // Not for infinities: inf - inf is NaN, and inf times the zero mid of a short factor is too; numbers from 2^104 and sums from
-// 2^80 on are infinite here as well.  A wavefront whose finished accumulators are not all finite takes its tile again with the
-// fp32 instruction, from the original filters (split_tile_again), so infinities and NaN come out as the fp32 kernels bring them.
+// 2^80 on are infinite here as well.  A wavefront whose finished accumulators are not all finite computes its tile with the
+// fp32 instruction too, from the original filters (split_tile_again), and every sum that is not finite takes that value: the
+// others keep theirs, whatever stands beside them in the tile.
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -325,7 +326,15 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
 #pragma unroll
             for (int v = 0; v < 16; v++) finite = __builtin_fmaf(acc[tm][tn][v], 0.0f, finite);
     const int m_first = m0 + wm * TM * 32, n_first = n0 + wn * TN * 32;
-    if (__any(finite != 0.0f)) split_tile_again<TM, TN>(p, acc, rsrc_in, rsrc_in2, m_first, n_first, step_lo, step_hi, lane);
+    if (__any(finite != 0.0f)) {
+        split_tile_again<TM, TN>(p, small, rsrc_in, rsrc_in2, m_first, n_first, step_lo, step_hi, lane);
+#pragma unroll
+        for (int tm = 0; tm < TM; tm++)
+#pragma unroll
+            for (int tn = 0; tn < TN; tn++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[tm][tn][v] = acc[tm][tn][v] * 0.0f == 0.0f ? acc[tm][tn][v] : small[tm][tn][v];
+    }
 
     if (split) {
         store_partial<TM, TN>(p, acc, local_tile, slice, wave, lane);

@@ -257,9 +257,9 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * number as an exact sum of three bf16 numbers (scaled by 2^24, so that subnormal numbers keep their bits too), the six
  * largest of their nine products on the bf16 matrix instructions, fp32 sums.  Its error against exact sums is below the fp32
  * instruction's (fewer roundings per sum) over the whole range of the inputs; infinities and NaN come out as the fp32 kernels
- * bring them (a tile whose scaled sums are not finite - numbers from 2^104 or sums from 2^80 on, too - is computed with
- * the fp32 instruction, 32 channels of a tap at a time: a sum that overflows in only one order of its terms can differ
- * from those kernels').  Workspace: the
+ * bring them (scaled sums that are not finite - numbers from 2^104 or sums from 2^80 on, too - are computed with the fp32
+ * instruction, 32 channels of a tap at a time: a sum that overflows in only one order of its terms can differ from those
+ * kernels').  No output's bits depend on the inputs of another.  Workspace: the
  * split filters, 6 bytes a weight, unless registered; never taken by eddlhip_conv2d_fwd_noalloc.
  *
  * eddlhip_conv2d_last_kernel() names the kernel the calling thread's last eddlhip_conv2d_fwd

@@ -1330,3 +1330,27 @@ def test_conv2d_split_form_keeps_24_bits_of_small_and_large_numbers(hip, plan, e
     ref = np.einsum("kc,nchw->nkhw", w[:, :, 0, 0].astype(np.float64), x.astype(np.float64))
     err = np.linalg.norm(O.numpy() - ref) / np.linalg.norm(ref)
     assert err <= 2.0 ** -21, err
+
+
+@pytest.mark.parametrize("plan", [(16, 1), (17, 1), (18, 1), (19, 2)])
+def test_conv2d_split_form_infinity_leaves_the_other_outputs_alone(hip, plan):
+    """An infinity changes the outputs whose window holds it and not a bit of any other, of its own image or another's."""
+    rng = np.random.default_rng(1798)
+    N, C, H, W, Kf = 3, 48, 7, 9, 40
+    x = rng.standard_normal((N, C, H, W), dtype=np.float32)
+    w = (rng.standard_normal((Kf, C, 3, 3)) * 0.05).astype(np.float32)
+    Wd, clean, marked = hip.array(w), hip.empty((N, Kf, H, W)), hip.empty((N, Kf, H, W))
+    y = x.copy()
+    y[1, 5, 3, 4] = np.inf
+    window = np.zeros((N, Kf, H, W), bool)
+    window[1, :, 2:5, 3:6] = True
+    try:
+        hip.force_conv_plan(*plan)
+        hip.conv2D(hip.array(x), Wd, None, clean, 1, 1, 1, 1)
+        hip.conv2D(hip.array(y), Wd, None, marked, 1, 1, 1, 1)
+        assert hip.last_conv_kernel().startswith("conv_split")
+    finally:
+        hip.force_conv_plan(-1, 1)
+    got = marked.numpy()
+    assert np.array_equal(np.isinf(got), window) and not np.isnan(got).any()
+    assert np.array_equal(got[~window], clean.numpy()[~window])

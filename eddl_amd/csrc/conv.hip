@@ -2799,7 +2799,7 @@ int conv2d_winograd_fused(int variant, int slices, int dev, const float *I, cons
 int conv2d_up2x2(int variant, int dev, const float *I, const float *K, const float *bias, float *O, int N, int C, int H, int W, int Kf, int P, int Q, const float *bn_g,
                  const float *bn_b, const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu);
 
-int conv2d_split(const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs);
+int conv2d_split(bool no_alloc, const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room);
 
 // Whether a convolution is the one conv_up2x2_kernel computes: a 2x2 stride-1 filter on ONE tensor upsampled twice in both
 // directions, no padding above or to the left (below and to the right the image is followed by zeros, as many as the
@@ -3169,12 +3169,15 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     if ((wino_ok && (g_force_tile == 4 || (g_wino && g_force_tile < 0 && !g_tuning))) || (fold_ok && g_force_tile == 5))
         return conv2d_winograd(g_force_tile == 5, R, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top, pad_left, P, Q, bn_g, bn_b,
                                bn_mean, bn_var, bn_eps, residual, relu);
-    // the split form: any filter shape, as long as a chunk of the input is addressed like the direct kernels do; never from the
-    // fixed scratch array (its filters take half as much again as the repacked ones)
-    const bool split_ok = !gemm && !no_alloc && g_algo == 0 && split_applies(C, Kf, R, S);
+    // the split form: any filter shape, as long as a chunk of the input is addressed like the direct kernels do; from the fixed
+    // scratch array where its filters (half as much again as the repacked ones) and partial tiles fit, else the planner's plan
+    const bool split_ok = !gemm && g_algo == 0 && split_applies(C, Kf, R, S);
+    bool no_room = false;
     if (split_ok && is_split_tile(g_force_tile)) {
         const int tile = g_force_tile - SPLIT_TILE0;
-        return conv2d_split(ksplit[tile], forced_plan(ksplit, tile, g_force_slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p, chunk_imgs);
+        const int rc = conv2d_split(no_alloc, ksplit[tile], forced_plan(ksplit, tile, g_force_slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p,
+                                    chunk_imgs, &no_room);
+        if (!no_room) return rc;
     }
     const bool query = gemm != nullptr && gemm->need_out != nullptr;  // report the workspace need, launch nothing
     bool plan_open = false;                                         // a search could still pick any plan for this geometry
@@ -3213,7 +3216,9 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
                                          bn_b, bn_mean, bn_var, bn_eps, residual, relu);
         if (found != nullptr && is_split_tile(found->tile) && split_ok) {
             const int tile = found->tile - SPLIT_TILE0;
-            return conv2d_split(ksplit[tile], forced_plan(ksplit, tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p, chunk_imgs);
+            const int rc = conv2d_split(no_alloc, ksplit[tile], forced_plan(ksplit, tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev,
+                                        p, chunk_imgs, &no_room);
+            if (!no_room) return rc;
         }
         if (found != nullptr && found->tile >= 0 && found->tile < 4)
             plan = forced_plan(family, found->tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu);
@@ -3697,8 +3702,9 @@ int conv2d_winograd_fused(int variant, int slices, int dev, const float *I, cons
 }
 
 // The split form (conv_split.h) of the call that `call` describes, under a plan of split steps.
-// Workspace: [split filters unless kept][partial tiles].
-int conv2d_split(const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs) {
+// Workspace: [split filters unless kept][partial tiles].  no_alloc: from the fixed scratch array; nothing is launched and *no_room
+// is set if that is too small.
+int conv2d_split(bool no_alloc, const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room) {
     hipStream_t st = state(dev).stream;
     const int RS = call.R * call.S, N = call.N;
     EH_REQUIRE(plan.tiles <= 0x3fffffffLL, "conv2d: too many tiles");
@@ -3710,7 +3716,7 @@ int conv2d_split(const Variant &v, const Plan &plan, int dev, const ConvParams &
         std::lock_guard<std::mutex> lock(g_cache_mutex);
         for (CachedFilters &e : g_cache[dev]) {
             if (e.K == call.K && e.Kf == call.Kf && e.C == call.C && e.R == call.R && e.S == call.S) {
-                if (e.Wsplit == nullptr && !state(dev).capturing) {
+                if (e.Wsplit == nullptr && !state(dev).capturing && !no_alloc) {
                     if (hipMalloc(&e.Wsplit, w_bytes) != hipSuccess) {
                         e.Wsplit = nullptr;
                         (void)hipGetLastError();
@@ -3728,7 +3734,15 @@ int conv2d_split(const Variant &v, const Plan &plan, int dev, const ConvParams &
     }
     const size_t ws_filters = Ws ? 0 : ((w_bytes + 255) & ~(size_t)255);
     void *ws = nullptr;
-    if (ws_filters + partial_bytes > 0) EH_TRY(get_workspace(dev, ws_filters + partial_bytes, &ws));
+    if (no_alloc) {
+        if (ws_filters + partial_bytes > (size_t)EDDLHIP_CONV_NOALLOC_SCRATCH_BYTES) {
+            *no_room = true;
+            return 0;
+        }
+        ws = g_scratch_ptr[dev];
+    } else if (ws_filters + partial_bytes > 0) {
+        EH_TRY(get_workspace(dev, ws_filters + partial_bytes, &ws));
+    }
     if (Ws == nullptr) {
         EH_TRY(launch_split_filters(dev, call.K, ws, call.Kf, call.C, RS, call.Mp));
         Ws = ws;

@@ -188,10 +188,11 @@ int eddlhip_conv2d_fwd_maxpool(int dev, const float *I, const float *I_second, i
 
 /* eddlhip_conv2d_fwd for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid it).  No counterpart in the reference.  Same arguments, same kernels,
- * same launch plan and therefore the same result, bit for bit, as eddlhip_conv2d_fwd; the difference is where
- * the call's scratch memory comes from (the repacked filters unless they are registered with
- * eddlhip_conv2d_cache_filters, the tap table of filter shapes other than 1x1 / 2x2 / 3x3, the partial tiles of
- * a K-split launch): a fixed array of EDDLHIP_CONV_NOALLOC_SCRATCH_BYTES in the library's device image, one copy
+ * same launch plan and therefore the same result, bit for bit, as eddlhip_conv2d_fwd, except under a plan of
+ * eddlhip_conv2d_autotune that names a Winograd or upsampled-input form or split filters that do not fit (below): then the
+ * planner's own choice.  The difference is where the call's scratch memory comes from (the repacked or split filters unless
+ * they are registered with eddlhip_conv2d_cache_filters, the tap table of filter shapes other than 1x1 / 2x2 / 3x3, the
+ * partial tiles of a K-split launch): a fixed array of EDDLHIP_CONV_NOALLOC_SCRATCH_BYTES in the library's device image, one copy
  * per device, instead of the grow-only workspace.  The call makes no hipMalloc / hipFree and no allocating
  * library call.  It returns EDDLHIP_EINVAL, and launches nothing, when
  *   - the device has not been initialised (call eddlhip_init(dev) once beforehand; that call allocates),
@@ -260,7 +261,8 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * bring them (scaled sums that are not finite - numbers from 2^104 or sums from 2^80 on, too - are computed with the fp32
  * instruction, 32 channels of a tap at a time: a sum that overflows in only one order of its terms can differ from those
  * kernels').  No output's bits depend on the inputs of another.  Workspace: the
- * split filters, 6 bytes a weight, unless registered; never taken by eddlhip_conv2d_fwd_noalloc.
+ * split filters, 6 bytes a weight, unless registered, and the partial tiles of a K-split plan; where that is more than
+ * eddlhip_conv2d_fwd_noalloc has (11 million unregistered weights), that entry point runs the planner's own choice.
  *
  * eddlhip_conv2d_last_kernel() names the kernel the calling thread's last eddlhip_conv2d_fwd
  * launched, followed by " +ksplit(T tiles x S)" when T tiles were divided into S slices; for the Winograd form

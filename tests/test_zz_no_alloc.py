@@ -142,3 +142,65 @@ def test_noalloc_refused_while_profiling(hip):
     finally:
         hip.conv_profile(False)
     assert rc == -1 and "profile" in hip.lib.eddlhip_last_error().decode()
+
+
+# (N, C, H, W, Kf, R, stride, pad), plan tile and K slices: the split form kept for a geometry
+SPLIT_PLANS = {"1x1": ((4, 96, 15, 17, 200, 1, 1, 0), 17, 4), "3x3 stride 2": ((3, 64, 28, 28, 128, 3, 2, 1), 19, 1), "3x3": ((2, 128, 13, 11, 72, 3, 1, 1), 18, 6)}
+
+
+@pytest.mark.parametrize("registered", [False, True])
+@pytest.mark.parametrize("name", sorted(SPLIT_PLANS))
+def test_noalloc_runs_the_split_plan_that_was_found(hip, tmp_path, name, registered):
+    """A plan of the split form is used like any found plan: same kernel and bits as conv2d_fwd, nothing allocated."""
+    (N, C, H, W, Kf, R, stride, pad), tile, slices = SPLIT_PLANS[name]
+    P, Q = _out_dim(H, R, stride, pad, pad), _out_dim(W, R, stride, pad, pad)
+    path = tmp_path / "plans.txt"
+    path.write_text("%d %d %d %d %d %d %d %d %d 1 | %d %d\n" % (N, C, Kf, R, R, stride, stride, P, Q, tile, slices))
+    rng = np.random.default_rng(74)
+    dx, dw = hip.array(rng.standard_normal((N, C, H, W), dtype=np.float32)), hip.array((rng.standard_normal((Kf, C, R, R)) * 0.05).astype(np.float32))
+    O1, O2 = hip.full((N, Kf, P, Q), float("nan")), hip.full((N, Kf, P, Q), float("nan"))
+    args = lambda O: (hip.dev, dx.ptr, dw.ptr, None, O.ptr, N, C, H, W, Kf, R, R, stride, stride, pad, pad, P, Q, None, None, None, None, 0.0, None, 0)
+    hip.conv_autotune(-1)
+    try:
+        hip.conv_tuned_load(str(path))
+        hip.conv_autotune(True)
+        if registered:
+            hip.cache_conv_filters(dw)
+        hip.synchronize()
+        hip.workspace_trim()
+        hip._check(hip.lib.eddlhip_conv2d_fwd_noalloc(*args(O1)))
+        kernel = hip.last_conv_kernel()
+        assert kernel.startswith("conv_split") and ("+ksplit" in kernel) == (slices > 1), kernel
+        assert hip.workspace_bytes() == 0
+        hip._check(hip.lib.eddlhip_conv2d_fwd(*args(O2)))
+        assert hip.last_conv_kernel() == kernel
+        assert np.array_equal(O1.numpy(), O2.numpy())
+        hip.fill_(O1, float("nan"))
+        hip._check(hip.lib.eddlhip_conv2d_fwd_noalloc(*args(O1)))   # (registered: with the split copy that conv2d_fwd has made)
+        assert np.array_equal(O1.numpy(), O2.numpy())
+    finally:
+        hip.conv_autotune(-1)
+        hip.uncache_conv_filters(dw)
+
+
+def test_noalloc_takes_the_planners_plan_where_the_split_filters_do_not_fit(hip, tmp_path):
+    """6 bytes a weight are beyond the array, the repacked 4 are not: the call is accepted as without a found plan."""
+    N, C, H, W, Kf = 1, 3840, 8, 8, 3072
+    assert 4 * C * Kf < SCRATCH_BYTES < 6 * C * Kf
+    path = tmp_path / "plans.txt"
+    path.write_text("%d %d %d 1 1 1 1 %d %d 1 | 17 1\n" % (N, C, Kf, H, W))
+    rng = np.random.default_rng(75)
+    dx, dw = hip.array(rng.standard_normal((N, C, H, W), dtype=np.float32)), hip.full((Kf, C, 1, 1), 0.25)
+    O1, O2 = hip.empty((N, Kf, H, W)), hip.empty((N, Kf, H, W))
+    args = lambda O: (hip.dev, dx.ptr, dw.ptr, None, O.ptr, N, C, H, W, Kf, 1, 1, 1, 1, 0, 0, H, W, None, None, None, None, 0.0, None, 0)
+    hip.conv_autotune(-1)
+    try:
+        hip._check(hip.lib.eddlhip_conv2d_fwd_noalloc(*args(O1)))
+        kernel = hip.last_conv_kernel()
+        hip.conv_tuned_load(str(path))
+        hip.conv_autotune(True)
+        hip._check(hip.lib.eddlhip_conv2d_fwd_noalloc(*args(O2)))
+        assert hip.last_conv_kernel() == kernel
+        assert np.array_equal(O1.numpy(), O2.numpy())
+    finally:
+        hip.conv_autotune(-1)

@@ -2256,7 +2256,7 @@ int prof_end(hipStream_t st) {
 thread_local char g_last_kernel[128] = "";
 int g_split = 1;  // divide the tiles left over after a whole number per CU along K (set_algo 5 turns it off)
 bool g_wino = false;  // set_algo(7): the Winograd form wherever it applies (8: only where a searched plan asks for it)
-bool g_wino_never = false;  // set_algo(9): no Winograd form at all, not in the plan search and not from a kept plan
+bool g_wino_never = false;  // set_algo(9): no Winograd and no split form at all, not in the plan search and not from a kept plan
 thread_local int g_force_tile = -1, g_force_slices = -1;  // eddlhip_conv2d_force_plan (per calling thread: the plan search steers its own launches with them)
 unsigned long long *g_trace = nullptr;       // eddlhip_conv2d_trace
 long long g_trace_wgs = 0;
@@ -3171,7 +3171,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
                                bn_mean, bn_var, bn_eps, residual, relu);
     // the split form: any filter shape, as long as a chunk of the input is addressed like the direct kernels do; from the fixed
     // scratch array where its filters (half as much again as the repacked ones) and partial tiles fit, else the planner's plan
-    const bool split_ok = !gemm && g_algo == 0 && split_applies(C, Kf, R, S);
+    const bool split_ok = !gemm && g_algo == 0 && !g_wino_never && split_applies(C, Kf, R, S);
     bool no_room = false;
     if (split_ok && is_split_tile(g_force_tile)) {
         const int tile = g_force_tile - SPLIT_TILE0;

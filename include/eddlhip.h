@@ -215,8 +215,9 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * written by the load unit straight into LDS (what 0 and 1 select); 5 / 6 = switch off / on the
  * division along K of the tiles left over after a whole number of tiles per CU (on by default;
  * independent of 0-4); 7 / 8 = switch on / off the Winograd form for every convolution it applies to
- * (off by default; independent of 5 / 6; only under 0); 9 = no Winograd form at all: the plan search does not try
- * it and a kept plan that names it runs the planner's own choice instead (8 returns to the default).
+ * (off by default; independent of 5 / 6; only under 0); 9 = no Winograd form and no split form at all: the plan search
+ * does not try them, which leaves the fp32 matrix instruction's sums, and a kept plan that names one runs the planner's own
+ * choice instead (8 returns to the default).
  *
  * The Winograd form, F(2x2, 3x3): a 3x3 stride-1 convolution (any paddings, one or two input tensors, stored or
  * upsampled image) computed as an input transform, 16 products of [Kf x C] by [C x blocks of 2x2 outputs] matrices -

@@ -1354,3 +1354,43 @@ def test_conv2d_split_form_infinity_leaves_the_other_outputs_alone(hip, plan):
     got = marked.numpy()
     assert np.array_equal(np.isinf(got), window) and not np.isnan(got).any()
     assert np.array_equal(got[~window], clean.numpy()[~window])
+
+
+def _one_plan(hip, tmp_path, N, C, Kf, R, stride, P, Q, tile, slices):
+    """The plan search's table with one geometry in it."""
+    path = tmp_path / "plans.txt"
+    path.write_text("%d %d %d %d %d %d %d %d %d 1 | %d %d\n" % (N, C, Kf, R, R, stride, stride, P, Q, tile, slices))
+    hip.conv_autotune(-1)
+    hip.conv_tuned_load(str(path))
+    hip.conv_autotune(True)
+
+
+def test_conv2d_winograd_never_refuses_the_split_form_too(hip, tmp_path):
+    """set_conv_algo("winograd_never") leaves fp32 sums of the direct form: no split form, forced, searched or kept."""
+    rng = np.random.default_rng(1799)
+    N, C, H, W, Kf = 2, 64, 14, 14, 64
+    X, Wd = hip.array(rng.standard_normal((N, C, H, W), dtype=np.float32)), hip.array((rng.standard_normal((Kf, C, 1, 1)) * 0.1).astype(np.float32))
+    O = hip.empty((N, Kf, H, W))
+    hip.conv2D(X, Wd, None, O, 1, 1, 0, 0)
+    planned, kernel = O.numpy(), hip.last_conv_kernel()
+    try:
+        hip.set_conv_algo("winograd_never")
+        hip.force_conv_plan(17, 1)
+        hip.conv2D(X, Wd, None, O, 1, 1, 0, 0)
+        assert hip.last_conv_kernel() == kernel
+        hip.force_conv_plan(-1, 1)
+        _one_plan(hip, tmp_path, N, C, Kf, 1, 1, H, W, 17, 1)
+        hip.conv2D(X, Wd, None, O, 1, 1, 0, 0)
+        assert hip.last_conv_kernel() == kernel and np.array_equal(O.numpy(), planned)
+        hip.conv_autotune(-1)
+        hip.conv_autotune(True)
+        hip.conv2D(X, Wd, None, O, 1, 1, 0, 0)
+        assert hip.conv_tuned_plans() == 1 and not hip.last_conv_kernel().startswith("conv_split")
+        hip.set_conv_algo("winograd_off")
+        _one_plan(hip, tmp_path, N, C, Kf, 1, 1, H, W, 17, 1)
+        hip.conv2D(X, Wd, None, O, 1, 1, 0, 0)
+        assert hip.last_conv_kernel().startswith("conv_split")
+    finally:
+        hip.force_conv_plan(-1, 1)
+        hip.set_conv_algo("winograd_off")
+        hip.conv_autotune(-1)

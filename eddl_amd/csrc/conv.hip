@@ -2526,6 +2526,41 @@ int repack(int dev, CachedFilters &e) {
     return 0;
 }
 
+// Which of the forms' own copies a registered filter tensor has (none if it is not registered).
+struct FilterCopies {
+    bool wino, fused, up, split;
+};
+CachedFilters *registered_filters(int dev, const float *K, int Kf, int C, int R, int S) {
+    for (CachedFilters &e : g_cache[dev])
+        if (e.K == K && e.Kf == Kf && e.C == C && e.R == R && e.S == S) return &e;
+    return nullptr;
+}
+FilterCopies copies_held(int dev, const float *K, int Kf, int C, int R, int S) {
+    std::lock_guard<std::mutex> lock(g_cache_mutex);
+    const CachedFilters *e = registered_filters(dev, K, Kf, C, R, S);
+    if (e == nullptr) return {false, false, false, false};
+    return {e->Wwino != nullptr, e->Wfused != nullptr, e->Wup != nullptr, e->Wsplit != nullptr};
+}
+// Frees the copies that a tensor has beyond `keep` (what a plan search made for forms that it did not keep).
+int drop_copies(int dev, const float *K, int Kf, int C, int R, int S, const FilterCopies &keep) {
+    std::lock_guard<std::mutex> lock(g_cache_mutex);
+    CachedFilters *e = registered_filters(dev, K, Kf, C, R, S);
+    if (e == nullptr) return 0;
+    bool synced = false;
+    auto drop = [&](auto &copy, bool kept) -> int {
+        if (kept || copy == nullptr) return 0;
+        if (!synced) EH_TRY_HIP(hipStreamSynchronize(state(dev).stream));
+        synced = true;
+        EH_TRY_HIP(hipFree(copy));
+        copy = nullptr;
+        return 0;
+    };
+    EH_TRY(drop(e->Wwino, keep.wino));
+    EH_TRY(drop(e->Wfused, keep.fused));
+    EH_TRY(drop(e->Wup, keep.up));
+    return drop(e->Wsplit, keep.split);
+}
+
 }  // namespace
 
 namespace eddlhip {
@@ -3196,8 +3231,16 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
             TunedPlan best;
             memcpy(best.key, key, sizeof(key));
             const size_t ws_before = state(dev).workspace_bytes;
+            FilterCopies keep = copies_held(dev, K, Kf, C, R, S);  // (those that other geometries' plans, and graphs, may use)
             const int src = search_plan(call, family, plan, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, split_ok, &best);
             if (src < 0) return -src;  // a runtime error inside the search
+            if (src == 0) {
+                keep.wino = keep.wino || best.tile == 4 || best.tile == 5;
+                keep.fused = keep.fused || (best.tile >= FUSED_TILE0 && best.tile < FUSED_TILE0 + NUM_FUSED);
+                keep.up = keep.up || best.tile == UP2X2_TILE || best.tile == UP2X2_TILE + 1;
+                keep.split = keep.split || is_split_tile(best.tile);
+            }
+            if (!gemm) EH_TRY(drop_copies(dev, K, Kf, C, R, S, keep));
             // the candidates may have taken far more workspace than the plan that stays: let it grow back to what is needed
             // (not inside another convolution's call, whose buffers live there)
             if (!gemm && state(dev).workspace_bytes > ws_before) EH_TRY(release_workspace(dev));

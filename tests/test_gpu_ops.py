@@ -1394,3 +1394,37 @@ def test_conv2d_winograd_never_refuses_the_split_form_too(hip, tmp_path):
         hip.force_conv_plan(-1, 1)
         hip.set_conv_algo("winograd_off")
         hip.conv_autotune(-1)
+
+
+@pytest.mark.parametrize("kernel", [1, 3])
+def test_conv2d_search_keeps_only_the_filter_copy_of_its_plan(hip, tmp_path, kernel):
+    """A search tries every form on a registered filter tensor; what stays allocated is the kept plan's copy of the filters."""
+    import torch
+    rng = np.random.default_rng(1800)
+    N, C, H, W, Kf = 8, 1024, 14, 14, 1024
+    X, O = hip.array(rng.standard_normal((N, C, H, W), dtype=np.float32)), hip.empty((N, Kf, H, W))
+    Wd = hip.array((rng.standard_normal((Kf, C, kernel, kernel)) * 0.02).astype(np.float32))
+    hip.cache_conv_filters(Wd)
+    hip.conv_autotune(-1)
+
+    def free():
+        hip.synchronize()
+        hip.workspace_trim()
+        return torch.cuda.mem_get_info(0)[0]
+    try:
+        hip.conv2D(X, Wd, None, O, 1, 1, kernel // 2, kernel // 2)
+        before = free()
+        hip.conv_autotune(True)
+        hip.conv2D(X, Wd, None, O, 1, 1, kernel // 2, kernel // 2)
+        after = free()
+        path = tmp_path / "plans.txt"
+        hip.conv_tuned_save(str(path))
+        head = "%d %d %d %d %d " % (N, C, Kf, kernel, kernel)
+        tiles = [int(l.split("|")[1].split()[0]) for l in path.read_text().splitlines() if l.startswith(head)]
+        assert len(tiles) == 1
+        weights = C * Kf * kernel * kernel
+        copy = weights * 6 if tiles[0] >= 16 else C * Kf * 16 * 4 if 4 <= tiles[0] <= 7 else 0
+        assert before - after <= copy + (4 << 20), (tiles, before - after, copy)  # (allocations come in pages of 2 MiB)
+    finally:
+        hip.conv_autotune(-1)
+        hip.uncache_conv_filters(Wd)

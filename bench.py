@@ -25,7 +25,23 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_FP32_MFMA_TFLOPS = 157.3  # MI355X dense fp32 matrix peak (256 CUs x 256 flop/clk x 2.4 GHz)
+# the split form: six products on the bf16 matrix instruction, which does 16 times the work of the fp32 one, per product of fp32 numbers
+PEAK_SPLIT_TFLOPS = PEAK_FP32_MFMA_TFLOPS * 16 / 6
 PEAK_HBM_GBS = 8000.0
+
+
+def form_of_plan(tile):
+    """The form of convolution that a plan's tile number names in a plans file (eddlhip_conv2d_force_plan)."""
+    for first, last, form in ((-1, -1, "planner"), (0, 3, "direct_tile"), (4, 4, "winograd_three_kernels"), (5, 5, "winograd_folded"),
+                              (6, 7, "winograd_one_launch"), (8, 9, "upsampled_2x2"), (16, 19, "split")):
+        if first <= tile <= last:
+            return form
+    raise ValueError("bench.py: plan tile %d names no form" % tile)
+
+
+def peak_of_form(form):
+    """What a layer's kernel could multiply at most, in TFLOP/s of fp32 products."""
+    return PEAK_SPLIT_TFLOPS if form == "split" else PEAK_FP32_MFMA_TFLOPS
 
 WORKLOADS = {
     # name -> (builder kwargs, seed, input distribution, description)
@@ -173,7 +189,9 @@ def oracle_parity(workload, device_output, max_images):
             "bound": PARITY_BOUND, "ok": bool(err <= PARITY_BOUND * scale)}
 
 
-RIDGE_FLOP_PER_BYTE = PEAK_FP32_MFMA_TFLOPS * 1e3 / PEAK_HBM_GBS  # 19.7: below it a layer is bound by HBM, not by the matrix cores
+def ridge_of_form(form):
+    """flop/byte below which a layer is bound by HBM, not by the matrix cores: 19.7, 52.4 in the split form."""
+    return peak_of_form(form) * 1e3 / PEAK_HBM_GBS
 
 
 def measure(hip, workload, steps, warmup, fused=True, graph=False, tune=True, plans=None):
@@ -209,11 +227,9 @@ def measure(hip, workload, steps, warmup, fused=True, graph=False, tune=True, pl
         with tempfile.NamedTemporaryFile("r", suffix=".txt") as fh:
             hip.conv_tuned_save(fh.name)
             lines = sorted(l.strip() for l in open(fh.name) if l.strip() and not l.startswith("#"))
-        forms = {"planner": 0, "direct_tile": 0, "winograd_three_kernels": 0, "winograd_folded": 0, "winograd_one_launch": 0, "upsampled_2x2": 0}
+        forms = {"planner": 0, "direct_tile": 0, "winograd_three_kernels": 0, "winograd_folded": 0, "winograd_one_launch": 0, "upsampled_2x2": 0, "split": 0}
         for l in lines:
-            tile = int(l.split("|")[1].split()[0])
-            forms["planner" if tile < 0 else "direct_tile" if tile < 4 else "winograd_three_kernels" if tile == 4 else "winograd_folded" if tile == 5
-                  else "winograd_one_launch" if tile < 8 else "upsampled_2x2"] += 1
+            forms[form_of_plan(int(l.split("|")[1].split()[0]))] += 1
         plans_info = {"geometries": len(lines), "sha16": hashlib.sha256("\n".join(lines).encode()).hexdigest()[:16], "kept": forms,
                       "workspace_bytes_after_search": hip.workspace_bytes()}
     step = model.run
@@ -242,7 +258,7 @@ def measure(hip, workload, steps, warmup, fused=True, graph=False, tune=True, pl
             # kernel_flops: what the timed kernel itself multiplies.  The Winograd form times its product launch (16 products
             # of [Kf x C] by [C x blocks] matrices, 2.25 times fewer multiplications than the layer's direct count); the two
             # transform kernels around it are in the op's own time only
-            kernel_flops, form = op.flops, "direct"
+            kernel_flops, form = op.flops, "split" if kern.startswith("conv_split_kernel") else "direct"
             if kern.startswith("winograd["):
                 blocks = int(kern[kern.rindex(",") + 1:].split()[0])
                 kern = kern[len("winograd["):kern.rindex(",")]
@@ -260,7 +276,8 @@ def measure(hip, workload, steps, warmup, fused=True, graph=False, tune=True, pl
                 n_out, kf = conv.out_shape[0] * conv.out_shape[2] * conv.out_shape[3], conv.out_shape[1]
                 c_in = op.flops // (2 * conv.kr * conv.kc * n_out * kf)
                 kernel_flops, form = 2 * 9 * kf * c_in * blocks, "upsampled2x2"
-            row.update(kernel=kern.split(" +ksplit")[0], kernel_ms=kms, kernel_launches=kl, kernel_flops=kernel_flops, form=form)
+            row.update(kernel=kern.split(" +ksplit")[0], kernel_ms=kms, kernel_launches=kl, kernel_flops=kernel_flops, form=form,
+                       kernel_peak_tflops=peak_of_form(form))
         if op.kind in ("conv2d", "dense") and ms > 0:
             row["tflops"] = op.flops / ms / 1e9
             row["frac_fp32_mfma_peak"] = row["tflops"] / PEAK_FP32_MFMA_TFLOPS
@@ -279,8 +296,10 @@ def measure(hip, workload, steps, warmup, fused=True, graph=False, tune=True, pl
     dom_flops, dom_ms = sum(r["kernel_flops"] for r in dom), sum(r["kernel_ms"] for r in dom)
     dom_launches = sum(r["kernel_launches"] for r in dom)
     achieved = dom_flops / dom_ms / 1e9 if dom_ms > 0 else 0.0
-    roofline = {"bound": "mfma", "achieved": achieved, "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s",
-                "frac": achieved / PEAK_FP32_MFMA_TFLOPS, "traffic": None,
+    dom_form = dom[0].get("form")
+    dom_peak = peak_of_form(dom_form)
+    roofline = {"bound": "mfma", "achieved": achieved, "peak": dom_peak, "unit": "TFLOP/s",
+                "frac": achieved / dom_peak, "traffic": None, "form": dom_form,
                 "kernel": dom_name, "launches_per_step": dom_launches, "layers": len(dom),
                 "flops_per_launch": dom_flops / max(dom_launches, 1), "avg_launch_ms": dom_ms / max(dom_launches, 1),
                 "algorithmic_bytes_per_launch": sum(r["bytes"] for r in dom) / max(dom_launches, 1)}
@@ -308,10 +327,11 @@ def measure(hip, workload, steps, warmup, fused=True, graph=False, tune=True, pl
     hbm_bound = [{"name": r["name"], "kernel": r.get("kernel"), "ms": r.get("kernel_ms", r["ms"]),
                   "flop_per_byte": r["flops"] / r["bytes"], "gbs": r["bytes"] / r.get("kernel_ms", r["ms"]) / 1e6,
                   "frac_hbm_peak": r["bytes"] / r.get("kernel_ms", r["ms"]) / 1e6 / PEAK_HBM_GBS}
-                 for r in conv_rows if r["bytes"] > 0 and r["flops"] / r["bytes"] < RIDGE_FLOP_PER_BYTE and r.get("kernel_ms", r["ms"]) > 0]
+                 for r in conv_rows if r["bytes"] > 0 and r["flops"] / r["bytes"] < ridge_of_form(r.get("form")) and r.get("kernel_ms", r["ms"]) > 0]
     conv_ms = sum(r["ms"] for r in conv_rows)
     conv_flops = sum(r["flops"] for r in conv_rows)
     executed_flops = sum(r.get("kernel_flops", r["flops"]) for r in conv_rows)  # what the launches multiply (Winograd layers: 2.25x less)
+    mfma_ms = sum(r.get("kernel_flops", r["flops"]) / peak_of_form(r.get("form")) for r in conv_rows) / 1e9  # ... at each layer's own peak
     summary = {"value": batch * steps / wall, "unit": "images/sec", "ms_per_step": wall * 1e3 / steps, "steps": steps, "warmup": warmup,
                "batch": batch, "fused_ops": len(model.ops), "roofline": roofline, "hbm_bound_convs": hbm_bound,
                # the layers' direct-form flop count over their device time: layers that run in the Winograd form multiply 2.25
@@ -322,8 +342,9 @@ def measure(hip, workload, steps, warmup, fused=True, graph=False, tune=True, pl
                               "flops_counted": "direct form", "layers": len(conv_rows),
                               # the flops the launches really multiply over the same time: the matrix pipe's useful share
                               "executed_gflop": executed_flops / 1e9,
-                              "mfma_util": (executed_flops / conv_ms / 1e9 / PEAK_FP32_MFMA_TFLOPS) if conv_ms else 0.0,
-                              "winograd_layers": sum(1 for r in conv_rows if r.get("form") == "winograd")},
+                              "mfma_util": mfma_ms / conv_ms if conv_ms else 0.0,
+                              "winograd_layers": sum(1 for r in conv_rows if r.get("form") == "winograd"),
+                              "split_layers": sum(1 for r in conv_rows if r.get("form") == "split")},
                "device_ms_sum_of_ops": sum(op_ms), "plans": plans_info, "workspace_bytes": hip.workspace_bytes()}
     del model
     return summary, rows, out_host, desc
@@ -431,7 +452,7 @@ def main():
         roofline["device_probe"] = {"unit": "TFLOP/s", "pure_mfma_constant_operands": const_mean,
                                     "pure_mfma_varying_operands_mean": vary_mean, "varying_best_launch": vary_best,
                                     "varying_worst_launch": vary_worst,
-                                    "frac_of_varying_mean": achieved / vary_mean if vary_mean > 0 else None}
+                                    "frac_of_varying_mean": achieved / vary_mean if vary_mean > 0 and roofline["form"] != "split" else None}
         # and what plain read / write / copy streams over 1 GiB buffers sustain, beside the 8 TB/s HBM peak
         rd, wr, cp = hip.probe_hbm(1 << 30)
         roofline["device_probe"].update(hbm_unit="GB/s", hbm_read_stream=rd, hbm_write_stream=wr, hbm_copy_stream=cp)
@@ -466,7 +487,7 @@ def main():
             sm, _, out_w, desc_w = measure(hip, w, steps, warmup, tune=not args.no_tune)
             entry = {"workload": desc_w, "value": sm["value"], "unit": "images/sec", "ms_per_step": sm["ms_per_step"], "steps": steps,
                      "warmup": warmup, "batch": sm["batch"], "dominant_kernel": sm["roofline"]["kernel"],
-                     "frac": sm["roofline"]["frac"], "achieved_tflops": sm["roofline"]["achieved"],
+                     "frac": sm["roofline"]["frac"], "achieved_tflops": sm["roofline"]["achieved"], "peak_tflops": sm["roofline"]["peak"],
                      "avg_launch_ms": sm["roofline"]["avg_launch_ms"], "launches_per_step": sm["roofline"]["launches_per_step"],
                      "conv_total": sm["conv_total"], "hbm_bound_convs": sm["hbm_bound_convs"], "plans": sm["plans"],
                      "workspace_bytes": sm["workspace_bytes"], "traffic": sm["roofline"].get("traffic")}
@@ -485,13 +506,13 @@ def main():
     table = ["# ms = device time between two events around the op; an event pair around a one-element fill reads %.4f ms"
              % event_floor_ms,
              "# TFLOP/s = the layer's direct-form flop count over that time (a layer in the Winograd form multiplies 2.25 times less: "
-             "its rate is an effective one)",
+             "its rate is an effective one); %mfma against the fp32 instruction's 157.3 (a layer in the split form: up to 267)",
              "%-44s %9s %9s %8s %9s %7s" % ("op", "ms", "TFLOP/s", "%mfma", "GB/s", "%hbm")]
     for r in rows:
         table.append("%-44s %9.4f %9s %8s %9.1f %7.2f  %s" % (
             r["name"][:44], r["ms"], "%.2f" % r["tflops"] if "tflops" in r else "-",
             "%.1f" % (100 * r["frac_fp32_mfma_peak"]) if "tflops" in r else "-", r.get("gbs", 0.0), 100 * r.get("frac_hbm_peak", 0.0),
-            ("winograd: " if r.get("form") == "winograd" else "upsampled 2x2: " if r.get("form") == "upsampled2x2" else "") + r.get("kernel", "")))
+            {"winograd": "winograd: ", "upsampled2x2": "upsampled 2x2: ", "split": "split: "}.get(r.get("form"), "") + r.get("kernel", "")))
     if args.layers:
         print("\n".join(table), file=sys.stderr)
     out_dir = args.out

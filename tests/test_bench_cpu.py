@@ -7,6 +7,7 @@ import subprocess
 import sys
 
 import numpy as np
+import pytest
 
 from conftest import ROOT
 
@@ -30,6 +31,26 @@ def test_workload_flops_match_the_configurations():
                 N, Kf, P, Q = cd.out_shape
                 flops += 2 * N * Kf * cd.kz * cd.kr * cd.kc * P * Q
         assert abs(flops - want[name]) / want[name] < 2e-3, (name, flops)
+
+
+def test_every_plan_number_has_a_form_and_the_split_form_a_peak_of_its_own(tmp_path):
+    """The benchmark names every plan that the library's loader accepts and no other, and prices the split form by the bf16 instruction."""
+    sys.path.insert(0, ROOT)
+    import bench
+    from eddl_amd import _lib
+    lib = _lib.load()
+    path = tmp_path / "plans.txt"
+    for tile in range(-2, 30):
+        path.write_text("4 128 64 1 1 1 1 28 28 1 | %d 1\n" % tile)
+        if lib.eddlhip_conv2d_tuned_load(0, str(path).encode()) == 0:
+            assert (bench.form_of_plan(tile) == "split") == (tile >= 16)
+            assert (bench.form_of_plan(tile) == "upsampled_2x2") == (tile in (8, 9))
+        else:
+            with pytest.raises(ValueError):
+                bench.form_of_plan(tile)
+    lib.eddlhip_conv2d_autotune(-1)
+    assert bench.peak_of_form("direct") == bench.peak_of_form("winograd") == 157.3
+    assert bench.peak_of_form("split") == pytest.approx(16 * 157.3 / 6)
 
 
 def test_cpu_baseline_leg_runs_on_a_small_sample(monkeypatch):

@@ -20,6 +20,7 @@ import sys
 
 HBM_PEAK_GBS = 8000.0
 FP32_MFMA_PEAK_TFLOPS = 157.3
+BF16_MFMA_PEAK_TFLOPS = 16 * FP32_MFMA_PEAK_TFLOPS
 COPY_PROBE_KIB = 262144.0  # bench.py --copy-probe: one ReLU over 2^26 floats reads 256 MiB and writes 256 MiB
 HOT = ("conv_", "wino_", "maxpool", "avgpool", "dense", "bn_", "add_kernel", "concat", "scale_", "unary_kernel", "pad_", "softmax", "upsample")
 
@@ -189,11 +190,12 @@ def traffic(workload, trace_dir, fetch_dir, write_dir, log, out, out_json=None, 
             fh.write("\n")
 
 
-MFMA_COUNTERS = "SQ_INSTS_VALU_MFMA_MOPS_F32 SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CU_CYCLES GRBM_GUI_ACTIVE"
+MFMA_COUNTERS = "SQ_INSTS_VALU_MFMA_MOPS_F32 SQ_INSTS_VALU_MFMA_MOPS_BF16 SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CU_CYCLES GRBM_GUI_ACTIVE"
 
 
 def mfma(workload, directory, out):
     mops, busy, gui = counter(directory, "SQ_INSTS_VALU_MFMA_MOPS_F32"), counter(directory, "SQ_VALU_MFMA_BUSY_CYCLES"), counter(directory, "GRBM_GUI_ACTIVE")
+    bf16 = counter(directory, "SQ_INSTS_VALU_MFMA_MOPS_BF16")
     dur = durations(directory)
     o = ["Matrix-core counters of the %s benchmark kernels (MI355X, gfx950)%s" % (workload, ("; library at commit %s" % commit()) if commit() else ""),
          "commands (from the repository root):",
@@ -206,7 +208,9 @@ def mfma(workload, directory, out):
         m = mean(mops[probe[0]])
         o += ["SQ_INSTS_VALU_MFMA_MOPS_F32 counts fp32 matrix operations in units of 512 flops: the pure-MFMA probe kernel of the same run",
               "(mfma_f32_probe_kernel, 1.0737e12 flops per launch by construction) reads %.4g, i.e. %.1f flops per count." % (m, 1.0737e12 / m)]
-    o += ["columns: calls = dispatches; avg us = mean of End_Timestamp - Start_Timestamp in THIS run (kernels run a few % slower while",
+    o += ["conv_split_kernel: SQ_INSTS_VALU_MFMA_MOPS_BF16 in the same unit, %%peak against the bf16 instruction's %.0f TFLOP/s; six bf16" % BF16_MFMA_PEAK_TFLOPS,
+          "products are one fp32 product, so a sixth of its exec GFLOP and TFLOP/s are those of fp32 work.",
+          "columns: calls = dispatches; avg us = mean of End_Timestamp - Start_Timestamp in THIS run (kernels run a few % slower while",
           "counters are collected); exec GFLOP = mean SQ_INSTS_VALU_MFMA_MOPS_F32 per dispatch x 512 / 1e9 (includes the zero taps of a",
           "padded K range); TFLOP/s = exec GFLOP / avg us / 1000; %peak = TFLOP/s / 157.3 x 100; busy % = SQ_VALU_MFMA_BUSY_CYCLES /",
           "(GRBM_GUI_ACTIVE / 8 XCDs x 1024 SIMDs) x 100; GHz = GRBM_GUI_ACTIVE / 8 / avg us / 1000 (the shader clock the kernel ran at:",
@@ -214,13 +218,15 @@ def mfma(workload, directory, out):
           "",
           "%-88s %6s %9s %12s %9s %7s %7s %6s" % ("kernel", "calls", "avg us", "exec GFLOP", "TFLOP/s", "%peak", "busy %", "GHz")]
     for k in mops:
-        if not any(t in k for t in ("conv_tap", "conv_gen", "conv_pointwise", "wino_fused_kernel", "dense_partial", "mfma_f32_probe")):
+        if not any(t in k for t in ("conv_tap", "conv_gen", "conv_split", "conv_pointwise", "wino_fused_kernel", "dense_partial", "mfma_f32_probe")):
             continue
         us = mean(dur[k])
-        fl = mean(mops[k]) * 512.0
+        split = "conv_split" in k
+        fl = mean((bf16 if split else mops)[k]) * 512.0
+        peak = BF16_MFMA_PEAK_TFLOPS if split else FP32_MFMA_PEAK_TFLOPS
         cyc = mean(gui[k]) / 8.0
         o.append("%-88s %6d %9.1f %12.2f %9.1f %7.1f %7.1f %6.2f"
-                 % (short(k, 88), len(dur[k]), us, fl / 1e9, fl / us / 1e6, fl / us / 1e6 / FP32_MFMA_PEAK_TFLOPS * 100, 100 * mean(busy[k]) / (cyc * 1024.0), cyc / us / 1e3))
+                 % (short(k, 88), len(dur[k]), us, fl / 1e9, fl / us / 1e6, fl / us / 1e6 / peak * 100, 100 * mean(busy[k]) / (cyc * 1024.0), cyc / us / 1e3))
     write(out, o, workload)
 
 

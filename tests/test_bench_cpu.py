@@ -83,3 +83,25 @@ def test_cpu_baseline_leg_checks_a_device_output_against_the_oracle(monkeypatch)
     assert good["ok"] and good["images"] == 1 and good["max_abs_err"] == 0.0
     bad = bench.cpu_baseline("block", want_seconds=0.1, device_output=full + 1e-3 * np.abs(full).max())["parity"]
     assert not bad["ok"] and bad["err_over_max_ref"] > bench.PARITY_BOUND
+
+
+def test_matrix_counter_table_counts_the_split_kernel_in_bf16_products(tmp_path):
+    """The counter summary has a row for every kind of matrix kernel, the split one from the bf16 counter and at that peak."""
+    from eddl_amd import profsum
+    names = ["void (anonymous namespace)::%s(ConvParams)" % k for k in ("conv_split_kernel<4, 1, 1, 2, 3>", "conv_tap_kernel<2, 2, 1, 1, 1, 1, 16, true>")]
+    with open(tmp_path / "m_counter_collection.csv", "w") as fh:
+        fh.write("Dispatch_Id,Kernel_Name,Counter_Name,Counter_Value\n")
+        for i, k in enumerate(names):
+            for counter, value in (("SQ_INSTS_VALU_MFMA_MOPS_F32", 2e6 * i), ("SQ_INSTS_VALU_MFMA_MOPS_BF16", 2e7 * (1 - i)),
+                                   ("SQ_VALU_MFMA_BUSY_CYCLES", 1024e4), ("GRBM_GUI_ACTIVE", 16e4)):
+                fh.write('%d,"%s",%s,%f\n' % (i, k, counter, value))
+    with open(tmp_path / "m_kernel_trace.csv", "w") as fh:
+        fh.write("Kernel_Name,Start_Timestamp,End_Timestamp\n")
+        for k in names:
+            fh.write('"%s",1000,11000\n' % k)
+    profsum.mfma("resnet50", str(tmp_path), str(tmp_path / "out.txt"))
+    rows = {l.split("<")[0]: l.split("(ConvParams)")[1].split() for l in open(tmp_path / "out.txt") if "(ConvParams)" in l}
+    assert set(rows) == {"conv_split_kernel", "conv_tap_kernel"}
+    for name, ops, peak in (("conv_split_kernel", 2e7, 16 * 157.3), ("conv_tap_kernel", 2e6, 157.3)):
+        rate = ops * 512 / 10e-6 / 1e12        # TFLOP/s of a 10 us dispatch
+        assert float(rows[name][3]) == round(rate, 1) and float(rows[name][4]) == round(100 * rate / peak, 1)

@@ -6,7 +6,7 @@
 // output block over a slice of k: per pair of k it loads ONE float4 of B per lane (lane l of a
 // half wavefront covers columns 4l..4l+3: 512 contiguous bytes per k row) and one dword of the
 // activations, and issues four v_mfma_f32_32x32x2_f32, one per column phase
-// (accumulator j holds columns 4l + j).  Except for one row or few short ones (reads_rows), the
+// (accumulator j holds columns 4l + j).  Except for one row, or few with not too many weights (reads_rows), the
 // activations are transposed first (At[k][32], a few MB, L2-resident) so that their loads are coalesced too.  k is split over wavefronts so the
 // whole device streams B; the per-slice partial blocks go to the private workspace and a second
 // kernel adds them in slice order (fixed summation order, no atomics).
@@ -170,10 +170,15 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(const float *__restri
 namespace {
 
 // Whether a product reads the activations where they are instead of from a transposed copy.  The copy is a launch of its own,
-// about 3 us: one row, 2048 x 1000 13.9 -> 10.9 us, 4096 x 4096 22.6 -> 19.6; 32 rows 16.4 -> 13.5, 26.0 -> 24.3.  Rows of
-// 25088 taps, read once per column tile from as many cache lines as there are rows, lose it again: 25088 x 4096 (413 MB, the
-// copy's 84 us are 4.9 TB/s) one row 83.9 -> 81.5 us, two 83.6 -> 86.6, 32 rows 91 -> 138.
-bool reads_rows(int m, int k) { return m == 1 || (m <= 32 && k <= 4096); }
+// 2 to 6 us.  In place a lane reads its own row, a cache line a row and not one for 32, and the wavefronts beside it read those
+// lines again while they stream the weights: the more rows and the more weights, the less of that the caches hold.  Measured over
+// 29 matrices of 512 .. 25088 x 128 .. 25088, the weights from memory (us, in place against the copy): one row is faster in place
+// everywhere (4096 x 1000 14.8 against 17.5, 25088 x 4096 81.8 against 83.2).  More rows are up to 17 M weights, whatever the
+// shape (32 rows: 4096 x 4096 26.4 against 28.9, 16384 x 1000 30.0 against 35.3; 6144 x 2048 alone 27.2 against 26.7).  At 25 M
+// up to 16 rows are (eight: 4096 x 6144 31.1 against 33.5, 25088 x 1000 40.0 against 43.0; sixteen 33.5 against 34.8, 45.2 against
+// 44.2) and 32 are not (43.7 against 38.2); from 34 M on only one row is (8192 x 4096: two rows 38.8 against 39.8, eight 42.9
+// against 41.4, 32 58.9 against 47.5).
+bool reads_rows(int m, int k, int n) { return m == 1 || (m <= 32 && (size_t)k * n <= (size_t)(m <= 16 ? 28 : 20) << 20); }
 
 int dense_impl(int dev, const float *A, const float *B, float *C, int m, int k, int n, int incC, const float *bias, int relu,
                const char *what) {
@@ -197,7 +202,7 @@ int dense_impl(int dev, const float *A, const float *B, float *C, int m, int k, 
     int kslice = ((k + nslices - 1) / nslices + 1) & ~1;  // even, so MFMA tap pairs do not straddle slices
     nslices = (k + kslice - 1) / kslice;
     EH_REQUIRE(nslices <= 65535 && mgroups <= 65535, "%s: shape out of range", what);
-    const bool direct = reads_rows(m, k);
+    const bool direct = reads_rows(m, k, n);
     const size_t at_bytes = direct ? 0 : ((size_t)mt * k * 32 * sizeof(float) + 255) & ~(size_t)255;
     void *ws = nullptr;
     EH_TRY(get_workspace(dev, at_bytes + (size_t)nslices * m * n * sizeof(float), &ws));

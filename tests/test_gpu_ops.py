@@ -962,6 +962,17 @@ def test_dense_rows_read_in_place_equal_the_transposed_ones(hip, m, k, n):
     assert np.array_equal(C.numpy(), D.numpy()[:m])
 
 
+@pytest.mark.parametrize("m,k,n", [(16, 2048, 14336), (16, 2048, 14340), (17, 2048, 10240), (17, 2048, 10244), (32, 8192, 2564), (1, 25088, 1204)])
+def test_dense_rows_on_either_side_of_the_line_between_the_two_ways(hip, m, k, n):
+    """28 and 20 times 2^20 weights, the lines that the rows' way of being read changes at: the same bits as among 33 rows."""
+    A, W, C, D = hip.empty((33, k)), hip.empty((k, n)), hip.full((m, n), 7.0), hip.empty((33, n))
+    hip.rand_normal(A, 0.0, 1.0, 11)
+    hip.rand_normal(W, 0.0, 0.03, 12)
+    hip.mult2D(hip.array(A.numpy()[:m]), W, C)
+    hip.mult2D(A, W, D)
+    assert np.array_equal(C.numpy(), D.numpy()[:m])
+
+
 def test_dense_sigmoid_softmax_within_tolerance(hip, oracle):
     rng = np.random.default_rng(405)
     for m, k, n in [(32, 512, 1000), (5, 37, 300), (64, 2048, 10), (33, 100, 65), (70, 1001, 131), (32, 3136, 4096), (1, 2, 1),

@@ -2904,8 +2904,8 @@ size_t winograd_workspace(bool fold, int N, int C, int Kf, int fs, int P, int Q,
 // launches, after the planner's plan has run for 25 ms (settled clocks), re-times the plans near the front in turns, and
 // takes each plan's FASTEST batch (noise only ever adds time).  Then, so that two searches of one geometry agree:
 // of all plans within 3 % of the fastest one it keeps the first in a fixed order of preference - the planner's own plan,
-// the one-launch Winograd form, the direct tiles, the Winograd forms with a transformed input in memory; within a form
-// fewer K slices first.  Returns 0 with *out filled, 1 when these tensors cannot be searched on (the output overlaps an
+// the one-launch Winograd form (or the upsampled-input form of a 2x2 filter), the split form, the direct tiles, the Winograd
+// forms with a transformed input in memory; within a form fewer K slices first.  Returns 0 with *out filled, 1 when these tensors cannot be searched on (the output overlaps an
 // input: repeating the call would change what it reads), or minus the error code of a runtime failure.
 int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, long long chunk_pix, bool wino_ok, bool fold_ok, bool fused_ok, bool up_ok,
                 bool split_ok, TunedPlan *out) {

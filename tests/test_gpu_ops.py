@@ -1246,9 +1246,10 @@ def test_conv2d_split_form_is_no_further_from_64_bits_than_the_fp32_form(hip, ca
     finally:
         hip.force_conv_plan(-1, 1)
     ref = _conv64(x, w, stride, pad, P, Q)
-    scale = np.linalg.norm(ref)
-    # the result's own rounding to fp32 (2^-24 of a value at most, both forms have it) beside the fp32 form's error
-    assert np.linalg.norm(got - ref) <= np.linalg.norm(fp32 - ref) + 2.0 ** -24 * scale
+    # (the case of one output is decided by chance: a sum is rounded at least twice, as it ends and as its small parts join it, 2^-24
+    # of it each time; the fp32 form's error in every other case is above that)
+    assert np.linalg.norm(got - ref) <= max(np.linalg.norm(fp32 - ref), 2.0 ** -23 * np.linalg.norm(ref))
+    assert np.prod(ref.shape) == 1 or np.linalg.norm(got - ref) <= np.linalg.norm(fp32 - ref)
     assert_conv_close(ref, got, case)
 
 

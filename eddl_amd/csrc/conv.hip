@@ -2326,11 +2326,12 @@ constexpr int UP2X2_TILE = FUSED_TILE0 + NUM_FUSED;  // plan "tiles" of the upsa
 constexpr int NUM_PLAN_TILES = UP2X2_TILE + 2;
 
 // The split form (conv_split.h): plan "tiles" from 16 on (10 .. 15 name nothing and stay refused in a plans file).
-// Tile shapes, measured at batch 64 (us; fp32 tiles before): 128x128 for many tiles of long K (256 channels 3x3 on 56x56, batch
-// 32: 826 -> 537, 220 TFLOP/s of fp32 work: the engine clock falls to 1.73 GHz under it and the matrix pipe is busy 69 % of
-// that), 128x64 for most 1x1 layers (1024 -> 256 on 14x14: 60 -> 42; 256 -> 1024: 60 -> 44; 64 -> 256 on 56x56: 73 -> 63, of
-// which 256 MB of traffic are 43), 64x128 where there are 64 filters (256 -> 64 on 56x56: 68 -> 54), 64x64 for few tiles.
-// A 128x64 tile gives every wavefront filters of its own and all the pixels: its filters then cross L1 once, not twice.
+// Tile shapes, measured at batch 64 (us; the best fp32 tile before): 128x128 for many tiles of long K (256 channels 3x3 on 56x56,
+// batch 32: 827 -> 559, 212 TFLOP/s of fp32 work; a U-Net's 1024 -> 512 2x2 step, 220 TFLOP/s, keeps the matrix pipe busy 63 % of
+// the cycles at 2.0 GHz), 128x64 for most 1x1 layers (1024 -> 256 on 14x14: 60 -> 43; 256 -> 1024: 60 -> 45; 512 -> 128 on 28x28:
+// 58 -> 42; 3x3 stride 2 of 128 on 56x56: 120 -> 91; 64 -> 256 on 56x56: 70 -> 67, of which 256 MB of traffic are 43; in a
+// ResNet-50 the pipe is busy 28 % of the cycles), 64x128 where there are 64 filters (256 -> 64 on 56x56: 60 -> 52), 64x64 for few
+// tiles.  A 128x64 tile gives every wavefront filters of its own and all the pixels: its filters then cross L1 once, not twice.
 #define SPLIT(WM, WN, TM, TN, WGS)                                                                                                           \
     {                                                                                                                                        \
         "conv_split_kernel<" #WM "," #WN "," #TM "," #TN "," #WGS ">", WM *TM * 32, WN *TN * 32, SPLIT_K, conv_split_kernel<WM, WN, TM, TN, WGS>, \

@@ -46,6 +46,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -2224,6 +2225,7 @@ __global__ __launch_bounds__(256) void wino_fused_reduce_kernel(const ConvParams
 }
 
 #include "conv_split.h"
+#include "wino_split.h"
 
 // ---------------------------------------------------------------- host side
 int g_algo = 0;
@@ -2314,14 +2316,26 @@ struct FusedVariant {
     void (*kernel)(const ConvParams);
     void (*kernel_wide)(const ConvParams);  // the build that loads the pixels 16 bytes per lane (conv2d_winograd_fused decides)
     void (*reduce)(const ConvParams);
+    int threads;
+    bool split;  // on the bf16 matrix instructions (wino_split.h)
 };
 #define FUSED(FM, FN, CK, WPE)                                                                                                       \
     {"wino_fused_kernel<" #FM "," #FN "," #CK "," #WPE ">", "wino_fused_kernel<" #FM "," #FN "," #CK "," #WPE ",true>", FM, FN, CK,  \
-     wino_fused_kernel<FM, FN, CK, WPE, false>,         wino_fused_kernel<FM, FN, CK, WPE, true>, wino_fused_reduce_kernel<FM, FN>}
+     wino_fused_kernel<FM, FN, CK, WPE, false>,         wino_fused_kernel<FM, FN, CK, WPE, true>, wino_fused_reduce_kernel<FM, FN>, 256, false}
 const FusedVariant kfused[] = {FUSED(1, 1, 4, 4), FUSED(2, 1, 4, 3)};
 constexpr int NUM_FUSED = (int)(sizeof(kfused) / sizeof(kfused[0]));
 constexpr int FUSED_TILE0 = 6;      // plan "tile" numbers 6 .. 6 + NUM_FUSED - 1 name these shapes (0..3: direct tiles, 4 / 5: the other Winograd forms)
 constexpr int FUSED_ROW_ALIGN = 8;  // the transformed filters are padded to whole K-steps of every variant
+// The same on the bf16 matrix instructions (wino_split.h): plan "tile" 32.  Channel counts that are multiples of 16, of each tensor
+// of a folded Concat too.  The search tries it from 512 blocks on: a filter is 96 bytes a channel here, and below that the
+// launches are bound by reading them (512 channels on 14x14, best plans of the other forms / this one: 1 image 18.3 / 27.0 us,
+// 4 images 34.4 / 42.8, 8 images 56.0 / 59.4, 16 images 85.1 / 81.1; 1024 channels, 392 blocks 151 / 186, 1024 blocks 290 / 241).
+const FusedVariant kwsplit[] = {
+    {"wino_split_kernel<false>", "wino_split_kernel<true>", 2, 1, 16, wino_split_kernel<false>, wino_split_kernel<true>, wino_fused_reduce_kernel<2, 1>, 256, true}};
+constexpr int NUM_WSPLIT = (int)(sizeof(kwsplit) / sizeof(kwsplit[0]));
+constexpr int WSPLIT_TILE0 = 32;
+constexpr long long WSPLIT_SEARCH_BLOCKS = 512;
+bool is_wsplit_tile(int tile) { return tile >= WSPLIT_TILE0 && tile < WSPLIT_TILE0 + NUM_WSPLIT; }
 constexpr int UP2X2_TILE = FUSED_TILE0 + NUM_FUSED;  // plan "tiles" of the upsampled-input form of a 2x2 convolution: conv_up2x2_kernel<3>, <2>
 constexpr int NUM_PLAN_TILES = UP2X2_TILE + 2;
 
@@ -2341,7 +2355,7 @@ const Variant ksplit[] = {SPLIT(2, 2, 2, 2, 2), SPLIT(4, 1, 1, 2, 3), SPLIT(2, 2
 constexpr int NUM_SPLIT = (int)(sizeof(ksplit) / sizeof(ksplit[0]));
 constexpr int SPLIT_TILE0 = 16;
 bool is_split_tile(int tile) { return tile >= SPLIT_TILE0 && tile < SPLIT_TILE0 + NUM_SPLIT; }
-bool is_plan_tile(int tile) { return (tile >= -1 && tile < NUM_PLAN_TILES) || is_split_tile(tile); }
+bool is_plan_tile(int tile) { return (tile >= -1 && tile < NUM_PLAN_TILES) || is_split_tile(tile) || is_wsplit_tile(tile); }
 int split_steps(int C, int RS) { return (C + SPLIT_K - 1) / SPLIT_K * RS; }
 size_t split_filter_bytes(int C, int RS, int Mp) { return (size_t)split_steps(C, RS) * 2 * (Mp / 32) * SPLIT_UNIT; }
 // Whether the split form can run a convolution: filters within a buffer descriptor, and channels in whole groups of eight also
@@ -2478,6 +2492,7 @@ struct CachedFilters {
     int wino_rows;
     float *Wfused;  // 3x3 filters: the transformed filters of the one-launch Winograd form [fused_rows][16][Mp], made on first use
     int fused_rows;
+    void *Wwsplit;  // 3x3 filters: the transformed filters as three bf16 parts (wino_split_filter_kernel), made on first use
     void *Wsplit;  // the filters as three bf16 parts in the operand order of the split form (split_filter_kernel), made on first use
     float *Wup;  // 2x2 filters: the nine weight-sum rows per channel of the upsampled-input form [C][9][Mp] (up2x2_filter_kernel), made on first use
     bool stale;  // K was written through this library since the last repack
@@ -2503,6 +2518,14 @@ int launch_split_filters(int dev, const float *K, void *Ws, int Kf, int C, int R
     return 0;
 }
 
+int launch_wino_split_filters(int dev, const float *K, void *Ws, int Kf, int C, int Mp) {
+    const int mblocks = Mp / 32, k16s = C / 16;
+    hipLaunchKernelGGL(wino_split_filter_kernel, dim3((unsigned)(((size_t)k16s * mblocks * 64 + 255) / 256)), dim3(256), 0, state(dev).stream, K, (uintx4 *)Ws, Kf, C,
+                       mblocks, k16s);
+    EH_CHECK_LAUNCH();
+    return 0;
+}
+
 int repack(int dev, CachedFilters &e) {
     hipLaunchKernelGGL(pack_filters_kernel, dim3((e.rows + 31) / 32, e.Mp / 32), dim3(256), 0, state(dev).stream, e.K, e.Wp, e.Kf,
                        e.C * e.R * e.S, e.Mp, e.rows);
@@ -2523,13 +2546,14 @@ int repack(int dev, CachedFilters &e) {
         EH_CHECK_LAUNCH();
     }
     if (e.Wsplit != nullptr) EH_TRY(launch_split_filters(dev, e.K, e.Wsplit, e.Kf, e.C, e.R * e.S, e.Mp));
+    if (e.Wwsplit != nullptr) EH_TRY(launch_wino_split_filters(dev, e.K, e.Wwsplit, e.Kf, e.C, e.Mp));
     e.stale = false;
     return 0;
 }
 
 // Which of the forms' own copies a registered filter tensor has (none if it is not registered).
 struct FilterCopies {
-    bool wino, fused, up, split;
+    bool wino, fused, up, split, wsplit;
 };
 CachedFilters *registered_filters(int dev, const float *K, int Kf, int C, int R, int S) {
     for (CachedFilters &e : g_cache[dev])
@@ -2539,8 +2563,8 @@ CachedFilters *registered_filters(int dev, const float *K, int Kf, int C, int R,
 FilterCopies copies_held(int dev, const float *K, int Kf, int C, int R, int S) {
     std::lock_guard<std::mutex> lock(g_cache_mutex);
     const CachedFilters *e = registered_filters(dev, K, Kf, C, R, S);
-    if (e == nullptr) return {false, false, false, false};
-    return {e->Wwino != nullptr, e->Wfused != nullptr, e->Wup != nullptr, e->Wsplit != nullptr};
+    if (e == nullptr) return {false, false, false, false, false};
+    return {e->Wwino != nullptr, e->Wfused != nullptr, e->Wup != nullptr, e->Wsplit != nullptr, e->Wwsplit != nullptr};
 }
 // Frees the copies that a tensor has beyond `keep` (what a plan search made for forms that it did not keep).
 int drop_copies(int dev, const float *K, int Kf, int C, int R, int S, const FilterCopies &keep) {
@@ -2559,6 +2583,7 @@ int drop_copies(int dev, const float *K, int Kf, int C, int R, int S, const Filt
     EH_TRY(drop(e->Wwino, keep.wino));
     EH_TRY(drop(e->Wfused, keep.fused));
     EH_TRY(drop(e->Wup, keep.up));
+    EH_TRY(drop(e->Wwsplit, keep.wsplit));
     return drop(e->Wsplit, keep.split);
 }
 
@@ -2603,6 +2628,7 @@ void conv_filters_released(int dev, const void *base, size_t bytes) {
             if (c[i].Wfused) (void)hipFree(c[i].Wfused);
             if (c[i].Wup) (void)hipFree(c[i].Wup);
             if (c[i].Wsplit) (void)hipFree(c[i].Wsplit);
+            if (c[i].Wwsplit) (void)hipFree(c[i].Wwsplit);
             c[i] = c.back();
             c.pop_back();
         } else {
@@ -2639,6 +2665,7 @@ int eddlhip_conv2d_cache_filters(int dev, const float *K, int Kf, int C, int R, 
     e.fused_rows = 0;
     e.Wup = nullptr;
     e.Wsplit = nullptr;
+    e.Wwsplit = nullptr;
     e.stale = true;
     EH_REQUIRE((size_t)e.rows * e.Mp * sizeof(float) < ((size_t)1 << 31),
                "conv2d_cache_filters: the repacked filter matrix (%d taps x %d channels) exceeds the 2 GiB a buffer descriptor covers", e.rows, e.Mp);
@@ -2667,6 +2694,7 @@ int eddlhip_conv2d_uncache_filters(int dev, const float *K) {
             if (c[i].Wfused) EH_TRY_HIP(hipFree(c[i].Wfused));
             if (c[i].Wup) EH_TRY_HIP(hipFree(c[i].Wup));
             if (c[i].Wsplit) EH_TRY_HIP(hipFree(c[i].Wsplit));
+            if (c[i].Wwsplit) EH_TRY_HIP(hipFree(c[i].Wwsplit));
             c[i] = c.back();
             c.pop_back();
         } else {
@@ -2679,8 +2707,8 @@ int eddlhip_conv2d_uncache_filters(int dev, const float *K) {
 int eddlhip_conv2d_force_plan(int tile, int slices) {
     EH_REQUIRE(is_plan_tile(tile),
                "conv2d_force_plan: tile is -1 (automatic), 0..3, 4 .. %d (the Winograd forms where they apply), %d, %d (a 2x2 filter on an input upsampled twice) "
-               "or %d .. %d (the split form where it applies)",
-               UP2X2_TILE - 1, UP2X2_TILE, UP2X2_TILE + 1, SPLIT_TILE0, SPLIT_TILE0 + NUM_SPLIT - 1);
+               "%d .. %d (the split form where it applies) or %d (the one-launch Winograd form in that arithmetic)",
+               UP2X2_TILE - 1, UP2X2_TILE, UP2X2_TILE + 1, SPLIT_TILE0, SPLIT_TILE0 + NUM_SPLIT - 1, WSPLIT_TILE0);
     g_force_tile = tile;
     g_force_slices = slices;
     return 0;
@@ -2828,7 +2856,7 @@ int conv2d_winograd(bool fold, int fs, int dev, const float *I, const float *I2,
                     int H, int W, int Kf, int pad_top, int pad_left, int P, int Q, const float *bn_g, const float *bn_b, const float *bn_mean,
                     const float *bn_var, float bn_eps, const float *residual, int relu);
 
-int conv2d_winograd_fused(int variant, int slices, int dev, const float *I, const float *I2, int uh, int uw, const float *K, const float *bias, float *O,
+int conv2d_winograd_fused(const FusedVariant &fv, int slices, int dev, const float *I, const float *I2, int uh, int uw, const float *K, const float *bias, float *O,
                           int N, int C, int H, int W, int Kf, int pad_top, int pad_left, int P, int Q, const float *bn_g, const float *bn_b,
                           const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu);
 
@@ -2909,7 +2937,7 @@ size_t winograd_workspace(bool fold, int N, int C, int Kf, int fs, int P, int Q,
 // forms with a transformed input in memory; within a form fewer K slices first.  Returns 0 with *out filled, 1 when these tensors cannot be searched on (the output overlaps an
 // input: repeating the call would change what it reads), or minus the error code of a runtime failure.
 int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, long long chunk_pix, bool wino_ok, bool fold_ok, bool fused_ok, bool up_ok,
-                bool split_ok, TunedPlan *out) {
+                bool split_ok, bool wsplit_ok, TunedPlan *out) {
     {
         const size_t out_bytes = (size_t)c.N * c.Kf * c.P * c.Q * 4, in_bytes = (size_t)c.N * (c.I2 ? c.C / 2 : c.C) * c.H * c.W * 4;
         const char *o_lo = (const char *)c.O, *o_hi = o_lo + out_bytes;
@@ -2986,6 +3014,16 @@ int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, l
                 if (ns == last_slices) continue;  // the same plan as the one before
                 last_slices = ns;
                 time_plan(1 + (NUM_FUSED - 1 - fv), FUSED_TILE0 + fv, sl);
+            }
+        }
+    if (wsplit_ok && (long long)c.N * ((c.P + 1) / 2) * ((c.Q + 1) / 2) >= WSPLIT_SEARCH_BLOCKS)  // ... and on the bf16 matrix instructions
+        for (int v = 0; v < NUM_WSPLIT; v++) {
+            int last_slices = 0;
+            for (int sl : kSearchSlices) {
+                const int ns = fused_slices(kwsplit[v], sl, (long long)c.N * ((c.P + 1) / 2) * ((c.Q + 1) / 2), c.C, c.Kf, num_cu);
+                if (ns == last_slices) continue;
+                last_slices = ns;
+                time_plan(3 + v, WSPLIT_TILE0 + v, sl);
             }
         }
     if (split_ok)  // the split form: its tile shapes, undivided and with the left-over tiles in K slices
@@ -3200,7 +3238,12 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     if (up_ok && (g_force_tile == UP2X2_TILE || g_force_tile == UP2X2_TILE + 1))
         return conv2d_up2x2(g_force_tile - UP2X2_TILE, dev, I, K, bias, O, N, C, H, W, Kf, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
     if (fused_ok && g_force_tile >= FUSED_TILE0 && g_force_tile < FUSED_TILE0 + NUM_FUSED)
-        return conv2d_winograd_fused(g_force_tile - FUSED_TILE0, g_force_slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top,
+        return conv2d_winograd_fused(kfused[g_force_tile - FUSED_TILE0], g_force_slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top,
+                                     pad_left, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
+    // the one-launch form in the split arithmetic: whole K-steps of 16 channels, each of one tensor
+    const bool wsplit_ok = fused_ok && C % 16 == 0 && (!two || C % 32 == 0) && (long long)(C / 16) * (p.Mp / 32) * WSPLIT_UNIT < (1LL << 31);
+    if (wsplit_ok && is_wsplit_tile(g_force_tile))
+        return conv2d_winograd_fused(kwsplit[g_force_tile - WSPLIT_TILE0], g_force_slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top,
                                      pad_left, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
     if ((wino_ok && (g_force_tile == 4 || (g_wino && g_force_tile < 0 && !g_tuning))) || (fold_ok && g_force_tile == 5))
         return conv2d_winograd(g_force_tile == 5, R, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top, pad_left, P, Q, bn_g, bn_b,
@@ -3233,13 +3276,14 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
             memcpy(best.key, key, sizeof(key));
             const size_t ws_before = state(dev).workspace_bytes;
             FilterCopies keep = copies_held(dev, K, Kf, C, R, S);  // (those that other geometries' plans, and graphs, may use)
-            const int src = search_plan(call, family, plan, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, split_ok, &best);
+            const int src = search_plan(call, family, plan, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, split_ok, wsplit_ok, &best);
             if (src < 0) return -src;  // a runtime error inside the search
             if (src == 0) {
                 keep.wino = keep.wino || best.tile == 4 || best.tile == 5;
                 keep.fused = keep.fused || (best.tile >= FUSED_TILE0 && best.tile < FUSED_TILE0 + NUM_FUSED);
                 keep.up = keep.up || best.tile == UP2X2_TILE || best.tile == UP2X2_TILE + 1;
                 keep.split = keep.split || is_split_tile(best.tile);
+                keep.wsplit = keep.wsplit || is_wsplit_tile(best.tile);
             }
             if (!gemm) EH_TRY(drop_copies(dev, K, Kf, C, R, S, keep));
             // the candidates may have taken far more workspace than the plan that stays: let it grow back to what is needed
@@ -3256,8 +3300,11 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
         if (found != nullptr && (found->tile == UP2X2_TILE || found->tile == UP2X2_TILE + 1) && up_ok)
             return conv2d_up2x2(found->tile - UP2X2_TILE, dev, I, K, bias, O, N, C, H, W, Kf, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
         if (found != nullptr && found->tile >= FUSED_TILE0 && found->tile < FUSED_TILE0 + NUM_FUSED && fused_ok)
-            return conv2d_winograd_fused(found->tile - FUSED_TILE0, found->slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top, pad_left, P, Q, bn_g,
+            return conv2d_winograd_fused(kfused[found->tile - FUSED_TILE0], found->slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top, pad_left, P, Q, bn_g,
                                          bn_b, bn_mean, bn_var, bn_eps, residual, relu);
+        if (found != nullptr && is_wsplit_tile(found->tile) && wsplit_ok)
+            return conv2d_winograd_fused(kwsplit[found->tile - WSPLIT_TILE0], found->slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top,
+                                         pad_left, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
         if (found != nullptr && is_split_tile(found->tile) && split_ok) {
             const int tile = found->tile - SPLIT_TILE0;
             const int rc = conv2d_split(no_alloc, ksplit[tile], forced_plan(ksplit, tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev,
@@ -3630,18 +3677,17 @@ int conv2d_up2x2(int variant, int dev, const float *I, const float *K, const flo
 
 // The one-launch Winograd form of a 3x3 stride-1 convolution (wino_fused_kernel).  Workspace: the transformed filters,
 // unless a registered filter tensor keeps them, and the partial output tiles of a K-split plan.
-int conv2d_winograd_fused(int variant, int slices, int dev, const float *I, const float *I2, int uh, int uw, const float *K, const float *bias, float *O,
+int conv2d_winograd_fused(const FusedVariant &fv, int slices, int dev, const float *I, const float *I2, int uh, int uw, const float *K, const float *bias, float *O,
                           int N, int C, int H, int W, int Kf, int pad_top, int pad_left, int P, int Q, const float *bn_g, const float *bn_b,
                           const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu) {
     hipStream_t st = state(dev).stream;
-    const FusedVariant &fv = kfused[variant];
     // a max-pool asked for with this convolution is taken into the epilogue where every 2x2 block of outputs is whole
     PoolRequest *const pool = (g_pool_req != nullptr && !g_tuning && P % 2 == 0 && Q % 2 == 0) ? g_pool_req : nullptr;
     if (pool != nullptr) pool->done = true;
     const int th = (P + 1) / 2, tw = (Q + 1) / 2;
     const int rows = (C + FUSED_ROW_ALIGN - 1) / FUSED_ROW_ALIGN * FUSED_ROW_ALIGN, Mp = (Kf + M_ALIGN - 1) / M_ALIGN * M_ALIGN;
-    const size_t u_floats = (size_t)16 * rows * Mp;
-    EH_REQUIRE(u_floats * sizeof(float) < ((size_t)1 << 31), "conv2d: the transformed filters (16 x %d x %d) exceed 2 GiB", rows, Mp);
+    const size_t u_size = fv.split ? (size_t)(C / 16) * (Mp / 32) * WSPLIT_UNIT : (size_t)16 * rows * Mp * sizeof(float);
+    EH_REQUIRE(u_size < ((size_t)1 << 31), "conv2d: the transformed filters (16 x %d x %d) exceed 2 GiB", rows, Mp);
 
     // a launch covers one batch chunk: input within the 2 GiB a buffer descriptor addresses, fewer than 2^30 blocks
     const int Cimg = I2 ? C / 2 : C;
@@ -3658,51 +3704,57 @@ int conv2d_winograd_fused(int variant, int slices, int dev, const float *I, cons
     // image or outside it as a whole and is aligned in memory (image rows of a multiple of four pixels, stored as they are
     // read, 16-byte aligned tensors), and where rows of blocks are long enough that the widened pixel rows of a tile's
     // segments fit its 16 slots per block (at most 2 + 30 / tw segments, each pixel row at most 6 slots longer than it needs to be).
-    const bool wide = uh == 1 && uw == 1 && W % 4 == 0 && tw >= 6 && pad_left <= 4 && (uintptr_t)I % 16 == 0 && (I2 == nullptr || (uintptr_t)I2 % 16 == 0);
+    // (The split kernel reads the middle pair of a patch row at once, which the widened rows align for odd paddings.)
+    const bool wide = uh == 1 && uw == 1 && W % 4 == 0 && tw >= 6 && pad_left <= 4 && (!fv.split || pad_left % 2 == 1) && (uintptr_t)I % 16 == 0 && (I2 == nullptr || (uintptr_t)I2 % 16 == 0);
     const size_t partial_bytes = (size_t)nslices * leftover * tile_floats * sizeof(float);
 
-    const float *U = nullptr;
+    const void *U = nullptr;
     {
         std::lock_guard<std::mutex> lock(g_cache_mutex);
         for (CachedFilters &e : g_cache[dev]) {
             if (e.K == K && e.Kf == Kf && e.C == C && e.R == 3 && e.S == 3) {
-                if (e.Wfused == nullptr && !state(dev).capturing) {
-                    if (hipMalloc((void **)&e.Wfused, u_floats * sizeof(float)) != hipSuccess) {
-                        e.Wfused = nullptr;
+                void *&kept = fv.split ? e.Wwsplit : (void *&)e.Wfused;
+                if (kept == nullptr && !state(dev).capturing) {
+                    if (hipMalloc(&kept, u_size) != hipSuccess) {
+                        kept = nullptr;
                         (void)hipGetLastError();
                         break;  // no room to keep them: transform per call
                     }
-                    e.fused_rows = rows;
+                    if (!fv.split) e.fused_rows = rows;
                     e.stale = true;
                 }
-                if (e.Wfused != nullptr) {
+                if (kept != nullptr) {
                     if (e.stale) EH_TRY(repack(dev, e));
-                    U = e.Wfused;
+                    U = kept;
                 }
                 break;
             }
         }
     }
-    const size_t u_bytes = U ? 0 : ((u_floats * sizeof(float) + 255) & ~(size_t)255);
+    const size_t u_bytes = U ? 0 : ((u_size + 255) & ~(size_t)255);
     void *ws = nullptr;
     if (u_bytes + partial_bytes > 0) EH_TRY(get_workspace(dev, u_bytes + partial_bytes, &ws));
     if (U == nullptr) {
-        const dim3 grid((unsigned)(((size_t)rows * Mp + 255) / 256));
-        hipLaunchKernelGGL(wino_filter_kernel<4>, grid, dim3(256), 0, st, K, (float *)ws, Kf, C, Mp, rows, 1);
-        EH_CHECK_LAUNCH();
-        U = (const float *)ws;
+        if (fv.split) {
+            EH_TRY(launch_wino_split_filters(dev, K, ws, Kf, C, Mp));
+        } else {
+            const dim3 grid((unsigned)(((size_t)rows * Mp + 255) / 256));
+            hipLaunchKernelGGL(wino_filter_kernel<4>, grid, dim3(256), 0, st, K, (float *)ws, Kf, C, Mp, rows, 1);
+            EH_CHECK_LAUNCH();
+        }
+        U = ws;
     }
 
     ConvParams q;
     memset(&q, 0, sizeof(q));
     q.Csplit = I2 ? C / 2 : C; q.Cimg = Cimg; q.uh = uh; q.uw = uw;
-    q.Wp = U; q.K = K;
+    q.Wp = (const float *)U; q.K = K;
     q.bias = bias; q.bn_g = bn_g; q.bn_b = bn_b; q.bn_mean = bn_mean; q.bn_var = bn_var;
     q.bn_eps = bn_eps; q.relu = relu;
     q.C = C; q.H = H; q.W = W; q.Kf = Kf; q.R = 3; q.S = 3; q.sr = 1; q.sc = 1; q.pt = pad_top; q.pl = pad_left; q.P = P; q.Q = Q;
     q.CRS = C * 9; q.Mp = Mp; q.PQ = P * Q;
     q.nsteps = (C + fv.ck - 1) / fv.ck;
-    q.wp_bytes = (unsigned)(u_floats * sizeof(float));
+    q.wp_bytes = (unsigned)u_size;
     q.wth = th; q.wtw = tw; q.wP = P; q.wQ = Q; q.wps = 4;
     q.gm = (Kf + 32 * fv.fm - 1) / (32 * fv.fm);
     q.partial = (float *)((char *)ws + u_bytes);
@@ -3731,7 +3783,7 @@ int conv2d_winograd_fused(int variant, int slices, int dev, const float *I, cons
         const long long wgs = q.main_tiles + split_tiles * q.nslices;
         q.trace = (g_trace != nullptr && wgs <= g_trace_wgs) ? g_trace : nullptr;
         EH_TRY(prof_begin(st));
-        hipLaunchKernelGGL(wide ? fv.kernel_wide : fv.kernel, dim3((unsigned)wgs), dim3(256), 0, st, q);
+        hipLaunchKernelGGL(wide ? fv.kernel_wide : fv.kernel, dim3((unsigned)wgs), dim3(fv.threads), 0, st, q);
         EH_CHECK_LAUNCH();
         EH_TRY(prof_end(st));
         if (split_tiles > 0) {

@@ -264,6 +264,10 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * kernels').  No output's bits depend on the inputs of another.  Workspace: the
  * split filters, 6 bytes a weight, unless registered, and the partial tiles of a K-split plan; where that is more than
  * eddlhip_conv2d_fwd_noalloc has (11 million unregistered weights), that entry point runs the planner's own choice.
+ * The one-launch Winograd form in that arithmetic (force_plan(32, .), or the search from 512 blocks of outputs on; channel counts
+ * that are multiples of 16): transformed pixels and filters are fp32 numbers as in the third Winograd form, their products and
+ * sums those of the split form, so its error is below that form's too.  Non-finite inputs as in the Winograd forms.  Its filters take
+ * 96 bytes per filter and channel.
  *
  * eddlhip_conv2d_last_kernel() names the kernel the calling thread's last eddlhip_conv2d_fwd
  * launched, followed by " +ksplit(T tiles x S)" when T tiles were divided into S slices; for the Winograd form
@@ -277,7 +281,7 @@ const char *eddlhip_conv2d_last_kernel(void);
  * shape x K slices and the Winograd forms, every launch timed by itself, the fastest of three to nine launches per plan,
  * on the call's own tensors) and remembers one; later calls with that geometry take it.  Which one: of all plans within
  * 3 % of the fastest, the first in a fixed order of preference (the planner's own plan, the one-launch Winograd form, the
- * split form, the direct tiles, the Winograd forms that keep a transformed input in memory - those are tried only below 512 MB of
+ * same in the split arithmetic, the split form, the direct tiles, the Winograd forms that keep a transformed input in memory - those are tried only below 512 MB of
  * workspace; within a form fewer K slices first), so that two searches of one geometry agree unless two plans differ by
  * just that margin.  A caller that needs run-to-run identical bits loads a plans file instead of searching.  The call's
  * tensors must not alias: when the output overlaps an input or the residual, nothing is searched or recorded and the
@@ -307,7 +311,8 @@ int eddlhip_conv2d_tuned_load(int dev, const char *host_path);
  * (1 = none).  tile = 4: the Winograd form wherever it applies (its product launch is planned or searched as usual),
  * 5: its folded form wherever that applies, 6 / 7: its one-launch form on tiles of 32 / 64 filters x 32 blocks, `slices`
  * K slices for the left-over tiles as above; 8 / 9: the upsampled-input form of a 2x2 filter, built for three / two
- * workgroups per CU; 16 .. 19: the split form on tiles of 128x128, 128x64, 64x128, 64x64 outputs; the planner's choice
+ * workgroups per CU; 16 .. 19: the split form on tiles of 128x128, 128x64, 64x128, 64x64 outputs; 32: the one-launch Winograd
+ * form in the split arithmetic on tiles of 64 filters x 32 blocks; the planner's choice
  * wherever a form does not apply.  Acts on the calling thread only. */
 int eddlhip_conv2d_force_plan(int tile, int slices);
 

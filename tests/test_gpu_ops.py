@@ -1440,3 +1440,163 @@ def test_conv2d_search_keeps_only_the_filter_copy_of_its_plan(hip, tmp_path, ker
     finally:
         hip.conv_autotune(-1)
         hip.uncache_conv_filters(Wd)
+
+
+# ------------------------------------------------------------------ the one-launch Winograd form in the split arithmetic
+# N C H W Kf pads(top, left) output size: edges of the tile (64 filters x 32 blocks) and of an image, one K-step of 16 channels and
+# many, odd planes, single rows and columns of blocks, 16- and 4-byte pixel loads (rows of a multiple of four pixels, odd left padding)
+WSPLIT_CASES = {
+    "one block": (1, 16, 2, 2, 1, (1, 1), None),
+    "one pixel": (2, 32, 1, 1, 65, (1, 1), None),
+    "64 filters x 32 blocks": (2, 16, 8, 8, 64, (1, 1), None),
+    "33 blocks, 65 filters": (1, 48, 2, 66, 65, (1, 1), None),
+    "columns of one block": (3, 32, 37, 2, 40, (1, 1), None),
+    "odd planes": (3, 64, 13, 17, 70, (1, 1), None),
+    "no padding": (2, 32, 11, 20, 33, (0, 0), None),
+    "two and three columns of padding": (2, 32, 12, 24, 64, (2, 3), None),
+    "rows of six blocks": (5, 16, 6, 12, 64, (1, 1), None),
+    "rows cut by the output size": (2, 16, 10, 28, 16, (0, 1), (9, 25)),
+    "long K": (1, 512, 14, 16, 64, (1, 1), None),
+}
+
+
+def _conv64_padded(x, w, pad, P, Q):
+    """3x3, stride 1, in doubles: `pad` zeros above and to the left, as many below and to the right as P x Q outputs ask for."""
+    N, C, H, W = x.shape
+    big = np.zeros((N, C, P + 2, Q + 2))
+    rows, cols = min(H, P + 2 - pad[0]), min(W, Q + 2 - pad[1])
+    big[:, :, pad[0]:pad[0] + rows, pad[1]:pad[1] + cols] = x[:, :, :rows, :cols]
+    return _conv64(big, w, (1, 1), (0, 0), P, Q)
+
+
+@pytest.mark.parametrize("slices", [1, 3, 16])
+@pytest.mark.parametrize("case", sorted(WSPLIT_CASES))
+def test_conv2d_winograd_split_is_no_further_from_64_bits_than_the_fp32_one(hip, case, slices):
+    N, C, H, W, Kf, pad, out = WSPLIT_CASES[case]
+    P, Q = out or (H + 2 * pad[0] - 2, W + 2 * pad[1] - 2)
+    rng = np.random.default_rng(1900 + sorted(WSPLIT_CASES).index(case))
+    x = rng.standard_normal((N, C, H, W), dtype=np.float32)
+    w = (rng.standard_normal((Kf, C, 3, 3)) * np.sqrt(2.0 / (C * 9))).astype(np.float32)
+    X, Wd, O = hip.array(x), hip.array(w), hip.full((N, Kf, P, Q), np.nan)
+    try:
+        hip.force_conv_plan(7, 1)
+        hip.conv2D(X, Wd, None, O, 1, 1, *pad)
+        assert "wino_fused_kernel" in hip.last_conv_kernel()
+        fp32 = O.numpy()
+        hip.force_conv_plan(32, slices)
+        hip.fill_(O, np.nan)
+        hip.conv2D(X, Wd, None, O, 1, 1, *pad)
+        name = hip.last_conv_kernel()
+        assert "wino_split_kernel" in name and ("+ksplit" in name) == (slices > 1 and C > 16), name
+        assert ("true>" in name) == (W % 4 == 0 and pad[1] % 2 == 1 and Q > 10), name
+        got = O.numpy()
+        hip.cache_conv_filters(Wd)                      # from registered filters: the same bits
+        hip.fill_(O, np.nan)
+        hip.conv2D(X, Wd, None, O, 1, 1, *pad)
+        assert np.array_equal(got, O.numpy())
+        hip.uncache_conv_filters(Wd)
+    finally:
+        hip.force_conv_plan(-1, 1)
+    ref = _conv64_padded(x, w, pad, P, Q)
+    # (few outputs are decided by chance: the transforms round at least four times along a sum, 2^-24 of their terms each time)
+    floor = 2.0 ** -22 * np.linalg.norm(ref) if ref.size < 1000 else 0.0
+    assert np.linalg.norm(got - ref) <= max(np.linalg.norm(fp32 - ref), floor)
+    assert_conv_close(ref, got, case)
+
+
+@pytest.mark.parametrize("slices", [1, 2])
+def test_conv2d_winograd_split_reads_folded_inputs_applies_the_epilogue_and_pools(hip, slices):
+    """A folded Concat and a folded UpSampling give the bits of the stored tensor; epilogue and pool those of the separate calls."""
+    rng = np.random.default_rng(1990)
+    N, C, H, W, Kf = 2, 64, 6, 10, 72
+    a, b = rng.standard_normal((2, N, C // 2, H, W), dtype=np.float32)
+    w = (rng.standard_normal((Kf, C, 3, 3)) * 0.06).astype(np.float32)
+    bias = rng.standard_normal(Kf).astype(np.float32)
+    g, bb, mean = rng.uniform(0.8, 1.2, Kf).astype(np.float32), *(rng.standard_normal((2, Kf)) * 0.1).astype(np.float32)
+    var = rng.uniform(0.5, 1.5, Kf).astype(np.float32)
+    A, B, AB, Wd = hip.array(a), hip.array(b), hip.array(np.concatenate([a, b], 1)), hip.array(w)
+    up = hip.array(np.repeat(np.repeat(np.concatenate([a, b], 1), 2, 2), 3, 3))
+    try:
+        hip.force_conv_plan(32, slices)
+        O1, O2 = hip.empty((N, Kf, H, W)), hip.empty((N, Kf, H, W))
+        hip.conv2D(A, Wd, None, O1, 1, 1, 1, 1, second=B)
+        assert "wino_split_kernel" in hip.last_conv_kernel()
+        hip.conv2D(AB, Wd, None, O2, 1, 1, 1, 1)
+        assert np.array_equal(O1.numpy(), O2.numpy())
+        U1, U2 = hip.empty((N, Kf, 2 * H, 3 * W)), hip.empty((N, Kf, 2 * H, 3 * W))
+        hip.conv2D(AB, Wd, None, U1, 1, 1, 1, 1, upsample=(2, 3))
+        hip.conv2D(up, Wd, None, U2, 1, 1, 1, 1)
+        assert np.array_equal(U1.numpy(), U2.numpy())
+        res = rng.standard_normal((N, Kf, H, W), dtype=np.float32)
+        epilogue = dict(bn=tuple(hip.array(v) for v in (g, bb, mean, var)) + (1e-5,), residual=hip.array(res), relu=True)
+        E = hip.empty((N, Kf, H, W))
+        hip.conv2D(AB, Wd, hip.array(bias), E, 1, 1, 1, 1, **epilogue)
+        col = lambda v: v[None, :, None, None]
+        t = O2.numpy() + col(bias)
+        t = (t - col(mean)) / col(np.sqrt(var + np.float32(1e-5))) * col(g) + col(bb) + res
+        assert np.array_equal(E.numpy(), np.maximum(t, np.float32(0)))
+        want, got = ([hip.full((N, Kf, H // 2, W // 2), 9.0) for _ in range(3)] for _ in range(2))
+        hip.mpool2D(E, *want, (2, 2), (2, 2), (0, 0, 0, 0))
+        hip.conv2D(AB, Wd, hip.array(bias), O1, 1, 1, 1, 1, pool=tuple(got), keep=False, **epilogue)
+        assert all(np.array_equal(p.numpy(), q.numpy()) for p, q in zip(want, got))
+    finally:
+        hip.force_conv_plan(-1, 1)
+
+
+@pytest.mark.parametrize("slices", [1, 2])
+def test_conv2d_winograd_split_keeps_what_is_not_finite_and_the_largest_numbers(hip, slices):
+    """Infinities, NaN and numbers that round up to infinity in 16 bits, in the image and in a filter: what the fp32 kernel of this
+    form gives, and not a bit of a block whose patch holds none of them."""
+    rng = np.random.default_rng(1995)
+    N, C, H, W, Kf = 2, 32, 12, 12, 64
+    x = rng.standard_normal((N, C, H, W), dtype=np.float32)
+    w = (rng.standard_normal((Kf, C, 3, 3)) * 0.05).astype(np.float32)
+    clean_x = x.copy()
+    x[0, 3, 2, 2], x[0, 9, 8, 8], x[1, 0, 0, 0], x[1, 5, 6, 6] = np.inf, -np.inf, np.nan, 3.4e38
+    x[1, 7, 11, 11] = 1e-40
+    bad = w.copy()
+    bad[60, 2, 1, 1] = np.inf
+    O, C1 = hip.empty((N, Kf, H, W)), hip.empty((N, Kf, H, W))
+    X = hip.array(x)
+    try:
+        hip.force_conv_plan(7, slices)
+        hip.conv2D(X, hip.array(bad), None, O, 1, 1, 1, 1)
+        want = O.numpy()
+        assert np.isnan(want).any() and np.isfinite(want).any()
+        hip.force_conv_plan(32, slices)
+        hip.conv2D(X, hip.array(bad), None, O, 1, 1, 1, 1)
+        assert "wino_split_kernel" in hip.last_conv_kernel()
+        hip.conv2D(hip.array(clean_x), hip.array(w), None, C1, 1, 1, 1, 1)
+    finally:
+        hip.force_conv_plan(-1, 1)
+    got = O.numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    assert np.array_equal(np.isneginf(got), np.isneginf(want))
+    ok = np.isfinite(want)
+    assert np.allclose(got[ok], want[ok], rtol=1e-4, atol=1e-5)
+    # (a patch is four rows and columns from 2 ty - 1, 2 tx - 1 on)
+    touched = np.zeros((N, H // 2, W // 2), bool)
+    for n, y, v in ((0, 2, 2), (0, 8, 8), (1, 0, 0), (1, 6, 6), (1, 11, 11)):
+        touched[n, max(0, (y - 1) // 2):(y + 1) // 2 + 1, max(0, (v - 1) // 2):(v + 1) // 2 + 1] = True
+    clean = np.broadcast_to(~np.repeat(np.repeat(touched, 2, 1), 2, 2)[:, None], got.shape).copy()
+    clean[:, 60] = False
+    assert np.array_equal(got[clean], C1.numpy()[clean])
+
+
+@pytest.mark.parametrize("e_pixels,e_filters", [(-112, 90), (90, -112), (-126, 100), (100, -120), (-140, 100), (-60, -60), (110, -60), (-60, 110), (40, 45), (60, 60)])
+def test_conv2d_winograd_split_keeps_24_bits_of_small_and_large_numbers(hip, e_pixels, e_filters):
+    """Pixels or filters anywhere in the fp32 range: no further from 64 bits than the fp32 kernel of this form."""
+    rng = np.random.default_rng(1997)
+    N, C, H, W, Kf = 1, 64, 10, 12, 70
+    x, w = _small_or_large(rng, (N, C, H, W), e_pixels), _small_or_large(rng, (Kf, C, 3, 3), e_filters)
+    O, err = hip.full((N, Kf, H, W), np.nan), {}
+    ref = _conv64_padded(x, w, (1, 1), H, W)
+    try:
+        for plan in (7, 32):
+            hip.force_conv_plan(plan, 1)
+            hip.conv2D(hip.array(x), hip.array(w), None, O, 1, 1, 1, 1)
+            assert ("wino_split_kernel" in hip.last_conv_kernel()) == (plan == 32)
+            err[plan] = np.linalg.norm(O.numpy() - ref) / np.linalg.norm(ref)
+    finally:
+        hip.force_conv_plan(-1, 1)
+    assert err[32] <= max(err[7], 2.0 ** -22), err

@@ -2226,6 +2226,7 @@ __global__ __launch_bounds__(256) void wino_fused_reduce_kernel(const ConvParams
 
 #include "conv_split.h"
 #include "wino_split.h"
+#include "conv_up_split.h"
 
 // ---------------------------------------------------------------- host side
 int g_algo = 0;
@@ -2355,8 +2356,24 @@ const Variant ksplit[] = {SPLIT(2, 2, 2, 2, 2), SPLIT(4, 1, 1, 2, 3), SPLIT(2, 2
 constexpr int NUM_SPLIT = (int)(sizeof(ksplit) / sizeof(ksplit[0]));
 constexpr int SPLIT_TILE0 = 16;
 bool is_split_tile(int tile) { return tile >= SPLIT_TILE0 && tile < SPLIT_TILE0 + NUM_SPLIT; }
-bool is_plan_tile(int tile) { return (tile >= -1 && tile < NUM_PLAN_TILES) || is_split_tile(tile) || is_wsplit_tile(tile); }
+// The upsampled-input form in the split arithmetic (conv_up_split.h): plan "tiles" 33 (128 filters x 64 blocks) and 34 (64 x 128, half
+// of a 128-filter tile would idle under 64 filters).  Measured, us, the best of the fp32 and of the direct split plans before -> this
+// (4 images, stored side x channels -> filters): 32 x 1024 -> 512 314 -> 203, 64 x 512 -> 256 280 -> 179, 128 x 256 -> 128 288 -> 182 (34: 192),
+// 256 x 128 -> 64 314 -> 225 (33: 339); 1 image: 23 x 1024 -> 512 67 -> 57, 184 x 128 -> 64 62 -> 42.
+struct UpSplitVariant {
+    const char *name;
+    int fm, fn;  // filters and blocks of a workgroup over 32
+    void (*kernel)(const ConvParams);
+    void (*reduce)(const ConvParams);
+};
+const UpSplitVariant kupsplit[] = {{"conv_up2x2_split_kernel<4,1>", 4, 2, conv_up2x2_split_kernel<4, 1>, wino_fused_reduce_kernel<4, 2>},
+                                   {"conv_up2x2_split_kernel<2,2>", 2, 4, conv_up2x2_split_kernel<2, 2>, wino_fused_reduce_kernel<2, 4>}};
+constexpr int NUM_UPSPLIT = (int)(sizeof(kupsplit) / sizeof(kupsplit[0]));
+constexpr int UPSPLIT_TILE0 = WSPLIT_TILE0 + NUM_WSPLIT;
+bool is_upsplit_tile(int tile) { return tile >= UPSPLIT_TILE0 && tile < UPSPLIT_TILE0 + NUM_UPSPLIT; }
+bool is_plan_tile(int tile) { return is_upsplit_tile(tile) || (tile >= -1 && tile < NUM_PLAN_TILES) || is_split_tile(tile) || is_wsplit_tile(tile); }
 int split_steps(int C, int RS) { return (C + SPLIT_K - 1) / SPLIT_K * RS; }
+size_t upsplit_filter_bytes(int C, int Mp) { return (size_t)split_steps(C, 1) * 2 * (Mp / 32) * UPSPLIT_UNIT; }
 size_t split_filter_bytes(int C, int RS, int Mp) { return (size_t)split_steps(C, RS) * 2 * (Mp / 32) * SPLIT_UNIT; }
 // Whether the split form can run a convolution: filters within a buffer descriptor, and channels in whole groups of eight also
 // where a folded Concat has two tensors for them.
@@ -2366,9 +2383,9 @@ bool split_applies(int C, int Kf, int R, int S) {
 
 // K slices of the left-over tiles of a one-launch Winograd plan that asks for `slices` of them (T blocks in the launch):
 // the tiles beyond a whole number per CU are divided, as in forced_plan; 1 = nothing is divided
-int fused_slices(const FusedVariant &fv, int slices, long long T, int C, int Kf, int num_cu, long long *leftover_out = nullptr, int *slice_steps_out = nullptr) {
-    const int nsteps = (C + fv.ck - 1) / fv.ck;
-    const long long tiles = (long long)((Kf + 32 * fv.fm - 1) / (32 * fv.fm)) * ((T + 32 * fv.fn - 1) / (32 * fv.fn));
+int fused_slices(int fm, int fn, int ck, int slices, long long T, int C, int Kf, int num_cu, long long *leftover_out = nullptr, int *slice_steps_out = nullptr) {
+    const int nsteps = (C + ck - 1) / ck;
+    const long long tiles = (long long)((Kf + 32 * fm - 1) / (32 * fm)) * ((T + 32 * fn - 1) / (32 * fn));
     const long long leftover = tiles % num_cu;
     const int want = slices < 1 ? 1 : (slices > nsteps ? nsteps : slices);
     int slice_steps = (nsteps + want - 1) / want;
@@ -2378,6 +2395,9 @@ int fused_slices(const FusedVariant &fv, int slices, long long T, int C, int Kf,
     if (leftover_out) *leftover_out = nslices > 1 ? leftover : 0;
     if (slice_steps_out) *slice_steps_out = slice_steps;
     return nslices;
+}
+int fused_slices(const FusedVariant &fv, int slices, long long T, int C, int Kf, int num_cu, long long *leftover_out = nullptr, int *slice_steps_out = nullptr) {
+    return fused_slices(fv.fm, fv.fn, fv.ck, slices, T, C, Kf, num_cu, leftover_out, slice_steps_out);
 }
 
 // Launch plan: tile shape and, for the tiles that do not divide evenly over the CUs, the number
@@ -2494,6 +2514,7 @@ struct CachedFilters {
     int fused_rows;
     void *Wwsplit;  // 3x3 filters: the transformed filters as three bf16 parts (wino_split_filter_kernel), made on first use
     void *Wsplit;  // the filters as three bf16 parts in the operand order of the split form (split_filter_kernel), made on first use
+    void *Wupsplit;  // 2x2 filters: those rows as three bf16 parts (up2x2_split_filter_kernel), made on first use
     float *Wup;  // 2x2 filters: the nine weight-sum rows per channel of the upsampled-input form [C][9][Mp] (up2x2_filter_kernel), made on first use
     bool stale;  // K was written through this library since the last repack
 };
@@ -2526,6 +2547,14 @@ int launch_wino_split_filters(int dev, const float *K, void *Ws, int Kf, int C, 
     return 0;
 }
 
+int launch_up_split_filters(int dev, const float *K, void *Ws, int Kf, int C, int Mp) {
+    const int mblocks = Mp / 32, k16s = split_steps(C, 1) * 2;
+    hipLaunchKernelGGL(up2x2_split_filter_kernel, dim3((unsigned)(((size_t)k16s * mblocks * 64 + 255) / 256)), dim3(256), 0, state(dev).stream, K, (uintx4 *)Ws, Kf, C,
+                       mblocks, k16s);
+    EH_CHECK_LAUNCH();
+    return 0;
+}
+
 int repack(int dev, CachedFilters &e) {
     hipLaunchKernelGGL(pack_filters_kernel, dim3((e.rows + 31) / 32, e.Mp / 32), dim3(256), 0, state(dev).stream, e.K, e.Wp, e.Kf,
                        e.C * e.R * e.S, e.Mp, e.rows);
@@ -2545,6 +2574,7 @@ int repack(int dev, CachedFilters &e) {
         hipLaunchKernelGGL(up2x2_filter_kernel, dim3((unsigned)(((size_t)e.C * e.Mp + 255) / 256)), dim3(256), 0, state(dev).stream, e.K, e.Wup, e.Kf, e.C, e.Mp);
         EH_CHECK_LAUNCH();
     }
+    if (e.Wupsplit != nullptr) EH_TRY(launch_up_split_filters(dev, e.K, e.Wupsplit, e.Kf, e.C, e.Mp));
     if (e.Wsplit != nullptr) EH_TRY(launch_split_filters(dev, e.K, e.Wsplit, e.Kf, e.C, e.R * e.S, e.Mp));
     if (e.Wwsplit != nullptr) EH_TRY(launch_wino_split_filters(dev, e.K, e.Wwsplit, e.Kf, e.C, e.Mp));
     e.stale = false;
@@ -2553,7 +2583,7 @@ int repack(int dev, CachedFilters &e) {
 
 // Which of the forms' own copies a registered filter tensor has (none if it is not registered).
 struct FilterCopies {
-    bool wino, fused, up, split, wsplit;
+    bool wino, fused, up, split, wsplit, upsplit;
 };
 CachedFilters *registered_filters(int dev, const float *K, int Kf, int C, int R, int S) {
     for (CachedFilters &e : g_cache[dev])
@@ -2563,8 +2593,8 @@ CachedFilters *registered_filters(int dev, const float *K, int Kf, int C, int R,
 FilterCopies copies_held(int dev, const float *K, int Kf, int C, int R, int S) {
     std::lock_guard<std::mutex> lock(g_cache_mutex);
     const CachedFilters *e = registered_filters(dev, K, Kf, C, R, S);
-    if (e == nullptr) return {false, false, false, false, false};
-    return {e->Wwino != nullptr, e->Wfused != nullptr, e->Wup != nullptr, e->Wsplit != nullptr, e->Wwsplit != nullptr};
+    if (e == nullptr) return {false, false, false, false, false, false};
+    return {e->Wwino != nullptr, e->Wfused != nullptr, e->Wup != nullptr, e->Wsplit != nullptr, e->Wwsplit != nullptr, e->Wupsplit != nullptr};
 }
 // Frees the copies that a tensor has beyond `keep` (what a plan search made for forms that it did not keep).
 int drop_copies(int dev, const float *K, int Kf, int C, int R, int S, const FilterCopies &keep) {
@@ -2584,6 +2614,7 @@ int drop_copies(int dev, const float *K, int Kf, int C, int R, int S, const Filt
     EH_TRY(drop(e->Wfused, keep.fused));
     EH_TRY(drop(e->Wup, keep.up));
     EH_TRY(drop(e->Wwsplit, keep.wsplit));
+    EH_TRY(drop(e->Wupsplit, keep.upsplit));
     return drop(e->Wsplit, keep.split);
 }
 
@@ -2629,6 +2660,7 @@ void conv_filters_released(int dev, const void *base, size_t bytes) {
             if (c[i].Wup) (void)hipFree(c[i].Wup);
             if (c[i].Wsplit) (void)hipFree(c[i].Wsplit);
             if (c[i].Wwsplit) (void)hipFree(c[i].Wwsplit);
+            if (c[i].Wupsplit) (void)hipFree(c[i].Wupsplit);
             c[i] = c.back();
             c.pop_back();
         } else {
@@ -2666,6 +2698,7 @@ int eddlhip_conv2d_cache_filters(int dev, const float *K, int Kf, int C, int R, 
     e.Wup = nullptr;
     e.Wsplit = nullptr;
     e.Wwsplit = nullptr;
+    e.Wupsplit = nullptr;
     e.stale = true;
     EH_REQUIRE((size_t)e.rows * e.Mp * sizeof(float) < ((size_t)1 << 31),
                "conv2d_cache_filters: the repacked filter matrix (%d taps x %d channels) exceeds the 2 GiB a buffer descriptor covers", e.rows, e.Mp);
@@ -2695,6 +2728,7 @@ int eddlhip_conv2d_uncache_filters(int dev, const float *K) {
             if (c[i].Wup) EH_TRY_HIP(hipFree(c[i].Wup));
             if (c[i].Wsplit) EH_TRY_HIP(hipFree(c[i].Wsplit));
             if (c[i].Wwsplit) EH_TRY_HIP(hipFree(c[i].Wwsplit));
+            if (c[i].Wupsplit) EH_TRY_HIP(hipFree(c[i].Wupsplit));
             c[i] = c.back();
             c.pop_back();
         } else {
@@ -2707,8 +2741,8 @@ int eddlhip_conv2d_uncache_filters(int dev, const float *K) {
 int eddlhip_conv2d_force_plan(int tile, int slices) {
     EH_REQUIRE(is_plan_tile(tile),
                "conv2d_force_plan: tile is -1 (automatic), 0..3, 4 .. %d (the Winograd forms where they apply), %d, %d (a 2x2 filter on an input upsampled twice) "
-               "%d .. %d (the split form where it applies) or %d (the one-launch Winograd form in that arithmetic)",
-               UP2X2_TILE - 1, UP2X2_TILE, UP2X2_TILE + 1, SPLIT_TILE0, SPLIT_TILE0 + NUM_SPLIT - 1, WSPLIT_TILE0);
+               "%d .. %d (the split form where it applies) or %d, %d .. %d (the one-launch Winograd and the upsampled-input form in that arithmetic)",
+               UP2X2_TILE - 1, UP2X2_TILE, UP2X2_TILE + 1, SPLIT_TILE0, SPLIT_TILE0 + NUM_SPLIT - 1, WSPLIT_TILE0, UPSPLIT_TILE0, UPSPLIT_TILE0 + NUM_UPSPLIT - 1);
     g_force_tile = tile;
     g_force_slices = slices;
     return 0;
@@ -2860,7 +2894,7 @@ int conv2d_winograd_fused(const FusedVariant &fv, int slices, int dev, const flo
                           int N, int C, int H, int W, int Kf, int pad_top, int pad_left, int P, int Q, const float *bn_g, const float *bn_b,
                           const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu);
 
-int conv2d_up2x2(int variant, int dev, const float *I, const float *K, const float *bias, float *O, int N, int C, int H, int W, int Kf, int P, int Q, const float *bn_g,
+int conv2d_up2x2(int tile, int slices, int dev, const float *I, const float *K, const float *bias, float *O, int N, int C, int H, int W, int Kf, int P, int Q, const float *bn_g,
                  const float *bn_b, const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu);
 
 int conv2d_split(bool no_alloc, const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room);
@@ -2937,7 +2971,7 @@ size_t winograd_workspace(bool fold, int N, int C, int Kf, int fs, int P, int Q,
 // forms with a transformed input in memory; within a form fewer K slices first.  Returns 0 with *out filled, 1 when these tensors cannot be searched on (the output overlaps an
 // input: repeating the call would change what it reads), or minus the error code of a runtime failure.
 int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, long long chunk_pix, bool wino_ok, bool fold_ok, bool fused_ok, bool up_ok,
-                bool split_ok, bool wsplit_ok, TunedPlan *out) {
+                bool split_ok, bool wsplit_ok, bool upsplit_ok, TunedPlan *out) {
     {
         const size_t out_bytes = (size_t)c.N * c.Kf * c.P * c.Q * 4, in_bytes = (size_t)c.N * (c.I2 ? c.C / 2 : c.C) * c.H * c.W * 4;
         const char *o_lo = (const char *)c.O, *o_hi = o_lo + out_bytes;
@@ -3006,6 +3040,16 @@ int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, l
         time_plan(1, UP2X2_TILE, 1);
         time_plan(2, UP2X2_TILE + 1, 1);
     }
+    if (upsplit_ok)  // ... in the split arithmetic
+        for (int v = 0; v < NUM_UPSPLIT; v++) {
+            int last_slices = 0;
+            for (int sl : kSearchSlices) {
+                const int ns = fused_slices(kupsplit[v].fm, kupsplit[v].fn, SPLIT_K, sl, (long long)c.N * ((c.P + 1) / 2) * ((c.Q + 1) / 2), c.C, c.Kf, num_cu);
+                if (ns == last_slices) continue;
+                last_slices = ns;
+                time_plan(3 + v, UPSPLIT_TILE0 + v, sl);
+            }
+        }
     if (fused_ok)  // the one-launch Winograd form: its tile shapes, each undivided and with the left-over tiles in K slices
         for (int fv = NUM_FUSED - 1; fv >= 0; fv--) {
             int last_slices = 0;
@@ -3235,8 +3279,9 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     // the upsampled-input form of a 2x2 filter: a geometry of its own in the plans table (kind 2 / 3), since the same
     // shapes on a stored tensor cannot take it
     const bool up_ok = !gemm && !no_alloc && g_algo == 0 && up2x2_applies(N, C, H, W, Kf, R, S, sr, sc, uh, uw, two, pad_top, pad_left, P, Q);
-    if (up_ok && (g_force_tile == UP2X2_TILE || g_force_tile == UP2X2_TILE + 1))
-        return conv2d_up2x2(g_force_tile - UP2X2_TILE, dev, I, K, bias, O, N, C, H, W, Kf, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
+    const bool upsplit_ok = up_ok && !g_wino_never && C % 16 == 0 && upsplit_filter_bytes(C, p.Mp) < ((size_t)1 << 31);
+    if ((up_ok && (g_force_tile == UP2X2_TILE || g_force_tile == UP2X2_TILE + 1)) || (upsplit_ok && is_upsplit_tile(g_force_tile)))
+        return conv2d_up2x2(g_force_tile, g_force_slices, dev, I, K, bias, O, N, C, H, W, Kf, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
     if (fused_ok && g_force_tile >= FUSED_TILE0 && g_force_tile < FUSED_TILE0 + NUM_FUSED)
         return conv2d_winograd_fused(kfused[g_force_tile - FUSED_TILE0], g_force_slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top,
                                      pad_left, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
@@ -3276,13 +3321,14 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
             memcpy(best.key, key, sizeof(key));
             const size_t ws_before = state(dev).workspace_bytes;
             FilterCopies keep = copies_held(dev, K, Kf, C, R, S);  // (those that other geometries' plans, and graphs, may use)
-            const int src = search_plan(call, family, plan, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, split_ok, wsplit_ok, &best);
+            const int src = search_plan(call, family, plan, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, split_ok, wsplit_ok, upsplit_ok, &best);
             if (src < 0) return -src;  // a runtime error inside the search
             if (src == 0) {
                 keep.wino = keep.wino || best.tile == 4 || best.tile == 5;
                 keep.fused = keep.fused || (best.tile >= FUSED_TILE0 && best.tile < FUSED_TILE0 + NUM_FUSED);
                 keep.up = keep.up || best.tile == UP2X2_TILE || best.tile == UP2X2_TILE + 1;
                 keep.split = keep.split || is_split_tile(best.tile);
+                keep.upsplit = keep.upsplit || is_upsplit_tile(best.tile);
                 keep.wsplit = keep.wsplit || is_wsplit_tile(best.tile);
             }
             if (!gemm) EH_TRY(drop_copies(dev, K, Kf, C, R, S, keep));
@@ -3297,8 +3343,8 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
         if (found != nullptr && ((found->tile == 4 && wino_ok) || (found->tile == 5 && fold_ok)))
             return conv2d_winograd(found->tile == 5, R, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top, pad_left, P, Q, bn_g,
                                    bn_b, bn_mean, bn_var, bn_eps, residual, relu);
-        if (found != nullptr && (found->tile == UP2X2_TILE || found->tile == UP2X2_TILE + 1) && up_ok)
-            return conv2d_up2x2(found->tile - UP2X2_TILE, dev, I, K, bias, O, N, C, H, W, Kf, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
+        if (found != nullptr && (((found->tile == UP2X2_TILE || found->tile == UP2X2_TILE + 1) && up_ok) || (is_upsplit_tile(found->tile) && upsplit_ok)))
+            return conv2d_up2x2(found->tile, found->slices, dev, I, K, bias, O, N, C, H, W, Kf, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
         if (found != nullptr && found->tile >= FUSED_TILE0 && found->tile < FUSED_TILE0 + NUM_FUSED && fused_ok)
             return conv2d_winograd_fused(kfused[found->tile - FUSED_TILE0], found->slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top, pad_left, P, Q, bn_g,
                                          bn_b, bn_mean, bn_var, bn_eps, residual, relu);
@@ -3609,69 +3655,91 @@ int conv2d_winograd(bool fold, int fs, int dev, const float *I, const float *I2,
 
 // A 2x2 convolution of an input upsampled twice, as four convolutions of the stored image (conv_up2x2_kernel; see
 // up2x2_filter_kernel).  Workspace: the nine filter rows per channel, unless a registered filter tensor keeps them.
-int conv2d_up2x2(int variant, int dev, const float *I, const float *K, const float *bias, float *O, int N, int C, int H, int W, int Kf, int P, int Q, const float *bn_g,
+int conv2d_up2x2(int tile, int slices, int dev, const float *I, const float *K, const float *bias, float *O, int N, int C, int H, int W, int Kf, int P, int Q, const float *bn_g,
                  const float *bn_b, const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu) {
     hipStream_t st = state(dev).stream;
     PoolRequest *const pool = (g_pool_req != nullptr && !g_tuning && P % 2 == 0 && Q % 2 == 0) ? g_pool_req : nullptr;
     if (pool != nullptr) pool->done = true;
     const int th = (P + 1) / 2, tw = (Q + 1) / 2;
-    const int T = N * th * tw, Tp = (T + 127) / 128 * 128;
+    const UpSplitVariant *const sv = is_upsplit_tile(tile) ? &kupsplit[tile - UPSPLIT_TILE0] : nullptr;
+    const int T = N * th * tw, Tp = sv ? T : (T + 127) / 128 * 128;
     const int Mp = (Kf + M_ALIGN - 1) / M_ALIGN * M_ALIGN;
-    const size_t u_floats = (size_t)9 * C * Mp;
-    const float *U = nullptr;
+    const size_t u_size = sv ? upsplit_filter_bytes(C, Mp) : (size_t)9 * C * Mp * sizeof(float);
+    long long leftover = 0;
+    int slice_steps = 0;
+    const int nslices = sv ? fused_slices(sv->fm, sv->fn, SPLIT_K, slices, T, C, Kf, state(dev).num_cu, &leftover, &slice_steps) : 1;
+    const size_t partial_bytes = sv ? (size_t)nslices * leftover * (32 * sv->fm) * (32 * sv->fn) * 4 * sizeof(float) : 0;
+    const void *U = nullptr;
     {
         std::lock_guard<std::mutex> lock(g_cache_mutex);
         for (CachedFilters &e : g_cache[dev]) {
             if (e.K == K && e.Kf == Kf && e.C == C && e.R == 2 && e.S == 2) {
-                if (e.Wup == nullptr && !state(dev).capturing) {
-                    if (hipMalloc((void **)&e.Wup, u_floats * sizeof(float)) != hipSuccess) {
-                        e.Wup = nullptr;
+                void *&kept = sv ? e.Wupsplit : (void *&)e.Wup;
+                if (kept == nullptr && !state(dev).capturing) {
+                    if (hipMalloc(&kept, u_size) != hipSuccess) {
+                        kept = nullptr;
                         (void)hipGetLastError();
                         break;  // no room to keep them: made per call
                     }
                     e.stale = true;
                 }
-                if (e.Wup != nullptr) {
+                if (kept != nullptr) {
                     if (e.stale) EH_TRY(repack(dev, e));
-                    U = e.Wup;
+                    U = kept;
                 }
                 break;
             }
         }
     }
+    const size_t u_bytes = U ? 0 : ((u_size + 255) & ~(size_t)255);
+    void *ws = nullptr;
+    if (u_bytes + partial_bytes > 0) EH_TRY(get_workspace(dev, u_bytes + partial_bytes, &ws));
     if (U == nullptr) {
-        void *ws = nullptr;
-        EH_TRY(get_workspace(dev, u_floats * sizeof(float), &ws));
-        hipLaunchKernelGGL(up2x2_filter_kernel, dim3((unsigned)(((size_t)C * Mp + 255) / 256)), dim3(256), 0, st, K, (float *)ws, Kf, C, Mp);
-        EH_CHECK_LAUNCH();
-        U = (const float *)ws;
+        if (sv) {
+            EH_TRY(launch_up_split_filters(dev, K, ws, Kf, C, Mp));
+        } else {
+            hipLaunchKernelGGL(up2x2_filter_kernel, dim3((unsigned)(((size_t)C * Mp + 255) / 256)), dim3(256), 0, st, K, (float *)ws, Kf, C, Mp);
+            EH_CHECK_LAUNCH();
+        }
+        U = ws;
     }
     ConvParams q;
     memset(&q, 0, sizeof(q));
     q.I = I; q.I2 = I; q.Csplit = C; q.Cimg = C; q.uh = 1; q.uw = 1;
-    q.Wp = U; q.w_img_stride = 0; q.K = K; q.O = O;
+    q.Wp = (const float *)U; q.w_img_stride = 0; q.K = K; q.O = O;
     q.bias = bias; q.bn_g = bn_g; q.bn_b = bn_b; q.bn_mean = bn_mean; q.bn_var = bn_var; q.residual = residual;
     q.bn_eps = bn_eps; q.relu = relu;
     q.N = N; q.C = C; q.H = H; q.W = W; q.Kf = Kf; q.R = 2; q.S = 2; q.sr = 1; q.sc = 1; q.P = 1; q.Q = Tp;
     q.CRS = 4 * C; q.Mp = Mp; q.PQ = Tp; q.npix = Tp;
-    q.gm = (Kf + 63) / 64; q.gn = Tp / 128;
+    const int bm = sv ? 32 * sv->fm : 64, bn = sv ? 32 * sv->fn : 128;
+    q.gm = (Kf + bm - 1) / bm; q.gn = (Tp + bn - 1) / bn;
     q.in_bytes = (unsigned)((size_t)N * C * H * W * sizeof(float));
-    q.wp_bytes = (unsigned)(u_floats * sizeof(float));
-    q.main_tiles = q.gm * q.gn; q.nslices = 1;
+    q.wp_bytes = (unsigned)u_size;
+    q.main_tiles = (int)((long long)q.gm * q.gn - leftover); q.nslices = nslices;
+    q.partial = (float *)((char *)ws + u_bytes);
     q.wth = th; q.wtw = tw; q.wT = T; q.wP = P; q.wQ = Q; q.wps = 3;
     if (pool != nullptr) {
         q.pool_O = pool->O; q.pool_ix = pool->ix; q.pool_iy = pool->iy;
         if (!pool->keep) q.O = nullptr;
     }
     EH_REQUIRE((long long)q.gm * q.gn <= 0x3fffffffLL, "conv2d: internal error, launch of the upsampled 2x2 form");
-    q.nsteps = C / 4;
-    q.slice_steps = q.nsteps;
+    q.nsteps = sv ? split_steps(C, 1) : C / 4;
+    q.slice_steps = sv ? slice_steps : q.nsteps;
+    const long long wgs = q.main_tiles + leftover * nslices;
+    if (sv) q.trace = (g_trace != nullptr && wgs <= g_trace_wgs) ? g_trace : nullptr;
     EH_TRY(prof_begin(st));
-    if (variant == 0) hipLaunchKernelGGL(conv_up2x2_kernel<3>, dim3((unsigned)q.main_tiles), dim3(256), 0, st, q);
+    if (sv) hipLaunchKernelGGL(sv->kernel, dim3((unsigned)wgs), dim3(256), 0, st, q);
+    else if (tile == UP2X2_TILE) hipLaunchKernelGGL(conv_up2x2_kernel<3>, dim3((unsigned)q.main_tiles), dim3(256), 0, st, q);
     else hipLaunchKernelGGL(conv_up2x2_kernel<2>, dim3((unsigned)q.main_tiles), dim3(256), 0, st, q);
     EH_CHECK_LAUNCH();
     EH_TRY(prof_end(st));
-    snprintf(g_last_kernel, sizeof(g_last_kernel), "upsampled2x2[conv_up2x2_kernel<%d>, %d blocks]", variant == 0 ? 3 : 2, Tp);
+    if (leftover > 0) {
+        hipLaunchKernelGGL(sv->reduce, dim3((unsigned)(leftover * sv->fm * sv->fn)), dim3(256), 0, st, q);
+        EH_CHECK_LAUNCH();
+    }
+    if (leftover > 0) snprintf(g_last_kernel, sizeof(g_last_kernel), "upsampled2x2[%s +ksplit(%lld tiles x %d), %d blocks]", sv->name, leftover, nslices, Tp);
+    else if (sv) snprintf(g_last_kernel, sizeof(g_last_kernel), "upsampled2x2[%s, %d blocks]", sv->name, Tp);
+    else snprintf(g_last_kernel, sizeof(g_last_kernel), "upsampled2x2[conv_up2x2_kernel<%d>, %d blocks]", tile == UP2X2_TILE ? 3 : 2, Tp);
     return 0;
 }
 

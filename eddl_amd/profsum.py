@@ -208,7 +208,7 @@ def mfma(workload, directory, out):
         m = mean(mops[probe[0]])
         o += ["SQ_INSTS_VALU_MFMA_MOPS_F32 counts fp32 matrix operations in units of 512 flops: the pure-MFMA probe kernel of the same run",
               "(mfma_f32_probe_kernel, 1.0737e12 flops per launch by construction) reads %.4g, i.e. %.1f flops per count." % (m, 1.0737e12 / m)]
-    o += ["conv_split_kernel, wino_split_kernel: SQ_INSTS_VALU_MFMA_MOPS_BF16 in the same unit, %%peak against the bf16 instruction's %.0f TFLOP/s; six bf16" % BF16_MFMA_PEAK_TFLOPS,
+    o += ["conv_split, wino_split and conv_up2x2_split kernels: SQ_INSTS_VALU_MFMA_MOPS_BF16 in the same unit, %%peak against the bf16 instruction's %.0f TFLOP/s; six bf16" % BF16_MFMA_PEAK_TFLOPS,
           "products are one fp32 product, so a sixth of its exec GFLOP and TFLOP/s are those of fp32 work.",
           "columns: calls = dispatches; avg us = mean of End_Timestamp - Start_Timestamp in THIS run (kernels run a few % slower while",
           "counters are collected); exec GFLOP = mean SQ_INSTS_VALU_MFMA_MOPS_F32 per dispatch x 512 / 1e9 (includes the zero taps of a",
@@ -218,10 +218,10 @@ def mfma(workload, directory, out):
           "",
           "%-88s %6s %9s %12s %9s %7s %7s %6s" % ("kernel", "calls", "avg us", "exec GFLOP", "TFLOP/s", "%peak", "busy %", "GHz")]
     for k in mops:
-        if not any(t in k for t in ("conv_tap", "conv_gen", "conv_split", "conv_pointwise", "wino_fused_kernel", "wino_split_kernel", "dense_partial", "mfma_f32_probe")):
+        if not any(t in k for t in ("conv_tap", "conv_gen", "conv_split", "conv_pointwise", "wino_fused_kernel", "wino_split_kernel", "conv_up2x2_split", "dense_partial", "mfma_f32_probe")):
             continue
         us = mean(dur[k])
-        split = "conv_split" in k or "wino_split" in k
+        split = any(t in k for t in ("conv_split", "wino_split", "up2x2_split"))
         fl = mean((bf16 if split else mops)[k]) * 512.0
         peak = BF16_MFMA_PEAK_TFLOPS if split else FP32_MFMA_PEAK_TFLOPS
         cyc = mean(gui[k]) / 8.0

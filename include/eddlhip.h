@@ -267,7 +267,9 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * The one-launch Winograd form in that arithmetic (force_plan(32, .), or the search from 512 blocks of outputs on; channel counts
  * that are multiples of 16): transformed pixels and filters are fp32 numbers as in the third Winograd form, their products and
  * sums those of the split form, so its error is below that form's too.  Non-finite inputs as in the Winograd forms.  Its filters take
- * 96 bytes per filter and channel.
+ * 96 bytes per filter and channel.  Likewise the upsampled-input form of a 2x2 filter (force_plan(33, .) / (34, .) on tiles of 128
+ * filters x 64 or 64 x 128 stored pixels, `slices` K slices for the left-over tiles, or the search; channel counts that are
+ * multiples of 16; 54 bytes per filter and channel).  Neither under set_algo(9).
  *
  * eddlhip_conv2d_last_kernel() names the kernel the calling thread's last eddlhip_conv2d_fwd
  * launched, followed by " +ksplit(T tiles x S)" when T tiles were divided into S slices; for the Winograd form
@@ -312,7 +314,7 @@ int eddlhip_conv2d_tuned_load(int dev, const char *host_path);
  * 5: its folded form wherever that applies, 6 / 7: its one-launch form on tiles of 32 / 64 filters x 32 blocks, `slices`
  * K slices for the left-over tiles as above; 8 / 9: the upsampled-input form of a 2x2 filter, built for three / two
  * workgroups per CU; 16 .. 19: the split form on tiles of 128x128, 128x64, 64x128, 64x64 outputs; 32: the one-launch Winograd
- * form in the split arithmetic on tiles of 64 filters x 32 blocks; the planner's choice
+ * form in the split arithmetic on tiles of 64 filters x 32 blocks, 33 / 34: the upsampled-input form in it; the planner's choice
  * wherever a form does not apply.  Acts on the calling thread only. */
 int eddlhip_conv2d_force_plan(int tile, int slices);
 

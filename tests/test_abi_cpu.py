@@ -98,8 +98,9 @@ def test_plans_of_the_split_form_are_accepted(tmp_path):
     lib.eddlhip_conv2d_autotune(-1)
 
 
-def test_plan_of_the_winograd_split_form_is_accepted(tmp_path):
-    """Plan number 32 names the one-launch Winograd form in the split arithmetic, 24 .. 31 and 33 nothing; the benchmark knows it."""
+def test_plans_of_the_other_forms_in_the_split_arithmetic_are_accepted(tmp_path):
+    """Plan numbers 32 and 33, 34 name the one-launch Winograd and the upsampled-input form in the split arithmetic, their neighbours
+    nothing; the benchmark knows them."""
     sys.path.insert(0, ROOT)
     import bench
     from eddl_amd import _lib
@@ -108,13 +109,14 @@ def test_plan_of_the_winograd_split_form_is_accepted(tmp_path):
     path = tmp_path / "plans.txt"
     for tile in range(24, 40):
         path.write_text("4 128 64 3 3 1 1 %d 28 1 | %d 2\n" % (tile, tile))
-        assert (lib.eddlhip_conv2d_tuned_load(0, str(path).encode()) == 0) == (tile == 32), tile
-        assert (lib.eddlhip_conv2d_force_plan(tile, 1) == 0) == (tile == 32), tile
-        if tile != 32:
+        assert (lib.eddlhip_conv2d_tuned_load(0, str(path).encode()) == 0) == (32 <= tile <= 34), tile
+        assert (lib.eddlhip_conv2d_force_plan(tile, 1) == 0) == (32 <= tile <= 34), tile
+        if not 32 <= tile <= 34:
             with pytest.raises(ValueError):
                 bench.form_of_plan(tile)
     lib.eddlhip_conv2d_force_plan(-1, 1)
     lib.eddlhip_conv2d_autotune(-1)
+    assert bench.form_of_plan(33) == bench.form_of_plan(34) == "upsampled_2x2_split" and bench.peak_of_form("upsampled2x2_split") == bench.peak_of_form("split")
     assert bench.form_of_plan(32) == "winograd_split" and bench.peak_of_form("winograd_split") == bench.peak_of_form("split")
 
 

@@ -1600,3 +1600,125 @@ def test_conv2d_winograd_split_keeps_24_bits_of_small_and_large_numbers(hip, e_p
     finally:
         hip.force_conv_plan(-1, 1)
     assert err[32] <= max(err[7], 2.0 ** -22), err
+
+
+# ------------------------------------------------------------------ the upsampled-input form of a 2x2 filter in the split arithmetic
+# N C H W (stored) Kf output size or None (2H x 2W): edges of the tiles (64 and 128 filters and blocks), half a K-step of 32 channels and
+# many, odd planes, output sizes that cut rows off and that ask for more zeros
+UPSPLIT_CASES = {
+    "one pixel": (1, 16, 1, 1, 1, None),
+    "65 filters": (2, 32, 6, 6, 65, None),
+    "129 filters, odd plane": (3, 48, 5, 7, 129, (9, 13)),
+    "129 blocks": (1, 80, 3, 43, 64, None),
+    "more zeros": (2, 64, 4, 4, 40, (9, 10)),
+    "long K": (1, 512, 6, 10, 64, None),
+}
+
+
+def _conv64_upsampled(x, w, P, Q):
+    up = np.repeat(np.repeat(x, 2, 2), 2, 3)
+    big = np.zeros(x.shape[:2] + (P + 1, Q + 1))
+    rows, cols = min(up.shape[2], P + 1), min(up.shape[3], Q + 1)
+    big[:, :, :rows, :cols] = up[:, :, :rows, :cols]
+    return _conv64(big, w, (1, 1), (0, 0), P, Q)
+
+
+@pytest.mark.parametrize("plan", [(33, 1), (33, 3), (34, 1), (34, 16)])
+@pytest.mark.parametrize("case", sorted(UPSPLIT_CASES))
+def test_conv2d_upsampled_2x2_split_is_no_further_from_64_bits_than_the_fp32_one(hip, case, plan):
+    N, C, H, W, Kf, out = UPSPLIT_CASES[case]
+    P, Q = out or (2 * H, 2 * W)
+    rng = np.random.default_rng(2000 + sorted(UPSPLIT_CASES).index(case))
+    x = rng.standard_normal((N, C, H, W), dtype=np.float32)
+    w = (rng.standard_normal((Kf, C, 2, 2)) * np.sqrt(2.0 / (C * 4))).astype(np.float32)
+    X, Wd, O = hip.array(x), hip.array(w), hip.full((N, Kf, P, Q), np.nan)
+    run = lambda to, **more: hip.conv2D(X, Wd, None, to, 1, 1, 0, 0, upsample=(2, 2), **more)
+    try:
+        hip.force_conv_plan(UP2X2_FORM, 1)
+        run(O)
+        fp32 = O.numpy()
+        hip.force_conv_plan(*plan)
+        hip.fill_(O, np.nan)
+        run(O)
+        name = hip.last_conv_kernel()
+        assert name.startswith("upsampled2x2[conv_up2x2_split_kernel") and ("+ksplit" in name) == (plan[1] > 1 and C > 32), name
+        got = O.numpy()
+        hip.cache_conv_filters(Wd)                      # from registered filters, which follow a write
+        Wd.copy_from(2.0 * w)
+        run(O)
+        assert np.array_equal(O.numpy(), 2.0 * got)
+        Wd.copy_from(w)
+        # the epilogue and the pool: those of the separate calls
+        bias, g, bb, mean = (rng.standard_normal(Kf).astype(np.float32) for _ in range(4))
+        var, res = rng.uniform(0.5, 1.5, Kf).astype(np.float32), rng.standard_normal((N, Kf, P, Q), dtype=np.float32)
+        E = hip.full((N, Kf, P, Q), np.nan)
+        epilogue = dict(bn=tuple(hip.array(v) for v in (g, bb, mean, var)) + (1e-5,), residual=hip.array(res), relu=True)
+        hip.conv2D(X, Wd, hip.array(bias), E, 1, 1, 0, 0, upsample=(2, 2), **epilogue)
+        col = lambda v: v[None, :, None, None]
+        t = (got + col(bias) - col(mean)) / col(np.sqrt(var + np.float32(1e-5))) * col(g) + col(bb) + res
+        assert np.array_equal(E.numpy(), np.maximum(t, np.float32(0)))
+        if P % 2 == 0 and Q % 2 == 0:
+            want, pooled = ([hip.full((N, Kf, P // 2, Q // 2), 9.0) for _ in range(3)] for _ in range(2))
+            hip.mpool2D(O2 := hip.array(got), *want, (2, 2), (2, 2), (0, 0, 0, 0))
+            run(O2, pool=tuple(pooled), keep=False)
+            assert all(np.array_equal(p.numpy(), q.numpy()) for p, q in zip(want, pooled))
+    finally:
+        hip.force_conv_plan(-1, 1)
+        hip.uncache_conv_filters(Wd)
+    ref = _conv64_upsampled(x, w, P, Q)
+    # (few outputs are decided by chance: a weight sum rounds up to three times, a sum of products at least twice, 2^-24 each)
+    floor = 2.0 ** -22 * np.linalg.norm(ref) if ref.size < 1000 else 0.0
+    assert np.linalg.norm(got - ref) <= max(np.linalg.norm(fp32 - ref), floor)
+    assert_conv_close(ref, got, case)
+
+
+@pytest.mark.parametrize("plan", [(33, 1), (34, 2)])
+def test_conv2d_upsampled_2x2_split_keeps_what_is_not_finite_and_the_largest_numbers(hip, plan):
+    """What the fp32 kernel of this form gives, and not a bit of an output whose pixels are finite."""
+    rng = np.random.default_rng(2095)
+    N, C, H, W, Kf = 2, 64, 7, 9, 72
+    clean = rng.standard_normal((N, C, H, W), dtype=np.float32)
+    x = clean.copy()
+    x[0, 3, 2, 2], x[0, 9, 5, 7], x[1, 0, 0, 0], x[1, 5, 4, 4] = np.inf, -np.inf, np.nan, 3.4e38
+    x[1, 7, 6, 8] = 1e-40
+    w = (rng.standard_normal((Kf, C, 2, 2)) * 0.05).astype(np.float32)
+    Wd, O, C1 = hip.array(w), hip.empty((N, Kf, 2 * H, 2 * W)), hip.empty((N, Kf, 2 * H, 2 * W))
+    try:
+        hip.force_conv_plan(UP2X2_FORM, 1)
+        hip.conv2D(hip.array(x), Wd, None, O, 1, 1, 0, 0, upsample=(2, 2))
+        want = O.numpy()
+        hip.force_conv_plan(*plan)
+        hip.conv2D(hip.array(x), Wd, None, O, 1, 1, 0, 0, upsample=(2, 2))
+        assert "conv_up2x2_split" in hip.last_conv_kernel()
+        hip.conv2D(hip.array(clean), Wd, None, C1, 1, 1, 0, 0, upsample=(2, 2))
+    finally:
+        hip.force_conv_plan(-1, 1)
+    got = O.numpy()
+    assert np.isinf(want).any() and np.isnan(want).any()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    assert np.array_equal(np.isneginf(got), np.isneginf(want))
+    ok = np.isfinite(want)
+    assert np.allclose(got[ok], want[ok], rtol=1e-4, atol=1e-5)
+    # output (p, q) reads stored rows p / 2 .. (p + 1) / 2 and columns likewise
+    seen = np.zeros((N, Kf, 2 * H, 2 * W), bool)
+    for n, y, v in ((0, 2, 2), (0, 5, 7), (1, 0, 0), (1, 4, 4), (1, 6, 8)):
+        seen[n, :, max(0, 2 * y - 1):2 * y + 2, max(0, 2 * v - 1):2 * v + 2] = True
+    assert np.array_equal(got[~seen], C1.numpy()[~seen])
+
+
+@pytest.mark.parametrize("e_pixels,e_filters", [(-112, 90), (90, -112), (-140, 100), (-60, -60), (110, -60), (-60, 110), (60, 60)])
+def test_conv2d_upsampled_2x2_split_keeps_24_bits_of_small_and_large_numbers(hip, e_pixels, e_filters):
+    """Pixels or filters anywhere in the fp32 range: no further from 64 bits than the fp32 kernel of this form."""
+    rng = np.random.default_rng(2097)
+    N, C, H, W, Kf = 1, 64, 5, 6, 70
+    x, w = _small_or_large(rng, (N, C, H, W), e_pixels), _small_or_large(rng, (Kf, C, 2, 2), e_filters)
+    O, err = hip.full((N, Kf, 2 * H, 2 * W), np.nan), {}
+    ref = _conv64_upsampled(x, w, 2 * H, 2 * W)
+    try:
+        for plan in (UP2X2_FORM, 33, 34):
+            hip.force_conv_plan(plan, 1)
+            hip.conv2D(hip.array(x), hip.array(w), None, O, 1, 1, 0, 0, upsample=(2, 2))
+            err[plan] = np.linalg.norm(O.numpy() - ref) / np.linalg.norm(ref)
+    finally:
+        hip.force_conv_plan(-1, 1)
+    assert max(err[33], err[34]) <= max(err[UP2X2_FORM], 2.0 ** -22), err

@@ -36,6 +36,14 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned &hi, unsig
     lo = split_round(ra - __builtin_bit_cast(float, mid << 16), rb - __builtin_bit_cast(float, mid & 0xffff0000u));
 }
 
+// The same of numbers that are known in 64 bits (transformed filters): the three parts, each rounded to nearest, hold 26 bits of them.
+__device__ __forceinline__ void split_pair(double a, double b, unsigned &hi, unsigned &mid, unsigned &lo) {
+    hi = split_round((float)a, (float)b);
+    const double ra = a - (double)__builtin_bit_cast(float, hi << 16), rb = b - (double)__builtin_bit_cast(float, hi & 0xffff0000u);
+    mid = split_round((float)ra, (float)rb);
+    lo = split_round((float)(ra - (double)__builtin_bit_cast(float, mid << 16)), (float)(rb - (double)__builtin_bit_cast(float, mid & 0xffff0000u)));
+}
+
 constexpr float SPLIT_UP = 16777216.0f;                    // 2^24, of pixels and filters
 constexpr float SPLIT_DOWN = 1.0f / SPLIT_UP / SPLIT_UP;   // of their products
 

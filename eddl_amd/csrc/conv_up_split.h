@@ -1,23 +1,20 @@
 // The 2x2 convolution of an image upsampled twice (conv_up2x2_kernel) in the split arithmetic of conv_split.h (included by conv.hip
-// only): the nine weight sums per filter and channel, added up in fp32 as there, and the stored pixels are split exactly into three
+// only): the nine weight sums per filter and channel, added up in 64 bits, and the stored pixels are split into three
 // bf16 numbers, the six largest products summed in one fp32 accumulator per output, the smallest first - six roundings per 16
-// channels and tap where the fp32 instruction makes eight.
+// channels and tap where the fp32 instruction makes eight.  What the instruction's rounding downwards adds to every sum
+// cancels as in wino_split.h: opposite signs in the middle half of the steps, and for the outputs (0,1) and (1,0) of a block.
 
 constexpr int UPSPLIT_UNIT = 9 * SPLIT_UNIT;  // bytes of 32 filters x 16 channels, all nine weight sums
 
 // Weight sum `row` (up2x2_filter_kernel's numbering) of the 2x2 filter at k.
-__device__ __forceinline__ float up2x2_sum(const float *k, int row) {
-    const float w00 = k[0], w01 = k[1], w10 = k[2], w11 = k[3];
-    return row == 0   ? __fadd_rn(__fadd_rn(w00, w01), __fadd_rn(w10, w11))
-           : row == 1 ? __fadd_rn(w00, w10)
-           : row == 2 ? __fadd_rn(w01, w11)
-           : row == 3 ? __fadd_rn(w00, w01)
-           : row == 4 ? __fadd_rn(w10, w11)
-                      : k[row - 5];
+template <typename T>
+__device__ __forceinline__ T up2x2_sum(const float *k, int row) {
+    const T w00 = k[0], w01 = k[1], w10 = k[2], w11 = k[3];
+    return row == 0 ? (w00 + w01) + (w10 + w11) : row == 1 ? w00 + w10 : row == 2 ? w01 + w11 : row == 3 ? w00 + w01 : row == 4 ? w10 + w11 : (T)k[row - 5];
 }
 
 // K[Kf][C][2][2] -> Ws[c / 16][Mp / 32][weight sum][part][lane][8], operands of the matrix instruction as in split_filter_kernel;
-// channels past C and filters past Kf are zeros.  Bound by the write (54 bytes per filter and channel).
+// channels past C and filters past Kf are zeros; the sums of the outputs (0,1) and (1,0) negated.  Bound by the write (54 bytes per filter and channel).
 __global__ __launch_bounds__(256) void up2x2_split_filter_kernel(const float *__restrict__ K, uintx4 *__restrict__ Ws, int Kf, int C, int mblocks, int k16s) {
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= (size_t)k16s * mblocks * 64) return;
@@ -27,6 +24,7 @@ __global__ __launch_bounds__(256) void up2x2_split_filter_kernel(const float *__
     uintx4 *dst = Ws + (size_t)unit * (9 * 192) + lane;
 #pragma unroll
     for (int row = 0; row < 9; row++) {
+        const double up = row >= 1 && row <= 4 ? -SPLIT_UP : SPLIT_UP;
         uintx4 hi, mid, lo;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -34,7 +32,7 @@ __global__ __launch_bounds__(256) void up2x2_split_filter_kernel(const float *__
             const float *k = K + ((size_t)(m < Kf ? m : 0) * C + (c < C ? c : 0)) * 4;  // (channels come in pairs: C is a multiple of 16)
             const bool ok = m < Kf && c < C;
             unsigned h, md, l;
-            split_pair(ok ? SPLIT_UP * up2x2_sum(k, row) : 0.0f, ok ? SPLIT_UP * up2x2_sum(k + 4, row) : 0.0f, h, md, l);
+            split_pair(ok ? up * up2x2_sum<double>(k, row) : 0.0, ok ? up * up2x2_sum<double>(k + 4, row) : 0.0, h, md, l);
             hi[q] = h;
             mid[q] = md;
             lo[q] = l;
@@ -60,7 +58,7 @@ __device__ __forceinline__ void up2x2_block_again(const ConvParams &p, floatx16 
         for (int t = 0; t < 4; t++) {
             if ((t & parity) != t) continue;  // (uniform: tap (t / 2, t % 2) is seen by the parities that have its bits)
             const int row = parity == 0 ? 0 : (parity == 1 ? 1 + t : (parity == 2 ? 3 + t / 2 : 5 + t));
-            const float a = up2x2_sum(k, row), b = buf_load(in, voff[t] == OOB ? OOB : voff[t] + c * HW4, 0);
+            const float a = up2x2_sum<float>(k, row), b = buf_load(in, voff[t] == OOB ? OOB : voff[t] + c * HW4, 0);
             sum = __builtin_amdgcn_mfma_f32_32x32x2f32(m < p.Kf ? a : 0.0f, b, sum, 0, 0, 0);
         }
     }
@@ -120,14 +118,16 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
             for (int j = 0; j < 8; j++, soff += HW4) raw[chunk][j] = buf_load(rsrc, voff[tap], soff);
         }
     };
-    auto put_pixels = [&](int buf) __attribute__((always_inline)) {
+    const SignOfStep sign(step_lo, step_hi);
+    auto put_pixels = [&](int buf, int step) __attribute__((always_inline)) {
+        const float up = sign.negative(step) ? -SPLIT_UP : SPLIT_UP;
 #pragma unroll
         for (int chunk = 0; chunk < CHUNKS; chunk++) {
             uintx4 hi, mid, lo;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 unsigned h, m, l;
-                split_pair(SPLIT_UP * raw[chunk][2 * j], SPLIT_UP * raw[chunk][2 * j + 1], h, m, l);
+                split_pair(up * raw[chunk][2 * j], up * raw[chunk][2 * j + 1], h, m, l);
                 hi[j] = h;
                 mid[j] = m;
                 lo[j] = l;
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
     load_a(0, 2 * step_lo, 0);
     ChannelEpilogue chan = {0.0f, 0.0f, 1.0f, 1.0f, 0.0f};
     if (!split) chan = fetch_channel_constants<BM>(p, m0, tid);
-    put_pixels(0);
+    put_pixels(0, step_lo);
     load_pixels(step_lo, 1);
     if (!split) put_channel_constants<BM>(epi, chan, tid);
 
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
                 acc[parity][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[set][kA[k]]), __builtin_bit_cast(bf16x8, b[tn][kB[k]]), acc[parity][tn], 0, 0, 0);
         if constexpr (G == 0 && S == 0) {
             // the next tap's pixels into the other buffer, those of the tap after it in their place
-            put_pixels((TAP & 1) ^ 1);
+            put_pixels((TAP & 1) ^ 1, TAP < 3 ? step : step + 1);
             load_pixels(TAP < 2 ? step : step + 1, (TAP + 2) & 3);
 #pragma unroll
             for (int i = 0; i < 12; i++) {
@@ -210,13 +210,18 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
         group(std::integral_constant<int, 1>());
         __syncthreads();
     };
-    for (int step = step_lo; step < step_hi; step++) {
-        const int next = step + 1 < step_hi ? step + 1 : step;
-        one_tap(step, next, std::integral_constant<int, 0>());
-        one_tap(step, next, std::integral_constant<int, 1>());
-        one_tap(step, next, std::integral_constant<int, 2>());
-        one_tap(step, next, std::integral_constant<int, 3>());
+    for (int run_lo = step_lo, run_hi; run_lo < step_hi; run_lo = run_hi) {  // (one to three runs of steps of one sign)
+        run_hi = sign.run_end(run_lo, step_hi);
+        for (int step = run_lo; step < run_hi; step++) {
+            const int next = step + 1 < step_hi ? step + 1 : step;
+            one_tap(step, next, std::integral_constant<int, 0>());
+            one_tap(step, next, std::integral_constant<int, 1>());
+            one_tap(step, next, std::integral_constant<int, 2>());
+            one_tap(step, next, std::integral_constant<int, 3>());
+        }
+        if (run_hi < step_hi) negate(acc);
     }
+    const float down = sign.negative(step_hi - 1) ? -SPLIT_DOWN : SPLIT_DOWN;
     trace_mark(p, 2);
 
     const int m_first = m0 + wm * 32 + (lane & 31);
@@ -229,7 +234,7 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
         for (int e = 0; e < 4; e++)
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                y[e >> 1][e & 1][v] = SPLIT_DOWN * acc[e][tn][v];
+                y[e >> 1][e & 1][v] = (e == 1 || e == 2 ? -down : down) * acc[e][tn][v];
                 finite = __builtin_fmaf(y[e >> 1][e & 1][v], 0.0f, finite);
             }
         if (__any(finite != 0.0f)) {

@@ -1,13 +1,19 @@
 // The one-launch Winograd form F(2x2, 3x3) on the bf16 matrix instructions (included by conv.hip only).  Loop order, tiles and
 // output transform are wino_fused_kernel's, the arithmetic of the products is conv_split.h's: the transformed pixels V = B^T d B
 // are computed in fp32 by the same operations, enlarged 2^24 times and split exactly into three bf16 numbers by the lane that
-// multiplies them; the transformed filters U are split once per registered filter tensor.  The six largest of the nine products
+// multiplies them; the filters are transformed in 64 bits and split once per registered filter tensor (an error in U is the same in
+// every pixel of a plane: rounded to fp32 as in the other Winograd forms it is what remains of theirs in a plane's mean).  The six largest of the nine products
 // of two such sums go into ONE fp32 accumulator, the smallest first: six roundings per 16 channels where the fp32 instruction
 // (two channels each) makes eight, so the error against 64 bits is below that form's (512 channels 5.8e-7 against 6.9e-7
-// relative in the 2-norm, 64 channels 2.1e-7 against 2.6e-7).  Sums that are not finite - infinities and NaN, and with the
+// relative in the 2-norm, 64 channels 2.1e-7 against 2.6e-7).  That instruction rounds what it shifts out on the way to an
+// accumulator downwards, not to nearest: 1.4e-8 of the outputs' root mean square for all sums of 512 channels, which the output
+// transform makes -9, 3, 3 and -1 times that of and no pool averages away (logits of ResNet-50, 16 images: 4.9e-7 from 64 bits, 4.2e-7
+// with the fp32 kernel).  So the middle half of a sum's steps is accumulated with the opposite sign, and so are the positions (i, j) of
+// odd i + j throughout: 4.2e-7.
+// Sums that are not finite - infinities and NaN, and with the
 // enlargement numbers from 2^104 and sums from 2^80 on - are computed with the fp32 instruction too and take that value.
 
-// K[Kf][C][3][3] -> Ws[c / 16][Mp / 32][position][part][lane][8]: the transformed filters U (wino_filter_kernel's operations) as
+// K[Kf][C][3][3] -> Ws[c / 16][Mp / 32][position][part][lane][8]: the transformed filters U = G g G^T, in 64 bits, as
 // operands of the matrix instruction: lane l holds filter l % 32 of the block, channels 8 (l / 32) .. + 7 of the 16.
 // C is a multiple of 16; filters past Kf are zeros.  Bound by the write (96 bytes per filter and channel).
 __global__ __launch_bounds__(256) void wino_split_filter_kernel(const float *__restrict__ K, uintx4 *__restrict__ Ws, int Kf, int C, int mblocks, int k16s) {
@@ -19,20 +25,17 @@ __global__ __launch_bounds__(256) void wino_split_filter_kernel(const float *__r
     uintx4 *dst = Ws + (size_t)unit * (16 * 192) + lane;
 #pragma unroll 1
     for (int i = 0; i < 4; i++) {  // a position row at a time: 4 x 8 values
-        float u[8][4];
+        double u[8][4];
 #pragma unroll
         for (int ch = 0; ch < 8; ch++) {
-            float g[9], t[3];
+            double g[9], t[3];
 #pragma unroll
-            for (int e = 0; e < 9; e++) g[e] = m < Kf ? K[((size_t)m * C + c0 + ch) * 9 + e] : 0.0f;
+            for (int e = 0; e < 9; e++) g[e] = m < Kf ? (double)SPLIT_UP * (double)K[((size_t)m * C + c0 + ch) * 9 + e] : 0.0;
 #pragma unroll
-            for (int j = 0; j < 3; j++)
-                t[j] = i == 0 ? g[j]
-                              : (i == 3 ? g[6 + j]
-                                        : __fmul_rn(0.5f, __fadd_rn(i == 1 ? __fadd_rn(g[j], g[3 + j]) : __fsub_rn(g[j], g[3 + j]), g[6 + j])));
+            for (int j = 0; j < 3; j++) t[j] = i == 0 ? g[j] : (i == 3 ? g[6 + j] : 0.5 * ((i == 1 ? g[j] + g[3 + j] : g[j] - g[3 + j]) + g[6 + j]));
             u[ch][0] = t[0];
-            u[ch][1] = __fmul_rn(0.5f, __fadd_rn(__fadd_rn(t[0], t[1]), t[2]));
-            u[ch][2] = __fmul_rn(0.5f, __fadd_rn(__fsub_rn(t[0], t[1]), t[2]));
+            u[ch][1] = 0.5 * (t[0] + t[1] + t[2]);
+            u[ch][2] = 0.5 * (t[0] - t[1] + t[2]);
             u[ch][3] = t[2];
         }
 #pragma unroll
@@ -41,7 +44,7 @@ __global__ __launch_bounds__(256) void wino_split_filter_kernel(const float *__r
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 unsigned h, md, l;
-                split_pair(SPLIT_UP * u[2 * q][j], SPLIT_UP * u[2 * q + 1][j], h, md, l);
+                split_pair(u[2 * q][j], u[2 * q + 1][j], h, md, l);
                 hi[q] = h;
                 mid[q] = md;
                 lo[q] = l;
@@ -51,6 +54,30 @@ __global__ __launch_bounds__(256) void wino_split_filter_kernel(const float *__r
             dst[(4 * i + j) * 192 + 128] = lo;
         }
     }
+}
+
+// The sign that the steps [lo, hi) of a sum are accumulated with: the first quarter and the last are added, what lies between is
+// subtracted from the negated sum, so that an error of one sign per step cancels, also one that grows with the steps linearly.
+struct SignOfStep {
+    int first, second;  // the sign changes in front of these steps
+    __device__ __forceinline__ SignOfStep(int lo, int hi) {
+        const int n = hi - lo;
+        // (below eight steps too little comes together to be worth the two negations: 64 channels 5 % of the time)
+        first = n < 8 ? hi : lo + (n + 2) / 4;
+        second = n < 8 ? hi : first + (n + 1) / 2;
+    }
+    __device__ __forceinline__ bool negative(int step) const { return step >= first && step < second; }
+    // the end of the run of steps of one sign that `step` is in
+    __device__ __forceinline__ int run_end(int step, int hi) const { return min(step < first ? first : (step < second ? second : hi), hi); }
+};
+template <int A, int B>
+__device__ __forceinline__ void negate(floatx16 (&sum)[A][B]) {
+#pragma unroll
+    for (int a = 0; a < A; a++)
+#pragma unroll
+        for (int b = 0; b < B; b++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) sum[a][b][v] = -sum[a][b][v];
 }
 
 constexpr int WSPLIT_UNIT = 16 * SPLIT_UNIT;  // bytes of 32 filters x 16 channels, all positions
@@ -231,6 +258,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int ra_off = half * 8 * SLOTS + my_base + ra * my_stride, rb_off = half * 8 * SLOTS + my_base + rb * my_stride;
     typedef const __attribute__((address_space(3))) floatx2 *lds_f2;
     uintx4 b[4][3];
+    const SignOfStep sign(step_lo, step_hi);
+    float up = ((wave & 1) != 0) != sign.negative(step_lo) ? -SPLIT_UP : SPLIT_UP;  // of the step whose operands are made (odd positions of a row: the other sign)
     float s1[8], s2[8], u3[8];  // what positions 2 and 3 are made of, from the turn of 0 and 1 to their own
     float d[2][2][4];           // [channel of a pair][patch row][column]
     auto read_pair = [&](const lds_float *rs, int q) __attribute__((always_inline)) {
@@ -256,7 +285,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         b[j][1][q] = m;
         b[j][2][q] = l;
     };
-    // positions 0 and 1 of a pair of channels: u0 - u2, u1 + u2
+    // positions 0 and 1 of a pair of channels: u0 - u2, -(u1 + u2)
     auto first = [&](int q) __attribute__((always_inline)) {
         float v[2][2];
 #pragma unroll
@@ -264,19 +293,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             float u[4];
 #pragma unroll
             for (int c = 0; c < 4; c++) u[c] = __builtin_fmaf(d[e][1][c], sgn, d[e][0][c]);
-            s1[2 * q + e] = SPLIT_UP * u[1];
-            s2[2 * q + e] = SPLIT_UP * u[2];
+            s1[2 * q + e] = up * u[1];
+            s2[2 * q + e] = up * u[2];
             u3[2 * q + e] = u[3];
-            v[0][e] = __builtin_fmaf(SPLIT_UP, u[0], -s2[2 * q + e]);
-            v[1][e] = __fadd_rn(s1[2 * q + e], s2[2 * q + e]);
+            v[0][e] = __builtin_fmaf(up, u[0], -s2[2 * q + e]);
+            v[1][e] = __fsub_rn(-s1[2 * q + e], s2[2 * q + e]);
         }
         put(0, q, v[0][0], v[0][1]);
         put(1, q, v[1][0], v[1][1]);
     };
-    // positions 2 and 3: u2 - u1, u1 - u3
+    // positions 2 and 3: u2 - u1, -(u1 - u3)
     auto second = [&](int q) __attribute__((always_inline)) {
         put(2, q, __fsub_rn(s2[2 * q], s1[2 * q]), __fsub_rn(s2[2 * q + 1], s1[2 * q + 1]));
-        put(3, q, __builtin_fmaf(-SPLIT_UP, u3[2 * q], s1[2 * q]), __builtin_fmaf(-SPLIT_UP, u3[2 * q + 1], s1[2 * q + 1]));
+        put(3, q, __builtin_fmaf(up, u3[2 * q], -s1[2 * q]), __builtin_fmaf(up, u3[2 * q + 1], -s1[2 * q + 1]));
     };
     constexpr int kA[6] = {2, 1, 1, 0, 0, 0}, kB[6] = {0, 1, 0, 2, 1, 0};
     auto multiply = [&](int j, int k) __attribute__((always_inline)) {  // product k of a position, the filters' smallest parts first
@@ -290,54 +319,63 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         first(q);
         if (q < 3) read_pair(rs_of(0), q + 1);
     }
-    for (int step = step_lo; step < step_hi; step++) {
-        const int cur = (step - step_lo) & 1;
-        const int next = step + 1 < step_hi ? step + 1 : step;
-        const lds_float *rs = rs_of(cur ^ 1);
+    for (int run_lo = step_lo, run_hi; run_lo < step_hi; run_lo = run_hi) {  // (one to three runs of steps of one sign)
+        run_hi = sign.run_end(run_lo, step_hi);
+        for (int step = run_lo; step < run_hi; step++) {
+            const int cur = (step - step_lo) & 1;
+            const int next = step + 1 < step_hi ? step + 1 : step;
+            const lds_float *rs = rs_of(cur ^ 1);
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (j == 2) {
-                // The next step's pixels were requested a step ago; of what was requested since then only this position's
-                // filters may still be on their way.  Behind the barrier nobody reads this step's pixels any more.
-                __builtin_amdgcn_s_waitcnt(0x0F70 | (3 * FM));
-                __syncthreads();
-                load_step(step + 2, rs_of(cur));
-                __builtin_amdgcn_sched_barrier(0);
-                read_pair(rs, 0);
-            }
-#pragma unroll
-            for (int h = 0; h < 2; h++) {  // half of a position's products
-                const int q = 2 * (j & 1) + h;
-#pragma unroll
-                for (int k = 3 * h; k < 3 * h + 3; k++) multiply(j, k);
-                if (j < 2) {
-                    second(q);
-                } else {
-                    first(q);
-                    if (q < 3) read_pair(rs, q + 1);
+            for (int j = 0; j < 4; j++) {
+                if (j == 2) {
+                    // The next step's pixels were requested a step ago; of what was requested since then only this position's
+                    // filters may still be on their way.  Behind the barrier nobody reads this step's pixels any more.
+                    __builtin_amdgcn_s_waitcnt(0x0F70 | (3 * FM));
+                    __syncthreads();
+                    load_step(step + 2, rs_of(cur));
+                    up = ((wave & 1) != 0) != sign.negative(step + 1) ? -SPLIT_UP : SPLIT_UP;
+                    __builtin_amdgcn_sched_barrier(0);
+                    read_pair(rs, 0);
                 }
-                const int js = j < 3 ? step : next, jn = (j + 1) & 3;
-                if (h == 0) load_a(2, js, jn), load_a(1, js, jn);
-                else load_a(0, js, jn);
 #pragma unroll
-                for (int t = 0; t < 3 * FM; t++) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    if (j < 2) __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
-                    else __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
-                    if (j >= 2 && q < 3 && (t == 1 || t == 2)) __builtin_amdgcn_sched_group_barrier(0x100, WIDE ? 6 : 4, 0);
-                    if (h == 0 && (t == FM || t == 3 * FM - 1)) __builtin_amdgcn_sched_group_barrier(0x020, FM, 0);
+                for (int h = 0; h < 2; h++) {  // half of a position's products
+                    const int q = 2 * (j & 1) + h;
+#pragma unroll
+                    for (int k = 3 * h; k < 3 * h + 3; k++) multiply(j, k);
+                    if (j < 2) {
+                        second(q);
+                    } else {
+                        first(q);
+                        if (q < 3) read_pair(rs, q + 1);
+                    }
+                    const int js = j < 3 ? step : next, jn = (j + 1) & 3;
+                    if (h == 0) load_a(2, js, jn), load_a(1, js, jn);
+                    else load_a(0, js, jn);
+#pragma unroll
+                    for (int t = 0; t < 3 * FM; t++) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        if (j < 2) __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+                        else __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+                        if (j >= 2 && q < 3 && (t == 1 || t == 2)) __builtin_amdgcn_sched_group_barrier(0x100, WIDE ? 6 : 4, 0);
+                        if (h == 0 && (t == FM || t == 3 * FM - 1)) __builtin_amdgcn_sched_group_barrier(0x020, FM, 0);
+                    }
+                    if (h == 1) __builtin_amdgcn_sched_group_barrier(0x020, FM, 0);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                if (h == 1) __builtin_amdgcn_sched_group_barrier(0x020, FM, 0);
-                __builtin_amdgcn_sched_barrier(0);
             }
         }
+        if (run_hi < step_hi) negate(acc);
     }
+    const float down = ((wave & 1) != 0) != sign.negative(step_hi - 1) ? -SPLIT_DOWN : SPLIT_DOWN;
     trace_mark(p, 2);
 
     // ---- output transform: along the position row in registers, across the rows through LDS
     const size_t plane = (size_t)p.wP * p.wQ;
+    // (the lane's number once more, so that nothing that follows from it lives through the loop: registers)
+    const unsigned lane_again = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    const int lane_e = (int)lane_again, l32_e = lane_e & 31, half_e = lane_e >> 5;
     const bool pair = (p.wQ % 2 == 0) && (((size_t)p.O | (size_t)(p.residual ? p.residual : p.O)) % 8 == 0);
-    floatx4 *xch = reinterpret_cast<floatx4 *>(&lds[0]);  // [filter group][position row][b][v / 4][lane] of v % 4
+    floatx4 *xch = reinterpret_cast<floatx4 *>(&lds[0]);  // [filter group][position row][b][v / 4][lane_e] of v % 4
     __builtin_amdgcn_s_waitcnt(0x0F70);                    // (the zeros behind the last step)
     __syncthreads();
     float finite = 0.0f;
@@ -350,14 +388,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             for (int k = 0; k < 4; k++) {
                 float m[4];
 #pragma unroll
-                for (int j = 0; j < 4; j++) m[j] = SPLIT_DOWN * acc[j][fm][4 * q + k];  // (the sums are 2^48 times too large)
+                for (int j = 0; j < 4; j++) m[j] = (j & 1 ? -down : down) * acc[j][fm][4 * q + k];  // (the sums are 2^48 times too large)
                 t[0][k] = __fadd_rn(__fadd_rn(m[0], m[1]), m[2]);
                 t[1][k] = __fsub_rn(__fsub_rn(m[1], m[2]), m[3]);
                 finite = __builtin_fmaf(t[0][k], 0.0f, finite);
                 finite = __builtin_fmaf(t[1][k], 0.0f, finite);
             }
 #pragma unroll
-            for (int b2 = 0; b2 < 2; b2++) xch[(((fm * 4 + wave) * 2 + b2) * 4 + q) * 64 + lane] = t[b2];
+            for (int b2 = 0; b2 < 2; b2++) xch[(((fm * 4 + wave) * 2 + b2) * 4 + q) * 64 + lane_e] = t[b2];
         }
     if (__any(finite != 0.0f)) {
         const __amdgpu_buffer_rsrc_t in1 = __builtin_amdgcn_make_buffer_rsrc((void *)p.I, 0, p.in_bytes, RSRC_WORD3);
@@ -368,47 +406,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll 1
             for (int j = 0; j < 4; j++) {
                 floatx16 sum;
-                wino_block_again(p, sum, in1, in2, m0 + fm * 32 + l32, n0 + l32, wave, j, step_lo * CK, step_hi * CK, half);
+                wino_block_again(p, sum, in1, in2, m0 + fm * 32 + l32_e, n0 + l32_e, wave, j, step_lo * CK, step_hi * CK, half_e);
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
                     const float x0 = j == 0 ? acc[0][0][v] : (j == 1 ? acc[1][0][v] : (j == 2 ? acc[2][0][v] : acc[3][0][v]));
                     const float x1 = j == 0 ? acc[0][1][v] : (j == 1 ? acc[1][1][v] : (j == 2 ? acc[2][1][v] : acc[3][1][v]));
-                    const float x = SPLIT_DOWN * (fm == 0 ? x0 : x1), m = x * 0.0f == 0.0f ? x : sum[v];
+                    const float x = (j & 1 ? -down : down) * (fm == 0 ? x0 : x1), m = x * 0.0f == 0.0f ? x : sum[v];
                     t0[v] = j == 0 ? m : (j == 3 ? t0[v] : __fadd_rn(t0[v], m));
                     t1[v] = j == 1 ? m : __fsub_rn(t1[v], m);
                 }
             }
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                xch[(((fm * 4 + wave) * 2 + 0) * 4 + q) * 64 + lane] = (floatx4){t0[4 * q], t0[4 * q + 1], t0[4 * q + 2], t0[4 * q + 3]};
-                xch[(((fm * 4 + wave) * 2 + 1) * 4 + q) * 64 + lane] = (floatx4){t1[4 * q], t1[4 * q + 1], t1[4 * q + 2], t1[4 * q + 3]};
+                xch[(((fm * 4 + wave) * 2 + 0) * 4 + q) * 64 + lane_e] = (floatx4){t0[4 * q], t0[4 * q + 1], t0[4 * q + 2], t0[4 * q + 3]};
+                xch[(((fm * 4 + wave) * 2 + 1) * 4 + q) * 64 + lane_e] = (floatx4){t1[4 * q], t1[4 * q + 1], t1[4 * q + 2], t1[4 * q + 3]};
             }
         }
     }
     __syncthreads();
-    const int n = n0 + l32;
+    const int n = n0 + l32_e;
     const int nc = n < p.wT ? n : 0;
     const int img = nc / per_img, r = nc - img * per_img, ty = r / p.wtw, tx = r - ty * p.wtw;
 #pragma unroll
     for (int fm = 0; fm < FM; fm++) {
-        float yk[4][2][2];  // [k][a][b]: output (2 ty + a, 2 tx + b) of filter row 8 wave + 4 half + k of the block
+        float yk[4][2][2];  // [k][a][b]: output (2 ty + a, 2 tx + b) of filter row 8 wave + 4 half_e + k of the block
 #pragma unroll
         for (int b2 = 0; b2 < 2; b2++) {
             floatx4 t[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) t[i] = xch[(((fm * 4 + i) * 2 + b2) * 4 + wave) * 64 + lane];
+            for (int i = 0; i < 4; i++) t[i] = xch[(((fm * 4 + i) * 2 + b2) * 4 + wave) * 64 + lane_e];
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 yk[k][0][b2] = __fadd_rn(__fadd_rn(t[0][k], t[1][k]), t[2][k]);
                 yk[k][1][b2] = __fsub_rn(__fsub_rn(t[1][k], t[2][k]), t[3][k]);
             }
         }
-        const int ml0 = fm * 32 + 8 * wave + 4 * half;
+        const int ml0 = fm * 32 + 8 * wave + 4 * half_e;
         if (split) {
             const size_t tiles = (gridDim.x - (unsigned)p.main_tiles) / p.nslices;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                floatx4 *dst = reinterpret_cast<floatx4 *>(p.partial) + (((((size_t)slice * tiles + local_tile) * FM + fm) * 4 + wave) * 4 + k) * 64 + lane;
+                floatx4 *dst = reinterpret_cast<floatx4 *>(p.partial) + (((((size_t)slice * tiles + local_tile) * FM + fm) * 4 + wave) * 4 + k) * 64 + lane_e;
                 floatx4 yv;
                 yv.x = yk[k][0][0], yv.y = yk[k][0][1], yv.z = yk[k][1][0], yv.w = yk[k][1][1];
                 *dst = yv;

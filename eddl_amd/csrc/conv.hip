@@ -2347,13 +2347,17 @@ constexpr int NUM_PLAN_TILES = UP2X2_TILE + 2;
 // 58 -> 42; 3x3 stride 2 of 128 on 56x56: 120 -> 91; 64 -> 256 on 56x56: 70 -> 67, of which 256 MB of traffic are 43; in a
 // ResNet-50 the pipe is busy 28 % of the cycles), 64x128 where there are 64 filters (256 -> 64 on 56x56: 60 -> 52), 64x64 for few
 // tiles.  A 128x64 tile gives every wavefront filters of its own and all the pixels: its filters then cross L1 once, not twice.
-#define SPLIT(WM, WN, TM, TN, WGS)                                                                                                           \
-    {                                                                                                                                        \
-        "conv_split_kernel<" #WM "," #WN "," #TM "," #TN "," #WGS ">", WM *TM * 32, WN *TN * 32, SPLIT_K, conv_split_kernel<WM, WN, TM, TN, WGS>, \
-            conv_reduce_kernel<WM, WN, TM, TN>, 0                                                                                            \
+// Each tile comes in three builds, by how a step finds its pixel (SplitTaps).
+#define SPLIT(WM, WN, TM, TN, WGS, TAPS)                                                                       \
+    {                                                                                                          \
+        "conv_split_kernel<" #WM "," #WN "," #TM "," #TN "," #WGS "," #TAPS ">", WM *TM * 32, WN *TN * 32,     \
+            SPLIT_K, conv_split_kernel<WM, WN, TM, TN, WGS, TAPS>, conv_reduce_kernel<WM, WN, TM, TN>, 0       \
     }
-const Variant ksplit[] = {SPLIT(2, 2, 2, 2, 2), SPLIT(4, 1, 1, 2, 3), SPLIT(2, 2, 1, 2, 3), SPLIT(2, 2, 1, 1, 4)};
-constexpr int NUM_SPLIT = (int)(sizeof(ksplit) / sizeof(ksplit[0]));
+#define SPLITS(TAPS) {SPLIT(2, 2, 2, 2, 2, TAPS), SPLIT(4, 1, 1, 2, 3, TAPS), SPLIT(2, 2, 1, 2, 3, TAPS), SPLIT(2, 2, 1, 1, 4, TAPS)}
+const Variant ksplits[][4] = {SPLITS(UPSAMPLED), SPLITS(STORED), SPLITS(ONE_TAP)};
+const Variant *const ksplit = ksplits[UPSAMPLED];  // (the tile shapes, which the plans are made for)
+constexpr int NUM_SPLIT = (int)(sizeof(ksplits[0]) / sizeof(ksplits[0][0]));
+const Variant &split_build(int tile, int RS, int uh, int uw) { return ksplits[RS == 1 ? ONE_TAP : uh * uw == 1 ? STORED : UPSAMPLED][tile]; }
 constexpr int SPLIT_TILE0 = 16;
 bool is_split_tile(int tile) { return tile >= SPLIT_TILE0 && tile < SPLIT_TILE0 + NUM_SPLIT; }
 // The upsampled-input form in the split arithmetic (conv_up_split.h): plan "tiles" 33 (128 filters x 64 blocks) and 34 (64 x 128, half
@@ -3299,7 +3303,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     bool no_room = false;
     if (split_ok && is_split_tile(g_force_tile)) {
         const int tile = g_force_tile - SPLIT_TILE0;
-        const int rc = conv2d_split(no_alloc, ksplit[tile], forced_plan(ksplit, tile, g_force_slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p,
+        const int rc = conv2d_split(no_alloc, split_build(tile, R * S, uh, uw), forced_plan(ksplit, tile, g_force_slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p,
                                     chunk_imgs, &no_room);
         if (!no_room) return rc;
     }
@@ -3353,7 +3357,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
                                          pad_left, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
         if (found != nullptr && is_split_tile(found->tile) && split_ok) {
             const int tile = found->tile - SPLIT_TILE0;
-            const int rc = conv2d_split(no_alloc, ksplit[tile], forced_plan(ksplit, tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev,
+            const int rc = conv2d_split(no_alloc, split_build(tile, R * S, uh, uw), forced_plan(ksplit, tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev,
                                         p, chunk_imgs, &no_room);
             if (!no_room) return rc;
         }

@@ -152,7 +152,14 @@ __device__ __forceinline__ void split_tile_again(const ConvParams &p, floatx16 (
 // one output position for 8 or 16 channels (coalesced along the image row), splits them and puts them into LDS in the
 // operand layout, [buffer][part][8 channels][pixel][8 bf16]: every LDS access is 16 bytes per lane of consecutive lanes.
 // Split filters go from L2 straight to registers (two wavefronts read the same 1 KB; the second meets the first's in L1).
-template <int WM, int WN, int TM, int TN, int WGS>
+// How a step finds its pixel.  UPSAMPLED: any convolution; STORED: of the image as it is stored; ONE_TAP: the filter has one tap, so
+// that the offset is the same in every step.  A general offset takes two divisions (25 vector instructions a step and thread, beside
+// the 52 that split its eight pixels), which slow a kernel that multiplies little per pixel (batch 64, best plans, us, all on one card;
+// UPSAMPLED -> ONE_TAP: 256 -> 64 on 56x56 55.8 -> 52.4, 512 -> 256 on 28x28 78.4 -> 76.5, 128 -> 512 53.1 -> 51.2, 256 -> 1024 on
+// 14x14 46.6 -> 45.2, 1024 -> 256 45.2 -> 43.2, 2048 -> 512 on 7x7 51.8 -> 49.5; UPSAMPLED -> STORED: 128 3x3 stride 2 on 56x56
+// 91.2 -> 89.9, tile 128x128 95.8 -> 94.4).
+enum SplitTaps { UPSAMPLED, STORED, ONE_TAP };
+template <int WM, int WN, int TM, int TN, int WGS, SplitTaps TAPS>
 __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p) {
     static_assert(WM * WN == 4, "four wavefronts per workgroup");
     constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
@@ -202,9 +209,16 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
         ld_kx = tap - ld_ky * p.S;
     }
     float raw[CHUNKS][8];
+    const int origin = (base + ih0 * p.W + iw0) * 4;  // (the window's first pixel, which may lie outside)
+    const int only = split_pixel(p, magic_h, magic_w, pvalid, base, ih0, iw0, 0, 0);
     // (the channel counts of this form are multiples of 16, of each tensor's of 8: eight channels are one tensor's or nobody's)
     auto load_pixels = [&](int chunk) {
-        const int voff = split_pixel(p, magic_h, magic_w, pvalid, base, ih0, iw0, ld_ky, ld_kx);
+        int voff = only;
+        if constexpr (TAPS == UPSAMPLED) voff = split_pixel(p, magic_h, magic_w, pvalid, base, ih0, iw0, ld_ky, ld_kx);
+        if constexpr (TAPS == STORED) {
+            const bool ok = pvalid && (unsigned)(ih0 + ld_ky) < (unsigned)p.H && (unsigned)(iw0 + ld_kx) < (unsigned)p.W;
+            voff = ok ? origin + (ld_ky * p.W + ld_kx) * 4 : OOB;
+        }
         const int c0 = ld_c + (kgroup + chunk) * 8;
         const bool second = c0 >= p.Csplit;
         const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(second ? p.I2 : p.I), 0, c0 < p.C ? p.in_bytes : 0u, RSRC_WORD3);
@@ -215,6 +229,10 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
     auto next_load_step = [&]() {
         // (selects: a branch would end the block that the matrix instructions are scheduled in; behind the last step the
         // channels run past the last and the loads bring zeros without touching memory)
+        if constexpr (TAPS == ONE_TAP) {
+            ld_c += SPLIT_K;
+            return;
+        }
         const int kx = ld_kx + 1, wrap_x = kx == p.S ? 1 : 0, ky = ld_ky + wrap_x, wrap_y = ky == p.R ? 1 : 0;
         ld_kx = wrap_x ? 0 : kx;
         ld_ky = wrap_y ? 0 : ky;

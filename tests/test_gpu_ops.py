@@ -1442,6 +1442,41 @@ def test_conv2d_search_keeps_only_the_filter_copy_of_its_plan(hip, tmp_path, ker
         hip.uncache_conv_filters(Wd)
 
 
+@pytest.mark.parametrize("tile", [16, 17, 18, 19])
+def test_conv2d_split_form_gives_the_same_bits_however_it_finds_its_pixels(hip, tile):
+    """The builds for one tap, for stored and for upsampled images: a filter of one tap is the middle of one of nine (the sums then only
+    gain zeros), an upsampled image one that is stored."""
+    rng = np.random.default_rng(1380 + tile)
+
+    def run(x, w, P, Q, taps, *geometry, upsample=(1, 1)):
+        O = hip.full((x.shape[0], w.shape[0], P, Q), np.nan)
+        hip.conv2D(hip.array(x), hip.array(w), None, O, *geometry, upsample=upsample)
+        name = hip.last_conv_kernel()
+        assert name.startswith("conv_split_kernel") and taps in name, name
+        return O.numpy()
+
+    hip.force_conv_plan(tile, 1)
+    try:
+        # (one pixel, an edge of every tile, more zeros around the image than pixels in it)
+        for N, C, H, W, Kf, stride, pad in ((1, 16, 1, 1, 1, 1, 0), (3, 48, 13, 11, 130, 1, 0), (2, 32, 14, 9, 65, 2, 0), (1, 16, 2, 3, 40, 1, 3)):
+            x = rng.standard_normal((N, C, H, W), dtype=np.float32)
+            w = rng.standard_normal((Kf, C, 1, 1), dtype=np.float32)
+            P, Q = (H + 2 * pad - 1) // stride + 1, (W + 2 * pad - 1) // stride + 1
+            nine = np.zeros((Kf, C, 3, 3), np.float32)
+            nine[:, :, 1:2, 1:2] = w
+            want = run(x, nine, P, Q, "STORED", stride, stride, pad + 1, pad + 1)
+            assert np.array_equal(run(x, w, P, Q, "ONE_TAP", stride, stride, pad, pad), want)
+            up = np.repeat(np.repeat(x, 2, 2), 3, 3)
+            full = rng.standard_normal((Kf, C, 3, 3), dtype=np.float32)
+            for f, name, py in ((full, "STORED", 2), (w, "ONE_TAP", 0)):
+                P, Q = (2 * H + 2 * py - f.shape[2]) // stride + 1, (3 * W + 2 * py - f.shape[3]) // stride + 1
+                want = run(up, f, P, Q, name, stride, stride, py, py)
+                got = run(x, f, P, Q, "UPSAMPLED" if name == "STORED" else name, stride, stride, py, py, upsample=(2, 3))
+                assert np.array_equal(got, want)
+    finally:
+        hip.force_conv_plan(-1, 1)
+
+
 # ------------------------------------------------------------------ the one-launch Winograd form in the split arithmetic
 # N C H W Kf pads(top, left) output size: edges of the tile (64 filters x 32 blocks) and of an image, one K-step of 16 channels and
 # many, odd planes, single rows and columns of blocks, 16- and 4-byte pixel loads (rows of a multiple of four pixels, odd left padding)

@@ -3,13 +3,19 @@
 // are computed in fp32 by the same operations, enlarged 2^24 times and split exactly into three bf16 numbers by the lane that
 // multiplies them; the filters are transformed in 64 bits and split once per registered filter tensor (an error in U is the same in
 // every pixel of a plane: rounded to fp32 as in the other Winograd forms it is what remains of theirs in a plane's mean).  The six largest of the nine products
-// of two such sums go into ONE fp32 accumulator, the smallest first: six roundings per 16 channels where the fp32 instruction
-// (two channels each) makes eight, so the error against 64 bits is below that form's (512 channels 5.8e-7 against 6.9e-7
-// relative in the 2-norm, 64 channels 2.1e-7 against 2.6e-7).  That instruction rounds what it shifts out on the way to an
-// accumulator downwards, not to nearest: 1.4e-8 of the outputs' root mean square for all sums of 512 channels, which the output
-// transform makes -9, 3, 3 and -1 times that of and no pool averages away (logits of ResNet-50, 16 images: 4.9e-7 from 64 bits, 4.2e-7
-// with the fp32 kernel).  So the middle half of a sum's steps is accumulated with the opposite sign, and so are the positions (i, j) of
-// odd i + j throughout: 4.2e-7.
+// of two such sums are added to fp32 accumulators, the smallest first: six roundings per 16 channels where the fp32 instruction
+// (two channels each) makes eight.  That instruction rounds what it shifts out on the way to an accumulator downwards, not to
+// nearest, and several times on the way (a product at a time or a few): in an accumulator of a long sum that costs more than the
+// eight roundings of the fp32 instruction.  Two things keep the form more accurate than the fp32 one-launch kernel all the same:
+//   * The positions (i, 1) of a patch, where pixels of one sign add up and whose sums are the largest by far behind a ReLU, have their
+//     six products of a step summed from zero and added to the long sum by vector instructions: one rounding to nearest per 16 channels.
+//   * The error that remains has one sign.  Position (i, 2) is accumulated with the opposite sign, so are the position rows 1 and 3,
+//     and so is every other block (2x2 outputs) of a plane: what is left in an output is a small fraction of its rounding, and
+//     the means of planes, which no pool and no later layer would average away, hold none of it.
+// Error against 64 bits on the inputs that the layers of the networks have, relative to the outputs' root mean square, of the fp32 one-launch kernel -> of
+// this one (in brackets with all products in one accumulator): 64 channels 1.5e-7 -> 1.1e-7 (1.4e-7), 128 2.0e-7 -> 1.1e-7 (1.9e-7), 256
+// 2.5e-7 -> 1.4e-7 (2.7e-7), 512 3.4e-7 -> 1.6e-7 (3.6e-7), 1024 4.8e-7 -> 2.3e-7 (5.2e-7); of the mean of a plane: 64 channels on 56x56
+// 4.6e-8 -> 4e-9, 256 on 14x14 6.0e-8 -> 1.6e-8, 512 on 7x7 9.5e-8 -> 4.4e-8.  On normally distributed pixels 2.6e-7 -> 1.8e-7 (64 channels).
 // Sums that are not finite - infinities and NaN, and with the
 // enlargement numbers from 2^104 and sums from 2^80 on - are computed with the fp32 instruction too and take that value.
 
@@ -133,9 +139,11 @@ __device__ __forceinline__ void wino_block_again(const ConvParams &p, floatx16 &
 //     layout), two steps ahead;
 //   * a lane reads the two patch rows of its block and position row for its eight channels, forms the four operands and
 //     splits them (64 vector instructions per pair of channels).  Positions 0 and 1 of step t + 1 are made during the matrix
-//     instructions of positions 2 and 3 of step t, positions 2 and 3 during those of 0 and 1: that keeps 48 operand
-//     and 24 intermediate registers alive instead of 96;
-//   * filters go from L2 straight to registers (a fragment is one wavefront's alone), each part of the next position's into
+//     instructions of positions 2 and 3 of step t, positions 2 and 3 are split during those of 0 and 1: that keeps 48 operand
+//     and 16 intermediate registers alive instead of 96;
+//   * a step is eight groups of six products (a position and 32 filters).  Position 1's alternate with position 0's: the sum of
+//     a group is added to the long one while the next group multiplies, so that 16 registers hold it and nothing waits for it;
+//   * filters go from L2 straight to registers (a fragment is one wavefront's alone), two groups ahead, each part into
 //     the place of the one that has been multiplied last.
 // Why this tile: filters are used for 32 blocks only (192 KB per step and two workgroups, 64 bytes a cycle and CU if the matrix
 // pipe never waited, which is what L2 delivers: 138 GB/s per CU measured, 100 where 25 MB of filters come from the last-level
@@ -168,12 +176,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void *)p.Wp, 0, p.wp_bytes, RSRC_WORD3);
     const int a_voff = lane * 16;
     const int a_base = (m0 / 32) * WSPLIT_UNIT + 4 * wave * SPLIT_UNIT, a_step = p.Mp / 32 * WSPLIT_UNIT;
-    uintx4 a[FM][3];
-    auto load_a = [&](int part, int step, int j) __attribute__((always_inline)) {
-#pragma unroll
-        for (int fm = 0; fm < FM; fm++)
-            a[fm][part] = __builtin_bit_cast(
-                uintx4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, a_voff + part * 1024, a_base + step * a_step + fm * WSPLIT_UNIT + j * SPLIT_UNIT, 0));
+    constexpr int GROUPS = 4 * FM, kPos[GROUPS] = {1, 0, 1, 0, 2, 2, 3, 3}, kFm[GROUPS] = {0, 0, 1, 1, 0, 1, 0, 1};  // a step's groups of products
+    uintx4 a[2][3];  // of this group and the next
+    auto load_a = [&](int part, int step, int i) __attribute__((always_inline)) {
+        a[i & 1][part] = __builtin_bit_cast(
+            uintx4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, a_voff + part * 1024, a_base + step * a_step + kFm[i] * WSPLIT_UNIT + kPos[i] * SPLIT_UNIT, 0));
     };
 
     // ---- where the tile's pixels go in LDS and this lane's patch lies there (wino_fused_kernel; a wavefront loads one or two groups of 64 slots)
@@ -182,7 +189,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int CPW = WIDE ? CK * KG / 4 : CK;
     const int my_k = wave % KG, my_c = wave / KG * CPW;
     const int per_img = p.wth * p.wtw;
-    int voff[WLC], my_base = WIDE ? 1 : 0, my_stride = 0;
+    int voff[WLC], my_base = WIDE ? 1 : 0, my_stride = 0, my_odd = 0;  // (my_odd: the parity of this lane's block in its plane)
 #pragma unroll
     for (int k = 0; k < WLC; k++) voff[k] = OOB;
     {
@@ -211,7 +218,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             }
             {
                 const int n = n0 + l32;
-                if (n >= seg_n && n < seg_n + cnt) my_base = base + shift + 2 * (n - seg_n), my_stride = WIDE ? 4 * gpr : width;
+                if (n >= seg_n && n < seg_n + cnt) my_base = base + shift + 2 * (n - seg_n), my_stride = WIDE ? 4 * gpr : width, my_odd = (ty + tx0 + n - seg_n) & 1;
             }
             base += WIDE ? 16 * gpr : 4 * width;
             seg_n += cnt;
@@ -238,29 +245,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     };
     load_step(step_lo, rs_of(0));
 #pragma unroll
-    for (int part = 2; part >= 0; part--) load_a(part, step_lo, 0);
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int part = 2; part >= 0; part--) load_a(part, step_lo, i);
     if (!split) stage_channel_constants<MF>(p, epi, m0, tid);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
     load_step(step_lo + 1, rs_of(1));
     trace_mark(p, 1);
 
-    floatx16 acc[4][FM];
+    floatx16 acc[4][FM];  // (position 1's are sum1)
 #pragma unroll
     for (int j = 0; j < 4; j++)
 #pragma unroll
         for (int fm = 0; fm < FM; fm++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[j][fm][v] = 0.0f;
+    float sum1[FM][16];
+#pragma unroll
+    for (int fm = 0; fm < FM; fm++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) sum1[fm][v] = 0.0f;
 
     const int ra = wave == 0 ? 0 : (wave == 2 ? 2 : 1), rb = wave == 0 ? 2 : (wave == 1 ? 2 : (wave == 2 ? 1 : 3));
     const float sgn = wave == 1 ? 1.0f : -1.0f;
     const int ra_off = half * 8 * SLOTS + my_base + ra * my_stride, rb_off = half * 8 * SLOTS + my_base + rb * my_stride;
     typedef const __attribute__((address_space(3))) floatx2 *lds_f2;
     uintx4 b[4][3];
-    const SignOfStep sign(step_lo, step_hi);
-    float up = ((wave & 1) != 0) != sign.negative(step_lo) ? -SPLIT_UP : SPLIT_UP;  // of the step whose operands are made (odd positions of a row: the other sign)
-    float s1[8], s2[8], u3[8];  // what positions 2 and 3 are made of, from the turn of 0 and 1 to their own
+    const float up = ((wave ^ my_odd) & 1) != 0 ? -SPLIT_UP : SPLIT_UP;  // (position 2 has the other sign)
+    float v2[8], v3[8];  // positions 2 and 3, from the turn of 0 and 1 to their own
     float d[2][2][4];           // [channel of a pair][patch row][column]
     auto read_pair = [&](const lds_float *rs, int q) __attribute__((always_inline)) {
 #pragma unroll
@@ -285,7 +298,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         b[j][1][q] = m;
         b[j][2][q] = l;
     };
-    // positions 0 and 1 of a pair of channels: u0 - u2, -(u1 + u2)
+    // positions 0 and 1 of a pair of channels: u0 - u2, u1 + u2 (and 2 and 3: -(u2 - u1), u1 - u3)
     auto first = [&](int q) __attribute__((always_inline)) {
         float v[2][2];
 #pragma unroll
@@ -293,25 +306,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             float u[4];
 #pragma unroll
             for (int c = 0; c < 4; c++) u[c] = __builtin_fmaf(d[e][1][c], sgn, d[e][0][c]);
-            s1[2 * q + e] = up * u[1];
-            s2[2 * q + e] = up * u[2];
-            u3[2 * q + e] = u[3];
-            v[0][e] = __builtin_fmaf(up, u[0], -s2[2 * q + e]);
-            v[1][e] = __fsub_rn(-s1[2 * q + e], s2[2 * q + e]);
+            const float s1 = up * u[1], s2 = up * u[2];
+            v[0][e] = __builtin_fmaf(up, u[0], -s2);
+            v[1][e] = __fadd_rn(s1, s2);
+            v2[2 * q + e] = __fsub_rn(s1, s2);
+            v3[2 * q + e] = __builtin_fmaf(-up, u[3], s1);
         }
         put(0, q, v[0][0], v[0][1]);
         put(1, q, v[1][0], v[1][1]);
     };
-    // positions 2 and 3: u2 - u1, -(u1 - u3)
     auto second = [&](int q) __attribute__((always_inline)) {
-        put(2, q, __fsub_rn(s2[2 * q], s1[2 * q]), __fsub_rn(s2[2 * q + 1], s1[2 * q + 1]));
-        put(3, q, __builtin_fmaf(up, u3[2 * q], -s1[2 * q]), __builtin_fmaf(up, u3[2 * q + 1], -s1[2 * q + 1]));
+        put(2, q, v2[2 * q], v2[2 * q + 1]);
+        put(3, q, v3[2 * q], v3[2 * q + 1]);
     };
     constexpr int kA[6] = {2, 1, 1, 0, 0, 0}, kB[6] = {0, 1, 0, 2, 1, 0};
-    auto multiply = [&](int j, int k) __attribute__((always_inline)) {  // product k of a position, the filters' smallest parts first
-#pragma unroll
-        for (int fm = 0; fm < FM; fm++)
-            acc[j][fm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[fm][kA[k]]), __builtin_bit_cast(bf16x8, b[j][kB[k]]), acc[j][fm], 0, 0, 0);
+    floatx16 own;  // position 1's products of one step and 32 filters
+    auto multiply = [&](int i, int k) __attribute__((always_inline)) {  // product k of group i, the filters' smallest parts first
+        const floatx16 zero = {0.0f};
+        floatx16 &sum = kPos[i] == 1 ? own : acc[kPos[i]][kFm[i]];
+        sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[i & 1][kA[k]]), __builtin_bit_cast(bf16x8, b[kPos[i]][kB[k]]), kPos[i] == 1 && k == 0 ? zero : sum,
+                                                      0, 0, 0);
     };
     read_pair(rs_of(0), 0);
 #pragma unroll
@@ -319,54 +333,50 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         first(q);
         if (q < 3) read_pair(rs_of(0), q + 1);
     }
-    for (int run_lo = step_lo, run_hi; run_lo < step_hi; run_lo = run_hi) {  // (one to three runs of steps of one sign)
-        run_hi = sign.run_end(run_lo, step_hi);
-        for (int step = run_lo; step < run_hi; step++) {
-            const int cur = (step - step_lo) & 1;
-            const int next = step + 1 < step_hi ? step + 1 : step;
-            const lds_float *rs = rs_of(cur ^ 1);
+    for (int step = step_lo; step < step_hi; step++) {
+        const int cur = (step - step_lo) & 1;
+        const int next = step + 1 < step_hi ? step + 1 : step;
+        const lds_float *rs = rs_of(cur ^ 1);
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if (j == 2) {
-                    // The next step's pixels were requested a step ago; of what was requested since then only this position's
-                    // filters may still be on their way.  Behind the barrier nobody reads this step's pixels any more.
-                    __builtin_amdgcn_s_waitcnt(0x0F70 | (3 * FM));
-                    __syncthreads();
-                    load_step(step + 2, rs_of(cur));
-                    up = ((wave & 1) != 0) != sign.negative(step + 1) ? -SPLIT_UP : SPLIT_UP;
-                    __builtin_amdgcn_sched_barrier(0);
-                    read_pair(rs, 0);
-                }
-#pragma unroll
-                for (int h = 0; h < 2; h++) {  // half of a position's products
-                    const int q = 2 * (j & 1) + h;
-#pragma unroll
-                    for (int k = 3 * h; k < 3 * h + 3; k++) multiply(j, k);
-                    if (j < 2) {
-                        second(q);
-                    } else {
-                        first(q);
-                        if (q < 3) read_pair(rs, q + 1);
-                    }
-                    const int js = j < 3 ? step : next, jn = (j + 1) & 3;
-                    if (h == 0) load_a(2, js, jn), load_a(1, js, jn);
-                    else load_a(0, js, jn);
-#pragma unroll
-                    for (int t = 0; t < 3 * FM; t++) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        if (j < 2) __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
-                        else __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
-                        if (j >= 2 && q < 3 && (t == 1 || t == 2)) __builtin_amdgcn_sched_group_barrier(0x100, WIDE ? 6 : 4, 0);
-                        if (h == 0 && (t == FM || t == 3 * FM - 1)) __builtin_amdgcn_sched_group_barrier(0x020, FM, 0);
-                    }
-                    if (h == 1) __builtin_amdgcn_sched_group_barrier(0x020, FM, 0);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+        for (int i = 0; i < GROUPS; i++) {
+            if (i == GROUPS / 2) {
+                // The next step's pixels were requested a step ago; of what was requested since then only the filters of
+                // this group and the next may still be on their way.  Behind the barrier nobody reads this step's pixels any more.
+                __builtin_amdgcn_s_waitcnt(0x0F70 | 6);
+                __syncthreads();
+                load_step(step + 2, rs_of(cur));
+                __builtin_amdgcn_sched_barrier(0);
+                read_pair(rs, 0);
             }
+            const int q = i & 3;
+#pragma unroll
+            for (int k = 0; k < 6; k++) multiply(i, k);
+            if (i < GROUPS / 2) {
+                second(q);
+                if (i & 1) {
+#pragma unroll
+                    for (int v = 0; v < 16; v++) sum1[kFm[i]][v] = __fadd_rn(sum1[kFm[i]][v], own[v]);
+                }
+            } else {
+                first(q);
+                if (q < 3) read_pair(rs, q + 1);
+            }
+            const int in = (i + 2) % GROUPS, js = i + 2 < GROUPS ? step : next;
+            load_a(2, js, in), load_a(1, js, in), load_a(0, js, in);
+#pragma unroll
+            for (int t = 0; t < 6; t++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (i >= GROUPS / 2) __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+                else if (i & 1) __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+                else __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+                if (i >= GROUPS / 2 && q < 3 && (t == 1 || t == 2)) __builtin_amdgcn_sched_group_barrier(0x100, WIDE ? 6 : 4, 0);
+                if (t == 1 || t == 3) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if (run_hi < step_hi) negate(acc);
     }
-    const float down = ((wave & 1) != 0) != sign.negative(step_hi - 1) ? -SPLIT_DOWN : SPLIT_DOWN;
+    const float down = up * (SPLIT_DOWN / SPLIT_UP);
     trace_mark(p, 2);
 
     // ---- output transform: along the position row in registers, across the rows through LDS
@@ -388,7 +398,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             for (int k = 0; k < 4; k++) {
                 float m[4];
 #pragma unroll
-                for (int j = 0; j < 4; j++) m[j] = (j & 1 ? -down : down) * acc[j][fm][4 * q + k];  // (the sums are 2^48 times too large)
+                for (int j = 0; j < 4; j++) m[j] = (j == 2 ? -down : down) * (j == 1 ? sum1[fm][4 * q + k] : acc[j][fm][4 * q + k]);  // (the sums are 2^48 times too large)
                 t[0][k] = __fadd_rn(__fadd_rn(m[0], m[1]), m[2]);
                 t[1][k] = __fsub_rn(__fsub_rn(m[1], m[2]), m[3]);
                 finite = __builtin_fmaf(t[0][k], 0.0f, finite);
@@ -409,9 +419,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 wino_block_again(p, sum, in1, in2, m0 + fm * 32 + l32_e, n0 + l32_e, wave, j, step_lo * CK, step_hi * CK, half_e);
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
-                    const float x0 = j == 0 ? acc[0][0][v] : (j == 1 ? acc[1][0][v] : (j == 2 ? acc[2][0][v] : acc[3][0][v]));
-                    const float x1 = j == 0 ? acc[0][1][v] : (j == 1 ? acc[1][1][v] : (j == 2 ? acc[2][1][v] : acc[3][1][v]));
-                    const float x = (j & 1 ? -down : down) * (fm == 0 ? x0 : x1), m = x * 0.0f == 0.0f ? x : sum[v];
+                    const float x0 = j == 0 ? acc[0][0][v] : (j == 1 ? sum1[0][v] : (j == 2 ? acc[2][0][v] : acc[3][0][v]));
+                    const float x1 = j == 0 ? acc[0][1][v] : (j == 1 ? sum1[1][v] : (j == 2 ? acc[2][1][v] : acc[3][1][v]));
+                    const float x = (j == 2 ? -down : down) * (fm == 0 ? x0 : x1), m = x * 0.0f == 0.0f ? x : sum[v];
                     t0[v] = j == 0 ? m : (j == 3 ? t0[v] : __fadd_rn(t0[v], m));
                     t1[v] = j == 1 ? m : __fsub_rn(t1[v], m);
                 }

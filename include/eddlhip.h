@@ -265,8 +265,10 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * split filters, 6 bytes a weight, unless registered, and the partial tiles of a K-split plan; where that is more than
  * eddlhip_conv2d_fwd_noalloc has (11 million unregistered weights), that entry point runs the planner's own choice.
  * The one-launch Winograd form in that arithmetic (force_plan(32, .), or the search from 512 blocks of outputs on; channel counts
- * that are multiples of 16): transformed pixels and filters are fp32 numbers as in the third Winograd form, their products and
- * sums those of the split form, so its error is below that form's too.  Non-finite inputs as in the Winograd forms.  Its filters take
+ * that are multiples of 16): transformed pixels are fp32 numbers as in the third Winograd form, filters are transformed in 64 bits, the
+ * products are those of the split form, and the sums of the largest of a patch's positions are rounded once per 16 channels: its error
+ * against 64 bits is below that of the third form, by a third to a half on the inputs of this library's networks, and in the means of
+ * planes by more than half.  Non-finite inputs as in the Winograd forms.  Its filters take
  * 96 bytes per filter and channel.  Likewise the upsampled-input form of a 2x2 filter (force_plan(33, .) / (34, .) on tiles of 128
  * filters x 64 or 64 x 128 stored pixels, `slices` K slices for the left-over tiles, or the search; channel counts that are
  * multiples of 16; 54 bytes per filter and channel).  Neither under set_algo(9).

@@ -2327,8 +2327,8 @@ const FusedVariant kfused[] = {FUSED(1, 1, 4, 4), FUSED(2, 1, 4, 3)};
 constexpr int NUM_FUSED = (int)(sizeof(kfused) / sizeof(kfused[0]));
 constexpr int FUSED_TILE0 = 6;      // plan "tile" numbers 6 .. 6 + NUM_FUSED - 1 name these shapes (0..3: direct tiles, 4 / 5: the other Winograd forms)
 constexpr int FUSED_ROW_ALIGN = 8;  // the transformed filters are padded to whole K-steps of every variant
-// The same on the bf16 matrix instructions (wino_split.h): plan "tile" 32.  Channel counts that are multiples of 16, of each tensor
-// of a folded Concat too.  The search tries it from 512 blocks on: a filter is 96 bytes a channel here, and below that the
+// The same on the bf16 matrix instructions (wino_split.h): plan "tile" 32.  Channel counts that are multiples of 16.
+// The search tries it from 512 blocks on: a filter is 96 bytes a channel here, and below that the
 // launches are bound by reading them (512 channels on 14x14, best plans of the other forms / this one: 1 image 18.3 / 27.0 us,
 // 4 images 34.4 / 42.8, 8 images 56.0 / 59.4, 16 images 85.1 / 81.1; 1024 channels, 392 blocks 151 / 186, 1024 blocks 290 / 241).
 const FusedVariant kwsplit[] = {
@@ -3289,8 +3289,8 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     if (fused_ok && g_force_tile >= FUSED_TILE0 && g_force_tile < FUSED_TILE0 + NUM_FUSED)
         return conv2d_winograd_fused(kfused[g_force_tile - FUSED_TILE0], g_force_slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top,
                                      pad_left, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
-    // the one-launch form in the split arithmetic: whole K-steps of 16 channels, each of one tensor
-    const bool wsplit_ok = fused_ok && C % 16 == 0 && (!two || C % 32 == 0) && (long long)(C / 16) * (p.Mp / 32) * WSPLIT_UNIT < (1LL << 31);
+    // the one-launch form in the split arithmetic: whole K-steps of 16 channels
+    const bool wsplit_ok = fused_ok && C % 16 == 0 && (long long)(C / 16) * (p.Mp / 32) * WSPLIT_UNIT < (1LL << 31);
     if (wsplit_ok && is_wsplit_tile(g_force_tile))
         return conv2d_winograd_fused(kwsplit[g_force_tile - WSPLIT_TILE0], g_force_slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top,
                                      pad_left, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);

@@ -230,16 +230,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // (no branch: it would end the block that the matrix instructions are scheduled in; past the last step zeros arrive)
     auto load_step = [&](int want, lds_float *rs) __attribute__((always_inline)) {
         const int step = min(want, step_hi - 1);
-        const bool second = step * CK >= p.Csplit;
-        const int32x4 dma = second ? dma_in2 : dma_in;
-        const int c0 = step * CK - (second ? p.Csplit : 0) + my_c;
+        // (a folded Concat's tensors have multiples of eight channels: eight of a step are one tensor's, not always all sixteen)
 #pragma unroll
-        for (int k = 0; k < WLC; k++) {
-            const int at = want < step_hi ? voff[k] : OOB;
+        for (int c8 = 0; c8 < CPW; c8 += 8) {
+            const int first = step * CK + my_c + c8;
+            const bool second = first >= p.Csplit;
+            const int32x4 dma = second ? dma_in2 : dma_in;
+            const int c0 = first - (second ? p.Csplit : 0);
 #pragma unroll
-            for (int c = 0; c < CPW; c++) {
-                if constexpr (WIDE) lds_dma_b128(dma, rs + (my_c + c) * SLOTS + my_k * 256, at, (c0 + c) * HW4);
-                else lds_dma_b32(dma, rs + (my_c + c) * SLOTS + (my_k + KG * k) * 64, at, (c0 + c) * HW4);
+            for (int k = 0; k < WLC; k++) {
+                const int at = want < step_hi ? voff[k] : OOB;
+#pragma unroll
+                for (int c = 0; c < 8; c++) {
+                    if constexpr (WIDE) lds_dma_b128(dma, rs + (my_c + c8 + c) * SLOTS + my_k * 256, at, (c0 + c) * HW4);
+                    else lds_dma_b32(dma, rs + (my_c + c8 + c) * SLOTS + (my_k + KG * k) * 64, at, (c0 + c) * HW4);
+                }
             }
         }
     };

@@ -1613,6 +1613,35 @@ def test_conv2d_winograd_split_reads_folded_inputs_applies_the_epilogue_and_pool
 
 
 @pytest.mark.parametrize("slices", [1, 2])
+@pytest.mark.parametrize("C,H,W", [(16, 6, 10), (48, 6, 10), (48, 6, 12), (80, 4, 76), (64, 6, 12), (64, 4, 76), (96, 10, 64)])
+def test_conv2d_winograd_split_reads_two_tensors_in_both_builds_and_pools(hip, C, H, W, slices):
+    """A folded Concat, also of tensors whose channels end within a step of 16 (8, 24 and 40), with pixels of 4 and of 16 bytes per lane: the
+    same plan runs as on the stored tensor, with the same bits; the pool in the epilogue gives those of the separate call."""
+    rng = np.random.default_rng(1992 + C + W)
+    N, Kf = 2, 72
+    a, b = rng.standard_normal((2, N, C // 2, H, W), dtype=np.float32)
+    w = (rng.standard_normal((Kf, C, 3, 3)) * 0.06).astype(np.float32)
+    A, B, AB, Wd = hip.array(a), hip.array(b), hip.array(np.concatenate([a, b], 1)), hip.array(w)
+    O1, O2 = hip.full((N, Kf, H, W), np.nan), hip.full((N, Kf, H, W), np.nan)
+    build = "wino_split_kernel<true>" if W % 4 == 0 else "wino_split_kernel<false>"
+    want, got = ([hip.full((N, Kf, H // 2, W // 2), 9.0) for _ in range(3)] for _ in range(2))
+    try:
+        hip.force_conv_plan(32, slices)
+        hip.conv2D(AB, Wd, None, O2, 1, 1, 1, 1)
+        assert build in hip.last_conv_kernel()
+        hip.conv2D(A, Wd, None, O1, 1, 1, 1, 1, second=B)
+        assert build in hip.last_conv_kernel()
+        assert np.array_equal(O1.numpy(), O2.numpy())
+        hip.mpool2D(O2, *want, (2, 2), (2, 2), (0, 0, 0, 0))
+        hip.conv2D(A, Wd, None, O1, 1, 1, 1, 1, second=B, pool=tuple(got), keep=False)
+        assert build in hip.last_conv_kernel()
+        assert all(np.array_equal(p.numpy(), q.numpy()) for p, q in zip(want, got))
+    finally:
+        hip.force_conv_plan(-1, 1)
+    assert_conv_close(_conv64_padded(np.concatenate([a, b], 1), w, (1, 1), H, W), O2.numpy(), "%d channels" % C)
+
+
+@pytest.mark.parametrize("slices", [1, 2])
 def test_conv2d_winograd_split_keeps_what_is_not_finite_and_the_largest_numbers(hip, slices):
     """Infinities, NaN and numbers that round up to infinity in 16 bits, in the image and in a filter: what the fp32 kernel of this
     form gives, and not a bit of a block whose patch holds none of them."""

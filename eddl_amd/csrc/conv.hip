@@ -2894,7 +2894,7 @@ int conv2d_winograd(bool fold, int fs, int dev, const float *I, const float *I2,
                     int H, int W, int Kf, int pad_top, int pad_left, int P, int Q, const float *bn_g, const float *bn_b, const float *bn_mean,
                     const float *bn_var, float bn_eps, const float *residual, int relu);
 
-int conv2d_winograd_fused(const FusedVariant &fv, int slices, int dev, const float *I, const float *I2, int uh, int uw, const float *K, const float *bias, float *O,
+int conv2d_winograd_fused(bool no_alloc, bool *no_room, const FusedVariant &fv, int slices, int dev, const float *I, const float *I2, int uh, int uw, const float *K, const float *bias, float *O,
                           int N, int C, int H, int W, int Kf, int pad_top, int pad_left, int P, int Q, const float *bn_g, const float *bn_b,
                           const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu);
 
@@ -3278,8 +3278,9 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     const bool wino_ok = !gemm && !no_alloc && g_algo == 0 && !g_wino_never && winograd_applies(N, C, Kf, R, S, sr, sc, P, Q);
     const bool fold_ok = wino_ok && winograd_fold_applies(N, C, Kf, R, S, sr, sc, P, Q);
     // the one-launch form (3x3 filters only) needs no transformed copy of the input, so none of V's limits apply
-    const bool fused_ok = !gemm && !no_alloc && g_algo == 0 && !g_wino_never && R == 3 && S == 3 && sr == 1 && sc == 1 &&
-                          (long long)C * 16 * p.Mp * 4 < (1LL << 31);
+    const bool fused_fits = !gemm && g_algo == 0 && !g_wino_never && R == 3 && S == 3 && sr == 1 && sc == 1 && (long long)C * 16 * p.Mp * 4 < (1LL << 31);
+    const bool fused_ok = fused_fits && !no_alloc;
+    bool no_room = false;
     // the upsampled-input form of a 2x2 filter: a geometry of its own in the plans table (kind 2 / 3), since the same
     // shapes on a stored tensor cannot take it
     const bool up_ok = !gemm && !no_alloc && g_algo == 0 && up2x2_applies(N, C, H, W, Kf, R, S, sr, sc, uh, uw, two, pad_top, pad_left, P, Q);
@@ -3287,20 +3288,21 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     if ((up_ok && (g_force_tile == UP2X2_TILE || g_force_tile == UP2X2_TILE + 1)) || (upsplit_ok && is_upsplit_tile(g_force_tile)))
         return conv2d_up2x2(g_force_tile, g_force_slices, dev, I, K, bias, O, N, C, H, W, Kf, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
     if (fused_ok && g_force_tile >= FUSED_TILE0 && g_force_tile < FUSED_TILE0 + NUM_FUSED)
-        return conv2d_winograd_fused(kfused[g_force_tile - FUSED_TILE0], g_force_slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top,
+        return conv2d_winograd_fused(false, nullptr, kfused[g_force_tile - FUSED_TILE0], g_force_slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top,
                                      pad_left, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
-    // the one-launch form in the split arithmetic: whole K-steps of 16 channels
-    const bool wsplit_ok = fused_ok && C % 16 == 0 && (long long)(C / 16) * (p.Mp / 32) * WSPLIT_UNIT < (1LL << 31);
-    if (wsplit_ok && is_wsplit_tile(g_force_tile))
-        return conv2d_winograd_fused(kwsplit[g_force_tile - WSPLIT_TILE0], g_force_slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top,
-                                     pad_left, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
+    // the one-launch form in the split arithmetic: whole K-steps of 16 channels; from the fixed scratch array as the split form below
+    const bool wsplit_ok = fused_fits && C % 16 == 0 && (long long)(C / 16) * (p.Mp / 32) * WSPLIT_UNIT < (1LL << 31);
+    if (wsplit_ok && is_wsplit_tile(g_force_tile)) {
+        const int rc = conv2d_winograd_fused(no_alloc, &no_room, kwsplit[g_force_tile - WSPLIT_TILE0], g_force_slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W,
+                                             Kf, pad_top, pad_left, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
+        if (!no_room) return rc;
+    }
     if ((wino_ok && (g_force_tile == 4 || (g_wino && g_force_tile < 0 && !g_tuning))) || (fold_ok && g_force_tile == 5))
         return conv2d_winograd(g_force_tile == 5, R, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top, pad_left, P, Q, bn_g, bn_b,
                                bn_mean, bn_var, bn_eps, residual, relu);
     // the split form: any filter shape, as long as a chunk of the input is addressed like the direct kernels do; from the fixed
     // scratch array where its filters (half as much again as the repacked ones) and partial tiles fit, else the planner's plan
     const bool split_ok = !gemm && g_algo == 0 && !g_wino_never && split_applies(C, Kf, R, S);
-    bool no_room = false;
     if (split_ok && is_split_tile(g_force_tile)) {
         const int tile = g_force_tile - SPLIT_TILE0;
         const int rc = conv2d_split(no_alloc, split_build(tile, R * S, uh, uw), forced_plan(ksplit, tile, g_force_slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p,
@@ -3350,11 +3352,13 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
         if (found != nullptr && (((found->tile == UP2X2_TILE || found->tile == UP2X2_TILE + 1) && up_ok) || (is_upsplit_tile(found->tile) && upsplit_ok)))
             return conv2d_up2x2(found->tile, found->slices, dev, I, K, bias, O, N, C, H, W, Kf, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
         if (found != nullptr && found->tile >= FUSED_TILE0 && found->tile < FUSED_TILE0 + NUM_FUSED && fused_ok)
-            return conv2d_winograd_fused(kfused[found->tile - FUSED_TILE0], found->slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top, pad_left, P, Q, bn_g,
+            return conv2d_winograd_fused(false, nullptr, kfused[found->tile - FUSED_TILE0], found->slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top, pad_left, P, Q, bn_g,
                                          bn_b, bn_mean, bn_var, bn_eps, residual, relu);
-        if (found != nullptr && is_wsplit_tile(found->tile) && wsplit_ok)
-            return conv2d_winograd_fused(kwsplit[found->tile - WSPLIT_TILE0], found->slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H, W, Kf, pad_top,
-                                         pad_left, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
+        if (found != nullptr && is_wsplit_tile(found->tile) && wsplit_ok) {
+            const int rc = conv2d_winograd_fused(no_alloc, &no_room, kwsplit[found->tile - WSPLIT_TILE0], found->slices, dev, I, two ? I2 : nullptr, uh, uw, K, bias, O, N, C, H,
+                                                 W, Kf, pad_top, pad_left, P, Q, bn_g, bn_b, bn_mean, bn_var, bn_eps, residual, relu);
+            if (!no_room) return rc;
+        }
         if (found != nullptr && is_split_tile(found->tile) && split_ok) {
             const int tile = found->tile - SPLIT_TILE0;
             const int rc = conv2d_split(no_alloc, split_build(tile, R * S, uh, uw), forced_plan(ksplit, tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev,
@@ -3748,8 +3752,8 @@ int conv2d_up2x2(int tile, int slices, int dev, const float *I, const float *K, 
 }
 
 // The one-launch Winograd form of a 3x3 stride-1 convolution (wino_fused_kernel).  Workspace: the transformed filters,
-// unless a registered filter tensor keeps them, and the partial output tiles of a K-split plan.
-int conv2d_winograd_fused(const FusedVariant &fv, int slices, int dev, const float *I, const float *I2, int uh, int uw, const float *K, const float *bias, float *O,
+// unless a registered filter tensor keeps them, and the partial output tiles of a K-split plan.  no_alloc: as in conv2d_split.
+int conv2d_winograd_fused(bool no_alloc, bool *no_room, const FusedVariant &fv, int slices, int dev, const float *I, const float *I2, int uh, int uw, const float *K, const float *bias, float *O,
                           int N, int C, int H, int W, int Kf, int pad_top, int pad_left, int P, int Q, const float *bn_g, const float *bn_b,
                           const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu) {
     hipStream_t st = state(dev).stream;
@@ -3786,7 +3790,7 @@ int conv2d_winograd_fused(const FusedVariant &fv, int slices, int dev, const flo
         for (CachedFilters &e : g_cache[dev]) {
             if (e.K == K && e.Kf == Kf && e.C == C && e.R == 3 && e.S == 3) {
                 void *&kept = fv.split ? e.Wwsplit : (void *&)e.Wfused;
-                if (kept == nullptr && !state(dev).capturing) {
+                if (kept == nullptr && !state(dev).capturing && !no_alloc) {
                     if (hipMalloc(&kept, u_size) != hipSuccess) {
                         kept = nullptr;
                         (void)hipGetLastError();
@@ -3805,7 +3809,15 @@ int conv2d_winograd_fused(const FusedVariant &fv, int slices, int dev, const flo
     }
     const size_t u_bytes = U ? 0 : ((u_size + 255) & ~(size_t)255);
     void *ws = nullptr;
-    if (u_bytes + partial_bytes > 0) EH_TRY(get_workspace(dev, u_bytes + partial_bytes, &ws));
+    if (no_alloc) {
+        if (u_bytes + partial_bytes > (size_t)EDDLHIP_CONV_NOALLOC_SCRATCH_BYTES) {
+            *no_room = true;
+            return 0;
+        }
+        ws = g_scratch_ptr[dev];
+    } else if (u_bytes + partial_bytes > 0) {
+        EH_TRY(get_workspace(dev, u_bytes + partial_bytes, &ws));
+    }
     if (U == nullptr) {
         if (fv.split) {
             EH_TRY(launch_wino_split_filters(dev, K, ws, Kf, C, Mp));

@@ -271,7 +271,9 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * planes by more than half.  Non-finite inputs as in the Winograd forms.  Its filters take
  * 96 bytes per filter and channel.  Likewise the upsampled-input form of a 2x2 filter (force_plan(33, .) / (34, .) on tiles of 128
  * filters x 64 or 64 x 128 stored pixels, `slices` K slices for the left-over tiles, or the search; channel counts that are
- * multiples of 16; 54 bytes per filter and channel).  Neither under set_algo(9).
+ * multiples of 16; 54 bytes per filter and channel).  Neither under set_algo(9).  A plan of the one-launch form is run by
+ * eddlhip_conv2d_fwd_noalloc too where its filters (unless registered and used by eddlhip_conv2d_fwd before: 700 thousand filters
+ * times channels) and partial tiles fit.
  *
  * eddlhip_conv2d_last_kernel() names the kernel the calling thread's last eddlhip_conv2d_fwd
  * launched, followed by " +ksplit(T tiles x S)" when T tiles were divided into S slices; for the Winograd form

@@ -204,3 +204,59 @@ def test_noalloc_takes_the_planners_plan_where_the_split_filters_do_not_fit(hip,
         assert np.array_equal(O1.numpy(), O2.numpy())
     finally:
         hip.conv_autotune(-1)
+
+
+@pytest.mark.parametrize("registered", [False, True])
+@pytest.mark.parametrize("W,slices", [(14, 1), (16, 4)])
+def test_noalloc_runs_the_split_winograd_plan_that_was_found(hip, tmp_path, W, slices, registered):
+    """The one-launch Winograd form in the split arithmetic is used like any found plan: same kernel and bits as conv2d_fwd, nothing allocated."""
+    N, C, H, Kf = 3, 128, 18, 72
+    path = tmp_path / "plans.txt"
+    path.write_text("%d %d %d 3 3 1 1 %d %d 1 | 32 %d\n" % (N, C, Kf, H, W, slices))
+    rng = np.random.default_rng(76)
+    dx, dw = hip.array(rng.standard_normal((N, C, H, W), dtype=np.float32)), hip.array((rng.standard_normal((Kf, C, 3, 3)) * 0.05).astype(np.float32))
+    O1, O2 = hip.full((N, Kf, H, W), float("nan")), hip.full((N, Kf, H, W), float("nan"))
+    args = lambda O: (hip.dev, dx.ptr, dw.ptr, None, O.ptr, N, C, H, W, Kf, 3, 3, 1, 1, 1, 1, H, W, None, None, None, None, 0.0, None, 0)
+    hip.conv_autotune(-1)
+    try:
+        hip.conv_tuned_load(str(path))
+        hip.conv_autotune(True)
+        if registered:
+            hip.cache_conv_filters(dw)
+        hip.synchronize()
+        hip.workspace_trim()
+        hip._check(hip.lib.eddlhip_conv2d_fwd_noalloc(*args(O1)))
+        kernel = hip.last_conv_kernel()
+        assert "wino_split_kernel" in kernel and ("+ksplit" in kernel) == (slices > 1), kernel
+        assert hip.workspace_bytes() == 0
+        hip._check(hip.lib.eddlhip_conv2d_fwd(*args(O2)))
+        assert hip.last_conv_kernel() == kernel
+        assert np.array_equal(O1.numpy(), O2.numpy())
+        hip.fill_(O1, float("nan"))
+        hip._check(hip.lib.eddlhip_conv2d_fwd_noalloc(*args(O1)))   # (registered: with the copy that conv2d_fwd has made)
+        assert np.array_equal(O1.numpy(), O2.numpy())
+    finally:
+        hip.conv_autotune(-1)
+        hip.uncache_conv_filters(dw)
+
+
+def test_noalloc_takes_the_planners_plan_where_the_split_winograd_filters_do_not_fit(hip, tmp_path):
+    N, C, H, W, Kf = 1, 1024, 8, 8, 1024
+    assert 4 * 9 * C * Kf < SCRATCH_BYTES < 96 * C * Kf
+    path = tmp_path / "plans.txt"
+    path.write_text("%d %d %d 3 3 1 1 %d %d 1 | 32 1\n" % (N, C, Kf, H, W))
+    rng = np.random.default_rng(77)
+    dx, dw = hip.array(rng.standard_normal((N, C, H, W), dtype=np.float32)), hip.full((Kf, C, 3, 3), 0.25)
+    O1, O2 = hip.empty((N, Kf, H, W)), hip.empty((N, Kf, H, W))
+    args = lambda O: (hip.dev, dx.ptr, dw.ptr, None, O.ptr, N, C, H, W, Kf, 3, 3, 1, 1, 1, 1, H, W, None, None, None, None, 0.0, None, 0)
+    hip.conv_autotune(-1)
+    try:
+        hip._check(hip.lib.eddlhip_conv2d_fwd_noalloc(*args(O1)))
+        kernel = hip.last_conv_kernel()
+        hip.conv_tuned_load(str(path))
+        hip.conv_autotune(True)
+        hip._check(hip.lib.eddlhip_conv2d_fwd_noalloc(*args(O2)))
+        assert hip.last_conv_kernel() == kernel
+        assert np.array_equal(O1.numpy(), O2.numpy())
+    finally:
+        hip.conv_autotune(-1)

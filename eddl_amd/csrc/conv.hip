@@ -2362,8 +2362,8 @@ constexpr int SPLIT_TILE0 = 16;
 bool is_split_tile(int tile) { return tile >= SPLIT_TILE0 && tile < SPLIT_TILE0 + NUM_SPLIT; }
 // The upsampled-input form in the split arithmetic (conv_up_split.h): plan "tiles" 33 (128 filters x 64 blocks) and 34 (64 x 128, half
 // of a 128-filter tile would idle under 64 filters).  Measured, us, the best of the fp32 and of the direct split plans before -> this
-// (4 images, stored side x channels -> filters): 32 x 1024 -> 512 314 -> 203, 64 x 512 -> 256 280 -> 179, 128 x 256 -> 128 288 -> 182 (34: 192),
-// 256 x 128 -> 64 314 -> 225 (33: 339); 1 image: 23 x 1024 -> 512 67 -> 57, 184 x 128 -> 64 62 -> 42.
+// (4 images, stored side x channels -> filters): 32 x 1024 -> 512 314 -> 195, 64 x 512 -> 256 280 -> 182, 128 x 256 -> 128 288 -> 186 (34: 201),
+// 256 x 128 -> 64 314 -> 232 (33: 354); 1 image: 184 x 128 -> 64 62 -> 44.
 struct UpSplitVariant {
     const char *name;
     int fm, fn;  // filters and blocks of a workgroup over 32

@@ -1,8 +1,13 @@
 // The 2x2 convolution of an image upsampled twice (conv_up2x2_kernel) in the split arithmetic of conv_split.h (included by conv.hip
 // only): the nine weight sums per filter and channel, added up in 64 bits, and the stored pixels are split into three
-// bf16 numbers, the six largest products summed in one fp32 accumulator per output, the smallest first - six roundings per 16
-// channels and tap where the fp32 instruction makes eight.  What the instruction's rounding downwards adds to every sum
-// cancels as in wino_split.h: opposite signs in the middle half of the steps, and for the outputs (0,1) and (1,0) of a block.
+// bf16 numbers, the six largest products of two such sums summed in fp32, the smallest first.  The instruction rounds what it
+// shifts out on the way to an accumulator downwards and several times a step, so that products added straight to the long sums are up to
+// 14 % further from 64 bits than the fp32 kernel's behind a ReLU: as in wino_split.h the products of 16 channels (of one to three
+// weight sums of a parity) are summed from zero and added to the long sum by vector instructions, rounded once and to nearest.
+// What remains of the bias has opposite signs for the outputs (0,1) and (1,0) of a block and for every other block of a plane.
+// Error against 64 bits behind a ReLU relative to the outputs' root mean square, of the fp32 kernel -> of this one (in brackets with the products
+// added straight to the long sums): 16 channels 9.0e-8 -> 4.4e-8 (7.2e-8), 128 2.2e-7 -> 1.0e-7 (2.4e-7), 512 4.2e-7 -> 1.7e-7 (4.7e-7), 1024
+// 6.1e-7 -> 2.5e-7 (7.0e-7); of the mean of a plane at 512 channels 1.9e-8 -> 5.0e-9 (3.2e-8).
 
 constexpr int UPSPLIT_UNIT = 9 * SPLIT_UNIT;  // bytes of 32 filters x 16 channels, all nine weight sums
 
@@ -43,6 +48,11 @@ __global__ __launch_bounds__(256) void up2x2_split_filter_kernel(const float *__
     }
 }
 
+template <typename F, int... I>
+__device__ __forceinline__ void for_each_index(std::integer_sequence<int, I...>, F f) {
+    (f(std::integral_constant<int, I>()), ...);
+}
+
 // One 32x32 block of one parity's sums once more with the fp32 instruction (see split_tile_again), channels [c_lo, c_hi): this
 // lane's filter m, the byte offsets of its block's four stored pixels.
 __device__ __forceinline__ void up2x2_block_again(const ConvParams &p, floatx16 &sum, __amdgpu_buffer_rsrc_t in, int m, const int (&voff)[4], int parity, int c_lo,
@@ -68,9 +78,12 @@ __device__ __forceinline__ void up2x2_block_again(const ConvParams &p, floatx16 
 // (128 registers).  A K-step is 32 channels: their four stored pixels per block come one tap after the other as in
 // conv_split_kernel (loaded a tap ahead, split between the matrix instructions on their way into LDS), and tap t is multiplied by the
 // weight sums that see it - 4, 2, 2 and 1 of the nine - straight from L2, the next sum's requested while the current one
-// multiplies.  216 matrix instructions of a wavefront share four reads of the pixels, so there is one vector instruction per matrix
-// instruction: bound by the matrix pipe, 42-52 % of the bf16 instruction's rate at 2.4 GHz (256 -> 128 on 128x128, 4 images: 182 us for
-// 232 GFLOP of bf16 products; the fp32 kernel 288).
+// multiplies.  216 matrix instructions of a wavefront share four reads of the pixels; their splitting and the additions to the long
+// sums are three to four vector instructions per matrix instruction.  Measured (4 images, us, with the products added straight to the
+// long sums -> this): 1024 -> 512 on 32x32 193 -> 195, 512 -> 256 on 64x64 171 -> 182, 256 -> 128 on 128x128 175 -> 186, 128 -> 64 on
+// 256x256 (64 x 128 tile) 218 -> 232; the fp32 kernel 314, 280, 288, 314.  256 -> 128 is 232 GFLOP of bf16 products: half of the bf16
+// instruction's rate at 2.4 GHz.
+// All 256 registers are taken; three values of either build lie in scratch.
 template <int WM, int WN>
 __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvParams p) {
     static_assert(WM * WN == 4, "four wavefronts per workgroup");
@@ -107,35 +120,30 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
     int voff[4];
     pixels_of(n0 + pix, voff);
     float raw[CHUNKS][8];
-    auto load_pixels = [&](int step, int tap) __attribute__((always_inline)) {
+    auto load_pixels = [&](int step, int tap, int chunk) __attribute__((always_inline)) {
+        const int c0 = step * SPLIT_K + (kgroup + chunk) * 8;
+        const bool there = c0 < p.C;  // (past the last channel, and behind the last step: zeros, without touching memory)
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)p.I, 0, there ? p.in_bytes : 0u, RSRC_WORD3);
+        int soff = there ? c0 * HW4 : 0;
 #pragma unroll
-        for (int chunk = 0; chunk < CHUNKS; chunk++) {
-            const int c0 = step * SPLIT_K + (kgroup + chunk) * 8;
-            const bool there = c0 < p.C;  // (past the last channel, and behind the last step: zeros, without touching memory)
-            const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)p.I, 0, there ? p.in_bytes : 0u, RSRC_WORD3);
-            int soff = there ? c0 * HW4 : 0;
-#pragma unroll
-            for (int j = 0; j < 8; j++, soff += HW4) raw[chunk][j] = buf_load(rsrc, voff[tap], soff);
-        }
+        for (int j = 0; j < 8; j++, soff += HW4) raw[chunk][j] = buf_load(rsrc, voff[tap], soff);
     };
-    const SignOfStep sign(step_lo, step_hi);
-    auto put_pixels = [&](int buf, int step) __attribute__((always_inline)) {
-        const float up = sign.negative(step) ? -SPLIT_UP : SPLIT_UP;
+    // every other block of a plane is accumulated with the opposite sign
+    auto odd_block = [&](int n) { return ((n / p.wtw + n % p.wtw - n / per_img * p.wth) & 1) != 0; };
+    const float up = odd_block(n0 + pix) ? -SPLIT_UP : SPLIT_UP;
+    auto put_pixels = [&](int buf, int chunk) __attribute__((always_inline)) {
+        uintx4 hi, mid, lo;
 #pragma unroll
-        for (int chunk = 0; chunk < CHUNKS; chunk++) {
-            uintx4 hi, mid, lo;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                unsigned h, m, l;
-                split_pair(up * raw[chunk][2 * j], up * raw[chunk][2 * j + 1], h, m, l);
-                hi[j] = h;
-                mid[j] = m;
-                lo[j] = l;
-            }
-            Bs[buf][0][kgroup + chunk][pix] = hi;
-            Bs[buf][1][kgroup + chunk][pix] = mid;
-            Bs[buf][2][kgroup + chunk][pix] = lo;
+        for (int j = 0; j < 4; j++) {
+            unsigned h, m, l;
+            split_pair(up * raw[chunk][2 * j], up * raw[chunk][2 * j + 1], h, m, l);
+            hi[j] = h;
+            mid[j] = m;
+            lo[j] = l;
         }
+        Bs[buf][0][kgroup + chunk][pix] = hi;
+        Bs[buf][1][kgroup + chunk][pix] = mid;
+        Bs[buf][2][kgroup + chunk][pix] = lo;
     };
 
     const int a_voff = lane * 16, a_base = (m0 / 32 + wm) * UPSPLIT_UNIT, a_k16 = p.Mp / 32 * UPSPLIT_UNIT;
@@ -143,14 +151,15 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
     auto load_a = [&](int set, int k16, int row) __attribute__((always_inline)) {
 #pragma unroll
         for (int part = 0; part < 3; part++)
-            a[set][part] = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, a_voff + part * 1024, a_base + k16 * a_k16 + row * SPLIT_UNIT, 0));
+            a[set][part] = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, a_voff, a_base + k16 * a_k16 + row * SPLIT_UNIT + part * 1024, 0));
     };
-    load_pixels(step_lo, 0);
+#pragma unroll
+    for (int chunk = 0; chunk < CHUNKS; chunk++) load_pixels(step_lo, 0, chunk);
     load_a(0, 2 * step_lo, 0);
     ChannelEpilogue chan = {0.0f, 0.0f, 1.0f, 1.0f, 0.0f};
     if (!split) chan = fetch_channel_constants<BM>(p, m0, tid);
-    put_pixels(0, step_lo);
-    load_pixels(step_lo, 1);
+#pragma unroll
+    for (int chunk = 0; chunk < CHUNKS; chunk++) put_pixels(0, chunk), load_pixels(step_lo, 1, chunk);
     if (!split) put_channel_constants<BM>(epi, chan, tid);
 
     floatx16 acc[4][TN];  // [parity 2 i + j][block group]
@@ -163,71 +172,68 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
     __syncthreads();
     trace_mark(p, 1);
 
-    // tap t's weight sums and the parities they belong to
-    constexpr int kSums[4] = {4, 2, 2, 1}, kRow[4][4] = {{0, 1, 3, 5}, {2, 6, 0, 0}, {4, 7, 0, 0}, {8, 0, 0, 0}}, kParity[4][4] = {{0, 1, 2, 3}, {1, 3, 0, 0}, {2, 3, 0, 0}, {3, 0, 0, 0}};
+    // The step's 18 groups of products: tap, 16 channels and the parity that they belong to, two or three in a row of one parity where
+    // that can be, as their products are added up before they go to the long sum
+    constexpr int GROUPS = 18;
+    constexpr int kTap[GROUPS] = {0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1, 2, 2, 2, 2, 3, 3}, kHalf[GROUPS] = {0, 0, 0, 0, 1, 1, 1, 1, 0, 0, 1, 1, 0, 0, 1, 1, 0, 1};
+    constexpr int kParity[GROUPS] = {0, 1, 2, 3, 3, 2, 0, 1, 1, 3, 1, 3, 3, 2, 2, 3, 3, 3}, kRow[4][4] = {{0, 1, 3, 5}, {0, 2, 0, 6}, {0, 0, 4, 7}, {0, 0, 0, 8}};  // [tap][parity]
     constexpr int kA[6] = {2, 1, 1, 0, 0, 0}, kB[6] = {0, 1, 0, 2, 1, 0};  // the smallest products first
     uintx4 b[TN][3];
-    // weight sum s of tap TAP and 16 channels G of a step; the filters of the sum after it are requested first
-    auto one_sum = [&](int step, int next, auto tap_c, auto g_c, auto s_c) __attribute__((always_inline)) {
-        constexpr int TAP = decltype(tap_c)::value, G = decltype(g_c)::value, S = decltype(s_c)::value;
-        constexpr bool last_s = S + 1 == kSums[TAP], last_g = last_s && G == 1;
-        constexpr int tap_n = last_g ? (TAP + 1) & 3 : TAP, g_n = last_s ? G ^ 1 : G, s_n = last_s ? 0 : S + 1;
-        // (a tap has an even number of pairs, of its four, two, two and one sums twice)
-        constexpr int set = (G * kSums[TAP] + S) & 1, parity = kParity[TAP][S];
-        if constexpr (S == 0) {
+    floatx16 own[TN];  // the products of a run of groups of one parity
 #pragma unroll
-            for (int part = 0; part < 3; part++)
+    for (int v = 0; v < 16; v++) own[1][v] = 0.0f;
+    auto add_own = [&](int parity, int tn) __attribute__((always_inline)) {
 #pragma unroll
-                for (int tn = 0; tn < TN; tn++) b[tn][part] = Bs[TAP & 1][part][2 * G + half][wn * 64 + tn * 32 + (lane & 31)];
-        }
-        load_a(set ^ 1, 2 * (last_g && TAP == 3 ? next : step) + g_n, kRow[tap_n][s_n]);
+        for (int v = 0; v < 16; v++) acc[parity][tn][v] = __fadd_rn(acc[parity][tn][v], own[tn][v]);
+    };
+    // Group I of a step; the filters of the group after it are requested first.  Products of 32 blocks are added to their long sum
+    // while those of the next 32 multiply: the second 32 blocks' in the next group.
+    auto group = [&](int step, int next, auto i_c) __attribute__((always_inline)) {
+        constexpr int I = decltype(i_c)::value, N = (I + 1) % GROUPS, B = (I + GROUPS - 1) % GROUPS;
+        constexpr int tap = kTap[I], g = kHalf[I], parity = kParity[I], set = I & 1;
+        constexpr bool fresh = tap != kTap[B] || g != kHalf[B];
+        // (the build with twice the pixels in flight has the registers for runs of one group only: with longer ones it spills in the loop, 350 us instead of 232)
+        constexpr bool run_starts = CHUNKS == 2 || parity != kParity[B], run_ends = CHUNKS == 2 || parity != kParity[N];
+        constexpr bool put = fresh && g < CHUNKS;  // the next tap's pixels into the other buffer, those of the tap after it in their place
+        const floatx16 zero = {0.0f};
+        load_a(set ^ 1, 2 * (N == 0 ? next : step) + kHalf[N], kRow[kTap[N]][kParity[N]]);
 #pragma unroll
-        for (int k = 0; k < 6; k++)
+        for (int tn = 0; tn < TN; tn++) {
+            if (fresh) {
 #pragma unroll
-            for (int tn = 0; tn < TN; tn++)
-                acc[parity][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[set][kA[k]]), __builtin_bit_cast(bf16x8, b[tn][kB[k]]), acc[parity][tn], 0, 0, 0);
-        if constexpr (G == 0 && S == 0) {
-            // the next tap's pixels into the other buffer, those of the tap after it in their place
-            put_pixels((TAP & 1) ^ 1, TAP < 3 ? step : step + 1);
-            load_pixels(TAP < 2 ? step : step + 1, (TAP + 2) & 3);
-#pragma unroll
-            for (int i = 0; i < 12; i++) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 5 * CHUNKS, 0);
+                for (int part = 0; part < 3; part++) b[tn][part] = Bs[tap & 1][part][2 * g + half][wn * 64 + tn * 32 + (lane & 31)];
             }
+            if (tn == 0 ? run_starts : run_ends) add_own(tn == 0 ? kParity[B] : parity, tn ^ 1);
+#pragma unroll
+            for (int k = 0; k < 6; k++)
+                own[tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[set][kA[k]]), __builtin_bit_cast(bf16x8, b[tn][kB[k]]), k == 0 && run_starts ? zero : own[tn],
+                                                                  0, 0, 0);
+            if (put && tn == 0) put_pixels((tap & 1) ^ 1, g);
+            if (put && tn == 1) load_pixels(tap < 2 ? step : step + 1, (tap + 2) & 3, g);
+#pragma unroll
+            for (int i = 0; i < 6; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (put && tn == 0 && i > 0) __builtin_amdgcn_sched_group_barrier(0x002, 13, 0);
+                else if (i > 0 && i < 5) __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (tap != kTap[N]) __syncthreads();
     };
-    auto one_tap = [&](int step, int next, auto tap_c) __attribute__((always_inline)) {
-        constexpr int N = kSums[decltype(tap_c)::value];
-        auto group = [&](auto g_c) __attribute__((always_inline)) {
-            one_sum(step, next, tap_c, g_c, std::integral_constant<int, 0>());
-            if constexpr (N > 1) one_sum(step, next, tap_c, g_c, std::integral_constant<int, 1>());
-            if constexpr (N > 2) one_sum(step, next, tap_c, g_c, std::integral_constant<int, 2>());
-            if constexpr (N > 3) one_sum(step, next, tap_c, g_c, std::integral_constant<int, 3>());
-        };
-        group(std::integral_constant<int, 0>());
-        group(std::integral_constant<int, 1>());
-        __syncthreads();
-    };
-    for (int run_lo = step_lo, run_hi; run_lo < step_hi; run_lo = run_hi) {  // (one to three runs of steps of one sign)
-        run_hi = sign.run_end(run_lo, step_hi);
-        for (int step = run_lo; step < run_hi; step++) {
-            const int next = step + 1 < step_hi ? step + 1 : step;
-            one_tap(step, next, std::integral_constant<int, 0>());
-            one_tap(step, next, std::integral_constant<int, 1>());
-            one_tap(step, next, std::integral_constant<int, 2>());
-            one_tap(step, next, std::integral_constant<int, 3>());
-        }
-        if (run_hi < step_hi) negate(acc);
+    for (int step = step_lo; step < step_hi; step++) {
+        const int next = step + 1 < step_hi ? step + 1 : step;
+        for_each_index(std::make_integer_sequence<int, GROUPS>(), [&](auto i_c) __attribute__((always_inline)) { group(step, next, i_c); });
     }
-    const float down = sign.negative(step_hi - 1) ? -SPLIT_DOWN : SPLIT_DOWN;
+    add_own(3, 1);
     trace_mark(p, 2);
 
-    const int m_first = m0 + wm * 32 + (lane & 31);
+    // (the lane's number once more, so that nothing that follows from it lives through the loop: registers)
+    const int lane_e = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), half_e = lane_e >> 5;
+    const int m_first = m0 + wm * 32 + (lane_e & 31);
     auto finish = [&](auto tn_c) __attribute__((always_inline)) {
         constexpr int tn = decltype(tn_c)::value;
         const int n_first = n0 + wn * 64 + tn * 32;
+        const float down = odd_block(n_first + (lane_e & 31)) ? -SPLIT_DOWN : SPLIT_DOWN;
         floatx16 y[2][2];
         float finite = 0.0f;
 #pragma unroll
@@ -240,11 +246,11 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
         if (__any(finite != 0.0f)) {
             const __amdgpu_buffer_rsrc_t in = __builtin_amdgcn_make_buffer_rsrc((void *)p.I, 0, p.in_bytes, RSRC_WORD3);
             int at[4];
-            pixels_of(n_first + (lane & 31), at);
+            pixels_of(n_first + (lane_e & 31), at);
 #pragma unroll 1
             for (int e = 0; e < 4; e++) {
                 floatx16 sum;
-                up2x2_block_again(p, sum, in, m_first, at, e, step_lo * SPLIT_K, step_hi * SPLIT_K, half);
+                up2x2_block_again(p, sum, in, m_first, at, e, step_lo * SPLIT_K, step_hi * SPLIT_K, half_e);
 #pragma unroll
                 for (int s = 0; s < 4; s++)
 #pragma unroll
@@ -257,11 +263,11 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
         if (split) {
             // this slice's share, raw: wino_fused_reduce_kernel's layout
             const size_t tiles = (gridDim.x - (unsigned)p.main_tiles) / p.nslices;
-            floatx4 *dst = reinterpret_cast<floatx4 *>(p.partial) + (((size_t)slice * tiles + local_tile) * (WM * 2 * WN) + wm * (2 * WN) + wn * 2 + tn) * 16 * 64 + lane;
+            floatx4 *dst = reinterpret_cast<floatx4 *>(p.partial) + (((size_t)slice * tiles + local_tile) * (WM * 2 * WN) + wm * (2 * WN) + wn * 2 + tn) * 16 * 64 + lane_e;
 #pragma unroll
             for (int v = 0; v < 16; v++) dst[v * 64] = (floatx4){y[0][0][v], y[0][1][v], y[1][0][v], y[1][1][v]};
         } else {
-            wino_store_tile<BM>(p, y, epi, m0, wm * 32, n_first, lane);
+            wino_store_tile<BM>(p, y, epi, m0, wm * 32, n_first, lane_e);
         }
     };
     finish(std::integral_constant<int, 0>());

@@ -62,30 +62,6 @@ __global__ __launch_bounds__(256) void wino_split_filter_kernel(const float *__r
     }
 }
 
-// The sign that the steps [lo, hi) of a sum are accumulated with: the first quarter and the last are added, what lies between is
-// subtracted from the negated sum, so that an error of one sign per step cancels, also one that grows with the steps linearly.
-struct SignOfStep {
-    int first, second;  // the sign changes in front of these steps
-    __device__ __forceinline__ SignOfStep(int lo, int hi) {
-        const int n = hi - lo;
-        // (below eight steps too little comes together to be worth the two negations: 64 channels 5 % of the time)
-        first = n < 8 ? hi : lo + (n + 2) / 4;
-        second = n < 8 ? hi : first + (n + 1) / 2;
-    }
-    __device__ __forceinline__ bool negative(int step) const { return step >= first && step < second; }
-    // the end of the run of steps of one sign that `step` is in
-    __device__ __forceinline__ int run_end(int step, int hi) const { return min(step < first ? first : (step < second ? second : hi), hi); }
-};
-template <int A, int B>
-__device__ __forceinline__ void negate(floatx16 (&sum)[A][B]) {
-#pragma unroll
-    for (int a = 0; a < A; a++)
-#pragma unroll
-        for (int b = 0; b < B; b++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) sum[a][b][v] = -sum[a][b][v];
-}
-
 constexpr int WSPLIT_UNIT = 16 * SPLIT_UNIT;  // bytes of 32 filters x 16 channels, all positions
 
 // One 32x32 block of one position's sums once more with the fp32 instruction (see split_tile_again), channels [c_lo, c_hi), from

@@ -1770,6 +1770,36 @@ def test_conv2d_upsampled_2x2_split_is_no_further_from_64_bits_than_the_fp32_one
     assert_conv_close(ref, got, case)
 
 
+@pytest.mark.parametrize("plan", [(33, 1), (33, 4), (34, 1)])
+@pytest.mark.parametrize("C,H,W", [(16, 40, 40), (48, 32, 28), (64, 32, 32), (128, 20, 26), (256, 20, 20), (512, 11, 13), (1024, 12, 12)])
+def test_conv2d_upsampled_2x2_split_behind_a_relu(hip, C, H, W, plan):
+    """Pixels as deep layers have them behind a ReLU (the split Winograd form's test): outputs, each of the four of a stored pixel by itself, and
+    the means of planes are no further from 64 bits than with the fp32 kernel of this form, and no error is common to all planes."""
+    rng = np.random.default_rng(2060 + C + W)
+    N, Kf = max(2, 1024 // (H * W)), 64
+    g = rng.standard_normal((N, C, H + 2, W + 2))
+    smooth = sum(g[:, :, a:a + H, b:b + W] for a in range(3) for b in range(3)) / 3.0
+    x = np.maximum(rng.standard_normal((N, C, 1, 1)) + 0.25 * smooth, 0.0).astype(np.float32)
+    w = (rng.standard_normal((Kf, C, 2, 2)) * np.sqrt(2.0 / (C * 4))).astype(np.float32)
+    X, Wd, O, err, part = hip.array(x), hip.array(w), hip.full((N, Kf, 2 * H, 2 * W), np.nan), {}, {}
+    ref = _conv64_upsampled(x, w, 2 * H, 2 * W)
+    try:
+        for p in ((UP2X2_FORM, 1), plan):
+            hip.force_conv_plan(*p)
+            hip.fill_(O, np.nan)
+            hip.conv2D(X, Wd, None, O, 1, 1, 0, 0, upsample=(2, 2))
+            got = O.numpy()
+            err[p[0]] = _errors_behind_a_relu(got, ref)
+            part[p[0]] = [_errors_behind_a_relu(got[:, :, i::2, j::2], ref[:, :, i::2, j::2])[0] for i in (0, 1) for j in (0, 1)]
+        assert "conv_up2x2_split" in hip.last_conv_kernel()
+    finally:
+        hip.force_conv_plan(-1, 1)
+    fp32, split = err[UP2X2_FORM], err[plan[0]]
+    print("C %d %dx%d plan %s: fp32 %.2e planes %.2e mean %.1e, split %.2e planes %.2e mean %.1e" % ((C, H, W, plan) + fp32 + split), flush=True)
+    assert split[0] <= fp32[0] and split[1] <= fp32[1] and all(a <= b for a, b in zip(part[plan[0]], part[UP2X2_FORM]))
+    assert split[2] <= 0.1 * fp32[1]
+
+
 @pytest.mark.parametrize("plan", [(33, 1), (34, 2)])
 def test_conv2d_upsampled_2x2_split_keeps_what_is_not_finite_and_the_largest_numbers(hip, plan):
     """What the fp32 kernel of this form gives, and not a bit of an output whose pixels are finite."""

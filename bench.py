@@ -42,7 +42,12 @@ def form_of_plan(tile):
 
 def peak_of_form(form):
     """What a layer's kernel could multiply at most, in TFLOP/s of fp32 products."""
-    return PEAK_SPLIT_TFLOPS if form in ("split", "winograd_split", "upsampled2x2_split") else PEAK_FP32_MFMA_TFLOPS
+    return PEAK_SPLIT_TFLOPS if is_split_form(form) else PEAK_FP32_MFMA_TFLOPS
+
+
+def is_split_form(form):
+    """The forms that multiply on the bf16 matrix instructions, six products for one of fp32."""
+    return form is not None and form.endswith("split")
 
 WORKLOADS = {
     # name -> (builder kwargs, seed, input distribution, description)
@@ -277,7 +282,7 @@ def measure(hip, workload, steps, warmup, fused=True, graph=False, tune=True, pl
                 conv = [l for l in op.layers if "cd" in l.attrs][0].attrs["cd"]
                 n_out, kf = conv.out_shape[0] * conv.out_shape[2] * conv.out_shape[3], conv.out_shape[1]
                 c_in = op.flops // (2 * conv.kr * conv.kc * n_out * kf)
-                kernel_flops, form = 2 * 9 * kf * c_in * blocks, "upsampled2x2_split" if kern.startswith("conv_up2x2_split") else "upsampled2x2"
+                kernel_flops, form = 2 * 9 * kf * c_in * blocks, "upsampled_2x2_split" if kern.startswith("conv_up2x2_split") else "upsampled_2x2"
             row.update(kernel=kern.split(" +ksplit")[0], kernel_ms=kms, kernel_launches=kl, kernel_flops=kernel_flops, form=form,
                        kernel_peak_tflops=peak_of_form(form))
         if op.kind in ("conv2d", "dense") and ms > 0:
@@ -346,7 +351,7 @@ def measure(hip, workload, steps, warmup, fused=True, graph=False, tune=True, pl
                               "executed_gflop": executed_flops / 1e9,
                               "mfma_util": mfma_ms / conv_ms if conv_ms else 0.0,
                               "winograd_layers": sum(1 for r in conv_rows if r.get("form") in ("winograd", "winograd_split")),
-                              "split_layers": sum(1 for r in conv_rows if r.get("form") in ("split", "winograd_split", "upsampled2x2_split"))},
+                              "split_layers": sum(1 for r in conv_rows if is_split_form(r.get("form")))},
                "device_ms_sum_of_ops": sum(op_ms), "plans": plans_info, "workspace_bytes": hip.workspace_bytes()}
     del model
     return summary, rows, out_host, desc
@@ -454,7 +459,7 @@ def main():
         roofline["device_probe"] = {"unit": "TFLOP/s", "pure_mfma_constant_operands": const_mean,
                                     "pure_mfma_varying_operands_mean": vary_mean, "varying_best_launch": vary_best,
                                     "varying_worst_launch": vary_worst,
-                                    "frac_of_varying_mean": achieved / vary_mean if vary_mean > 0 and roofline["form"] not in ("split", "winograd_split", "upsampled2x2_split") else None}
+                                    "frac_of_varying_mean": achieved / vary_mean if vary_mean > 0 and not is_split_form(roofline["form"]) else None}
         # and what plain read / write / copy streams over 1 GiB buffers sustain, beside the 8 TB/s HBM peak
         rd, wr, cp = hip.probe_hbm(1 << 30)
         roofline["device_probe"].update(hbm_unit="GB/s", hbm_read_stream=rd, hbm_write_stream=wr, hbm_copy_stream=cp)
@@ -514,7 +519,7 @@ def main():
         table.append("%-44s %9.4f %9s %8s %9.1f %7.2f  %s" % (
             r["name"][:44], r["ms"], "%.2f" % r["tflops"] if "tflops" in r else "-",
             "%.1f" % (100 * r["frac_fp32_mfma_peak"]) if "tflops" in r else "-", r.get("gbs", 0.0), 100 * r.get("frac_hbm_peak", 0.0),
-            {"winograd": "winograd: ", "winograd_split": "winograd split: ", "upsampled2x2": "upsampled 2x2: ", "upsampled2x2_split": "upsampled 2x2 split: ", "split": "split: "}.get(r.get("form"), "") + r.get("kernel", "")))
+            {"winograd": "winograd: ", "winograd_split": "winograd split: ", "upsampled_2x2": "upsampled 2x2: ", "upsampled_2x2_split": "upsampled 2x2 split: ", "split": "split: "}.get(r.get("form"), "") + r.get("kernel", "")))
     if args.layers:
         print("\n".join(table), file=sys.stderr)
     out_dir = args.out

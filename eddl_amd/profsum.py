@@ -15,6 +15,7 @@ import csv
 import glob
 import json
 import os
+import re
 import subprocess
 import sys
 
@@ -22,6 +23,7 @@ HBM_PEAK_GBS = 8000.0
 FP32_MFMA_PEAK_TFLOPS = 157.3
 BF16_MFMA_PEAK_TFLOPS = 16 * FP32_MFMA_PEAK_TFLOPS
 COPY_PROBE_KIB = 262144.0  # bench.py --copy-probe: one ReLU over 2^26 floats reads 256 MiB and writes 256 MiB
+SPLIT_TAPS = ("UPSAMPLED", "STORED", "ONE_TAP")  # the enumerators of SplitTaps (csrc/conv_split.h), in their order
 HOT = ("conv_", "wino_", "maxpool", "avgpool", "dense", "bn_", "add_kernel", "concat", "scale_", "unary_kernel", "pad_", "softmax", "upsample")
 
 
@@ -78,6 +80,13 @@ def short(name, width):
     return name.replace("void (anonymous namespace)::", "").replace("(anonymous namespace)::", "")[:width]
 
 
+def library_name(name):
+    """A kernel's name as the library and the trace both have it: the trace spells out a defaulted last template argument and writes
+    enumerators as numbers."""
+    name = name.replace(" ", "").replace(",false>", ">")
+    return re.sub(r"\((?:\(anonymousnamespace\)::)?SplitTaps\)(\d)", lambda m: SPLIT_TAPS[int(m.group(1))], name)
+
+
 def mean(values):
     return sum(values) / len(values)
 
@@ -114,11 +123,12 @@ def trace(workload, trace_dir, log, out, extra=""):
               "  value %.1f %s, %.3f ms/step" % (bench["value"], bench["unit"], bench["ms_per_step"]),
               "  roofline kernel %s: %s launches/step, avg launch %.4f ms (HIP events inside bench.py), achieved %.2f %s = %.1f%% of %.1f"
               % (rf["kernel"], rf.get("launches_per_step"), rf.get("avg_launch_ms", 0.0), rf["achieved"], rf["unit"], 100 * rf["frac"], rf["peak"])]
-        key = rf["kernel"].replace(" ", "")
-        # (the trace spells out a kernel's defaulted last template argument, the library's name for it does not)
-        dom = [r for r in stats if key in r["Name"].replace(" ", "").replace(",false>", ">")]
+        key = library_name(rf["kernel"])
+        dom = [r for r in stats if key in library_name(r["Name"])]
         if dom:
             o.append("  same kernel in the trace above: average %.4f ms over %s calls" % (float(dom[0]["AverageNs"]) / 1e6, dom[0]["Calls"]))
+        else:
+            o.append("  same kernel in the trace above: NOT FOUND")
     write(out, o, workload)
 
 
@@ -258,7 +268,7 @@ def stalls(workload, sq_dir, tcp_dir, out):
          "",
          "%-64s %6s %9s %10s %9s %9s %7s %10s %10s" % ("kernel", "calls", "avg us", "mfma busy", "wait any", "wait lds", "issue", "tcp stall", "valu/vmem")]
     for k in a["SQ_WAVE_CYCLES"]:
-        if not ("conv_" in k or "wino_fused_kernel" in k) or k not in b["SQ_WAVE_CYCLES" if "SQ_WAVE_CYCLES" in b else "SQ_WAIT_ANY"]:
+        if not any(t in k for t in ("conv_", "wino_fused_kernel", "wino_split_kernel")) or k not in b["SQ_WAVE_CYCLES" if "SQ_WAVE_CYCLES" in b else "SQ_WAIT_ANY"]:
             continue
         m = lambda d, n: mean(d[n][k])
         cyc_a, cyc_b = m(a, "GRBM_GUI_ACTIVE") / 8.0, m(b, "GRBM_GUI_ACTIVE") / 8.0

@@ -105,3 +105,49 @@ def test_matrix_counter_table_counts_the_split_kernel_in_bf16_products(tmp_path)
     for name, ops, peak in (("conv_split_kernel", 2e7, 16 * 157.3), ("conv_tap_kernel", 2e6, 157.3)):
         rate = ops * 512 / 10e-6 / 1e12        # TFLOP/s of a 10 us dispatch
         assert float(rows[name][3]) == round(rate, 1) and float(rows[name][4]) == round(100 * rate / peak, 1)
+
+
+def test_stall_table_and_trace_find_the_split_kernels_under_the_traces_names(tmp_path):
+    """Every convolution kernel has its row of stall counters, and the benchmark's dominant kernel is found in a trace that writes enumerators as numbers."""
+    import json
+    import os
+    import re
+    from eddl_amd import profsum
+    split = "conv_split_kernel<4, 1, 1, 2, 3, ((anonymous namespace)::SplitTaps)2>"
+    names = ["void (anonymous namespace)::%s((anonymous namespace)::ConvParams)" % k for k in
+             (split, "wino_split_kernel<true>", "wino_fused_kernel<2, 1, 4, 3, true>", "conv_up2x2_split_kernel<4, 1>", "softmax_kernel")]
+    for d, counters in (("sq", profsum.STALL_SQ), ("tcp", profsum.STALL_TCP)):
+        os.makedirs(str(tmp_path / d))
+        with open(tmp_path / d / "m_counter_collection.csv", "w") as fh:
+            fh.write("Dispatch_Id,Kernel_Name,Counter_Name,Counter_Value\n")
+            for i, k in enumerate(names):
+                for c in counters.split():
+                    fh.write('%d,"%s",%s,1000\n' % (i, k, c))
+        with open(tmp_path / d / "m_kernel_trace.csv", "w") as fh:
+            fh.write("Kernel_Name,Start_Timestamp,End_Timestamp\n")
+            for k in names:
+                fh.write('"%s",1000,11000\n' % k)
+    profsum.stalls("vgg16", str(tmp_path / "sq"), str(tmp_path / "tcp"), str(tmp_path / "stalls.txt"))
+    text = open(tmp_path / "stalls.txt").read()
+    assert all(re.search("^%s<" % k, text, re.M) for k in ("conv_split_kernel", "wino_split_kernel", "wino_fused_kernel", "conv_up2x2_split_kernel"))
+    assert not re.search("^softmax", text, re.M)
+
+    with open(tmp_path / "t_kernel_stats.csv", "w") as fh:
+        fh.write("Name,Calls,TotalDurationNs,AverageNs,Percentage\n")
+        for i, k in enumerate(names):
+            fh.write('"%s",%d,1000,%d000,10\n' % (k, i + 1, i + 1))
+    for kernel, found in (("conv_split_kernel<4,1,1,2,3,ONE_TAP>", "average 0.0010 ms over 1 calls"), ("wino_split_kernel<true>", "average 0.0020 ms over 2 calls"),
+                          ("wino_fused_kernel<2,1,4,3,true>", "average 0.0030 ms over 3 calls"), ("conv_split_kernel<4,1,1,2,3,STORED>", "NOT FOUND")):
+        (tmp_path / "bench.log").write_text(json.dumps({"metric": "x", "value": 1.0, "unit": "u", "ms_per_step": 1.0,
+                                                        "roofline": {"kernel": kernel, "achieved": 1.0, "unit": "TFLOP/s", "frac": 0.1, "peak": 10.0}}) + "\n")
+        profsum.trace("vgg16", str(tmp_path), str(tmp_path / "bench.log"), str(tmp_path / "trace.txt"))
+        assert "same kernel in the trace above: %s" % found in open(tmp_path / "trace.txt").read()
+
+
+def test_a_form_has_one_name_and_its_peak():
+    import bench
+    for tile in (16, 19, 32, 33, 34):
+        assert bench.peak_of_form(bench.form_of_plan(tile)) == pytest.approx(16 * 157.3 / 6)
+    for tile in (-1, 0, 3, 4, 5, 6, 7, 8, 9):
+        assert bench.peak_of_form(bench.form_of_plan(tile)) == 157.3
+    assert bench.peak_of_form(None) == 157.3

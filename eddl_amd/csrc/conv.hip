@@ -2317,12 +2317,11 @@ struct FusedVariant {
     void (*kernel)(const ConvParams);
     void (*kernel_wide)(const ConvParams);  // the build that loads the pixels 16 bytes per lane (conv2d_winograd_fused decides)
     void (*reduce)(const ConvParams);
-    int threads;
     bool split;  // on the bf16 matrix instructions (wino_split.h)
 };
 #define FUSED(FM, FN, CK, WPE)                                                                                                       \
     {"wino_fused_kernel<" #FM "," #FN "," #CK "," #WPE ">", "wino_fused_kernel<" #FM "," #FN "," #CK "," #WPE ",true>", FM, FN, CK,  \
-     wino_fused_kernel<FM, FN, CK, WPE, false>,         wino_fused_kernel<FM, FN, CK, WPE, true>, wino_fused_reduce_kernel<FM, FN>, 256, false}
+     wino_fused_kernel<FM, FN, CK, WPE, false>,         wino_fused_kernel<FM, FN, CK, WPE, true>, wino_fused_reduce_kernel<FM, FN>, false}
 const FusedVariant kfused[] = {FUSED(1, 1, 4, 4), FUSED(2, 1, 4, 3)};
 constexpr int NUM_FUSED = (int)(sizeof(kfused) / sizeof(kfused[0]));
 constexpr int FUSED_TILE0 = 6;      // plan "tile" numbers 6 .. 6 + NUM_FUSED - 1 name these shapes (0..3: direct tiles, 4 / 5: the other Winograd forms)
@@ -2332,7 +2331,7 @@ constexpr int FUSED_ROW_ALIGN = 8;  // the transformed filters are padded to who
 // launches are bound by reading them (512 channels on 14x14, best plans of the other forms / this one: 1 image 18.3 / 27.0 us,
 // 4 images 34.4 / 42.8, 8 images 56.0 / 59.4, 16 images 85.1 / 81.1; 1024 channels, 392 blocks 151 / 186, 1024 blocks 290 / 241).
 const FusedVariant kwsplit[] = {
-    {"wino_split_kernel<false>", "wino_split_kernel<true>", 2, 1, 16, wino_split_kernel<false>, wino_split_kernel<true>, wino_fused_reduce_kernel<2, 1>, 256, true}};
+    {"wino_split_kernel<false>", "wino_split_kernel<true>", 2, 1, 16, wino_split_kernel<false>, wino_split_kernel<true>, wino_fused_reduce_kernel<2, 1>, true}};
 constexpr int NUM_WSPLIT = (int)(sizeof(kwsplit) / sizeof(kwsplit[0]));
 constexpr int WSPLIT_TILE0 = 32;
 constexpr long long WSPLIT_SEARCH_BLOCKS = 512;
@@ -3867,7 +3866,7 @@ int conv2d_winograd_fused(bool no_alloc, bool *no_room, const FusedVariant &fv, 
         const long long wgs = q.main_tiles + split_tiles * q.nslices;
         q.trace = (g_trace != nullptr && wgs <= g_trace_wgs) ? g_trace : nullptr;
         EH_TRY(prof_begin(st));
-        hipLaunchKernelGGL(wide ? fv.kernel_wide : fv.kernel, dim3((unsigned)wgs), dim3(fv.threads), 0, st, q);
+        hipLaunchKernelGGL(wide ? fv.kernel_wide : fv.kernel, dim3((unsigned)wgs), dim3(256), 0, st, q);
         EH_CHECK_LAUNCH();
         EH_TRY(prof_end(st));
         if (split_tiles > 0) {

@@ -1641,6 +1641,30 @@ def test_conv2d_winograd_split_reads_two_tensors_in_both_builds_and_pools(hip, C
     assert_conv_close(_conv64_padded(np.concatenate([a, b], 1), w, (1, 1), H, W), O2.numpy(), "%d channels" % C)
 
 
+@pytest.mark.parametrize("W", [14, 16])
+def test_conv2d_winograd_split_follows_a_write_to_registered_filters(hip, W):
+    """The split copy of registered filters, once it exists, is made again after the filters were written."""
+    rng = np.random.default_rng(1993)
+    N, C, H, Kf = 2, 32, 14, 65
+    X, w = hip.array(rng.standard_normal((N, C, H, W), dtype=np.float32)), (rng.standard_normal((Kf, C, 3, 3)) * 0.06).astype(np.float32)
+    Wd, O = hip.array(w), hip.full((N, Kf, H, W), np.nan)
+    try:
+        hip.cache_conv_filters(Wd)
+        hip.force_conv_plan(32, 1)
+        hip.conv2D(X, Wd, None, O, 1, 1, 1, 1)
+        assert "wino_split_kernel" in hip.last_conv_kernel()
+        first = O.numpy()
+        Wd.copy_from(2.0 * w)
+        hip.conv2D(X, Wd, None, O, 1, 1, 1, 1)
+        assert np.array_equal(O.numpy(), 2.0 * first)
+        Wd.copy_from(w)
+        hip.conv2D(X, Wd, None, O, 1, 1, 1, 1)
+        assert np.array_equal(O.numpy(), first)
+    finally:
+        hip.force_conv_plan(-1, 1)
+        hip.uncache_conv_filters(Wd)
+
+
 @pytest.mark.parametrize("slices", [1, 2])
 def test_conv2d_winograd_split_keeps_what_is_not_finite_and_the_largest_numbers(hip, slices):
     """Infinities, NaN and numbers that round up to infinity in 16 bits, in the image and in a filter: what the fp32 kernel of this

@@ -83,7 +83,11 @@ def short(name, width):
 def library_name(name):
     """A kernel's name as the library and the trace both have it: the trace spells out a defaulted last template argument and writes
     enumerators as numbers."""
-    name = name.replace(" ", "").replace(",false>", ">")
+    return enumerators_by_name(name).replace(",false>", ">")
+
+
+def enumerators_by_name(name):
+    name = name.replace(" ", "")
     return re.sub(r"\((?:\(anonymousnamespace\)::)?SplitTaps\)(\d)", lambda m: SPLIT_TAPS[int(m.group(1))], name)
 
 
@@ -183,14 +187,14 @@ def traffic(workload, trace_dir, fetch_dir, write_dir, log, out, out_json=None, 
         # parameter list), so that a later run finds its dominant kernel whichever plan its search kept
         table = {}
         for k, (b, calls, fb, wb) in per_kernel.items():
-            name = short(k, 10 ** 6).split("(")[0].replace(" ", "")
+            name = enumerators_by_name(short(k, 10 ** 6)).split("(")[0]
             table[name] = {"hbm_bytes_per_launch": b, "fetch_bytes_per_launch": fb, "write_bytes_per_launch": wb, "launches_in_counter_run": calls}
         # forwards in the counter run (warm-up, timed steps, bench.py's per-op timing passes): the dominant kernel's dispatches
         # over its launches per forward
         steps = None
         if bench and bench["roofline"].get("launches_per_step"):
-            dom = bench["roofline"]["kernel"].replace(" ", "")
-            hit = [v for k, v in table.items() if k.replace(",false>", ">") == dom]
+            dom = library_name(bench["roofline"]["kernel"])
+            hit = [v for k, v in table.items() if library_name(k) == dom]
             if hit:
                 steps = hit[0]["launches_in_counter_run"] / bench["roofline"]["launches_per_step"]
         with open(out_json, "w") as fh:

@@ -144,6 +144,30 @@ def test_stall_table_and_trace_find_the_split_kernels_under_the_traces_names(tmp
         assert "same kernel in the trace above: %s" % found in open(tmp_path / "trace.txt").read()
 
 
+def test_traffic_table_has_a_row_for_each_build_of_the_split_kernel(tmp_path):
+    import json
+    import os
+    from eddl_amd import profsum
+    names = ["void (anonymous namespace)::conv_split_kernel<4, 1, 1, 2, 3, ((anonymous namespace)::SplitTaps)%d>((anonymous namespace)::ConvParams)" % i for i in range(3)]
+    probe = "void (anonymous namespace)::unary_kernel<0>(float const*, float*, unsigned long)"
+    for d, c in (("f", "FETCH_SIZE"), ("w", "WRITE_SIZE")):
+        os.makedirs(str(tmp_path / d))
+        with open(tmp_path / d / "m_counter_collection.csv", "w") as fh:
+            fh.write("Dispatch_Id,Kernel_Name,Counter_Name,Counter_Value\n")
+            for i, k in enumerate(names + [probe]):
+                fh.write('%d,"%s",%s,%f\n' % (i, k, c, 262144.0 if k == probe else 1000.0 * (i + 1)))
+    with open(tmp_path / "t_kernel_stats.csv", "w") as fh:
+        fh.write("Name,Calls,TotalDurationNs,AverageNs,Percentage\n")
+        for k in names + [probe]:
+            fh.write('"%s",1,1000,1000,10\n' % k)
+    (tmp_path / "bench.log").write_text(json.dumps({"metric": "x", "value": 1.0, "unit": "u", "ms_per_step": 1.0, "roofline": {
+        "kernel": "conv_split_kernel<4,1,1,2,3,ONE_TAP>", "launches_per_step": 1, "achieved": 1.0, "unit": "TFLOP/s", "frac": 0.1, "peak": 10.0}}) + "\n")
+    profsum.traffic("resnet50", str(tmp_path), str(tmp_path / "f"), str(tmp_path / "w"), str(tmp_path / "bench.log"), str(tmp_path / "o.txt"), str(tmp_path / "o.json"))
+    table = json.load(open(tmp_path / "o.json"))
+    assert [table["kernels"]["conv_split_kernel<4,1,1,2,3,%s>" % t]["fetch_bytes_per_launch"] for t in ("UPSAMPLED", "STORED", "ONE_TAP")] == [1024e3, 2048e3, 3072e3]
+    assert table["steps_in_counter_run"] == 1.0
+
+
 def test_a_form_has_one_name_and_its_peak():
     import bench
     for tile in (16, 19, 32, 33, 34):

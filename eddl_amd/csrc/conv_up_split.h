@@ -240,7 +240,7 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
         for (int e = 0; e < 4; e++)
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                y[e >> 1][e & 1][v] = (e == 1 || e == 2 ? -down : down) * acc[e][tn][v];
+                y[e >> 1][e & 1][v] = __builtin_fmaf(e == 1 || e == 2 ? -down : down, acc[e][tn][v], 0.0f);  // (a sum of zeros is +0 under either sign)
                 finite = __builtin_fmaf(y[e >> 1][e & 1][v], 0.0f, finite);
             }
         if (__any(finite != 0.0f)) {

@@ -1824,6 +1824,26 @@ def test_conv2d_upsampled_2x2_split_behind_a_relu(hip, C, H, W, plan):
     assert split[2] <= 0.1 * fp32[1]
 
 
+@pytest.mark.parametrize("slices", [1, 2])
+def test_split_winograd_and_upsampled_sums_of_zeros_are_positive_zeros(hip, slices):
+    """As in the fp32 kernels: the sign that a block is accumulated with leaves none on a zero."""
+    rng = np.random.default_rng(2099)
+    X = hip.full((2, 64, 6, 7), 0.0)
+    O3, O2 = hip.full((2, 40, 6, 7), np.nan), hip.full((2, 40, 12, 14), np.nan)
+    try:
+        for plan in (32, 33, 34):
+            hip.force_conv_plan(plan, slices)
+            if plan == 32:
+                hip.conv2D(X, hip.array(rng.standard_normal((40, 64, 3, 3), dtype=np.float32)), None, O3, 1, 1, 1, 1)
+            else:
+                hip.conv2D(X, hip.array(rng.standard_normal((40, 64, 2, 2), dtype=np.float32)), None, O2, 1, 1, 0, 0, upsample=(2, 2))
+            assert ("wino_split_kernel" if plan == 32 else "conv_up2x2_split") in hip.last_conv_kernel()
+            got = (O3 if plan == 32 else O2).numpy()
+            assert (got == 0.0).all() and not np.signbit(got).any(), plan
+    finally:
+        hip.force_conv_plan(-1, 1)
+
+
 @pytest.mark.parametrize("plan", [(33, 1), (34, 2)])
 def test_conv2d_upsampled_2x2_split_keeps_what_is_not_finite_and_the_largest_numbers(hip, plan):
     """What the fp32 kernel of this form gives, and not a bit of an output whose pixels are finite."""

@@ -79,10 +79,11 @@ __device__ __forceinline__ void up2x2_block_again(const ConvParams &p, floatx16 
 // conv_split_kernel (loaded a tap ahead, split between the matrix instructions on their way into LDS), and tap t is multiplied by the
 // weight sums that see it - 4, 2, 2 and 1 of the nine - straight from L2, the next sum's requested while the current one
 // multiplies.  216 matrix instructions of a wavefront share four reads of the pixels; their splitting and the additions to the long
-// sums are three to four vector instructions per matrix instruction.  Measured (4 images, us, with the products added straight to the
+// sums are three to five vector instructions per matrix instruction.  Measured (4 images, us, with the products added straight to the
 // long sums -> this): 1024 -> 512 on 32x32 193 -> 195, 512 -> 256 on 64x64 171 -> 182, 256 -> 128 on 128x128 175 -> 186, 128 -> 64 on
-// 256x256 (64 x 128 tile) 218 -> 232; the fp32 kernel 314, 280, 288, 314.  256 -> 128 is 232 GFLOP of bf16 products: half of the bf16
-// instruction's rate at 2.4 GHz.
+// 256x256 (64 x 128 tile) 218 -> 232; the fp32 kernel 314, 280, 288, 314.  Bound: in U-Net's launches the matrix pipe is busy 49 % of the cycles
+// at 2.26 GHz (46 % of the bf16 instruction's rate; 64 x 128 tile 41 %), the vector L1 holds requests back half of them (every filter
+// comes from L2 for 64 or 128 blocks only) and a wavefront waits 37 %.
 // All 256 registers are taken; three values of either build lie in scratch.
 template <int WM, int WN>
 __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvParams p) {

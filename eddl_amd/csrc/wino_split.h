@@ -126,8 +126,11 @@ __device__ __forceinline__ void wino_block_again(const ConvParams &p, floatx16 &
 // cache), but two independent workgroups share a CU and cover each other's latencies, prologue and epilogue.  Tried: 64 filters x 64
 // blocks on eight wavefronts (half the filter traffic, one workgroup per CU): level on 512 channels, 17-25 % slower on 64 and 128;
 // the same on sixteen wavefronts with one position each: 1.5 times the time.
-// Bound: the matrix pipe is busy 52-58 % of the cycles at 1.75-2.0 GHz (2.4 with operands of zeros: power); without filter loads
-// a quarter of the time goes, without pixel loads a tenth.  Batch 32, us, wino_fused_kernel -> this one: conv 64->64 on 224x224 541
+// Bound: neither pipe is full. VGG-16's nine launches of the wide build at batch 32 keep the matrix pipe busy 36 % of the cycles, at 2.2 GHz (power:
+// 2.4 with operands of zeros); a wavefront issues 38 % of its cycles, 13 vector instructions per memory instruction, and waits for memory or LDS 28 %; the
+// vector L1 holds requests back 35 % of a CU's cycles.  Without filter loads a quarter of the time goes, without pixel loads a tenth.  Narrow build (planes 14
+// wide): 26 %, 34 % and 31 %; each step's pixels are four times as many load instructions, and its 62 scalar values beyond the register file lie in
+// vector registers (no scratch).  Batch 32, us, wino_fused_kernel -> this one: conv 64->64 on 224x224 541
 // -> 495, 128->128 on 112x112 492 -> 410, 256->256 on 56x56 462 -> 368, 512->512 on 28x28 462 -> 363, on 14x14 151 -> 129; 64->64 on
 // 512x512, batch 4, 359 -> 328; ResNet-50's at batch 64: 77 -> 65, 73 -> 61, 84 -> 70.
 template <bool WIDE>

@@ -1,6 +1,6 @@
 """The files that go into EDDL itself (integration/eddl): the binding translation unit, the generated stubs, the patch.
 
-With an EDDL tree at hand (/root/reference here; absent on the GPU box, where these tests skip) the three device-seam
+With an EDDL tree at hand (/root/reference here; where there is none, these tests skip) the three device-seam
 headers are parsed and every declaration must be defined exactly once, by hip_backend.cpp or by hip_stubs.cpp; every
 member the binding reads through a Tensor / ConvolDescriptor / PoolDescriptor pointer must exist in EDDL's classes; the
 patch must apply to the tree.  Without the tree, what does not need it still runs: the stubs parse as C++, and the

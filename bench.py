@@ -34,7 +34,7 @@ def form_of_plan(tile):
     """The form of convolution that a plan's tile number names in a plans file (eddlhip_conv2d_force_plan)."""
     for first, last, form in ((-1, -1, "planner"), (0, 3, "direct_tile"), (4, 4, "winograd_three_kernels"), (5, 5, "winograd_folded"),
                               (6, 7, "winograd_one_launch"), (8, 9, "upsampled_2x2"), (16, 19, "split"), (32, 32, "winograd_split"),
-                              (33, 34, "upsampled_2x2_split")):
+                              (33, 34, "upsampled_2x2_split"), (40, 41, "wave_split")):
         if first <= tile <= last:
             return form
     raise ValueError("bench.py: plan tile %d names no form" % tile)
@@ -234,7 +234,7 @@ def measure(hip, workload, steps, warmup, fused=True, graph=False, tune=True, pl
             hip.conv_tuned_save(fh.name)
             lines = sorted(l.strip() for l in open(fh.name) if l.strip() and not l.startswith("#"))
         forms = {"planner": 0, "direct_tile": 0, "winograd_three_kernels": 0, "winograd_folded": 0, "winograd_one_launch": 0, "upsampled_2x2": 0, "split": 0, "winograd_split": 0,
-                 "upsampled_2x2_split": 0}
+                 "upsampled_2x2_split": 0, "wave_split": 0}
         for l in lines:
             forms[form_of_plan(int(l.split("|")[1].split()[0]))] += 1
         plans_info = {"geometries": len(lines), "sha16": hashlib.sha256("\n".join(lines).encode()).hexdigest()[:16], "kept": forms,
@@ -265,7 +265,7 @@ def measure(hip, workload, steps, warmup, fused=True, graph=False, tune=True, pl
             # kernel_flops: what the timed kernel itself multiplies.  The Winograd form times its product launch (16 products
             # of [Kf x C] by [C x blocks] matrices, 2.25 times fewer multiplications than the layer's direct count); the two
             # transform kernels around it are in the op's own time only
-            kernel_flops, form = op.flops, "split" if kern.startswith("conv_split_kernel") else "direct"
+            kernel_flops, form = op.flops, "split" if kern.startswith("conv_split_kernel") else "wave_split" if kern.startswith("conv_wave_split") else "direct"
             if kern.startswith("winograd["):
                 blocks = int(kern[kern.rindex(",") + 1:].split()[0])
                 kern = kern[len("winograd["):kern.rindex(",")]
@@ -283,7 +283,7 @@ def measure(hip, workload, steps, warmup, fused=True, graph=False, tune=True, pl
                 n_out, kf = conv.out_shape[0] * conv.out_shape[2] * conv.out_shape[3], conv.out_shape[1]
                 c_in = op.flops // (2 * conv.kr * conv.kc * n_out * kf)
                 kernel_flops, form = 2 * 9 * kf * c_in * blocks, "upsampled_2x2_split" if kern.startswith("conv_up2x2_split") else "upsampled_2x2"
-            row.update(kernel=kern.split(" +ksplit")[0], kernel_ms=kms, kernel_launches=kl, kernel_flops=kernel_flops, form=form,
+            row.update(kernel=kern.split(" +")[0], kernel_ms=kms, kernel_launches=kl, kernel_flops=kernel_flops, form=form,
                        kernel_peak_tflops=peak_of_form(form))
         if op.kind in ("conv2d", "dense") and ms > 0:
             row["tflops"] = op.flops / ms / 1e9
@@ -519,7 +519,7 @@ def main():
         table.append("%-44s %9.4f %9s %8s %9.1f %7.2f  %s" % (
             r["name"][:44], r["ms"], "%.2f" % r["tflops"] if "tflops" in r else "-",
             "%.1f" % (100 * r["frac_fp32_mfma_peak"]) if "tflops" in r else "-", r.get("gbs", 0.0), 100 * r.get("frac_hbm_peak", 0.0),
-            {"winograd": "winograd: ", "winograd_split": "winograd split: ", "upsampled_2x2": "upsampled 2x2: ", "upsampled_2x2_split": "upsampled 2x2 split: ", "split": "split: "}.get(r.get("form"), "") + r.get("kernel", "")))
+            {"winograd": "winograd: ", "winograd_split": "winograd split: ", "upsampled_2x2": "upsampled 2x2: ", "upsampled_2x2_split": "upsampled 2x2 split: ", "split": "split: ", "wave_split": "split: "}.get(r.get("form"), "") + r.get("kernel", "")))
     if args.layers:
         print("\n".join(table), file=sys.stderr)
     out_dir = args.out

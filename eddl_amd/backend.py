@@ -261,7 +261,7 @@ class Backend:
     def force_conv_plan(self, tile=-1, slices=1):
         """Override the convolution launch planner (tile 0..3, K slices; tile 4 .. 7: the Winograd forms where they apply;
         8 / 9: the upsampled-input form of a 2x2 filter; 16 .. 19: the split form; 32: the one-launch Winograd form and
-        33 / 34 the upsampled-input form in the split arithmetic); tile -1 restores it."""
+        33 / 34 the upsampled-input form in the split arithmetic; 40 / 41: the split form for few tiles); tile -1 restores it."""
         self._check(self.lib.eddlhip_conv2d_force_plan(tile, slices))
 
     def last_conv_kernel(self):

@@ -45,6 +45,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <type_traits>
 #include <utility>
@@ -61,9 +62,15 @@ using namespace eddlhip;
 // conv_setup_device asks for the device address once per device and everything else uses that pointer.
 static __device__ __align__(256) unsigned char scratch[EDDLHIP_CONV_NOALLOC_SCRATCH_BYTES];
 
+// How many slices of a tile's rows have been written (conv_wave_split.h); who finishes the rows sets their count back to zero.
+// A launch takes the next stretch of the array (conv2d_wave_split), so that launches in flight on two streams never share one.
+constexpr unsigned TILE_COUNTS = 1u << 20;
+static __device__ unsigned tile_counts[TILE_COUNTS];
+
 namespace {
 
 void *g_scratch_ptr[EDDLHIP_MAX_DEVICES];  // device address of `scratch` on each initialised device
+unsigned *g_counts_ptr[EDDLHIP_MAX_DEVICES];  // ... and of `tile_counts`
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -111,6 +118,7 @@ struct ConvParams {
     // adds the slices and finishes those tiles.
     int main_tiles, nslices, slice_steps;
     float *partial;
+    unsigned *count;  // conv_wave_split_kernel only: how many slices of a tile's rows have been written, zero between launches
     // conv_gen_kernel only: one entry per tap of the padded K range (tap_table_kernel)
     const int32x4 *taps;
     // eddlhip_conv2d_trace: eight 64-bit words per workgroup (see trace_mark), or nullptr
@@ -184,15 +192,18 @@ __device__ __forceinline__ ChannelEpilogue load_channel(const ConvParams &p, int
     return e;
 }
 
-__device__ __forceinline__ float apply_epilogue(const ConvParams &p, const ChannelEpilogue &e, float v, size_t oidx) {
+__device__ __forceinline__ float finish_value(const ConvParams &p, const ChannelEpilogue &e, float v, float residual) {
     if (p.bias) v = __fadd_rn(v, e.bias);
     if (p.bn_mean) {
         v = __fdiv_rn(__fsub_rn(v, e.mean), e.sd);
         if (p.bn_g) v = __fadd_rn(__fmul_rn(v, e.g), e.b);
     }
-    if (p.residual) v = __fadd_rn(v, p.residual[oidx]);
+    if (p.residual) v = __fadd_rn(v, residual);
     if (p.relu) v = v > 0.0f ? v : 0.0f;
     return v;
+}
+__device__ __forceinline__ float apply_epilogue(const ConvParams &p, const ChannelEpilogue &e, float v, size_t oidx) {
+    return finish_value(p, e, v, p.residual ? p.residual[oidx] : 0.0f);
 }
 
 // LDS-direct load: the load unit writes the dword of lane i to LDS address dst + 4*i (out-of-range
@@ -2227,6 +2238,7 @@ __global__ __launch_bounds__(256) void wino_fused_reduce_kernel(const ConvParams
 #include "conv_split.h"
 #include "wino_split.h"
 #include "conv_up_split.h"
+#include "conv_wave_split.h"
 
 // ---------------------------------------------------------------- host side
 int g_algo = 0;
@@ -2359,6 +2371,28 @@ constexpr int NUM_SPLIT = (int)(sizeof(ksplits[0]) / sizeof(ksplits[0][0]));
 const Variant &split_build(int tile, int RS, int uh, int uw) { return ksplits[RS == 1 ? ONE_TAP : uh * uw == 1 ? STORED : UPSAMPLED][tile]; }
 constexpr int SPLIT_TILE0 = 16;
 bool is_split_tile(int tile) { return tile >= SPLIT_TILE0 && tile < SPLIT_TILE0 + NUM_SPLIT; }
+// The split form for few tiles (conv_wave_split.h): plan "tiles" 40 and 41 (32 and 64 filters x 32 pixels), their K slices divide every
+// tile, the channel count is any.  Best plan of the other forms -> best of these, us, launches back to back: 1 image, 256 -> 64 on 56x56
+// 8.8 -> 5.1, 64 3x3 on 56x56 11.2 -> 6.2, 512 -> 128 on 28x28 9.8 -> 5.5, 128 -> 512 8.2 -> 5.4, 256 3x3 on 14x14 12.6 -> 8.3, 256 -> 1024
+// 10.4 -> 5.4, 512 3x3 on 7x7 14.7 -> 8.8, 2048 -> 512 11.5 -> 7.1, 512 3x3 on 14x14 20.1 -> 14.0; 4 images, 512 -> 128 on 28x28 13.1 -> 7.6,
+// 256 3x3 on 14x14 17.3 -> 13.8, 512 3x3 on 7x7 21.2 -> 14.3, 2048 -> 512 13.8 -> 9.7.  No gain where four workgroups per CU do not hold
+// the tiles (4 images, 64 -> 256 on 56x56 10.3 against 21; 12 images, any), so the search tries no more.
+struct WaveSplitVariant {
+    const char *name[3];  // by SplitTaps
+    int tm, tn;           // 32 tm filters x 32 tn pixels
+    void (*kernel[3])(const WaveSplitParams);
+};
+#define WAVE_SPLIT_NAME(TM, TN, TAPS) "conv_wave_split_kernel<" #TM "," #TN "," #TAPS ">"
+#define WAVE_SPLIT(TM, TN)                                                                                                             \
+    {                                                                                                                                  \
+        {WAVE_SPLIT_NAME(TM, TN, UPSAMPLED), WAVE_SPLIT_NAME(TM, TN, STORED), WAVE_SPLIT_NAME(TM, TN, ONE_TAP)}, TM, TN,                \
+            {conv_wave_split_kernel<TM, TN, UPSAMPLED>, conv_wave_split_kernel<TM, TN, STORED>, conv_wave_split_kernel<TM, TN, ONE_TAP>} \
+    }
+const WaveSplitVariant kwave[] = {WAVE_SPLIT(1, 1), WAVE_SPLIT(2, 1)};
+constexpr int NUM_WAVE = (int)(sizeof(kwave) / sizeof(kwave[0]));
+constexpr int WAVE_TILE0 = 40;
+constexpr long long WAVE_MAX_TILES = 1024;  // of a divided launch: its stretch of tile_counts
+bool is_wave_tile(int tile) { return tile >= WAVE_TILE0 && tile < WAVE_TILE0 + NUM_WAVE; }
 // The upsampled-input form in the split arithmetic (conv_up_split.h): plan "tiles" 33 (128 filters x 64 blocks) and 34 (64 x 128, half
 // of a 128-filter tile would idle under 64 filters).  Measured, us, the best of the fp32 and of the direct split plans before -> this
 // (4 images, stored side x channels -> filters): 32 x 1024 -> 512 314 -> 195, 64 x 512 -> 256 280 -> 182, 128 x 256 -> 128 288 -> 186 (34: 201),
@@ -2374,7 +2408,7 @@ const UpSplitVariant kupsplit[] = {{"conv_up2x2_split_kernel<4,1>", 4, 2, conv_u
 constexpr int NUM_UPSPLIT = (int)(sizeof(kupsplit) / sizeof(kupsplit[0]));
 constexpr int UPSPLIT_TILE0 = WSPLIT_TILE0 + NUM_WSPLIT;
 bool is_upsplit_tile(int tile) { return tile >= UPSPLIT_TILE0 && tile < UPSPLIT_TILE0 + NUM_UPSPLIT; }
-bool is_plan_tile(int tile) { return is_upsplit_tile(tile) || (tile >= -1 && tile < NUM_PLAN_TILES) || is_split_tile(tile) || is_wsplit_tile(tile); }
+bool is_plan_tile(int tile) { return is_wave_tile(tile) || is_upsplit_tile(tile) || (tile >= -1 && tile < NUM_PLAN_TILES) || is_split_tile(tile) || is_wsplit_tile(tile); }
 int split_steps(int C, int RS) { return (C + SPLIT_K - 1) / SPLIT_K * RS; }
 size_t upsplit_filter_bytes(int C, int Mp) { return (size_t)split_steps(C, 1) * 2 * (Mp / 32) * UPSPLIT_UNIT; }
 size_t split_filter_bytes(int C, int RS, int Mp) { return (size_t)split_steps(C, RS) * 2 * (Mp / 32) * SPLIT_UNIT; }
@@ -2382,6 +2416,15 @@ size_t split_filter_bytes(int C, int RS, int Mp) { return (size_t)split_steps(C,
 // where a folded Concat has two tensors for them.
 bool split_applies(int C, int Kf, int R, int S) {
     return C % 16 == 0 && split_filter_bytes(C, R * S, (Kf + M_ALIGN - 1) / M_ALIGN * M_ALIGN) < ((size_t)1 << 31);
+}
+
+bool wave_applies(int C, int Kf, int R, int S) { return split_filter_bytes(C, R * S, (Kf + M_ALIGN - 1) / M_ALIGN * M_ALIGN) < ((size_t)1 << 31); }
+long long wave_tiles(const WaveSplitVariant &v, int Kf, long long npix) { return (long long)((Kf + 32 * v.tm - 1) / (32 * v.tm)) * ((npix + 32 * v.tn - 1) / (32 * v.tn)); }
+// K slices of a plan that asks for `slices`: no more than there are units of 16 channels under one tap for eight wavefronts each
+int wave_slices(const WaveSplitVariant &v, int slices, int Kf, int C, int RS, long long npix) {
+    const long long units = (long long)((C + 15) / 16) * RS, most = (units + WAVE_SPLIT_WAVES - 1) / WAVE_SPLIT_WAVES;
+    if (slices <= 1 || wave_tiles(v, Kf, npix) > WAVE_MAX_TILES) return 1;
+    return slices < most ? slices : (int)most;
 }
 
 // K slices of the left-over tiles of a one-launch Winograd plan that asks for `slices` of them (T blocks in the launch):
@@ -2633,6 +2676,9 @@ int conv_setup_device(int dev) {
     EH_TRY_HIP(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));
     EH_REQUIRE(ptr != nullptr, "device %d: no address for the convolution scratch array", dev);
     g_scratch_ptr[dev] = ptr;
+    EH_TRY_HIP(hipGetSymbolAddress(&ptr, HIP_SYMBOL(tile_counts)));
+    EH_REQUIRE(ptr != nullptr, "device %d: no address for the convolution's tile counts", dev);
+    g_counts_ptr[dev] = (unsigned *)ptr;
     for (const Variant(*fam)[4] : {k3x3, k1x1, k2x2, kgen})
         for (int d = 0; d < 2; d++) EH_TRY(family_occupancy(fam[d]));
     return 0;
@@ -2901,6 +2947,7 @@ int conv2d_up2x2(int tile, int slices, int dev, const float *I, const float *K, 
                  const float *bn_b, const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu);
 
 int conv2d_split(bool no_alloc, const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room);
+int conv2d_wave_split(bool no_alloc, const WaveSplitVariant &v, int slices, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room);
 
 // Whether a convolution is the one conv_up2x2_kernel computes: a 2x2 stride-1 filter on ONE tensor upsampled twice in both
 // directions, no padding above or to the left (below and to the right the image is followed by zeros, as many as the
@@ -2974,7 +3021,7 @@ size_t winograd_workspace(bool fold, int N, int C, int Kf, int fs, int P, int Q,
 // forms with a transformed input in memory; within a form fewer K slices first.  Returns 0 with *out filled, 1 when these tensors cannot be searched on (the output overlaps an
 // input: repeating the call would change what it reads), or minus the error code of a runtime failure.
 int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, long long chunk_pix, bool wino_ok, bool fold_ok, bool fused_ok, bool up_ok,
-                bool split_ok, bool wsplit_ok, bool upsplit_ok, TunedPlan *out) {
+                bool split_ok, bool wsplit_ok, bool upsplit_ok, bool wave_ok, TunedPlan *out) {
     {
         const size_t out_bytes = (size_t)c.N * c.Kf * c.P * c.Q * 4, in_bytes = (size_t)c.N * (c.I2 ? c.C / 2 : c.C) * c.H * c.W * 4;
         const char *o_lo = (const char *)c.O, *o_hi = o_lo + out_bytes;
@@ -3081,6 +3128,17 @@ int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, l
                 if (fp.nslices == last_slices) continue;
                 last_slices = fp.nslices;
                 time_plan(5 + v, SPLIT_TILE0 + v, sl);
+            }
+        }
+    if (wave_ok)  // the split form for few tiles: up to four workgroups per CU
+        for (int v = 0; v < NUM_WAVE; v++) {
+            const long long tiles = wave_tiles(kwave[v], c.Kf, chunk_pix);
+            int last_slices = 0;
+            for (int sl : kSearchSlices) {
+                const int ns = wave_slices(kwave[v], sl, c.Kf, c.C, c.R * c.S, chunk_pix);
+                if (ns == last_slices || tiles * ns > 4LL * num_cu) continue;
+                last_slices = ns;
+                time_plan(9, WAVE_TILE0 + v, sl);
             }
         }
     for (int tile = 0; tile < 4; tile++) {
@@ -3219,6 +3277,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     p.in_bytes = p.wp_bytes = 0;
     p.main_tiles = 0; p.nslices = 1; p.slice_steps = 0; p.partial = nullptr;
     p.trace = nullptr;
+    p.count = nullptr;
     p.w_img_stride = 0;
 
     if (g_algo == 2) {
@@ -3308,6 +3367,12 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
                                     chunk_imgs, &no_room);
         if (!no_room) return rc;
     }
+    // ... and for few tiles, any channel count
+    const bool wave_ok = !gemm && g_algo == 0 && !g_wino_never && wave_applies(C, Kf, R, S);
+    if (wave_ok && is_wave_tile(g_force_tile)) {
+        const int rc = conv2d_wave_split(no_alloc, kwave[g_force_tile - WAVE_TILE0], g_force_slices, dev, p, chunk_imgs, &no_room);
+        if (!no_room) return rc;
+    }
     const bool query = gemm != nullptr && gemm->need_out != nullptr;  // report the workspace need, launch nothing
     bool plan_open = false;                                         // a search could still pick any plan for this geometry
     if (g_autotune && g_force_tile < 0 && g_algo == 0 && g_split != 0) {
@@ -3326,13 +3391,13 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
             memcpy(best.key, key, sizeof(key));
             const size_t ws_before = state(dev).workspace_bytes;
             FilterCopies keep = copies_held(dev, K, Kf, C, R, S);  // (those that other geometries' plans, and graphs, may use)
-            const int src = search_plan(call, family, plan, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, split_ok, wsplit_ok, upsplit_ok, &best);
+            const int src = search_plan(call, family, plan, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, split_ok, wsplit_ok, upsplit_ok, wave_ok, &best);
             if (src < 0) return -src;  // a runtime error inside the search
             if (src == 0) {
                 keep.wino = keep.wino || best.tile == 4 || best.tile == 5;
                 keep.fused = keep.fused || (best.tile >= FUSED_TILE0 && best.tile < FUSED_TILE0 + NUM_FUSED);
                 keep.up = keep.up || best.tile == UP2X2_TILE || best.tile == UP2X2_TILE + 1;
-                keep.split = keep.split || is_split_tile(best.tile);
+                keep.split = keep.split || is_split_tile(best.tile) || is_wave_tile(best.tile);
                 keep.upsplit = keep.upsplit || is_upsplit_tile(best.tile);
                 keep.wsplit = keep.wsplit || is_wsplit_tile(best.tile);
             }
@@ -3362,6 +3427,10 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
             const int tile = found->tile - SPLIT_TILE0;
             const int rc = conv2d_split(no_alloc, split_build(tile, R * S, uh, uw), forced_plan(ksplit, tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev,
                                         p, chunk_imgs, &no_room);
+            if (!no_room) return rc;
+        }
+        if (found != nullptr && is_wave_tile(found->tile) && wave_ok) {
+            const int rc = conv2d_wave_split(no_alloc, kwave[found->tile - WAVE_TILE0], found->slices, dev, p, chunk_imgs, &no_room);
             if (!no_room) return rc;
         }
         if (found != nullptr && found->tile >= 0 && found->tile < 4)
@@ -3880,6 +3949,29 @@ int conv2d_winograd_fused(bool no_alloc, bool *no_room, const FusedVariant &fv, 
     return 0;
 }
 
+// The split copy of a registered filter tensor, made on first use; *Ws stays NULL where there is none.
+int kept_split_filters(bool no_alloc, int dev, const ConvParams &call, size_t w_bytes, const void **Ws) {
+    std::lock_guard<std::mutex> lock(g_cache_mutex);
+    for (CachedFilters &e : g_cache[dev]) {
+        if (e.K == call.K && e.Kf == call.Kf && e.C == call.C && e.R == call.R && e.S == call.S) {
+            if (e.Wsplit == nullptr && !state(dev).capturing && !no_alloc) {
+                if (hipMalloc(&e.Wsplit, w_bytes) != hipSuccess) {
+                    e.Wsplit = nullptr;
+                    (void)hipGetLastError();
+                    break;  // no room to keep them: split per call
+                }
+                e.stale = true;
+            }
+            if (e.Wsplit != nullptr) {
+                if (e.stale) EH_TRY(repack(dev, e));
+                *Ws = e.Wsplit;
+            }
+            break;
+        }
+    }
+    return 0;
+}
+
 // The split form (conv_split.h) of the call that `call` describes, under a plan of split steps.
 // Workspace: [split filters unless kept][partial tiles].  no_alloc: from the fixed scratch array; nothing is launched and *no_room
 // is set if that is too small.
@@ -3891,26 +3983,7 @@ int conv2d_split(bool no_alloc, const Variant &v, const Plan &plan, int dev, con
     const size_t w_bytes = split_filter_bytes(call.C, RS, call.Mp);
     const size_t partial_bytes = (size_t)plan.nslices * leftover * v.bm * v.bn * sizeof(float);
     const void *Ws = nullptr;
-    {
-        std::lock_guard<std::mutex> lock(g_cache_mutex);
-        for (CachedFilters &e : g_cache[dev]) {
-            if (e.K == call.K && e.Kf == call.Kf && e.C == call.C && e.R == call.R && e.S == call.S) {
-                if (e.Wsplit == nullptr && !state(dev).capturing && !no_alloc) {
-                    if (hipMalloc(&e.Wsplit, w_bytes) != hipSuccess) {
-                        e.Wsplit = nullptr;
-                        (void)hipGetLastError();
-                        break;  // no room to keep them: split per call
-                    }
-                    e.stale = true;
-                }
-                if (e.Wsplit != nullptr) {
-                    if (e.stale) EH_TRY(repack(dev, e));
-                    Ws = e.Wsplit;
-                }
-                break;
-            }
-        }
-    }
+    EH_TRY(kept_split_filters(no_alloc, dev, call, w_bytes, &Ws));
     const size_t ws_filters = Ws ? 0 : ((w_bytes + 255) & ~(size_t)255);
     void *ws = nullptr;
     if (no_alloc) {
@@ -3961,6 +4034,78 @@ int conv2d_split(bool no_alloc, const Variant &v, const Plan &plan, int dev, con
     }
     if (leftover > 0) snprintf(g_last_kernel, sizeof(g_last_kernel), "%s +ksplit(%lld tiles x %d)", v.name, leftover, plan.nslices);
     else snprintf(g_last_kernel, sizeof(g_last_kernel), "%s", v.name);
+    return 0;
+}
+
+// The split form for few tiles (conv_wave_split.h) of the call that `call` describes; workspace and no_alloc as conv2d_split.
+int conv2d_wave_split(bool no_alloc, const WaveSplitVariant &v, int slices, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room) {
+    static std::atomic<unsigned> next_count{0};
+    hipStream_t st = state(dev).stream;
+    const int RS = call.R * call.S, N = call.N;
+    const int nslices = wave_slices(v, slices, call.Kf, call.C, RS, chunk_imgs * call.PQ);
+    const size_t w_bytes = split_filter_bytes(call.C, RS, call.Mp);
+    const size_t partial_bytes = nslices > 1 ? (size_t)nslices * wave_tiles(v, call.Kf, chunk_imgs * call.PQ) * v.tm * v.tn * 4096 : 0;
+    const void *Ws = nullptr;
+    EH_TRY(kept_split_filters(no_alloc, dev, call, w_bytes, &Ws));
+    const size_t ws_filters = Ws ? 0 : ((w_bytes + 255) & ~(size_t)255);
+    void *ws = nullptr;
+    if (no_alloc) {
+        if (ws_filters + partial_bytes > (size_t)EDDLHIP_CONV_NOALLOC_SCRATCH_BYTES) {
+            *no_room = true;
+            return 0;
+        }
+        ws = g_scratch_ptr[dev];
+    } else if (ws_filters + partial_bytes > 0) {
+        EH_TRY(get_workspace(dev, ws_filters + partial_bytes, &ws));
+    }
+    if (Ws == nullptr) {
+        EH_TRY(launch_split_filters(dev, call.K, ws, call.Kf, call.C, RS, call.Mp));
+        Ws = ws;
+    }
+    // (channels past the last and units that lie in both tensors of a folded Concat are the general build's)
+    const bool whole = call.C % 16 == 0 && (call.Csplit == call.C || call.Csplit % 16 == 0) && call.uh * call.uw == 1;
+    const SplitTaps taps = !whole ? UPSAMPLED : RS == 1 ? ONE_TAP : STORED;
+    WaveSplitParams q;
+    static_cast<ConvParams &>(q) = call;
+    q.Wp = (const float *)Ws;
+    q.wp_bytes = (unsigned)w_bytes;
+    q.partial = (float *)((char *)ws + ws_filters);
+    q.nslices = nslices;
+    auto magic = [](int divisor) { return divisor == 1 ? 0u : 0xffffffffu / (unsigned)divisor + 1u; };
+    const int units = (call.C + 15) / 16 * RS, parts = nslices * WAVE_SPLIT_WAVES;
+    q.units_each = units / parts;
+    q.more = units % parts;
+    q.gm = (call.Kf + 32 * v.tm - 1) / (32 * v.tm);
+    const size_t img_elems = (size_t)call.Cimg * call.H * call.W, out_elems = (size_t)call.Kf * call.PQ;
+    for (long long b0 = 0; b0 < N; b0 += chunk_imgs) {
+        const int nb = (int)((N - b0 < chunk_imgs) ? N - b0 : chunk_imgs);
+        q.N = nb;
+        q.I = call.I + b0 * img_elems;
+        q.I2 = call.I2 + b0 * img_elems;
+        q.O = call.O + b0 * out_elems;
+        q.residual = call.residual ? call.residual + b0 * out_elems : nullptr;
+        q.npix = (long long)nb * call.PQ;
+        q.in_bytes = (unsigned)(nb * img_elems * sizeof(float));
+        const long long gn = (q.npix + 32 * v.tn - 1) / (32 * v.tn), wgs = gn * q.gm * nslices;
+        EH_REQUIRE(wgs <= 0x3fffffffLL, "conv2d: too many tiles");
+        q.gn = (int)gn;
+        q.magic_gn = magic(q.gn), q.magic_gm = magic(q.gm), q.magic_pq = magic(q.PQ), q.magic_q = magic(q.Q), q.magic_rs = magic(RS), q.magic_s = magic(q.S);
+        if (nslices > 1) {
+            // the next stretch of counts that does not run over the end of the array
+            const unsigned need = (unsigned)(gn * q.gm) * (WAVE_SPLIT_WAVES * WAVE_SPLIT_COUNT_WORDS);
+            unsigned at = next_count.load(), first;
+            do first = at + need > TILE_COUNTS ? 0 : at;
+            while (!next_count.compare_exchange_weak(at, first + need));
+            q.count = g_counts_ptr[dev] + first;
+        }
+        q.trace = (g_trace != nullptr && wgs <= g_trace_wgs) ? g_trace : nullptr;
+        EH_TRY(prof_begin(st));
+        hipLaunchKernelGGL(v.kernel[taps], dim3((unsigned)wgs), dim3(64 * WAVE_SPLIT_WAVES), 0, st, q);
+        EH_CHECK_LAUNCH();
+        EH_TRY(prof_end(st));
+    }
+    if (nslices > 1) snprintf(g_last_kernel, sizeof(g_last_kernel), "%s +slices(%d)", v.name[taps], nslices);
+    else snprintf(g_last_kernel, sizeof(g_last_kernel), "%s", v.name[taps]);
     return 0;
 }
 

@@ -93,11 +93,11 @@ __device__ __forceinline__ int split_pixel(const ConvParams &p, unsigned magic_h
     return ok ? at : OOB;
 }
 
-// The K-steps [step_lo, step_hi) of a wavefront's blocks once more with the fp32 instruction, two channels at a time in the
-// order of the split filters; reads the image and the original filters where they are.  Only infinities, NaN and numbers near
+// The K-steps [step_lo, step_hi) (of GROUP channels each) of a wavefront's blocks once more with the fp32 instruction, two channels at
+// a time in the order of the split sums; reads the image and the original filters where they are.  Only infinities, NaN and numbers near
 // the end of the fp32 range come here.  (The fp32 kernels take the channels slowest: a sum that overflows in one of the two
 // orders and not in the other can differ.)
-template <int TM, int TN>
+template <int TM, int TN, int GROUP>
 __device__ __forceinline__ void split_tile_again(const ConvParams &p, floatx16 (&acc)[TM][TN], __amdgpu_buffer_rsrc_t in1, __amdgpu_buffer_rsrc_t in2, int m_first,
                                                  int n_first, int step_lo, int step_hi, int lane) {
     const int RS = p.R * p.S, half = lane >> 5, HW4 = p.H * p.W * 4;
@@ -124,7 +124,7 @@ __device__ __forceinline__ void split_tile_again(const ConvParams &p, floatx16 (
     for (int step = step_lo; step < step_hi; step++) {
         const int cb = step / RS, tap = step - cb * RS, ky = tap / p.S, kx = tap - ky * p.S;
 #pragma unroll 1
-        for (int c0 = cb * SPLIT_K; c0 < cb * SPLIT_K + SPLIT_K && c0 < p.C; c0 += 2) {
+        for (int c0 = cb * GROUP; c0 < cb * GROUP + GROUP && c0 < p.C; c0 += 2) {
             const int c = c0 + half;
             float a[TM], b[TN];
 #pragma unroll
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
             for (int v = 0; v < 16; v++) finite = __builtin_fmaf(acc[tm][tn][v], 0.0f, finite);
     const int m_first = m0 + wm * TM * 32, n_first = n0 + wn * TN * 32;
     if (__any(finite != 0.0f)) {
-        split_tile_again<TM, TN>(p, small, rsrc_in, rsrc_in2, m_first, n_first, step_lo, step_hi, lane);
+        split_tile_again<TM, TN, SPLIT_K>(p, small, rsrc_in, rsrc_in2, m_first, n_first, step_lo, step_hi, lane);
 #pragma unroll
         for (int tm = 0; tm < TM; tm++)
 #pragma unroll

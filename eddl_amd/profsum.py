@@ -232,10 +232,10 @@ def mfma(workload, directory, out):
           "",
           "%-88s %6s %9s %12s %9s %7s %7s %6s" % ("kernel", "calls", "avg us", "exec GFLOP", "TFLOP/s", "%peak", "busy %", "GHz")]
     for k in mops:
-        if not any(t in k for t in ("conv_tap", "conv_gen", "conv_split", "conv_pointwise", "wino_fused_kernel", "wino_split_kernel", "conv_up2x2_split", "dense_partial", "mfma_f32_probe")):
+        if not any(t in k for t in ("conv_tap", "conv_gen", "conv_split", "conv_wave_split", "conv_pointwise", "wino_fused_kernel", "wino_split_kernel", "conv_up2x2_split", "dense_partial", "mfma_f32_probe")):
             continue
         us = mean(dur[k])
-        split = any(t in k for t in ("conv_split", "wino_split", "up2x2_split"))
+        split = any(t in k for t in ("conv_split", "wave_split", "wino_split", "up2x2_split"))
         fl = mean((bf16 if split else mops)[k]) * 512.0
         peak = BF16_MFMA_PEAK_TFLOPS if split else FP32_MFMA_PEAK_TFLOPS
         cyc = mean(gui[k]) / 8.0

@@ -274,9 +274,13 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * multiples of 16; 54 bytes per filter and channel).  Neither under set_algo(9).  A plan of the one-launch form is run by
  * eddlhip_conv2d_fwd_noalloc too where its filters (unless registered and used by eddlhip_conv2d_fwd before: 700 thousand filters
  * times channels) and partial tiles fit.
+ * The split form for launches of few tiles (force_plan(40 / 41, .), or the search; any filter, any channel count): the same arithmetic,
+ * tiles of 32 / 64 filters x 32 pixels whose K range is divided over eight wavefronts and `slices` workgroups, one launch also with slices.
+ * Filters, non-finite inputs, eddlhip_conv2d_fwd_noalloc and set_algo(9) as in the split form.
  *
  * eddlhip_conv2d_last_kernel() names the kernel the calling thread's last eddlhip_conv2d_fwd
- * launched, followed by " +ksplit(T tiles x S)" when T tiles were divided into S slices; for the Winograd form
+ * launched, followed by " +ksplit(T tiles x S)" when T tiles were divided into S slices (" +slices(S)" when all were, by the kernel
+ * that finishes them itself); for the Winograd form
  * "winograd[<kernel and plan of the product launch>, <blocks per product> blocks]", for the upsampled-input form
  * "upsampled2x2[<kernel>, <blocks> blocks]". */
 int eddlhip_conv2d_set_algo(int algo);
@@ -318,8 +322,8 @@ int eddlhip_conv2d_tuned_load(int dev, const char *host_path);
  * 5: its folded form wherever that applies, 6 / 7: its one-launch form on tiles of 32 / 64 filters x 32 blocks, `slices`
  * K slices for the left-over tiles as above; 8 / 9: the upsampled-input form of a 2x2 filter, built for three / two
  * workgroups per CU; 16 .. 19: the split form on tiles of 128x128, 128x64, 64x128, 64x64 outputs; 32: the one-launch Winograd
- * form in the split arithmetic on tiles of 64 filters x 32 blocks, 33 / 34: the upsampled-input form in it; the planner's choice
- * wherever a form does not apply.  Acts on the calling thread only. */
+ * form in the split arithmetic on tiles of 64 filters x 32 blocks, 33 / 34: the upsampled-input form in it; 40 / 41: the split form for few tiles, every tile in
+ * `slices`; the planner's choice wherever a form does not apply.  Acts on the calling thread only. */
 int eddlhip_conv2d_force_plan(int tile, int slices);
 
 /* Filters that stay fixed between calls (inference).  Every eddlhip_conv2d_fwd first repacks its

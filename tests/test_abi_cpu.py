@@ -216,3 +216,22 @@ def test_host_layer_links_against_the_c_abi():
                 "_ZN8eddl_hip28import_net_from_onnx_pointerEPKvmi",
                 "_ZN8eddl_hip21save_net_to_onnx_fileEPNS_3NetERKNSt7__cxx1112basic_stringIcSt11char_traitsIcESaIcEEE"):
         assert hasattr(h, sym), sym
+
+
+def test_plans_of_the_split_form_for_few_tiles_are_accepted(tmp_path):
+    """Plan numbers 40 and 41 name its tiles, their neighbours nothing; the benchmark knows them."""
+    sys.path.insert(0, ROOT)
+    import bench
+    from eddl_amd import _lib
+    lib = _lib.load()
+    lib.eddlhip_conv2d_autotune(-1)
+    path = tmp_path / "plans.txt"
+    for tile in range(38, 44):
+        path.write_text("1 %d 64 3 3 1 1 28 28 1 | %d 16\n" % (tile, tile))
+        known = tile in (40, 41)
+        assert (lib.eddlhip_conv2d_tuned_load(0, str(path).encode()) == 0) == known, tile
+        assert (lib.eddlhip_conv2d_force_plan(tile, 1) == 0) == known, tile
+        if known:
+            assert bench.form_of_plan(tile) == "wave_split" and bench.peak_of_form("wave_split") == bench.peak_of_form("split")
+    lib.eddlhip_conv2d_force_plan(-1, 1)
+    lib.eddlhip_conv2d_autotune(-1)

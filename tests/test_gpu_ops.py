@@ -1894,3 +1894,101 @@ def test_conv2d_upsampled_2x2_split_keeps_24_bits_of_small_and_large_numbers(hip
     finally:
         hip.force_conv_plan(-1, 1)
     assert max(err[33], err[34]) <= max(err[UP2X2_FORM], 2.0 ** -22), err
+
+
+# ------------------------------------------------------------------ the split form for few tiles (K range over wavefronts and workgroups)
+WAVE_CASES = dict(SPLIT_CASES, **{
+    "one channel": (1, 1, 9, 9, 8, 3, 3, (1, 1), (1, 1)),
+    "stem": (1, 3, 22, 23, 33, 7, 7, (2, 2), (3, 3)),
+    "33 channels": (2, 33, 8, 5, 96, 1, 1, (1, 1), (0, 0)),
+    "many slices": (1, 512, 4, 5, 64, 1, 1, (1, 1), (0, 0)),
+})
+
+
+@pytest.mark.parametrize("plan", [(40, 1), (40, 3), (40, 16), (41, 1), (41, 4)])
+@pytest.mark.parametrize("case", sorted(WAVE_CASES))
+def test_conv2d_split_form_for_few_tiles_is_no_further_from_64_bits_than_the_fp32_form(hip, case, plan):
+    """... from plain and registered filters and from the entry point that allocates nothing: the same bits, call after call (a launch
+    leaves the counts of its slices as it found them)."""
+    N, C, H, W, Kf, R, S, stride, pad = WAVE_CASES[case]
+    P, Q = (H + 2 * pad[0] - R) // stride[0] + 1, (W + 2 * pad[1] - S) // stride[1] + 1
+    rng = np.random.default_rng(2400 + sorted(WAVE_CASES).index(case))
+    x = rng.standard_normal((N, C, H, W), dtype=np.float32)
+    w = (rng.standard_normal((Kf, C, R, S)) * np.sqrt(2.0 / (C * R * S))).astype(np.float32)
+    X, Wd, O = hip.array(x), hip.array(w), hip.full((N, Kf, P, Q), np.nan)
+    outs = []
+
+    def noalloc():
+        hip._check(hip.lib.eddlhip_conv2d_fwd_noalloc(hip.dev, X.ptr, Wd.ptr, None, O.ptr, N, C, H, W, Kf, R, S, *stride, *pad, P, Q, None, None, None, None, 0.0, None, 0))
+    try:
+        hip.force_conv_plan(2, 1)
+        hip.conv2D(X, Wd, None, O, *stride, *pad)
+        fp32 = O.numpy()
+        hip.force_conv_plan(*plan)
+        for call in ("plain", "plain", "noalloc", "registered", "registered"):
+            if call == "registered":
+                hip.cache_conv_filters(Wd)
+            hip.fill_(O, np.nan)
+            noalloc() if call == "noalloc" else hip.conv2D(X, Wd, None, O, *stride, *pad)
+            assert hip.last_conv_kernel().startswith("conv_wave_split_kernel")
+            outs.append(O.numpy())
+    finally:
+        hip.force_conv_plan(-1, 1)
+        hip.uncache_conv_filters(Wd)
+    assert all(np.array_equal(outs[0], o) for o in outs[1:])
+    ref = _conv64(x, w, stride, pad, P, Q)
+    # (2^-23: as in the split form's own test, the case of few outputs is decided by chance)
+    assert np.linalg.norm(outs[0] - ref) <= max(np.linalg.norm(fp32 - ref), 2.0 ** -23 * np.linalg.norm(ref))
+    assert_conv_close(ref, outs[0], case)
+
+
+@pytest.mark.parametrize("plan", [(40, 1), (40, 4), (41, 3)])
+@pytest.mark.parametrize("C", [48, 96, 70, 6])
+def test_conv2d_split_form_for_few_tiles_reads_folded_inputs_and_applies_the_epilogue(hip, plan, C):
+    """A folded Concat (tensors of 24, 48, 35, 3 channels) and UpSampling give the bits of the stored tensor; infinities and NaN come out as
+    the fp32 kernels bring them; a graph replays the launch."""
+    rng = np.random.default_rng(2450 + C)
+    N, H, W, Kf = 2, 6, 10, 72
+    x = rng.standard_normal((N, C, H, W), dtype=np.float32)
+    w3 = (rng.standard_normal((Kf, C, 3, 3)) * np.sqrt(2.0 / (9 * C))).astype(np.float32)
+    w2 = (rng.standard_normal((Kf, C, 2, 2)) * np.sqrt(2.0 / (4 * C))).astype(np.float32)
+    X, Xa, Xb = hip.array(x), hip.array(x[:, :C // 2].copy()), hip.array(x[:, C // 2:].copy())
+    big = hip.array(x.repeat(2, 2).repeat(2, 3))
+    W3, W2 = hip.array(w3), hip.array(w2)
+    bn = tuple(hip.array(rng.uniform(0.5, 1.5, Kf).astype(np.float32)) for _ in range(4)) + (1e-5,)
+    res = hip.array(rng.standard_normal((N, Kf, H, W), dtype=np.float32))
+    A, B, Y = (hip.full((N, Kf, H, W), np.nan) for _ in range(3))
+    U, V = (hip.full((N, Kf, 2 * H - 1, 2 * W - 1), np.nan) for _ in range(2))
+    try:
+        hip.force_conv_plan(*plan)
+        hip.conv2D(X, W3, None, A, 1, 1, 1, 1)
+        hip.conv2D(Xa, W3, None, B, 1, 1, 1, 1, second=Xb)
+        assert hip.last_conv_kernel().startswith("conv_wave_split_kernel") and np.array_equal(A.numpy(), B.numpy())
+        hip.conv2D(big, W2, None, U, 1, 1, 0, 0)
+        hip.conv2D(X, W2, None, V, 1, 1, 0, 0, upsample=(2, 2))
+        assert np.array_equal(U.numpy(), V.numpy())
+        # the epilogue: the layers' own kernels on the plain output
+        hip.batchnorm_inference(A, B, hip.empty((N, Kf, H, W)), bn[2], bn[3], bn[0], bn[1], hip.empty((Kf,)), 1e-5)
+        hip.add(1.0, B, 1.0, res, Y, 0)
+        hip.relu(Y, Y)
+        hip.conv2D(X, W3, None, B, 1, 1, 1, 1, bn=bn, residual=res, relu=True)
+        assert np.array_equal(B.numpy(), Y.numpy())
+        g = hip.record(lambda: hip.conv2D(X, W3, None, B, 1, 1, 1, 1, bn=bn, residual=res, relu=True))
+        for _ in range(3):
+            hip.fill_(B, np.nan)
+            g.launch()
+            assert np.array_equal(B.numpy(), Y.numpy())
+        # not finite: as the direct fp32 tile has them; every other output keeps its bits
+        finite = A.numpy()
+        x[0, C // 2, 2, 3], x[1, 0, 5, 9] = np.inf, np.nan
+        X.copy_from(x)
+        hip.conv2D(X, W3, None, A, 1, 1, 1, 1)
+        got = A.numpy()
+        hip.force_conv_plan(2, 1)
+        hip.conv2D(X, W3, None, A, 1, 1, 1, 1)
+        fp32 = A.numpy()
+    finally:
+        hip.force_conv_plan(-1, 1)
+    ok = np.isfinite(fp32)
+    assert (~ok).any() and np.array_equal(np.isnan(fp32), np.isnan(got)) and np.array_equal(fp32[~ok & ~np.isnan(fp32)], got[~ok & ~np.isnan(fp32)])
+    assert np.array_equal(finite[ok], got[ok])

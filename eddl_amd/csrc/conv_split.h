@@ -148,6 +148,16 @@ __device__ __forceinline__ void split_tile_again(const ConvParams &p, floatx16 (
     }
 }
 
+// Issue order of a stretch of code: its VALU vector instructions behind its MFMA matrix instructions, evenly.
+template <int MFMA, int VALU>
+__device__ __forceinline__ void split_issue_order() {
+#pragma unroll
+    for (int i = 0; i < MFMA; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, (VALU + MFMA - 1) / MFMA, 0);
+    }
+}
+
 // Implicit GEMM, any filter shape and stride: a K-step is 32 channels of one filter tap.  A thread loads the tap's pixel of
 // one output position for 8 or 16 channels (coalesced along the image row), splits them and puts them into LDS in the
 // operand layout, [buffer][part][8 channels][pixel][8 bf16]: every LDS access is 16 bytes per lane of consecutive lanes.
@@ -165,6 +175,7 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
     constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
     constexpr int CHUNKS = SPLIT_K / (256 / BN) / 8;  // groups of 8 channels a thread loads per step
     static_assert(CHUNKS == 1 || CHUNKS == 2, "BN is 64 or 128");
+    constexpr int RD = CHUNKS == 1 ? 2 : 1;  // steps whose pixels are in registers or on their way there
     __shared__ uintx4 Bs[2][3][SPLIT_K / 8][BN];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -208,11 +219,11 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
         ld_ky = tap / p.S;
         ld_kx = tap - ld_ky * p.S;
     }
-    float raw[CHUNKS][8];
+    float raw[RD][CHUNKS][8];
     const int origin = (base + ih0 * p.W + iw0) * 4;  // (the window's first pixel, which may lie outside)
     const int only = split_pixel(p, magic_h, magic_w, pvalid, base, ih0, iw0, 0, 0);
     // (the channel counts of this form are multiples of 16, of each tensor's of 8: eight channels are one tensor's or nobody's)
-    auto load_pixels = [&](int chunk) {
+    auto load_pixels = [&](int at, int chunk) __attribute__((always_inline)) {
         int voff = only;
         if constexpr (TAPS == UPSAMPLED) voff = split_pixel(p, magic_h, magic_w, pvalid, base, ih0, iw0, ld_ky, ld_kx);
         if constexpr (TAPS == STORED) {
@@ -224,7 +235,7 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
         const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(second ? p.I2 : p.I), 0, c0 < p.C ? p.in_bytes : 0u, RSRC_WORD3);
         int soff = (second ? c0 - p.Csplit : c0) * HW4;
 #pragma unroll
-        for (int j = 0; j < 8; j++, soff += HW4) raw[chunk][j] = buf_load(rsrc, voff, soff);
+        for (int j = 0; j < 8; j++, soff += HW4) raw[at][chunk][j] = buf_load(rsrc, voff, soff);
     };
     auto next_load_step = [&]() {
         // (selects: a branch would end the block that the matrix instructions are scheduled in; behind the last step the
@@ -238,27 +249,25 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
         ld_ky = wrap_y ? 0 : ky;
         ld_c += wrap_y ? SPLIT_K : 0;
     };
-    auto put_pixels = [&](int chunk, int buf) {
-        uintx4 hi, mid, lo;
+    uintx4 parts[CHUNKS][3];
+    auto split_pixels = [&](int at, int chunk, int q) __attribute__((always_inline)) {  // pair q of the four
+        unsigned h, m, l;
+        split_pair(SPLIT_UP * raw[at][chunk][2 * q], SPLIT_UP * raw[at][chunk][2 * q + 1], h, m, l);
+        parts[chunk][0][q] = h;
+        parts[chunk][1][q] = m;
+        parts[chunk][2][q] = l;
+    };
+    auto put_pixels = [&](int chunk, int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            unsigned h, m, l;
-            split_pair(SPLIT_UP * raw[chunk][2 * j], SPLIT_UP * raw[chunk][2 * j + 1], h, m, l);
-            hi[j] = h;
-            mid[j] = m;
-            lo[j] = l;
-        }
-        Bs[buf][0][kgroup + chunk][pix] = hi;
-        Bs[buf][1][kgroup + chunk][pix] = mid;
-        Bs[buf][2][kgroup + chunk][pix] = lo;
+        for (int part = 0; part < 3; part++) Bs[buf][part][kgroup + chunk][pix] = parts[chunk][part];
     };
 
     // ---- filters: 3 x 16 bytes per lane, block and 16 channels
     const int mblocks = p.Mp / 32;
     const int a_voff = lane * 16 + (m0 / 32 + wm * TM) * SPLIT_UNIT;
     uintx4 a[2][TM][3];
-    auto load_a = [&](int g, int step) {
-        const int soff = (step * 2 + g) * mblocks * SPLIT_UNIT;
+    auto load_a = [&](int g, int step) __attribute__((always_inline)) {
+        const int soff = (min(step, step_hi - 1) * 2 + g) * mblocks * SPLIT_UNIT;
 #pragma unroll
         for (int tm = 0; tm < TM; tm++)
 #pragma unroll
@@ -277,64 +286,124 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
             for (int v = 0; v < 16; v++) acc[tm][tn][v] = small[tm][tn][v] = 0.0f;
 
     uintx4 b[TN][3];
-    auto read_b = [&](int g, int buf) {
+    auto read_b = [&](int part, int g, int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int part = 0; part < 3; part++)
-#pragma unroll
-            for (int tn = 0; tn < TN; tn++) b[tn][part] = Bs[buf][part][2 * g + (lane >> 5)][wn * TN * 32 + tn * 32 + (lane & 31)];
+        for (int tn = 0; tn < TN; tn++) b[tn][part] = Bs[buf][part][2 * g + (lane >> 5)][wn * TN * 32 + tn * 32 + (lane & 31)];
     };
-    auto multiply = [&](int g) {
-        constexpr int kA[6] = {0, 1, 2, 0, 1, 0}, kB[6] = {0, 0, 0, 1, 1, 2};
+    constexpr int kA[6] = {0, 1, 2, 0, 1, 0}, kB[6] = {0, 0, 0, 1, 1, 2};
+    auto multiply = [&](int g, int k) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < 6; k++)
+        for (int tm = 0; tm < TM; tm++)
 #pragma unroll
-            for (int tm = 0; tm < TM; tm++)
-#pragma unroll
-                for (int tn = 0; tn < TN; tn++) {
-                    floatx16 &d = k == 0 ? acc[tm][tn] : small[tm][tn];
-                    d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[g][tm][kA[k]]), __builtin_bit_cast(bf16x8, b[tn][kB[k]]), d, 0, 0, 0);
-                }
+            for (int tn = 0; tn < TN; tn++) {
+                floatx16 &d = k == 0 ? acc[tm][tn] : small[tm][tn];
+                d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[g][tm][kA[k]]), __builtin_bit_cast(bf16x8, b[tn][kB[k]]), d, 0, 0, 0);
+            }
     };
 
 #pragma unroll
-    for (int chunk = 0; chunk < CHUNKS; chunk++) load_pixels(chunk);
-    next_load_step();
+    for (int i = 0; i < RD; i++) {
+#pragma unroll
+        for (int chunk = 0; chunk < CHUNKS; chunk++) load_pixels(i, chunk);
+        next_load_step();
+    }
     load_a(0, step_lo);
 #pragma unroll
     for (int chunk = 0; chunk < CHUNKS; chunk++) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) split_pixels(0, chunk, q);
         put_pixels(chunk, 0);
-        load_pixels(chunk);
+        load_pixels(0, chunk);
     }
     next_load_step();
     __syncthreads();
     trace_mark(p, 1);
-    // Step t multiplies buffer t % 2, splits the pixels of step t + 1 (loaded during step t - 1) into the other buffer and
-    // loads those of step t + 2 in their place: a load has a whole step to arrive.  (In the last step nothing is loaded and
-    // what is put into the other buffer is not read.)
-    for (int step = step_lo; step < step_hi; step++) {
-        const int buf = (step - step_lo) & 1;
+    constexpr int T = TM * TN;
+    if constexpr (CHUNKS == 1) {
+        // Step t multiplies buffer t % 2, splits the pixels of step t + 1 into the other buffer and loads those of step t + 3.  (In the
+        // last steps nothing is loaded and what is put into the other buffer is not used.)  Two things keep the matrix
+        // pipe from waiting where a CU has one or two workgroups:
+        //   * the six products take the parts of the pixels in turn, so the registers of a part take the next 16 channels' as soon as its
+        //     last product has started, and the one barrier of a step stands where the first part of the next step is read, half
+        //     a step behind the last write;
+        //   * loads arrive in the order in which they were asked for, so a wait for filters waits for the pixels asked for before
+        //     them: pixels are asked for right behind the filters of the next half step, which makes theirs a whole step.
+        // 12 images, the loop below -> this: 256 3x3 on 14x14 58.7 -> 53.6 us (64x64 tile 49.9 -> 41.0), 128 3x3 stride 2 on 56x56 34.6 -> 31.0,
+        // 1024 -> 256 on 14x14 26.9 -> 25.3; 64 images 256 3x3 on 14x14 94.8 -> 91.1, 1x1 layers within 1 %.
 #pragma unroll
-        for (int g = 0; g < 2; g++) {
-            read_b(g, buf);
-            load_a(g ^ 1, g == 0 ? step : (step + 1 < step_hi ? step + 1 : step));
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(g);
-            if (g < CHUNKS) {
-                put_pixels(g, buf ^ 1);
-                load_pixels(g);
-            }
-            if (g == 1) next_load_step();
-            // issue order: the splitting between the matrix instructions, then what it is for
+        for (int part = 0; part < 3; part++) read_b(part, 0, 0);
+        auto whole_step = [&](int step, int s) __attribute__((always_inline)) {  // s: the step's place in the unrolled loop
+            const int buf = (step - step_lo) & 1;
 #pragma unroll
-            for (int i = 0; i < 6 * TM * TN; i++) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, TM * TN == 4 ? 3 : (TM * TN == 2 ? 6 : 10), 0);
+            for (int g = 0; g < 2; g++) {
+                const int next_buf = g == 0 ? buf : buf ^ 1;
+                load_a(g ^ 1, step + g);
+                if (g == 0) {
+#pragma unroll
+                    for (int q = 0; q < 3; q++) split_pixels((s + 1) % RD, 0, q);
+                    __builtin_amdgcn_sched_group_barrier(0x020, 3 * TM, 0);
+                } else {
+                    load_pixels((s + 1) % RD, 0);
+                    next_load_step();
+                    __builtin_amdgcn_sched_group_barrier(0x020, 3 * TM + 8, 0);
+                }
+#pragma unroll
+                for (int k = 0; k < 3; k++) multiply(g, k);
+                if (g == 0) split_issue_order<3 * T, 39>();
+                __builtin_amdgcn_sched_barrier(0);
+                if (g == 1) {
+                    __syncthreads();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                read_b(0, g ^ 1, next_buf);
+                __builtin_amdgcn_sched_barrier(0);
+                if (g == 0) split_pixels((s + 1) % RD, 0, 3);
+                multiply(g, 3);
+                multiply(g, 4);
+                if (g == 0) split_issue_order<2 * T, 13>();
+                __builtin_amdgcn_sched_barrier(0);
+                read_b(1, g ^ 1, next_buf);
+                if (g == 0) put_pixels(0, buf ^ 1);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(g, 5);
+                __builtin_amdgcn_sched_barrier(0);
+                read_b(2, g ^ 1, next_buf);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x200, 3, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, 8, 0);
-            __builtin_amdgcn_sched_barrier(0);
+        };
+        int step = step_lo;
+        for (; step + 2 <= step_hi; step += 2) {
+            whole_step(step, 0);
+            whole_step(step + 1, 1);
         }
-        __syncthreads();
+        if (step < step_hi) whole_step(step, 0);
+        __syncthreads();  // (the last reads, before the epilogue writes there)
+    } else {
+        // The same with a barrier at the end of a step and a chunk split in each half: more registers are not to be had, and the order
+        // above without them is 2-6 % slower here.
+        for (int step = step_lo; step < step_hi; step++) {
+            const int buf = (step - step_lo) & 1;
+#pragma unroll
+            for (int g = 0; g < 2; g++) {
+#pragma unroll
+                for (int part = 0; part < 3; part++) read_b(part, g, buf);
+                load_a(g ^ 1, step + g);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < 6; k++) multiply(g, k);
+#pragma unroll
+                for (int q = 0; q < 4; q++) split_pixels(0, g, q);
+                put_pixels(g, buf ^ 1);
+                load_pixels(0, g);
+                if (g == 1) next_load_step();
+                // issue order: the splitting between the matrix instructions, then what it is for
+                split_issue_order<6 * T, 72>();
+                __builtin_amdgcn_sched_group_barrier(0x200, 3, 0);
+                __builtin_amdgcn_sched_group_barrier(0x020, 8, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __syncthreads();
+        }
     }
     trace_mark(p, 2);
 #pragma unroll

@@ -174,6 +174,30 @@ struct ChannelEpilogue {
     float bias, mean, sd, g, b;
 };
 
+// x / sd rounded to nearest, for many x and one sd, without the division: with r + rl = 1 / sd to 48 bits (r rounded to nearest) the
+// quotient q = x r + x rl is within an ulp of x / sd, its remainder x - q sd is exact, and q plus r times it is then the correctly
+// rounded quotient (Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", 1990).  Nothing may over- or
+// underflow on the way: sd and |x| lie in [2^-60, 2^60] (out_of_quotient_range; zeros, infinities, NaN and the rest are divided).
+// Four instructions and one for the range instead of the division's fourteen issue slots: 64 -> 256 1x1 on 56x56 with batch norm, 64 images,
+// 80.7 -> 75.1 us, 3x3 64 -> 64 68.9 -> 67.3.
+struct Reciprocal {
+    float r, rl;
+};
+__device__ __forceinline__ Reciprocal reciprocal_of(float sd) {  // r = 0: not in the range
+    Reciprocal k;
+    const bool ok = sd >= 0x1p-60f && sd <= 0x1p60f;
+    k.r = ok ? __fdiv_rn(1.0f, sd) : 0.0f;
+    k.rl = ok ? __fdiv_rn(__builtin_fmaf(-k.r, sd, 1.0f), sd) : 0.0f;
+    return k;
+}
+__device__ __forceinline__ float quotient(float x, float sd, float r, float rl) {
+    const float q = __builtin_fmaf(x, r, __fmul_rn(x, rl));
+    return __builtin_fmaf(__builtin_fmaf(-q, sd, x), r, q);
+}
+// ... for a wavefront: the least and the largest |x| of its values, the least zero where a channel has no reciprocal.  (NaN passes, and
+// comes out as NaN.)
+__device__ __forceinline__ bool out_of_quotient_range(float least, float most) { return __any(!(least >= 0x1p-60f && most <= 0x1p60f)); }
+
 __device__ __forceinline__ ChannelEpilogue load_channel(const ConvParams &p, int k) {
     ChannelEpilogue e;
     e.bias = p.bias ? p.bias[k] : 0.0f;
@@ -288,8 +312,9 @@ __device__ __forceinline__ void store_partial(const ConvParams &p, floatx16 (&ac
             for (int v = 0; v < 16; v++) dst[((tm * TN + tn) * 16 + v) * 64] = acc[tm][tn][v];
 }
 
+constexpr int EPI_ROWS = 7;
 // The per-channel constants of a tile's BM channels reach the epilogue through LDS (layout:
-// bias[BM], mean[BM], sd[BM], g[BM], b[BM]).  Thread t < BM fetches those of channel m0 + t at the
+// bias[BM], mean[BM], sd[BM], g[BM], b[BM], r[BM], rl[BM], the last two of 1 / sd).  Thread t < BM fetches those of channel m0 + t at the
 // START of the kernel, so that their memory latency passes during the K loop instead of standing
 // between the last MFMA and the first store, and writes them to LDS after the loop; the caller
 // synchronises before and after that write.
@@ -307,6 +332,9 @@ __device__ __forceinline__ void put_channel_constants(float *epi, const ChannelE
         epi[2 * BM + tid] = e.sd;
         epi[3 * BM + tid] = e.g;
         epi[4 * BM + tid] = e.b;
+        const Reciprocal k = reciprocal_of(e.sd);
+        epi[5 * BM + tid] = k.r;
+        epi[6 * BM + tid] = k.rl;
     }
 }
 template <int BM>
@@ -366,10 +394,29 @@ __device__ __forceinline__ void store_tile_inside(const ConvParams &p, floatx16 
             if (has_bn) {
                 const floatx4 mean = *reinterpret_cast<const floatx4 *>(epi + BM + row0);
                 const floatx4 sd = *reinterpret_cast<const floatx4 *>(epi + 2 * BM + row0);
+                const floatx4 r = *reinterpret_cast<const floatx4 *>(epi + 5 * BM + row0), rl = *reinterpret_cast<const floatx4 *>(epi + 6 * BM + row0);
+                float least = 1.0f, most = 1.0f;
 #pragma unroll
-                for (int j = 0; j < 4; j++)
+                for (int j = 0; j < 4; j++) {
+                    least = r[j] > 0.0f ? least : 0.0f;
 #pragma unroll
-                    for (int tn = 0; tn < TN; tn++) x[j][tn] = __fdiv_rn(__fsub_rn(x[j][tn], mean[j]), sd[j]);
+                    for (int tn = 0; tn < TN; tn++) {
+                        x[j][tn] = __fsub_rn(x[j][tn], mean[j]);
+                        least = fminf(least, fabsf(x[j][tn]));
+                        most = fmaxf(most, fabsf(x[j][tn]));
+                    }
+                }
+                if (out_of_quotient_range(least, most)) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+#pragma unroll
+                        for (int tn = 0; tn < TN; tn++) x[j][tn] = __fdiv_rn(x[j][tn], sd[j]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+#pragma unroll
+                        for (int tn = 0; tn < TN; tn++) x[j][tn] = quotient(x[j][tn], sd[j], r[j], rl[j]);
+                }
                 if (affine) {
                     const floatx4 g = *reinterpret_cast<const floatx4 *>(epi + 3 * BM + row0);
                     const floatx4 b = *reinterpret_cast<const floatx4 *>(epi + 4 * BM + row0);
@@ -643,12 +690,35 @@ __device__ __forceinline__ void wino_store_rows(const ConvParams &p, const float
     }
     if (p.bn_mean) {
         const vec_t mean = *reinterpret_cast<const vec_t *>(epi + BM + ml), sd = *reinterpret_cast<const vec_t *>(epi + 2 * BM + ml);
+        const vec_t r = *reinterpret_cast<const vec_t *>(epi + 5 * BM + ml), rl = *reinterpret_cast<const vec_t *>(epi + 6 * BM + ml);
+        float least = 1.0f, most = 1.0f;
 #pragma unroll
-        for (int k = 0; k < NK; k++)
+        for (int k = 0; k < NK; k++) {
+            least = r[k] > 0.0f ? least : 0.0f;
 #pragma unroll
             for (int a = 0; a < 2; a++)
 #pragma unroll
-                for (int b = 0; b < 2; b++) x[k][a][b] = __fdiv_rn(__fsub_rn(x[k][a][b], mean[k]), sd[k]);
+                for (int b = 0; b < 2; b++) {
+                    x[k][a][b] = __fsub_rn(x[k][a][b], mean[k]);
+                    least = fminf(least, fabsf(x[k][a][b]));
+                    most = fmaxf(most, fabsf(x[k][a][b]));
+                }
+        }
+        if (out_of_quotient_range(least, most)) {
+#pragma unroll
+            for (int k = 0; k < NK; k++)
+#pragma unroll
+                for (int a = 0; a < 2; a++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++) x[k][a][b] = __fdiv_rn(x[k][a][b], sd[k]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < NK; k++)
+#pragma unroll
+                for (int a = 0; a < 2; a++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++) x[k][a][b] = quotient(x[k][a][b], sd[k], r[k], rl[k]);
+        }
         if (p.bn_g) {
             const vec_t g = *reinterpret_cast<const vec_t *>(epi + 3 * BM + ml), bb = *reinterpret_cast<const vec_t *>(epi + 4 * BM + ml);
 #pragma unroll
@@ -1875,7 +1945,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     constexpr int XCH_FLOATS = 4 * 2 * 16 * 64;  // the exchange of one 32x32 block: [position row][b][v][lane]
     constexpr int LDS_FLOATS = 2 * BUF_FLOATS > XCH_FLOATS ? 2 * BUF_FLOATS : XCH_FLOATS;
     __shared__ __attribute__((aligned(16))) float lds[LDS_FLOATS];
-    __shared__ __attribute__((aligned(16))) float epi[5 * MF];
+    __shared__ __attribute__((aligned(16))) float epi[EPI_ROWS * MF];
 
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -2790,8 +2860,10 @@ int eddlhip_conv2d_uncache_filters(int dev, const float *K) {
 int eddlhip_conv2d_force_plan(int tile, int slices) {
     EH_REQUIRE(is_plan_tile(tile),
                "conv2d_force_plan: tile is -1 (automatic), 0..3, 4 .. %d (the Winograd forms where they apply), %d, %d (a 2x2 filter on an input upsampled twice) "
-               "%d .. %d (the split form where it applies) or %d, %d .. %d (the one-launch Winograd and the upsampled-input form in that arithmetic)",
-               UP2X2_TILE - 1, UP2X2_TILE, UP2X2_TILE + 1, SPLIT_TILE0, SPLIT_TILE0 + NUM_SPLIT - 1, WSPLIT_TILE0, UPSPLIT_TILE0, UPSPLIT_TILE0 + NUM_UPSPLIT - 1);
+               "%d .. %d (the split form where it applies) or %d, %d .. %d (the one-launch Winograd and the upsampled-input form in that arithmetic) "
+               "or %d .. %d (the split form for few tiles)",
+               UP2X2_TILE - 1, UP2X2_TILE, UP2X2_TILE + 1, SPLIT_TILE0, SPLIT_TILE0 + NUM_SPLIT - 1, WSPLIT_TILE0, UPSPLIT_TILE0, UPSPLIT_TILE0 + NUM_UPSPLIT - 1,
+               WAVE_TILE0, WAVE_TILE0 + NUM_WAVE - 1);
     g_force_tile = tile;
     g_force_slices = slices;
     return 0;

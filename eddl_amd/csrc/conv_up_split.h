@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
     constexpr int CHUNKS = SPLIT_K / (256 / BN) / 8;
     static_assert(CHUNKS == 1 || CHUNKS == 2, "BN is 64 or 128");
     __shared__ uintx4 Bs[2][3][SPLIT_K / 8][BN];
-    __shared__ __attribute__((aligned(16))) float epi[5 * BM];
+    __shared__ __attribute__((aligned(16))) float epi[EPI_ROWS * BM];
 
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -138,7 +138,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int FM = 2, MF = 32 * FM, NB = 32, CK = 16, SLOTS = 16 * NB;
     constexpr int R_FLOATS = CK * SLOTS;
     __shared__ __attribute__((aligned(16))) float lds[2 * R_FLOATS];
-    __shared__ __attribute__((aligned(16))) float epi[5 * MF];
+    __shared__ __attribute__((aligned(16))) float epi[EPI_ROWS * MF];
     static_assert(2 * R_FLOATS >= FM * 4 * 2 * 16 * 64, "the exchange of the filter groups");
 
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;

@@ -1992,3 +1992,32 @@ def test_conv2d_split_form_for_few_tiles_reads_folded_inputs_and_applies_the_epi
     ok = np.isfinite(fp32)
     assert (~ok).any() and np.array_equal(np.isnan(fp32), np.isnan(got)) and np.array_equal(fp32[~ok & ~np.isnan(fp32)], got[~ok & ~np.isnan(fp32)])
     assert np.array_equal(finite[ok], got[ok])
+
+
+@pytest.mark.parametrize("plan", [(0, 1), (2, 1), (6, 1), (7, 1), (17, 1), (18, 1), (32, 1), (40, 1)])
+@pytest.mark.parametrize("e_pixels,e_deviation", [(0, 0), (-59, 3), (-61, 0), (-75, -20), (59, -3), (62, 0), (70, 20), (-130, 0), (0, -59), (0, -61), (0, 59), (0, 61)])
+def test_conv2d_epilogue_divides_as_the_batch_norm_kernel_does(hip, plan, e_pixels, e_deviation):
+    """The quotient by the reciprocal, on either side of the range that it is taken in, bit for bit: numbers and deviations around 2^-60 and
+    2^60, zeros of both signs, subnormal numbers, infinities."""
+    rng = np.random.default_rng(2600)
+    N, C, H, W, Kf = 2, 32, 8, 24, 64
+    x = np.ldexp(rng.standard_normal((N, C, H, W)), e_pixels).astype(np.float32)
+    x[0, :, :4] = 0.0
+    w = (rng.standard_normal((Kf, C, 3, 3)) * 0.1).astype(np.float32)
+    if abs(e_pixels) == 59:
+        x[1, 3, 6, 20] = np.inf
+    g, b = rng.uniform(0.8, 1.2, Kf).astype(np.float32), (rng.standard_normal(Kf) * 0.1).astype(np.float32)
+    mean = np.where(np.arange(Kf) % 3 == 0, 0.0, np.ldexp(rng.standard_normal(Kf) * 0.1, e_pixels)).astype(np.float32)
+    var = np.ldexp(rng.uniform(0.5, 1.5, Kf), 2 * e_deviation).astype(np.float32)
+    X, Wd, bn = hip.array(x), hip.array(w), tuple(hip.array(v) for v in (g, b, mean, var)) + (0.0,)
+    A, B, F = (hip.full((N, Kf, H, W), np.nan) for _ in range(3))
+    try:
+        hip.force_conv_plan(*plan)
+        hip.conv2D(X, Wd, None, A, 1, 1, 1, 1)
+        hip.conv2D(X, Wd, None, F, 1, 1, 1, 1, bn=bn)
+    finally:
+        hip.force_conv_plan(-1, 1)
+    hip.batchnorm_inference(A, B, hip.empty((N, Kf, H, W)), bn[2], bn[3], bn[0], bn[1], hip.empty((Kf,)), 0.0)
+    want, got = B.numpy(), F.numpy()
+    assert np.array_equal(np.isnan(want), np.isnan(got))
+    assert np.array_equal(want.view(np.uint32)[~np.isnan(want)], got.view(np.uint32)[~np.isnan(want)])

@@ -174,7 +174,7 @@ struct ChannelEpilogue {
     float bias, mean, sd, g, b;
 };
 
-// x / sd rounded to nearest, for many x and one sd, without the division: with r + rl = 1 / sd to 48 bits (r rounded to nearest) the
+// x / sd rounded to nearest, for many x and one sd, without the division: with r + rl = 1 / sd to 47 bits (r rounded to nearest) the
 // quotient q = x r + x rl is within an ulp of x / sd, its remainder x - q sd is exact, and q plus r times it is then the correctly
 // rounded quotient (Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", 1990).  Nothing may over- or
 // underflow on the way: sd and |x| lie in [2^-60, 2^60] (out_of_quotient_range; zeros, infinities, NaN and the rest are divided).
@@ -187,7 +187,7 @@ __device__ __forceinline__ Reciprocal reciprocal_of(float sd) {  // r = 0: not i
     Reciprocal k;
     const bool ok = sd >= 0x1p-60f && sd <= 0x1p60f;
     k.r = ok ? __fdiv_rn(1.0f, sd) : 0.0f;
-    k.rl = ok ? __fdiv_rn(__builtin_fmaf(-k.r, sd, 1.0f), sd) : 0.0f;
+    k.rl = __fmul_rn(__builtin_fmaf(-k.r, sd, 1.0f), k.r);
     return k;
 }
 __device__ __forceinline__ float quotient(float x, float sd, float r, float rl) {
@@ -318,23 +318,29 @@ constexpr int EPI_ROWS = 7;
 // START of the kernel, so that their memory latency passes during the K loop instead of standing
 // between the last MFMA and the first store, and writes them to LDS after the loop; the caller
 // synchronises before and after that write.
+struct TileChannel : ChannelEpilogue {
+    Reciprocal k;
+};
+constexpr TileChannel NO_CHANNEL = {{0.0f, 0.0f, 1.0f, 1.0f, 0.0f}, {0.0f, 0.0f}};
 template <int BM>
-__device__ __forceinline__ ChannelEpilogue fetch_channel_constants(const ConvParams &p, int m0, int tid) {
-    ChannelEpilogue e = {0.0f, 0.0f, 1.0f, 1.0f, 0.0f};
-    if (tid < BM && m0 + tid < p.Kf) e = load_channel(p, m0 + tid);
+__device__ __forceinline__ TileChannel fetch_channel_constants(const ConvParams &p, int m0, int tid) {
+    TileChannel e = NO_CHANNEL;
+    if (tid < BM && m0 + tid < p.Kf) {
+        static_cast<ChannelEpilogue &>(e) = load_channel(p, m0 + tid);
+        if (p.bn_mean) e.k = reciprocal_of(e.sd);
+    }
     return e;
 }
 template <int BM>
-__device__ __forceinline__ void put_channel_constants(float *epi, const ChannelEpilogue &e, int tid) {
+__device__ __forceinline__ void put_channel_constants(float *epi, const TileChannel &e, int tid) {
     if (tid < BM) {
         epi[tid] = e.bias;
         epi[BM + tid] = e.mean;
         epi[2 * BM + tid] = e.sd;
         epi[3 * BM + tid] = e.g;
         epi[4 * BM + tid] = e.b;
-        const Reciprocal k = reciprocal_of(e.sd);
-        epi[5 * BM + tid] = k.r;
-        epi[6 * BM + tid] = k.rl;
+        epi[5 * BM + tid] = e.k.r;
+        epi[6 * BM + tid] = e.k.rl;
     }
 }
 template <int BM>
@@ -406,7 +412,7 @@ __device__ __forceinline__ void store_tile_inside(const ConvParams &p, floatx16 
                         most = fmaxf(most, fabsf(x[j][tn]));
                     }
                 }
-                if (out_of_quotient_range(least, most)) {
+                if (__builtin_expect(out_of_quotient_range(least, most), 0)) {  // (out of line: a jump over it costs a small launch 0.1 us a time)
 #pragma unroll
                     for (int j = 0; j < 4; j++)
 #pragma unroll
@@ -704,7 +710,7 @@ __device__ __forceinline__ void wino_store_rows(const ConvParams &p, const float
                     most = fmaxf(most, fabsf(x[k][a][b]));
                 }
         }
-        if (out_of_quotient_range(least, most)) {
+        if (__builtin_expect(out_of_quotient_range(least, most), 0)) {  // (out of line: a jump over it costs a small launch 0.1 us a time)
 #pragma unroll
             for (int k = 0; k < NK; k++)
 #pragma unroll
@@ -848,7 +854,7 @@ __device__ __forceinline__ void conv_tap_body(const ConvParams &p) {
     const int step_hi = split ? min(step_lo + p.slice_steps, p.nsteps) : p.nsteps;
     const int m0 = m_tile * BM;
     const long long n0 = (long long)n_tile * BN;
-    ChannelEpilogue chan = {0.0f, 0.0f, 1.0f, 1.0f, 0.0f};
+    TileChannel chan = NO_CHANNEL;
     if (!split && !UP2) chan = fetch_channel_constants<BM>(p, m0, tid);  // (UP2 has no register to spare in its K loop: fetched after it)
 
     const __amdgpu_buffer_rsrc_t rsrc_in = __builtin_amdgcn_make_buffer_rsrc((void *)p.I, 0, p.in_bytes, RSRC_WORD3);
@@ -1277,7 +1283,7 @@ __global__ __launch_bounds__(256, (TM * TN >= 4 ? 3 : 4)) void conv_gen_kernel(c
     const int step_hi = split ? min(step_lo + p.slice_steps, p.nsteps) : p.nsteps;
     const int m0 = m_tile * BM;
     const long long n0 = (long long)n_tile * BN;
-    ChannelEpilogue chan = {0.0f, 0.0f, 1.0f, 1.0f, 0.0f};
+    TileChannel chan = NO_CHANNEL;
     if (!split) chan = fetch_channel_constants<BM>(p, m0, tid);
 
     const __amdgpu_buffer_rsrc_t rsrc_in = __builtin_amdgcn_make_buffer_rsrc((void *)p.I, 0, p.in_bytes, RSRC_WORD3);
@@ -1959,7 +1965,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     const int step_hi = split ? min(step_lo + p.slice_steps, p.nsteps) : p.nsteps;
     // Requested first, used last: the step's filter slice needs nothing but the tile's place, so it is on its way while
     // the lanes work out where the pixels go (below); so are the channel constants, which reach LDS after that.
-    ChannelEpilogue chan = {0.0f, 0.0f, 1.0f, 1.0f, 0.0f};
+    TileChannel chan = NO_CHANNEL;
 
     // filter slice: a wavefront instruction moves 256 consecutive floats of the slice, i.e. RPI whole rows of MF
     constexpr int RPI = 256 / MF, U_UNITS = U_FLOATS / 256, UPW = U_UNITS / 4;

@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
     const int step_hi = split ? min(step_lo + p.slice_steps, p.nsteps) : p.nsteps;
     const int m0 = m_tile * BM;
     const int n0 = n_tile * BN;
-    ChannelEpilogue chan = {0.0f, 0.0f, 1.0f, 1.0f, 0.0f};
+    TileChannel chan = NO_CHANNEL;
     if (!split) chan = fetch_channel_constants<BM>(p, m0, tid);
 
     const __amdgpu_buffer_rsrc_t rsrc_in = __builtin_amdgcn_make_buffer_rsrc((void *)p.I, 0, p.in_bytes, RSRC_WORD3);

@@ -157,7 +157,7 @@ __global__ __launch_bounds__(256, 2) void conv_up2x2_split_kernel(const ConvPara
 #pragma unroll
     for (int chunk = 0; chunk < CHUNKS; chunk++) load_pixels(step_lo, 0, chunk);
     load_a(0, 2 * step_lo, 0);
-    ChannelEpilogue chan = {0.0f, 0.0f, 1.0f, 1.0f, 0.0f};
+    TileChannel chan = NO_CHANNEL;
     if (!split) chan = fetch_channel_constants<BM>(p, m0, tid);
 #pragma unroll
     for (int chunk = 0; chunk < CHUNKS; chunk++) put_pixels(0, chunk), load_pixels(step_lo, 1, chunk);

@@ -2621,6 +2621,82 @@ Plan forced_plan(const Variant *family, int tile, int slices, int Kf, int C, int
 }
 
 
+// The planner's choice among the tiles of the split form (conv_split.h, conv_wave_split.h) for a convolution that the direct kernels
+// are expected to take `direct_us` for: tile -1 if none is expected to be faster.  It depends on the geometry alone, so that a convolution
+// has the same bits from registered filters, from others (splitting them costs a call what repacking them does: 10 bytes of
+// traffic a weight instead of 8) and from the entry point that allocates nothing - a choice whose filters and partial tiles do
+// not fit that one's scratch array is none.
+// Time of a workgroup step: `alone` with one workgroup on a CU, at least `shared` for every one that is there; of a workgroup around its
+// steps: `fixed` and `each` for every one there.  Fitted to 6200 timed plans of 281 convolutions (1 - 64 images, 7 - 368 pixels, 16 - 1024
+// channels, filters of 1 - 7, this library's networks among them), rms error 17-20 %; by its choices the 156 of them that have whole groups of
+// 16 channels take 1 / 1.43 of the direct kernels' time together (the best plan of each:
+// 1 / 1.5) and none takes more than 1.02 of it.  Below 7 us of direct kernel nothing is to be gained by this model, and the direct kernel stays.
+struct SplitChoice {
+    int tile, slices;
+    double cost_us;
+};
+SplitChoice plan_split(int Kf, int C, int RS, int Mp, long long npix, int num_cu, double direct_us, double traffic_us) {
+    static const struct {
+        double alone, shared, fixed, each;
+        int resident;
+    } kTile[NUM_SPLIT] = {{1.34, 0.978, 1.8, 1.04, 2}, {0.723, 0.48, 0.0334, 1.68, 3}, {0.976, 0.586, 0.00882, 1.76, 3}, {0.554, 0.345, 0.248, 1.01, 4}};
+    static const struct {
+        double launch, group, unit, slices;
+        int resident;
+    } kWave[NUM_WAVE] = {{1.1, 2.76, 0.762, 2.16, 2}, {0.211, 4.41, 1.02, 2.02, 1}};
+    static const int kSlices[6] = {1, 2, 3, 4, 6, 8};
+    SplitChoice best = {-1, 1, direct_us > traffic_us ? direct_us : traffic_us};
+    if (best.cost_us < 7.0 || C % 16 != 0) return best;
+    if (direct_us > traffic_us) best.cost_us = 0.9 * direct_us > traffic_us ? 0.9 * direct_us : traffic_us;  // (a tenth for the model's error)
+    const size_t filters = (split_filter_bytes(C, RS, Mp) + 255) & ~(size_t)255;
+    auto offer = [&](int tile, int slices, size_t partial, double us) {
+        us = us > traffic_us ? us : traffic_us;
+        if (us < best.cost_us && filters + partial <= (size_t)EDDLHIP_CONV_NOALLOC_SCRATCH_BYTES) best = {tile, slices, us};
+    };
+    for (int t = 0; t < NUM_SPLIT; t++) {
+        const auto &k = kTile[t];
+        auto step = [&](long long there) { return k.alone > k.shared * (double)there ? k.alone : k.shared * (double)there; };
+        int last = 0;
+        for (int want : kSlices) {
+            const Plan fp = forced_plan(ksplit, t, want, Kf, C, RS, npix, num_cu);
+            if (fp.nslices == last) continue;
+            last = fp.nslices;
+            const long long divided = fp.nslices > 1 ? fp.leftover : 0;
+            const long long whole = (fp.tiles - divided + num_cu - 1) / num_cu, parts = (divided * fp.nslices + num_cu - 1) / num_cu;  // on the busiest CU
+            auto group = [&](long long there, int steps) { return steps * step(there) + k.fixed + (double)there * k.each; };
+            const long long tail = whole % k.resident;
+            double us = 1.5 + (double)(whole / k.resident) * group(k.resident, fp.nsteps);
+            if (tail > 0) {
+                const long long there = tail + parts < k.resident ? tail + parts : k.resident;
+                us += group(there, fp.nsteps);
+                if (tail + parts > k.resident) us += fp.slice_steps * step(tail + parts - k.resident) + k.fixed;
+            } else if (parts > 0) {
+                us += (double)(parts / k.resident) * group(k.resident, fp.slice_steps);
+                if (parts % k.resident > 0) us += group(parts % k.resident, fp.slice_steps);
+            }
+            const size_t partial = (size_t)(divided * fp.nslices) * ksplit[t].bm * ksplit[t].bn * sizeof(float);
+            if (divided > 0) us += (double)partial * 2.0 / 3.0e6 + 4.0;
+            offer(SPLIT_TILE0 + t, fp.nslices, partial, us);
+        }
+    }
+    for (int t = 0; t < NUM_WAVE; t++) {
+        const auto &k = kWave[t];
+        const long long units = (long long)(C / 16) * RS;
+        int last = 0;
+        for (int want : kSlices) {
+            const int slices = wave_slices(kwave[t], want, Kf, C, RS, npix);
+            const long long tiles = wave_tiles(kwave[t], Kf, npix), here = (tiles * slices + num_cu - 1) / num_cu;
+            if (slices == last || tiles * slices > 8LL * num_cu) continue;
+            last = slices;
+            const double each = (double)((units + 8 * slices - 1) / (8 * slices)) * k.unit;
+            double us = k.launch + (double)(here / k.resident) * (k.group + each * k.resident) + (slices > 1 ? k.slices : 0.0);
+            if (here % k.resident > 0) us += k.group + each * (double)(here % k.resident);
+            offer(WAVE_TILE0 + t, slices, slices > 1 ? (size_t)(tiles * slices) * kwave[t].tm * kwave[t].tn * 4096 : 0, us);
+        }
+    }
+    return best;
+}
+
 // ---------------------------------------------------------------- cache of repacked filters
 // A caller that keeps its filters fixed between calls (inference) registers them once
 // (eddlhip_conv2d_cache_filters); eddlhip_conv2d_fwd then finds the repacked copy by the filter
@@ -2655,8 +2731,11 @@ int cache_rows(int C, int R, int S) {
 
 int launch_split_filters(int dev, const float *K, void *Ws, int Kf, int C, int RS, int Mp) {
     const int mblocks = Mp / 32, k16s = split_steps(C, RS) * 2;
-    hipLaunchKernelGGL(split_filter_kernel, dim3((unsigned)(((size_t)k16s * mblocks * 64 + 255) / 256)), dim3(256), 0, state(dev).stream, K, (uintx4 *)Ws, Kf, C, RS,
-                       mblocks, k16s);
+    if (RS > 1 && RS <= SPLIT_FILTER_TAPS && (long long)Kf * C * RS >= SPLIT_FILTER_MANY)  // (a workgroup for the zeros past an odd number of 16 channels, too)
+        hipLaunchKernelGGL(split_filter_taps_kernel, dim3((unsigned)(k16s / RS * mblocks)), dim3(256), 0, state(dev).stream, K, (uintx4 *)Ws, Kf, C, RS, mblocks);
+    else
+        hipLaunchKernelGGL(split_filter_kernel, dim3((unsigned)(((size_t)k16s * mblocks * 64 + 255) / 256)), dim3(256), 0, state(dev).stream, K, (uintx4 *)Ws, Kf, C, RS,
+                           mblocks, k16s);
     EH_CHECK_LAUNCH();
     return 0;
 }
@@ -3451,6 +3530,17 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
         const int rc = conv2d_wave_split(no_alloc, kwave[g_force_tile - WAVE_TILE0], g_force_slices, dev, p, chunk_imgs, &no_room);
         if (!no_room) return rc;
     }
+    // the planner's own choice: a tile of the split form where its model expects one to be faster (not under switches that ask for the
+    // fp32 instruction's sums, or for undivided tiles)
+    SplitChoice choice = {-1, 1, 0.0};
+    bool chosen = false;
+    auto choose = [&]() {
+        if (chosen) return;
+        chosen = true;
+        if (gemm || !split_ok || g_split == 0 || (g_force_tile >= 0 && g_force_tile < 4)) return;
+        const double traffic_us = 4.0 * ((double)chunk_imgs * C * H * W + (double)chunk_imgs * Kf * p.PQ) / 5.0e6;
+        choice = plan_split(Kf, C, R * S, p.Mp, (long long)chunk_imgs * p.PQ, state(dev).num_cu, plan.cost_us, traffic_us);
+    };
     const bool query = gemm != nullptr && gemm->need_out != nullptr;  // report the workspace need, launch nothing
     bool plan_open = false;                                         // a search could still pick any plan for this geometry
     if (g_autotune && g_force_tile < 0 && g_algo == 0 && g_split != 0) {
@@ -3469,13 +3559,16 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
             memcpy(best.key, key, sizeof(key));
             const size_t ws_before = state(dev).workspace_bytes;
             FilterCopies keep = copies_held(dev, K, Kf, C, R, S);  // (those that other geometries' plans, and graphs, may use)
-            const int src = search_plan(call, family, plan, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, split_ok, wsplit_ok, upsplit_ok, wave_ok, &best);
+            choose();
+            Plan planned = plan;
+            if (choice.tile >= 0) planned.tile = -1;  // (not one of the direct tiles)
+            const int src = search_plan(call, family, planned, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, split_ok, wsplit_ok, upsplit_ok, wave_ok, &best);
             if (src < 0) return -src;  // a runtime error inside the search
             if (src == 0) {
                 keep.wino = keep.wino || best.tile == 4 || best.tile == 5;
                 keep.fused = keep.fused || (best.tile >= FUSED_TILE0 && best.tile < FUSED_TILE0 + NUM_FUSED);
                 keep.up = keep.up || best.tile == UP2X2_TILE || best.tile == UP2X2_TILE + 1;
-                keep.split = keep.split || is_split_tile(best.tile) || is_wave_tile(best.tile);
+                keep.split = keep.split || is_split_tile(best.tile) || is_wave_tile(best.tile) || (best.tile < 0 && choice.tile >= 0);
                 keep.upsplit = keep.upsplit || is_upsplit_tile(best.tile);
                 keep.wsplit = keep.wsplit || is_wsplit_tile(best.tile);
             }
@@ -3511,8 +3604,21 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
             const int rc = conv2d_wave_split(no_alloc, kwave[found->tile - WAVE_TILE0], found->slices, dev, p, chunk_imgs, &no_room);
             if (!no_room) return rc;
         }
-        if (found != nullptr && found->tile >= 0 && found->tile < 4)
+        if (found != nullptr && found->tile >= 0 && found->tile < 4) {
             plan = forced_plan(family, found->tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu);
+            choice.tile = -1;
+            chosen = true;
+        }
+    }
+    choose();
+    if (choice.tile >= 0) {
+        no_room = false;
+        const int rc = is_wave_tile(choice.tile)
+                           ? conv2d_wave_split(no_alloc, kwave[choice.tile - WAVE_TILE0], choice.slices, dev, p, chunk_imgs, &no_room)
+                           : conv2d_split(no_alloc, split_build(choice.tile - SPLIT_TILE0, R * S, uh, uw),
+                                          forced_plan(ksplit, choice.tile - SPLIT_TILE0, choice.slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p, chunk_imgs,
+                                          &no_room);
+        if (!no_room) return rc;
     }
     if (query && plan_open) {
         // the largest partial-tile need of any plan the search tries

@@ -75,6 +75,49 @@ __global__ __launch_bounds__(256) void split_filter_kernel(const float *__restri
     dst[128] = lo;
 }
 
+// The same for filters of 2 ... 9 taps: a workgroup takes 32 filters and 16 channels, whose weights lie in 32 runs of memory, through LDS, so that
+// reads are whole lines (one weight at a time they are 4 bytes at the stride of the taps).  us with the launch,
+// one weight at a time -> this: 512 -> 512 16.6 -> 11.6, 1024 -> 1024 37 -> 15.9, 128 -> 128 3.2 -> 4.9, 256 -> 512 9.1 -> 11.2; so from 2 million weights on.
+constexpr int SPLIT_FILTER_TAPS = 9;
+constexpr long long SPLIT_FILTER_MANY = 2000000;
+__global__ __launch_bounds__(256) void split_filter_taps_kernel(const float *__restrict__ K, uintx4 *__restrict__ Ws, int Kf, int C, int RS, int mblocks) {
+    constexpr int PITCH = 16 * SPLIT_FILTER_TAPS + 1;  // odd: the 32 filters of a read lie in 32 banks
+    __shared__ float rows[32 * PITCH];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int mb = blockIdx.x % mblocks, c16 = blockIdx.x / mblocks, run = 16 * RS, there = min(run, C * RS - c16 * run);  // (fewer, or none, past C)
+    constexpr int PASSES = (16 * SPLIT_FILTER_TAPS + 63) / 64;
+    float w[8][PASSES];  // (all of a wavefront's eight runs are asked for before the first is stored)
+#pragma unroll
+    for (int f8 = 0; f8 < 8; f8++)
+#pragma unroll
+        for (int i = 0; i < PASSES; i++) {
+            const int m = mb * 32 + 8 * wave + f8, r = lane + 64 * i;
+            w[f8][i] = m < Kf && r < there ? K[((size_t)m * C + c16 * 16) * RS + r] : 0.0f;
+        }
+#pragma unroll
+    for (int f8 = 0; f8 < 8; f8++)
+#pragma unroll
+        for (int i = 0; i < PASSES; i++)
+            if (lane + 64 * i < run) rows[(8 * wave + f8) * PITCH + lane + 64 * i] = SPLIT_UP * w[f8][i];
+    __syncthreads();
+    for (int t = wave; t < RS; t += 4) {
+        const float *src = rows + (lane & 31) * PITCH + (lane >> 5) * 8 * RS + t;
+        uintx4 hi, mid, lo;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            unsigned h, md, l;
+            split_pair(src[2 * j * RS], src[(2 * j + 1) * RS], h, md, l);
+            hi[j] = h;
+            mid[j] = md;
+            lo[j] = l;
+        }
+        uintx4 *dst = Ws + ((size_t)(2 * ((c16 >> 1) * RS + t) + (c16 & 1)) * mblocks + mb) * 192 + lane;
+        dst[0] = hi;
+        dst[64] = mid;
+        dst[128] = lo;
+    }
+}
+
 // Division by an upsampling factor as one multiplication, with no branch (a branch would end the block that the matrix
 // instructions are scheduled in): magic = ceil(2^32 / factor), 0 for factor 1.  The sides of the enlarged image are at most
 // 2^20, so the product overestimates the quotient by less than 2^-12 and by one whole at most.

@@ -212,7 +212,7 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * 2 = the scalar direct kernel (one thread per output; taps summed in the reference's ky,kx,c
  * order with its rounding - used to cross-check the MFMA kernels on the device);
  * 3 = MFMA with the operand slices staged through registers; 4 = MFMA with the operand slices
- * written by the load unit straight into LDS (what 0 and 1 select); 5 / 6 = switch off / on the
+ * written by the load unit straight into LDS (what 1 selects, and 0 where no other form is chosen); 5 / 6 = switch off / on the
  * division along K of the tiles left over after a whole number of tiles per CU (on by default;
  * independent of 0-4); 7 / 8 = switch on / off the Winograd form for every convolution it applies to
  * (off by default; independent of 5 / 6; only under 0); 9 = no Winograd form and no split form at all: the plan search
@@ -264,6 +264,9 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * kernels').  No output's bits depend on the inputs of another.  Workspace: the
  * split filters, 6 bytes a weight, unless registered, and the partial tiles of a K-split plan; where that is more than
  * eddlhip_conv2d_fwd_noalloc has (11 million unregistered weights), that entry point runs the planner's own choice.
+ * The planner chooses a tile of this form, or of the one for few tiles below, by itself where its model expects it to be faster than the
+ * direct kernels: by the geometry alone (whole groups of 16 channels, filters and partial tiles that fit the fixed scratch array, a
+ * direct kernel of 7 us or more), so registered and other filters and all entry points give the same bits.  Not under set_algo(1 .. 5) or (9).
  * The one-launch Winograd form in that arithmetic (force_plan(32, .), or the search from 512 blocks of outputs on; channel counts
  * that are multiples of 16): transformed pixels are fp32 numbers as in the third Winograd form, filters are transformed in 64 bits, the
  * products are those of the split form, and the sums of the largest of a patch's positions are rounded once per 16 channels: its error

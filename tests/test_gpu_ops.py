@@ -2021,3 +2021,74 @@ def test_conv2d_epilogue_divides_as_the_batch_norm_kernel_does(hip, plan, e_pixe
     want, got = B.numpy(), F.numpy()
     assert np.array_equal(np.isnan(want), np.isnan(got))
     assert np.array_equal(want.view(np.uint32)[~np.isnan(want)], got.view(np.uint32)[~np.isnan(want)])
+
+
+# ------------------------------------------------------------------ the planner's choice of the split form
+# N C H W Kf R S strides pads: chosen (tiles of either kernel, undivided and in slices) and, the last two, not: 40 channels, too little work
+PLANNER_CASES = {
+    "1x1": ((8, 256, 28, 28, 256, 1, 1, (1, 1), (0, 0)), True),
+    "3x3": ((2, 128, 28, 30, 128, 3, 3, (1, 1), (1, 1)), True),
+    "3x3 stride 2": ((9, 64, 57, 41, 96, 3, 3, (2, 2), (1, 1)), True),
+    "5x5": ((3, 48, 33, 35, 72, 5, 5, (1, 1), (2, 2)), True),
+    "many pixels": ((16, 64, 56, 56, 128, 3, 3, (1, 1), (1, 1)), True),
+    "long K": ((1, 1024, 14, 14, 200, 1, 1, (1, 1), (0, 0)), True),
+    "40 channels": ((2, 40, 56, 56, 128, 3, 3, (1, 1), (1, 1)), False),
+    "little work": ((1, 64, 12, 12, 32, 1, 1, (1, 1), (0, 0)), False),
+}
+
+
+@pytest.mark.parametrize("case", sorted(PLANNER_CASES))
+def test_conv2d_planner_chooses_the_split_form_by_the_geometry_alone(hip, case):
+    """The same kernel and bits from plain and registered filters and the entry point that allocates nothing; no further from 64 bits than the
+    direct kernels, which are left alone under the switches that ask for them."""
+    (N, C, H, W, Kf, R, S, stride, pad), chosen = PLANNER_CASES[case]
+    P, Q = (H + 2 * pad[0] - R) // stride[0] + 1, (W + 2 * pad[1] - S) // stride[1] + 1
+    rng = np.random.default_rng(2700 + sorted(PLANNER_CASES).index(case))
+    x = rng.standard_normal((N, C, H, W), dtype=np.float32)
+    w = (rng.standard_normal((Kf, C, R, S)) * np.sqrt(2.0 / (C * R * S))).astype(np.float32)
+    X, Wd, O = hip.array(x), hip.array(w), hip.full((N, Kf, P, Q), np.nan)
+    split = lambda k: k.startswith("conv_split_kernel") or k.startswith("conv_wave_split_kernel")
+    outs, kernels = {}, {}
+    try:
+        for call in ("plain", "noalloc", "registered", "ksplit_off", "winograd_never", "mfma_staged"):
+            hip.fill_(O, np.nan)
+            if call == "registered":
+                hip.cache_conv_filters(Wd)
+            if call == "noalloc":
+                hip._check(hip.lib.eddlhip_conv2d_fwd_noalloc(hip.dev, X.ptr, Wd.ptr, None, O.ptr, N, C, H, W, Kf, R, S, *stride, *pad, P, Q, None, None, None, None,
+                                                              0.0, None, 0))
+            else:
+                if call in ("ksplit_off", "winograd_never", "mfma_staged"):
+                    hip.set_conv_algo(call)
+                hip.conv2D(X, Wd, None, O, *stride, *pad)
+                hip.set_conv_algo({"ksplit_off": "ksplit_on", "winograd_never": "winograd_off"}.get(call, "auto"))
+            outs[call], kernels[call] = O.numpy(), hip.last_conv_kernel()
+    finally:
+        hip.set_conv_algo("ksplit_on")
+        hip.set_conv_algo("winograd_off")
+        hip.set_conv_algo("auto")
+        hip.uncache_conv_filters(Wd)
+    assert split(kernels["plain"]) == chosen and kernels["plain"] == kernels["noalloc"] == kernels["registered"], kernels
+    assert np.array_equal(outs["plain"], outs["noalloc"]) and np.array_equal(outs["plain"], outs["registered"])
+    assert not any(split(kernels[k]) for k in ("ksplit_off", "winograd_never", "mfma_staged")), kernels
+    ref = _conv64(x, w, stride, pad, P, Q)
+    assert np.linalg.norm(outs["plain"] - ref) <= np.linalg.norm(outs["winograd_never"] - ref)
+    assert_conv_close(ref, outs["plain"], case)
+
+
+@pytest.mark.parametrize("R,S", [(1, 1), (2, 2), (3, 3), (1, 9), (5, 2)])
+def test_conv2d_split_filters_of_many_weights(hip, R, S):
+    """From two million weights on the taps of a filter are split together: the bits of the weights split one by one (a slice of the filters)."""
+    rng = np.random.default_rng(2750 + 10 * R + S)
+    C = 336 if R * S == 9 else 1008 if R * S == 4 else 700
+    Kf, few = (2000000 + C * R * S - 1) // (C * R * S) + 3, 70
+    x = rng.standard_normal((1, C, 6, 11), dtype=np.float32)
+    w = (rng.standard_normal((Kf, C, R, S)) * 0.03).astype(np.float32)
+    O, F = hip.empty((1, Kf, 7 - R, 12 - S)), hip.empty((1, few, 7 - R, 12 - S))
+    try:
+        hip.force_conv_plan(40, 1)
+        hip.conv2D(hip.array(x), hip.array(w), None, O, 1, 1, 0, 0)
+        hip.conv2D(hip.array(x), hip.array(w[Kf - few:].copy()), None, F, 1, 1, 0, 0)
+    finally:
+        hip.force_conv_plan(-1, 1)
+    assert np.array_equal(O.numpy()[:, Kf - few:], F.numpy())

@@ -672,7 +672,8 @@ __device__ __forceinline__ ChannelEpilogue channel_from_lds(const float *epi, in
 // decided once for the 4 NK values (the flags are the same for every lane), the channel constants of the rows come from
 // LDS in one read each (`epi`: stage_channel_constants' layout, ml = the first row's place in the tile, a multiple of
 // NK), one 64-bit address serves all stores, and the residual's loads are in flight together.
-template <int BM, int NK>
+// QUOTIENT: a kernel with no registers for the reciprocals divides.
+template <int BM, int NK, bool QUOTIENT = true>
 __device__ __forceinline__ void wino_store_rows(const ConvParams &p, const float *epi, int ml, int m, int img, int ty, int tx, size_t plane,
                                                 float (&x)[NK][2][2]) {
     static_assert(NK == 4 || NK == 2, "the constants of the rows are one 16-byte or one 8-byte read");
@@ -696,27 +697,36 @@ __device__ __forceinline__ void wino_store_rows(const ConvParams &p, const float
     }
     if (p.bn_mean) {
         const vec_t mean = *reinterpret_cast<const vec_t *>(epi + BM + ml), sd = *reinterpret_cast<const vec_t *>(epi + 2 * BM + ml);
-        const vec_t r = *reinterpret_cast<const vec_t *>(epi + 5 * BM + ml), rl = *reinterpret_cast<const vec_t *>(epi + 6 * BM + ml);
-        float least = 1.0f, most = 1.0f;
+        if constexpr (QUOTIENT) {
+            const vec_t r = *reinterpret_cast<const vec_t *>(epi + 5 * BM + ml), rl = *reinterpret_cast<const vec_t *>(epi + 6 * BM + ml);
+            float least = 1.0f, most = 1.0f;
 #pragma unroll
-        for (int k = 0; k < NK; k++) {
-            least = r[k] > 0.0f ? least : 0.0f;
-#pragma unroll
-            for (int a = 0; a < 2; a++)
-#pragma unroll
-                for (int b = 0; b < 2; b++) {
-                    x[k][a][b] = __fsub_rn(x[k][a][b], mean[k]);
-                    least = fminf(least, fabsf(x[k][a][b]));
-                    most = fmaxf(most, fabsf(x[k][a][b]));
-                }
-        }
-        if (__builtin_expect(out_of_quotient_range(least, most), 0)) {  // (out of line: a jump over it costs a small launch 0.1 us a time)
-#pragma unroll
-            for (int k = 0; k < NK; k++)
+            for (int k = 0; k < NK; k++) {
+                least = r[k] > 0.0f ? least : 0.0f;
 #pragma unroll
                 for (int a = 0; a < 2; a++)
 #pragma unroll
-                    for (int b = 0; b < 2; b++) x[k][a][b] = __fdiv_rn(x[k][a][b], sd[k]);
+                    for (int b = 0; b < 2; b++) {
+                        x[k][a][b] = __fsub_rn(x[k][a][b], mean[k]);
+                        least = fminf(least, fabsf(x[k][a][b]));
+                        most = fmaxf(most, fabsf(x[k][a][b]));
+                    }
+            }
+            if (__builtin_expect(out_of_quotient_range(least, most), 0)) {  // (out of line: a jump over it costs a small launch 0.1 us a time)
+#pragma unroll
+                for (int k = 0; k < NK; k++)
+#pragma unroll
+                    for (int a = 0; a < 2; a++)
+#pragma unroll
+                        for (int b = 0; b < 2; b++) x[k][a][b] = __fdiv_rn(x[k][a][b], sd[k]);
+            } else {
+#pragma unroll
+                for (int k = 0; k < NK; k++)
+#pragma unroll
+                    for (int a = 0; a < 2; a++)
+#pragma unroll
+                        for (int b = 0; b < 2; b++) x[k][a][b] = quotient(x[k][a][b], sd[k], r[k], rl[k]);
+            }
         } else {
 #pragma unroll
             for (int k = 0; k < NK; k++)
@@ -766,7 +776,7 @@ __device__ __forceinline__ void wino_store_rows(const ConvParams &p, const float
 // A wavefront's 32 filters x 32 blocks: lane = block (column) lane % 32, filter rows 8 * (v / 4) + 4 * (lane / 32) + v % 4.
 // `epi`: the tile's channel constants (stage_channel_constants); m_local: the wavefront's first row in the tile.
 // NK: filter rows finished at a time (wino_store_rows), or 1 for a caller that has no registers for that.
-template <int BM, int NK = 4>
+template <int BM, int NK = 4, bool QUOTIENT = true>
 __device__ __forceinline__ void wino_store_tile(const ConvParams &p, floatx16 (&y)[2][2], const float *epi, int m0, int m_local, int n_base,
                                                 int lane) {
     const int n = n_base + (lane & 31);
@@ -795,7 +805,7 @@ __device__ __forceinline__ void wino_store_tile(const ConvParams &p, floatx16 (&
                     for (int a = 0; a < 2; a++)
 #pragma unroll
                         for (int b = 0; b < 2; b++) x[k][a][b] = y[a][b][v0 + k];
-                wino_store_rows<BM, NK>(p, epi, ml, m0 + ml, img, ty, tx, plane, x);
+                wino_store_rows<BM, NK, QUOTIENT>(p, epi, ml, m0 + ml, img, ty, tx, plane, x);
             } else {
 #pragma unroll
                 for (int k = 0; k < NK; k++) {
@@ -1190,7 +1200,7 @@ __device__ __forceinline__ void conv_tap_body(const ConvParams &p) {
         float *epi = &As[0][0];
         put_channel_constants<BM>(epi, chan, tid);
         __syncthreads();
-        wino_store_tile<BM>(p, wy, epi, m0, wm * 32, (int)n0 + wn * 32, lane);
+        wino_store_tile<BM, 4, false>(p, wy, epi, m0, wm * 32, (int)n0 + wn * 32, lane);
     } else if constexpr (UP2) {
         // (launched with whole tiles only; a lane holds the four outputs of a block like the Winograd forms)
         float *epi = &As[0][0];
@@ -2254,7 +2264,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
                 }
             } else if (n < p.wT) {
                 if (pair && 2 * ty + 1 < p.wP && 2 * tx + 1 < p.wQ && m0 + ml0 + 3 < p.Kf) {
-                    wino_store_rows<MF, 4>(p, epi, ml0, m0 + ml0, img, ty, tx, plane, yk);
+                    wino_store_rows<MF, 4, FM == 1>(p, epi, ml0, m0 + ml0, img, ty, tx, plane, yk);
                 } else {
 #pragma unroll
                     for (int k = 0; k < 4; k++)

@@ -43,6 +43,8 @@ int release_workspace(int dev);
 // change is repacked before its next use and one that is freed is forgotten.
 void conv_filters_written(int dev, const void *dst, size_t bytes);
 void conv_filters_released(int dev, const void *base, size_t bytes);
+// A product of a dense layer in the split form of a convolution (conv.hip), if it is one for it.
+int dense_split(int dev, const float *A, const float *B, float *C, int m, int k, int n, int incC, const float *bias, int relu, bool *taken);
 // Per-device set-up of the convolution code (address of its fixed scratch array, kernel occupancies);
 // use_device calls it once, when it initialises the device.
 int conv_setup_device(int dev);

@@ -104,6 +104,7 @@ struct ConvParams {
     const float *bias, *bn_g, *bn_b, *bn_mean, *bn_var, *residual;
     float bn_eps;
     int relu;
+    int residual_row;  // the residual is one plane for all filters (a dense layer's bias, see dense_split)
     // The output is written with the streaming (non-temporal) hint: set by the host for a layer that is bound by its
     // output traffic and whose output is larger than the last-level cache, so that keeping it there helps no reader.
     int stream_out;
@@ -227,7 +228,7 @@ __device__ __forceinline__ float finish_value(const ConvParams &p, const Channel
     return v;
 }
 __device__ __forceinline__ float apply_epilogue(const ConvParams &p, const ChannelEpilogue &e, float v, size_t oidx) {
-    return finish_value(p, e, v, p.residual ? p.residual[oidx] : 0.0f);
+    return finish_value(p, e, v, p.residual ? p.residual[p.residual_row ? oidx % (size_t)p.PQ : oidx] : 0.0f);
 }
 
 // LDS-direct load: the load unit writes the dword of lane i to LDS address dst + 4*i (out-of-range
@@ -367,7 +368,7 @@ __device__ __forceinline__ void store_tile_inside(const ConvParams &p, floatx16 
         const unsigned pq = n - img * (unsigned)p.PQ;
         const size_t idx = ((size_t)img * p.Kf + (size_t)(m0 + m_local + 4 * half)) * plane + pq;
         optr[tn] = p.O + idx;
-        rptr[tn] = p.residual + idx;  // not dereferenced without a residual
+        rptr[tn] = p.residual + (p.residual_row ? (size_t)pq : idx);  // not dereferenced without a residual
     }
     const bool has_bias = p.bias != nullptr, has_bn = p.bn_mean != nullptr, affine = p.bn_g != nullptr;
     constexpr bool has_res = HAS_RES;
@@ -378,12 +379,13 @@ __device__ __forceinline__ void store_tile_inside(const ConvParams &p, floatx16 
         for (int q4 = 0; q4 < 4; q4++) {  // rows 8*q4 + 4*half + 0..3 of the block: v = 4*q4 + j
             const int row0 = m_local + tm * 32 + 8 * q4 + 4 * half;
             const size_t roff = (size_t)(tm * 32 + 8 * q4) * plane;
+            const size_t rplane = p.residual_row ? 0 : plane, rroff = p.residual_row ? 0 : roff;
             float res[4][TN];
             if constexpr (has_res) {
 #pragma unroll
                 for (int j = 0; j < 4; j++)
 #pragma unroll
-                    for (int tn = 0; tn < TN; tn++) res[j][tn] = rptr[tn][roff + (size_t)j * plane];
+                    for (int tn = 0; tn < TN; tn++) res[j][tn] = rptr[tn][rroff + (size_t)j * rplane];
             }
             float x[4][TN];
 #pragma unroll
@@ -512,7 +514,7 @@ __device__ __forceinline__ void store_tile_edge(const ConvParams &p, floatx16 (&
 #pragma unroll
                     for (int tn = 0; tn < TN; tn++) {
                         const size_t oidx = (mok && nok[tn]) ? obase[tn] + (size_t)(m0 + ml) * p.PQ : 0;
-                        res[vv][tn] = p.residual[oidx];
+                        res[vv][tn] = p.residual[p.residual_row ? oidx % (size_t)p.PQ : oidx];
                     }
                 }
             }
@@ -733,7 +735,7 @@ __device__ __forceinline__ void wino_store_rows(const ConvParams &p, const float
 #pragma unroll
                 for (int a = 0; a < 2; a++)
 #pragma unroll
-                    for (int b = 0; b < 2; b++) x[k][a][b] = quotient(x[k][a][b], sd[k], r[k], rl[k]);
+                    for (int b = 0; b < 2; b++) x[k][a][b] = __fdiv_rn(__fsub_rn(x[k][a][b], mean[k]), sd[k]);
         }
         if (p.bn_g) {
             const vec_t g = *reinterpret_cast<const vec_t *>(epi + 3 * BM + ml), bb = *reinterpret_cast<const vec_t *>(epi + 4 * BM + ml);
@@ -3425,7 +3427,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     p.uh = uh; p.uw = uw;
     p.K = K; p.O = O; p.Wp = nullptr;
     p.bias = bias; p.bn_g = bn_g; p.bn_b = bn_b; p.bn_mean = bn_mean; p.bn_var = bn_var; p.residual = residual;
-    p.bn_eps = bn_eps; p.relu = relu;
+    p.bn_eps = bn_eps; p.relu = relu; p.residual_row = 0;
     {
         // bound by its output traffic (arithmetic intensity under the ridge of 157.3 TFLOP/s over 8 TB/s) and an output that
         // the 256 MB last-level cache cannot hold for the next layer anyway
@@ -4304,6 +4306,41 @@ int conv2d_wave_split(bool no_alloc, const WaveSplitVariant &v, int slices, int 
 }
 
 }  // namespace
+
+namespace eddlhip {
+
+// C[m][n] (+)= A[m][k] B[k][n] (+ bias per column) (then ReLU) as the 1x1 convolution that it is in the split form: B an image of k channels
+// and n pixels, the rows of A its filters.  Sets *taken if the product is one that this is made for (dense.hip says which); false
+// leaves everything as it is.
+int dense_split(int dev, const float *A, const float *B, float *C, int m, int k, int n, int incC, const float *bias, int relu, bool *taken) {
+    *taken = false;
+    if (g_algo != 0 || g_wino_never || (incC && bias) || !split_applies(k, m, 1, 1) || (long long)k * n > (1LL << 28) || n > 0x7ffffe00) return 0;
+    *taken = true;
+    ConvParams p;
+    memset(&p, 0, sizeof(p));
+    p.I = p.I2 = B;
+    p.Csplit = p.Cimg = p.C = k;
+    p.uh = p.uw = 1;
+    p.K = A;
+    p.O = C;
+    p.residual = incC ? C : bias;
+    p.residual_row = incC ? 0 : 1;
+    p.relu = relu;
+    p.N = 1, p.H = 1, p.W = n, p.Kf = m, p.R = p.S = p.sr = p.sc = 1, p.P = 1, p.Q = n;
+    p.CRS = k, p.PQ = n, p.npix = n;
+    p.Mp = (m + M_ALIGN - 1) / M_ALIGN * M_ALIGN;
+    // 64x64 tiles up to 64 rows, 128x64 above; where the weights fill the last-level cache 64x128 ones, whose wavefronts ask for more at a time.  One or
+    // two workgroups on a CU, each with four steps of 32 channels at least.
+    const bool large = (long long)k * n > 1LL << 26;
+    const int tile = m > 64 ? 1 : large ? 2 : 3, fill = m > 64 && !large ? 1 : 2, num_cu = state(dev).num_cu, steps = split_steps(k, 1);
+    const long long tiles = (long long)((m + ksplit[tile].bm - 1) / ksplit[tile].bm) * ((n + ksplit[tile].bn - 1) / ksplit[tile].bn);
+    long long slices = (fill * num_cu + tiles - 1) / tiles;
+    slices = std::max(1LL, std::min(std::min(slices, 16LL), (long long)steps / 4));
+    bool no_room = false;
+    return conv2d_split(false, ksplits[ONE_TAP][tile], forced_plan(ksplit, tile, (int)slices, m, k, 1, n, num_cu), dev, p, 1, &no_room);
+}
+
+}  // namespace eddlhip
 
 extern "C" {
 

@@ -9,7 +9,7 @@
 // (accumulator j holds columns 4l + j).  Except for one row, or few with not too many weights (reads_rows), the
 // activations are transposed first (At[k][32], a few MB, L2-resident) so that their loads are coalesced too.  k is split over wavefronts so the
 // whole device streams B; the per-slice partial blocks go to the private workspace and a second
-// kernel adds them in slice order (fixed summation order, no atomics).
+// kernel adds them in slice order (fixed summation order, no atomics).  More rows than 48 take the split form (split_rows).
 #include <algorithm>
 
 #include "common.h"
@@ -180,6 +180,13 @@ namespace {
 // against 41.4, 32 58.9 against 47.5).
 bool reads_rows(int m, int k, int n) { return m == 1 || (m <= 32 && (size_t)k * n <= (size_t)(m <= 16 ? 28 : 20) << 20); }
 
+// Many rows are bound by the fp32 matrix instruction as much as by the weights, and take the split form of a convolution (dense_split) where that
+// can run it: whole groups of 16 inputs.  us, before -> after: 64 rows 25088 x 4096 159 -> 116, 4096 x 4096 39.3 -> 28.8, 4096 x 1000 26.4
+// -> 18.2; 128 rows 297 -> 171, 63.6 -> 37.2, 37.1 -> 21.6, 512 x 4096 38.5 -> 17.9; error against 64 bits 3.7e-7 -> 2.4e-7 ... 3.3e-7, 1.8e-7 ->
+// 1.0e-7, 1.6e-7 -> 9.7e-8.  33 to 48 rows would gain as much (48 rows 37.7 -> 28.7), but a few rows have the bits that they have
+// among 33, which this would end; up to 32 the weights are streamed no faster by it (25088 x 4096 110 against 112).
+bool split_rows(int m) { return m > 48; }
+
 int dense_impl(int dev, const float *A, const float *B, float *C, int m, int k, int n, int incC, const float *bias, int relu,
                const char *what) {
     EH_REQUIRE(m >= 0 && k > 0 && n > 0, "%s: bad shape %dx%d * %dx%d", what, m, k, k, n);
@@ -187,6 +194,11 @@ int dense_impl(int dev, const float *A, const float *B, float *C, int m, int k, 
     EH_REQUIRE(A && B && C, "%s: NULL tensor", what);
     EH_TRY(use_device(dev));
     hipStream_t st = state(dev).stream;
+    if (split_rows(m)) {
+        bool taken = false;
+        EH_TRY(dense_split(dev, A, B, C, m, k, n, incC, bias, relu, &taken));
+        if (taken) return 0;
+    }
     const int nt = (n + 127) / 128, mt = (m + 31) / 32;
     // Wavefronts to cover the device eight times over, in slices of at least 128 taps (shorter
     // slices cost more in partial blocks written and read back than they gain) - unless that

@@ -468,7 +468,8 @@ int eddlhip_sum2d_rowwise(int dev, const float *A, const float *B, float *C, int
 /* LDense::forward in one call: C[m,n] = A[m,k] * W[k,n], then + bias[column] when bias != NULL
  * (sum2D_rowwise), then ReLU when relu != 0 (the LActivation that commonly follows; 
  * src/hardware/cpu/nn/cpu_activations.cpp:18-33).  Each step is the separate call's fp32 operation,
- * so the result equals eddlhip_mult2d + eddlhip_sum2d_rowwise + eddlhip_relu bit for bit. */
+ * so the result equals eddlhip_mult2d + eddlhip_sum2d_rowwise + eddlhip_relu bit for bit.  Both run products of more than 48 rows and a
+ * multiple of 16 inputs in the split form of the convolutions (not under eddlhip_conv2d_set_algo(1 .. 4) or (9)). */
 int eddlhip_dense_fwd(int dev, const float *A, const float *W, const float *bias, float *C, int m, int k, int n, int relu);
 
 #ifdef __cplusplus

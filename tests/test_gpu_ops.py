@@ -2092,3 +2092,44 @@ def test_conv2d_split_filters_of_many_weights(hip, R, S):
     finally:
         hip.force_conv_plan(-1, 1)
     assert np.array_equal(O.numpy()[:, Kf - few:], F.numpy())
+
+
+@pytest.mark.parametrize("m,k,n", [(49, 16, 1), (49, 512, 131), (64, 4096, 64), (65, 2048, 1000), (128, 1040, 36), (130, 96, 4097), (52, 25088, 2700)])
+def test_dense_of_many_rows_is_no_further_from_64_bits_than_the_fp32_product(hip, m, k, n):
+    """... and the fused call equals the separate launches, with and without what C holds; infinities and NaN as the fp32 product has them."""
+    rng = np.random.default_rng(2800 + m)
+    a, w, bias = rng.standard_normal((m, k), dtype=np.float32), (rng.standard_normal((k, n)) / np.sqrt(k)).astype(np.float32), rng.standard_normal(n).astype(np.float32)
+    A, Wd, b = hip.array(a), hip.array(w), hip.array(bias)
+    C, F, G = (hip.full((m, n), np.nan) for _ in range(3))
+
+    def fp32(A, out, inc=0):
+        hip.set_conv_algo("winograd_never")
+        try:
+            hip.mult2D(A, Wd, out, inc)
+        finally:
+            hip.set_conv_algo("winograd_off")
+        return out.numpy()
+    direct = fp32(A, G)
+    hip.mult2D(A, Wd, C, 0)
+    got = C.numpy()
+    ref = a.astype(np.float64) @ w.astype(np.float64)
+    assert not np.array_equal(got, direct) or k == 16
+    # (2^-23: a sum of one group of 16 is rounded twice or three times in either form)
+    assert np.linalg.norm(got - ref) <= max(np.linalg.norm(direct - ref), 2.0 ** -23 * np.linalg.norm(ref))
+    assert_conv_close(ref, got, "%dx%dx%d" % (m, k, n))
+    hip.sum2D_rowwise(C, b, C)
+    hip.dense(A, Wd, b, F)
+    assert np.array_equal(C.numpy(), F.numpy())
+    hip.relu(C, C)
+    hip.dense(A, Wd, b, F, relu=True)
+    assert np.array_equal(C.numpy(), F.numpy())
+    before = F.numpy()
+    hip.mult2D(A, Wd, F, 1)
+    assert np.array_equal(F.numpy(), before + got)
+    a[3, k // 2], a[m - 1, 0] = np.inf, np.nan
+    A.copy_from(a)
+    hip.mult2D(A, Wd, C, 0)
+    x, y = C.numpy(), fp32(A, G)
+    assert np.array_equal(np.isnan(x), np.isnan(y)) and np.array_equal(x[3], y[3], equal_nan=True)
+    rest = [r for r in range(m) if r not in (3, m - 1)]
+    assert np.array_equal(x[rest], got[rest])

@@ -2641,7 +2641,7 @@ Plan forced_plan(const Variant *family, int tile, int slices, int Kf, int C, int
 // Time of a workgroup step: `alone` with one workgroup on a CU, at least `shared` for every one that is there; of a workgroup around its
 // steps: `fixed` and `each` for every one there.  Fitted to 6200 timed plans of 281 convolutions (1 - 64 images, 7 - 368 pixels, 16 - 1024
 // channels, filters of 1 - 7, this library's networks among them), rms error 17-20 %; by its choices the 156 of them that have whole groups of
-// 16 channels take 1 / 1.43 of the direct kernels' time together (the best plan of each:
+// 16 channels take 1 / 1.40 of the direct kernels' time together (the best plan of each:
 // 1 / 1.5) and none takes more than 1.02 of it.  Below 7 us of direct kernel nothing is to be gained by this model, and the direct kernel stays.
 struct SplitChoice {
     int tile, slices;
@@ -2659,7 +2659,9 @@ SplitChoice plan_split(int Kf, int C, int RS, int Mp, long long npix, int num_cu
     static const int kSlices[6] = {1, 2, 3, 4, 6, 8};
     SplitChoice best = {-1, 1, direct_us > traffic_us ? direct_us : traffic_us};
     if (best.cost_us < 7.0 || C % 16 != 0) return best;
-    if (direct_us > traffic_us) best.cost_us = 0.9 * direct_us > traffic_us ? 0.9 * direct_us : traffic_us;  // (a tenth for the model's error)
+    // a tenth for the model's error, a quarter where launches weigh as much as work (one of 11 us was chosen one of 13)
+    const double least = (direct_us < 15.0 ? 0.75 : 0.9) * direct_us;
+    if (direct_us > traffic_us) best.cost_us = least > traffic_us ? least : traffic_us;
     const size_t filters = (split_filter_bytes(C, RS, Mp) + 255) & ~(size_t)255;
     auto offer = [&](int tile, int slices, size_t partial, double us) {
         us = us > traffic_us ? us : traffic_us;
@@ -3253,7 +3255,8 @@ int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, l
         }
         if (rc != 0) fatal = rc;
     }
-    time_plan(0, -1, -1);
+    // (a choice of the split form is also among that form's tiles below and has no preference of its own: 3 % of every layer are too much for it)
+    time_plan(planned.tile >= 0 ? 0 : 30, -1, -1);
     if (fatal == 0 && cands.empty()) fatal = set_error(EDDLHIP_EINVAL, "conv2d plan search: the planner's own plan did not run");
     if (up_ok) {  // (2x2 filters only: no rank shared with the one-launch Winograd form of 3x3 filters)
         time_plan(1, UP2X2_TILE, 1);
@@ -3299,7 +3302,10 @@ int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, l
                 time_plan(5 + v, SPLIT_TILE0 + v, sl);
             }
         }
-    if (wave_ok)  // the split form for few tiles: up to four workgroups per CU
+    // the split form for few tiles: up to four workgroups per CU.  Large filters for more than two tiles of pixels are left to the other forms: the
+    // launches timed here find them in L2, where a network's come from memory and every tile of pixels waits for them again (VGG-16, one image,
+    // 445 -> 451 us with its 7 and 14 MB filters in this form, though the launches take 14 us for 20 here)
+    if (wave_ok && (chunk_pix <= 64 || split_filter_bytes(c.C, c.R * c.S, (c.Kf + M_ALIGN - 1) / M_ALIGN * M_ALIGN) <= ((size_t)4 << 20)))
         for (int v = 0; v < NUM_WAVE; v++) {
             const long long tiles = wave_tiles(kwave[v], c.Kf, chunk_pix);
             int last_slices = 0;

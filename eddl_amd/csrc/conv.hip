@@ -2508,6 +2508,12 @@ bool split_applies(int C, int Kf, int R, int S) {
 
 bool wave_applies(int C, int Kf, int R, int S) { return split_filter_bytes(C, R * S, (Kf + M_ALIGN - 1) / M_ALIGN * M_ALIGN) < ((size_t)1 << 31); }
 long long wave_tiles(const WaveSplitVariant &v, int Kf, long long npix) { return (long long)((Kf + 32 * v.tm - 1) / (32 * v.tm)) * ((npix + 32 * v.tn - 1) / (32 * v.tn)); }
+// Every tile of 32 pixels reads all filters.  A launch repeated by itself finds them in L2, a network's come from memory and are waited for by
+// every tile again, so neither the search nor the planner offers this form from 64 MB of such reads on (VGG-16, one image, 442 -> 457 us with its
+// 2 ... 14 MB filters in this form for 98 ... 7 tiles, though by itself the last takes 14 us for 20).
+bool wave_filters_fit(int C, int Kf, int RS, long long npix) {
+    return (double)split_filter_bytes(C, RS, (Kf + M_ALIGN - 1) / M_ALIGN * M_ALIGN) * (double)((npix + 31) / 32) <= 64e6;
+}
 // K slices of a plan that asks for `slices`: no more than there are units of 16 channels under one tap for eight wavefronts each
 int wave_slices(const WaveSplitVariant &v, int slices, int Kf, int C, int RS, long long npix) {
     const long long units = (long long)((C + 15) / 16) * RS, most = (units + WAVE_SPLIT_WAVES - 1) / WAVE_SPLIT_WAVES;
@@ -2693,7 +2699,7 @@ SplitChoice plan_split(int Kf, int C, int RS, int Mp, long long npix, int num_cu
             offer(SPLIT_TILE0 + t, fp.nslices, partial, us);
         }
     }
-    for (int t = 0; t < NUM_WAVE; t++) {
+    for (int t = 0; t < NUM_WAVE && wave_filters_fit(C, Kf, RS, npix); t++) {
         const auto &k = kWave[t];
         const long long units = (long long)(C / 16) * RS;
         int last = 0;
@@ -3302,10 +3308,7 @@ int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, l
                 time_plan(5 + v, SPLIT_TILE0 + v, sl);
             }
         }
-    // the split form for few tiles: up to four workgroups per CU.  Large filters for more than two tiles of pixels are left to the other forms: the
-    // launches timed here find them in L2, where a network's come from memory and every tile of pixels waits for them again (VGG-16, one image,
-    // 445 -> 451 us with its 7 and 14 MB filters in this form, though the launches take 14 us for 20 here)
-    if (wave_ok && (chunk_pix <= 64 || split_filter_bytes(c.C, c.R * c.S, (c.Kf + M_ALIGN - 1) / M_ALIGN * M_ALIGN) <= ((size_t)4 << 20)))
+    if (wave_ok && wave_filters_fit(c.C, c.Kf, c.R * c.S, chunk_pix))  // the split form for few tiles: up to four workgroups per CU
         for (int v = 0; v < NUM_WAVE; v++) {
             const long long tiles = wave_tiles(kwave[v], c.Kf, chunk_pix);
             int last_slices = 0;

@@ -2029,7 +2029,7 @@ PLANNER_CASES = {
     "1x1": ((8, 256, 28, 28, 256, 1, 1, (1, 1), (0, 0)), True),
     "3x3": ((2, 128, 28, 30, 128, 3, 3, (1, 1), (1, 1)), True),
     "3x3 stride 2": ((9, 256, 57, 41, 128, 3, 3, (2, 2), (1, 1)), True),
-    "5x5": ((3, 48, 33, 35, 72, 5, 5, (1, 1), (2, 2)), True),
+    "5x5": ((12, 64, 33, 35, 128, 5, 5, (1, 1), (2, 2)), True),
     "many pixels": ((16, 64, 56, 56, 128, 3, 3, (1, 1), (1, 1)), True),
     "long K": ((1, 1024, 14, 14, 200, 1, 1, (1, 1), (0, 0)), True),
     "40 channels": ((2, 40, 56, 56, 128, 3, 3, (1, 1), (1, 1)), False),

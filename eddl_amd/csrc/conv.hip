@@ -4324,6 +4324,10 @@ namespace eddlhip {
 int dense_split(int dev, const float *A, const float *B, float *C, int m, int k, int n, int incC, const float *bias, int relu, bool *taken) {
     *taken = false;
     if (g_algo != 0 || g_wino_never || (incC && bias) || !split_applies(k, m, 1, 1) || (long long)k * n > (1LL << 28) || n > 0x7ffffe00) return 0;
+    // (a tile is written while others still read the weights, and the rows where the sums are not finite; dense.hip's own kernels write the
+    // output in a launch behind the one that reads, so an output on an operand is theirs)
+    auto on_output = [&](const float *operand, size_t floats) { return operand < C + (size_t)m * n && C < operand + floats; };
+    if (on_output(A, (size_t)m * k) || on_output(B, (size_t)k * n)) return 0;
     *taken = true;
     ConvParams p;
     memset(&p, 0, sizeof(p));

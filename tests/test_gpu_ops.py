@@ -2133,3 +2133,27 @@ def test_dense_of_many_rows_is_no_further_from_64_bits_than_the_fp32_product(hip
     assert np.array_equal(np.isnan(x), np.isnan(y)) and np.array_equal(x[3], y[3], equal_nan=True)
     rest = [r for r in range(m) if r not in (3, m - 1)]
     assert np.array_equal(x[rest], got[rest])
+
+
+@pytest.mark.parametrize("m,k,n,onto", [(256, 256, 16384, "B"), (4096, 1024, 1024, "A"), (192, 512, 512, "A"), (192, 192, 512, "B")])
+def test_dense_of_many_rows_onto_an_operand(hip, m, k, n, onto):
+    """An output that lies on the rows, or on the weights, comes out as one of its own does: no launch writes it while another part of
+    the product is still to be read (infinities among the rows, which the split form reads again, included)."""
+    rng = np.random.default_rng(2860 + m)
+    a, w = rng.standard_normal((m, k), dtype=np.float32), (rng.standard_normal((k, n)) / np.sqrt(k)).astype(np.float32)
+    a[::67, 5] = np.inf
+    A, W, C = hip.array(a), hip.array(w), hip.full((m, n), np.nan)
+    hip.set_conv_algo("winograd_never")
+    try:
+        hip.mult2D(A, W, C)
+    finally:
+        hip.set_conv_algo("winograd_off")
+    out = A if onto == "A" else W
+    hip._check(hip.lib.eddlhip_mult2d(hip.dev, A.ptr, W.ptr, out.ptr, m, k, n, 0))
+    assert np.array_equal(out.numpy().reshape(m, n), C.numpy(), equal_nan=True)
+    # ... and on a part of it: the last rows of the output, in front of the operand
+    both = hip.array(np.concatenate([np.zeros((m - 1) * n, np.float32), (a if onto == "A" else w).ravel()]))
+    operand = both.ptr + 4 * (m - 1) * n
+    A.copy_from(a), W.copy_from(w)
+    hip._check(hip.lib.eddlhip_mult2d(hip.dev, operand if onto == "A" else A.ptr, operand if onto == "B" else W.ptr, both.ptr, m, k, n, 0))
+    assert np.array_equal(both.numpy()[:m * n].reshape(m, n), C.numpy(), equal_nan=True)

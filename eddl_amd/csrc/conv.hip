@@ -3123,7 +3123,9 @@ int conv2d_winograd_fused(bool no_alloc, bool *no_room, const FusedVariant &fv, 
 int conv2d_up2x2(int tile, int slices, int dev, const float *I, const float *K, const float *bias, float *O, int N, int C, int H, int W, int Kf, int P, int Q, const float *bn_g,
                  const float *bn_b, const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu);
 
-int conv2d_split(bool no_alloc, const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room);
+// Whose call a launch of the split form is: a convolution's, the same from the fixed scratch array, a dense layer's
+enum class SplitCall { CONV, CONV_NO_ALLOC, PRODUCT };
+int conv2d_split(SplitCall use, const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room);
 int conv2d_wave_split(bool no_alloc, const WaveSplitVariant &v, int slices, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room);
 
 // Whether a convolution is the one conv_up2x2_kernel computes: a 2x2 stride-1 filter on ONE tensor upsampled twice in both
@@ -3539,9 +3541,10 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     // the split form: any filter shape, as long as a chunk of the input is addressed like the direct kernels do; from the fixed
     // scratch array where its filters (half as much again as the repacked ones) and partial tiles fit, else the planner's plan
     const bool split_ok = !gemm && g_algo == 0 && !g_wino_never && split_applies(C, Kf, R, S);
+    const SplitCall split_use = no_alloc ? SplitCall::CONV_NO_ALLOC : SplitCall::CONV;
     if (split_ok && is_split_tile(g_force_tile)) {
         const int tile = g_force_tile - SPLIT_TILE0;
-        const int rc = conv2d_split(no_alloc, split_build(tile, R * S, uh, uw), forced_plan(ksplit, tile, g_force_slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p,
+        const int rc = conv2d_split(split_use, split_build(tile, R * S, uh, uw), forced_plan(ksplit, tile, g_force_slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p,
                                     chunk_imgs, &no_room);
         if (!no_room) return rc;
     }
@@ -3617,7 +3620,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
         }
         if (found != nullptr && is_split_tile(found->tile) && split_ok) {
             const int tile = found->tile - SPLIT_TILE0;
-            const int rc = conv2d_split(no_alloc, split_build(tile, R * S, uh, uw), forced_plan(ksplit, tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev,
+            const int rc = conv2d_split(split_use, split_build(tile, R * S, uh, uw), forced_plan(ksplit, tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev,
                                         p, chunk_imgs, &no_room);
             if (!no_room) return rc;
         }
@@ -3636,7 +3639,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
         no_room = false;
         const int rc = is_wave_tile(choice.tile)
                            ? conv2d_wave_split(no_alloc, kwave[choice.tile - WAVE_TILE0], choice.slices, dev, p, chunk_imgs, &no_room)
-                           : conv2d_split(no_alloc, split_build(choice.tile - SPLIT_TILE0, R * S, uh, uw),
+                           : conv2d_split(split_use, split_build(choice.tile - SPLIT_TILE0, R * S, uh, uw),
                                           forced_plan(ksplit, choice.tile - SPLIT_TILE0, choice.slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p, chunk_imgs,
                                           &no_room);
         if (!no_room) return rc;
@@ -4178,17 +4181,18 @@ int kept_split_filters(bool no_alloc, int dev, const ConvParams &call, size_t w_
 }
 
 // The split form (conv_split.h) of the call that `call` describes, under a plan of split steps.
-// Workspace: [split filters unless kept][partial tiles].  no_alloc: from the fixed scratch array; nothing is launched and *no_room
-// is set if that is too small.
-int conv2d_split(bool no_alloc, const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room) {
+// Workspace: [split filters unless kept][partial tiles].  CONV_NO_ALLOC: from the fixed scratch array; nothing is launched and *no_room
+// is set if that is too small.  PRODUCT: the rows that stand for filters are no registered tensor's, wherever they lie.
+int conv2d_split(SplitCall use, const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room) {
     hipStream_t st = state(dev).stream;
+    const bool no_alloc = use == SplitCall::CONV_NO_ALLOC;
     const int RS = call.R * call.S, N = call.N;
     EH_REQUIRE(plan.tiles <= 0x3fffffffLL, "conv2d: too many tiles");
     const long long leftover = plan.nslices > 1 ? plan.leftover : 0;
     const size_t w_bytes = split_filter_bytes(call.C, RS, call.Mp);
     const size_t partial_bytes = (size_t)plan.nslices * leftover * v.bm * v.bn * sizeof(float);
     const void *Ws = nullptr;
-    EH_TRY(kept_split_filters(no_alloc, dev, call, w_bytes, &Ws));
+    if (use != SplitCall::PRODUCT) EH_TRY(kept_split_filters(no_alloc, dev, call, w_bytes, &Ws));
     const size_t ws_filters = Ws ? 0 : ((w_bytes + 255) & ~(size_t)255);
     void *ws = nullptr;
     if (no_alloc) {
@@ -4350,7 +4354,7 @@ int dense_split(int dev, const float *A, const float *B, float *C, int m, int k,
     long long slices = (fill * num_cu + tiles - 1) / tiles;
     slices = std::max(1LL, std::min(std::min(slices, 16LL), (long long)steps / 4));
     bool no_room = false;
-    return conv2d_split(false, ksplits[ONE_TAP][tile], forced_plan(ksplit, tile, (int)slices, m, k, 1, n, num_cu), dev, p, 1, &no_room);
+    return conv2d_split(SplitCall::PRODUCT, ksplits[ONE_TAP][tile], forced_plan(ksplit, tile, (int)slices, m, k, 1, n, num_cu), dev, p, 1, &no_room);
 }
 
 }  // namespace eddlhip

@@ -2157,3 +2157,21 @@ def test_dense_of_many_rows_onto_an_operand(hip, m, k, n, onto):
     A.copy_from(a), W.copy_from(w)
     hip._check(hip.lib.eddlhip_mult2d(hip.dev, operand if onto == "A" else A.ptr, operand if onto == "B" else W.ptr, both.ptr, m, k, n, 0))
     assert np.array_equal(both.numpy()[:m * n].reshape(m, n), C.numpy(), equal_nan=True)
+
+
+def test_dense_rows_that_are_a_registered_filter_tensor(hip):
+    """A product reads its rows where they are, also where a copy of them is registered as the filters of a 1x1 convolution and a kernel has
+    written them since (the copy is the convolution's)."""
+    rng = np.random.default_rng(2870)
+    m, k, n = 64, 256, 512
+    A, W = hip.array(rng.standard_normal((m, k, 1, 1), dtype=np.float32)), hip.array(rng.standard_normal((k, n), dtype=np.float32))
+    C, D = hip.full((m, n), np.nan), hip.full((m, n), np.nan)
+    hip.cache_conv_filters(A)
+    try:
+        hip.mult2D(A.reshape((m, k)), W, C)
+        hip.relu(A, A)
+        hip.mult2D(A.reshape((m, k)), W, C)
+    finally:
+        hip.uncache_conv_filters(A)
+    hip.mult2D(A.reshape((m, k)), W, D)
+    assert np.array_equal(C.numpy(), D.numpy())

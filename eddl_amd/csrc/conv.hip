@@ -4182,17 +4182,18 @@ int kept_split_filters(bool no_alloc, int dev, const ConvParams &call, size_t w_
 
 // The split form (conv_split.h) of the call that `call` describes, under a plan of split steps.
 // Workspace: [split filters unless kept][partial tiles].  CONV_NO_ALLOC: from the fixed scratch array; nothing is launched and *no_room
-// is set if that is too small.  PRODUCT: the rows that stand for filters are no registered tensor's, wherever they lie.
+// is set if that is too small.  PRODUCT: the rows that stand for filters are no registered tensor's, wherever they lie, and the launch is
+// none that the convolutions' measuring hooks see (so it is also recorded while they collect).
 int conv2d_split(SplitCall use, const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room) {
     hipStream_t st = state(dev).stream;
-    const bool no_alloc = use == SplitCall::CONV_NO_ALLOC;
+    const bool no_alloc = use == SplitCall::CONV_NO_ALLOC, product = use == SplitCall::PRODUCT;
     const int RS = call.R * call.S, N = call.N;
     EH_REQUIRE(plan.tiles <= 0x3fffffffLL, "conv2d: too many tiles");
     const long long leftover = plan.nslices > 1 ? plan.leftover : 0;
     const size_t w_bytes = split_filter_bytes(call.C, RS, call.Mp);
     const size_t partial_bytes = (size_t)plan.nslices * leftover * v.bm * v.bn * sizeof(float);
     const void *Ws = nullptr;
-    if (use != SplitCall::PRODUCT) EH_TRY(kept_split_filters(no_alloc, dev, call, w_bytes, &Ws));
+    if (!product) EH_TRY(kept_split_filters(no_alloc, dev, call, w_bytes, &Ws));
     const size_t ws_filters = Ws ? 0 : ((w_bytes + 255) & ~(size_t)255);
     void *ws = nullptr;
     if (no_alloc) {
@@ -4231,16 +4232,17 @@ int conv2d_split(SplitCall use, const Variant &v, const Plan &plan, int dev, con
         q.nslices = split_tiles > 0 ? plan.nslices : 1;
         q.slice_steps = split_tiles > 0 ? plan.slice_steps : plan.nsteps;
         const long long wgs = q.main_tiles + split_tiles * q.nslices;
-        q.trace = (g_trace != nullptr && wgs <= g_trace_wgs) ? g_trace : nullptr;
-        EH_TRY(prof_begin(st));
+        q.trace = (!product && g_trace != nullptr && wgs <= g_trace_wgs) ? g_trace : nullptr;
+        if (!product) EH_TRY(prof_begin(st));
         hipLaunchKernelGGL(v.kernel, dim3((unsigned)wgs), dim3(256), 0, st, q);
         EH_CHECK_LAUNCH();
-        EH_TRY(prof_end(st));
+        if (!product) EH_TRY(prof_end(st));
         if (split_tiles > 0) {
             hipLaunchKernelGGL(v.reduce, dim3((unsigned)(split_tiles * (v.bm / 32) * (v.bn / 32))), dim3(256), 0, st, q);
             EH_CHECK_LAUNCH();
         }
     }
+    if (product) return 0;
     if (leftover > 0) snprintf(g_last_kernel, sizeof(g_last_kernel), "%s +ksplit(%lld tiles x %d)", v.name, leftover, plan.nslices);
     else snprintf(g_last_kernel, sizeof(g_last_kernel), "%s", v.name);
     return 0;

@@ -2175,3 +2175,30 @@ def test_dense_rows_that_are_a_registered_filter_tensor(hip):
         hip.uncache_conv_filters(A)
     hip.mult2D(A.reshape((m, k)), W, D)
     assert np.array_equal(C.numpy(), D.numpy())
+
+
+def test_dense_of_many_rows_is_no_convolution_to_the_measuring_hooks(hip):
+    """The convolutions' collection counts no product, their timeline and their label keep what the last convolution left there, and a product
+    is recorded while a collection is on."""
+    rng = np.random.default_rng(2880)
+    X, K, O = hip.array(rng.standard_normal((2, 64, 20, 20), dtype=np.float32)), hip.array(rng.standard_normal((64, 64, 3, 3), dtype=np.float32)), hip.empty((2, 64, 18, 18))
+    A, W, C, D = (hip.array(rng.standard_normal(s, dtype=np.float32)) for s in ((64, 256), (256, 512), (64, 512), (64, 512)))
+    bias = hip.array(rng.standard_normal(512).astype(np.float32))
+    trace = hip.conv_trace(4096)
+    try:
+        hip.conv2D(X, K, None, O, 1, 1, 0, 0)
+        kernel, marks = hip.last_conv_kernel(), trace.numpy().view(np.uint32)
+        hip.conv_profile(True)
+        hip.mult2D(A, W, C)
+        hip.dense(A, W, bias, C)
+        graph = hip.record(lambda: hip.dense(A, W, bias, D))
+        assert hip.conv_profile_read()[0] == 0
+    finally:
+        hip.conv_profile(False)
+        after = trace.numpy().view(np.uint32)
+        hip.conv_trace(0)
+    assert hip.last_conv_kernel() == kernel and marks.any() and np.array_equal(marks, after)
+    for _ in range(3):
+        hip.fill_(D, np.nan)
+        graph.launch()
+        assert np.array_equal(D.numpy(), C.numpy())

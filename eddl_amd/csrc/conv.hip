@@ -3562,7 +3562,8 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
         if (chosen) return;
         chosen = true;
         if (gemm || !split_ok || g_split == 0 || (g_force_tile >= 0 && g_force_tile < 4)) return;
-        const double traffic_us = 4.0 * ((double)chunk_imgs * C * H * W + (double)chunk_imgs * Kf * p.PQ) / 5.0e6;
+        // (of the input that the window passes over, not of what is stored: a folded UpSampling or Pad layer is the same convolution)
+        const double traffic_us = 4.0 * (double)chunk_imgs * p.PQ * ((double)C * sr * sc + Kf) / 5.0e6;
         choice = plan_split(Kf, C, R * S, p.Mp, (long long)chunk_imgs * p.PQ, state(dev).num_cu, plan.cost_us, traffic_us);
     };
     const bool query = gemm != nullptr && gemm->need_out != nullptr;  // report the workspace need, launch nothing

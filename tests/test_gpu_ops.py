@@ -2076,6 +2076,31 @@ def test_conv2d_planner_chooses_the_split_form_by_the_geometry_alone(hip, case):
     assert_conv_close(ref, outs["plain"], case)
 
 
+# N C Kf and the enlarged side lengths: each has other slices by what the stored input moves than by what the enlarged one does
+@pytest.mark.parametrize("N,C,Kf,P,Q", [(2, 512, 64, 224, 224), (4, 320, 64, 224, 224), (11, 512, 64, 208, 44), (13, 656, 48, 56, 136)])
+def test_conv2d_planner_chooses_alike_for_folded_and_stored_inputs(hip, N, C, Kf, P, Q):
+    """A folded UpSampling, Concat and Pad: the plan and the bits of the stored tensor, without a plan search."""
+    X, W, big = hip.empty((N, C, P // 2, Q // 2)), hip.empty((Kf, C, 1, 1)), hip.empty((N, C, P, Q))
+    hip.rand_normal(X, 0.0, 1.0, 21)
+    hip.rand_normal(W, 0.0, C ** -0.5, 22)
+    hip.scale(X, big, [P, Q])
+    A, B = hip.full((N, Kf, P, Q), np.nan), hip.full((N, Kf, P, Q), np.nan)
+    hip.conv2D(big, W, None, A, 1, 1, 0, 0)
+    stored = hip.last_conv_kernel()
+    hip.conv2D(X, W, None, B, 1, 1, 0, 0, upsample=(2, 2))
+    assert hip.last_conv_kernel() == stored and np.array_equal(A.numpy(), B.numpy())
+    host = big.numpy()
+    hip.conv2D(hip.array(host[:, :C // 2]), W, None, B, 1, 1, 0, 0, second=hip.array(host[:, C // 2:]))
+    assert hip.last_conv_kernel() == stored and np.array_equal(A.numpy(), B.numpy())
+    padded = hip.empty((N, C, P + 2, Q + 2))
+    hip.pad(big, padded, [1, 1, 1, 1])
+    A, B = hip.full((N, Kf, P + 2, Q + 2), np.nan), hip.full((N, Kf, P + 2, Q + 2), np.nan)
+    hip.conv2D(padded, W, None, A, 1, 1, 0, 0)
+    stored = hip.last_conv_kernel()
+    hip.conv2D(big, W, None, B, 1, 1, 1, 1)
+    assert hip.last_conv_kernel() == stored and np.array_equal(A.numpy(), B.numpy())
+
+
 @pytest.mark.parametrize("R,S", [(1, 1), (2, 2), (3, 3), (1, 9), (5, 2)])
 def test_conv2d_split_filters_of_many_weights(hip, R, S):
     """From two million weights on the taps of a filter are split together: the bits of the weights split one by one (a slice of the filters)."""

@@ -2372,7 +2372,7 @@ long long g_trace_wgs = 0;
 // (kind + 2).
 struct TunedPlan {
     int key[10];       // N C Kf R S sr sc P Q kind (0 / 1: register-staged / LDS-direct gather; + 2: see above)
-    int tile, slices;  // tile -1: the planner's own choice was the fastest; tile 4: the Winograd form
+    int tile, slices;  // tile -1: the planner's plan of the direct kernels (a file's -1 is the same launch as when it was found); tile 4: the Winograd form
 };
 bool g_autotune = false;
 thread_local bool g_tuning = false;  // this thread is inside a plan search: the convolutions it times start no search of their own
@@ -3195,9 +3195,10 @@ size_t winograd_workspace(bool fold, int N, int C, int Kf, int fs, int P, int Q,
 // tensors (each plan writes the same output, up to the rounding of its summation order) in batches of about 0.3 ms of
 // launches, after the planner's plan has run for 25 ms (settled clocks), re-times the plans near the front in turns, and
 // takes each plan's FASTEST batch (noise only ever adds time).  Then, so that two searches of one geometry agree:
-// of all plans within 3 % of the fastest one it keeps the first in a fixed order of preference - the planner's own plan,
-// the one-launch Winograd form (or the upsampled-input form of a 2x2 filter), the split form, the direct tiles, the Winograd
-// forms with a transformed input in memory; within a form fewer K slices first.  Returns 0 with *out filled, 1 when these tensors cannot be searched on (the output overlaps an
+// of all plans within 3 % of the fastest one it keeps the first in a fixed order of preference - the planner's plan of the direct
+// kernels, the one-launch Winograd form (or the upsampled-input form of a 2x2 filter), the same in the split arithmetic, the split form,
+// the split form for few tiles, the direct tiles, the Winograd forms with a transformed input in memory; within a form fewer K slices
+// first.  (The planner's choice among the split form's tiles has no preference of its own: with one, ResNet-50 of 16 images lost 2 %.)  Returns 0 with *out filled, 1 when these tensors cannot be searched on (the output overlaps an
 // input: repeating the call would change what it reads), or minus the error code of a runtime failure.
 int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, long long chunk_pix, bool wino_ok, bool fold_ok, bool fused_ok, bool up_ok,
                 bool split_ok, bool wsplit_ok, bool upsplit_ok, bool wave_ok, TunedPlan *out) {
@@ -3263,8 +3264,7 @@ int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, l
         }
         if (rc != 0) fatal = rc;
     }
-    // (a choice of the split form is also among that form's tiles below and has no preference of its own: 3 % of every layer are too much for it)
-    time_plan(planned.tile >= 0 ? 0 : 30, -1, -1);
+    time_plan(0, -1, -1);
     if (fatal == 0 && cands.empty()) fatal = set_error(EDDLHIP_EINVAL, "conv2d plan search: the planner's own plan did not run");
     if (up_ok) {  // (2x2 filters only: no rank shared with the one-launch Winograd form of 3x3 filters)
         time_plan(1, UP2X2_TILE, 1);
@@ -3554,18 +3554,8 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
         const int rc = conv2d_wave_split(no_alloc, kwave[g_force_tile - WAVE_TILE0], g_force_slices, dev, p, chunk_imgs, &no_room);
         if (!no_room) return rc;
     }
-    // the planner's own choice: a tile of the split form where its model expects one to be faster (not under switches that ask for the
-    // fp32 instruction's sums, or for undivided tiles)
-    SplitChoice choice = {-1, 1, 0.0};
-    bool chosen = false;
-    auto choose = [&]() {
-        if (chosen) return;
-        chosen = true;
-        if (gemm || !split_ok || g_split == 0 || (g_force_tile >= 0 && g_force_tile < 4)) return;
-        // (of the input that the window passes over, not of what is stored: a folded UpSampling or Pad layer is the same convolution)
-        const double traffic_us = 4.0 * (double)chunk_imgs * p.PQ * ((double)C * sr * sc + Kf) / 5.0e6;
-        choice = plan_split(Kf, C, R * S, p.Mp, (long long)chunk_imgs * p.PQ, state(dev).num_cu, plan.cost_us, traffic_us);
-    };
+    // whether a plan names the direct kernels: forced, found, or the one that a search times as the planner's
+    bool direct_plan = g_tuning || (g_force_tile >= 0 && g_force_tile < 4);
     const bool query = gemm != nullptr && gemm->need_out != nullptr;  // report the workspace need, launch nothing
     bool plan_open = false;                                         // a search could still pick any plan for this geometry
     if (g_autotune && g_force_tile < 0 && g_algo == 0 && g_split != 0) {
@@ -3584,16 +3574,13 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
             memcpy(best.key, key, sizeof(key));
             const size_t ws_before = state(dev).workspace_bytes;
             FilterCopies keep = copies_held(dev, K, Kf, C, R, S);  // (those that other geometries' plans, and graphs, may use)
-            choose();
-            Plan planned = plan;
-            if (choice.tile >= 0) planned.tile = -1;  // (not one of the direct tiles)
-            const int src = search_plan(call, family, planned, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, split_ok, wsplit_ok, upsplit_ok, wave_ok, &best);
+            const int src = search_plan(call, family, plan, (long long)chunk_imgs * p.PQ, wino_ok, fold_ok, fused_ok, up_ok, split_ok, wsplit_ok, upsplit_ok, wave_ok, &best);
             if (src < 0) return -src;  // a runtime error inside the search
             if (src == 0) {
                 keep.wino = keep.wino || best.tile == 4 || best.tile == 5;
                 keep.fused = keep.fused || (best.tile >= FUSED_TILE0 && best.tile < FUSED_TILE0 + NUM_FUSED);
                 keep.up = keep.up || best.tile == UP2X2_TILE || best.tile == UP2X2_TILE + 1;
-                keep.split = keep.split || is_split_tile(best.tile) || is_wave_tile(best.tile) || (best.tile < 0 && choice.tile >= 0);
+                keep.split = keep.split || is_split_tile(best.tile) || is_wave_tile(best.tile);
                 keep.upsplit = keep.upsplit || is_upsplit_tile(best.tile);
                 keep.wsplit = keep.wsplit || is_wsplit_tile(best.tile);
             }
@@ -3629,13 +3616,19 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
             const int rc = conv2d_wave_split(no_alloc, kwave[found->tile - WAVE_TILE0], found->slices, dev, p, chunk_imgs, &no_room);
             if (!no_room) return rc;
         }
-        if (found != nullptr && found->tile >= 0 && found->tile < 4) {
-            plan = forced_plan(family, found->tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu);
-            choice.tile = -1;
-            chosen = true;
+        if (found != nullptr && found->tile < 4) {
+            if (found->tile >= 0) plan = forced_plan(family, found->tile, found->slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu);
+            direct_plan = true;
         }
     }
-    choose();
+    // the planner's own choice: a tile of the split form where its model expects one to be faster than the direct kernels (not under
+    // switches that ask for the fp32 instruction's sums, or for undivided tiles, and not where a plan names the direct kernels)
+    SplitChoice choice = {-1, 1, 0.0};
+    if (!gemm && split_ok && g_split != 0 && !direct_plan) {
+        // (of the input that the window passes over, not of what is stored: a folded UpSampling or Pad layer is the same convolution)
+        const double traffic_us = 4.0 * (double)chunk_imgs * p.PQ * ((double)C * sr * sc + Kf) / 5.0e6;
+        choice = plan_split(Kf, C, R * S, p.Mp, (long long)chunk_imgs * p.PQ, state(dev).num_cu, plan.cost_us, traffic_us);
+    }
     if (choice.tile >= 0) {
         no_room = false;
         const int rc = is_wave_tile(choice.tile)

@@ -293,9 +293,10 @@ const char *eddlhip_conv2d_last_kernel(void);
  * device has not seen (N, C, Kf, R, S, strides, output size P x Q) runs that convolution under every launch plan (tile
  * shape x K slices and the Winograd forms, every launch timed by itself, the fastest of three to nine launches per plan,
  * on the call's own tensors) and remembers one; later calls with that geometry take it.  Which one: of all plans within
- * 3 % of the fastest, the first in a fixed order of preference (the planner's own plan, the one-launch Winograd form, the
- * same in the split arithmetic, the split form, the direct tiles, the Winograd forms that keep a transformed input in memory - those are tried only below 512 MB of
- * workspace; within a form fewer K slices first), so that two searches of one geometry agree unless two plans differ by
+ * 3 % of the fastest, the first in a fixed order of preference (the planner's plan of the direct kernels - tile -1 of the table, also in
+ * files that were saved before the planner chose among other tiles -, the one-launch Winograd form, the same in the split arithmetic, the split
+ * form, the split form for few tiles, the direct tiles, the Winograd forms that keep a transformed input in memory - those are tried only
+ * below 512 MB of workspace; within a form fewer K slices first), so that two searches of one geometry agree unless two plans differ by
  * just that margin.  A caller that needs run-to-run identical bits loads a plans file instead of searching.  The call's
  * tensors must not alias: when the output overlaps an input or the residual, nothing is searched or recorded and the
  * planner's plan runs (repeating such a call would change what it reads).  The reference does the same on a layer's first forward, with

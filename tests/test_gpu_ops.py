@@ -2101,6 +2101,32 @@ def test_conv2d_planner_chooses_alike_for_folded_and_stored_inputs(hip, N, C, Kf
     assert hip.last_conv_kernel() == stored and np.array_equal(A.numpy(), B.numpy())
 
 
+def test_conv2d_plan_that_names_the_planner_is_its_plan_of_the_direct_kernels(hip, tmp_path):
+    """Plan -1 of a table is the launch that it was when it was found, from a search or a file: the fp32 kernels, also where an unsearched
+    call takes a tile of the split form."""
+    N, C, H, W, Kf, R, S, stride, pad = PLANNER_CASES["3x3"][0]
+    rng = np.random.default_rng(2790)
+    X, K = hip.array(rng.standard_normal((N, C, H, W), dtype=np.float32)), hip.array((rng.standard_normal((Kf, C, R, S)) * 0.03).astype(np.float32))
+    O, F = hip.full((N, Kf, H, W), np.nan), hip.full((N, Kf, H, W), np.nan)
+    hip.conv2D(X, K, None, O, *stride, *pad)
+    assert "split_kernel" in hip.last_conv_kernel()
+    hip.set_conv_algo("winograd_never")
+    hip.conv2D(X, K, None, F, *stride, *pad)
+    hip.set_conv_algo("winograd_off")
+    kernel = hip.last_conv_kernel()
+    path = tmp_path / "plans.txt"
+    path.write_text("%d %d %d %d %d 1 1 %d %d 1 | -1 1\n" % (N, C, Kf, R, S, H, W))
+    hip.conv_autotune(-1)
+    try:
+        hip.conv_tuned_load(path)
+        hip.conv_autotune(True)
+        hip.fill_(O, np.nan)
+        hip.conv2D(X, K, None, O, *stride, *pad)
+        assert hip.last_conv_kernel() == kernel and np.array_equal(O.numpy(), F.numpy())
+    finally:
+        hip.conv_autotune(-1)
+
+
 @pytest.mark.parametrize("R,S", [(1, 1), (2, 2), (3, 3), (1, 9), (5, 2)])
 def test_conv2d_split_filters_of_many_weights(hip, R, S):
     """From two million weights on the taps of a filter are split together: the bits of the weights split one by one (a slice of the filters)."""

@@ -2731,10 +2731,13 @@ struct CachedFilters {
     float *Wfused;  // 3x3 filters: the transformed filters of the one-launch Winograd form [fused_rows][16][Mp], made on first use
     int fused_rows;
     void *Wwsplit;  // 3x3 filters: the transformed filters as three bf16 parts (wino_split_filter_kernel), made on first use
-    void *Wsplit;  // the filters as three bf16 parts in the operand order of the split form (split_filter_kernel), made on first use
+    // The filters as three bf16 parts in the operand order of the split form (split_filter_kernel).  Where the planner may choose that form they are
+    // made with the registration, so that no call, allocating or not, recorded or not, splits registered filters; elsewhere on first use.
+    void *Wsplit;
+    bool split_stale;  // K was written since they were made (a state of its own: a tensor that only one form reads is not redone for the other)
     void *Wupsplit;  // 2x2 filters: those rows as three bf16 parts (up2x2_split_filter_kernel), made on first use
     float *Wup;  // 2x2 filters: the nine weight-sum rows per channel of the upsampled-input form [C][9][Mp] (up2x2_filter_kernel), made on first use
-    bool stale;  // K was written through this library since the last repack
+    bool stale;  // K was written through this library since the last repack (of all copies but Wsplit)
 };
 std::mutex g_cache_mutex;
 std::vector<CachedFilters> g_cache[EDDLHIP_MAX_DEVICES];
@@ -2796,9 +2799,14 @@ int repack(int dev, CachedFilters &e) {
         EH_CHECK_LAUNCH();
     }
     if (e.Wupsplit != nullptr) EH_TRY(launch_up_split_filters(dev, e.K, e.Wupsplit, e.Kf, e.C, e.Mp));
-    if (e.Wsplit != nullptr) EH_TRY(launch_split_filters(dev, e.K, e.Wsplit, e.Kf, e.C, e.R * e.S, e.Mp));
     if (e.Wwsplit != nullptr) EH_TRY(launch_wino_split_filters(dev, e.K, e.Wwsplit, e.Kf, e.C, e.Mp));
     e.stale = false;
+    return 0;
+}
+
+int split_again(int dev, CachedFilters &e) {
+    EH_TRY(launch_split_filters(dev, e.K, e.Wsplit, e.Kf, e.C, e.R * e.S, e.Mp));
+    e.split_stale = false;
     return 0;
 }
 
@@ -2865,7 +2873,7 @@ void conv_filters_written(int dev, const void *dst, size_t bytes) {
     const char *lo = (const char *)dst, *hi = lo + bytes;
     for (CachedFilters &e : g_cache[dev]) {
         const char *klo = (const char *)e.K, *khi = klo + (size_t)e.Kf * e.C * e.R * e.S * sizeof(float);
-        if (lo < khi && klo < hi) e.stale = true;
+        if (lo < khi && klo < hi) e.stale = e.split_stale = true;
     }
 }
 
@@ -2907,7 +2915,8 @@ int eddlhip_conv2d_cache_filters(int dev, const float *K, int Kf, int C, int R, 
         if (e.K == K) {
             EH_REQUIRE(e.Kf == Kf && e.C == C && e.R == R && e.S == S,
                        "conv2d_cache_filters: pointer already registered with shape %dx%dx%dx%d", e.Kf, e.C, e.R, e.S);
-            return repack(dev, e);
+            EH_TRY(repack(dev, e));
+            return e.Wsplit != nullptr ? split_again(dev, e) : 0;
         }
     }
     CachedFilters e;
@@ -2923,13 +2932,22 @@ int eddlhip_conv2d_cache_filters(int dev, const float *K, int Kf, int C, int R, 
     e.Wsplit = nullptr;
     e.Wwsplit = nullptr;
     e.Wupsplit = nullptr;
-    e.stale = true;
+    e.stale = e.split_stale = true;
     EH_REQUIRE((size_t)e.rows * e.Mp * sizeof(float) < ((size_t)1 << 31),
                "conv2d_cache_filters: the repacked filter matrix (%d taps x %d channels) exceeds the 2 GiB a buffer descriptor covers", e.rows, e.Mp);
     EH_TRY_HIP(hipMalloc((void **)&e.Wp, (size_t)e.rows * e.Mp * sizeof(float)));
     int rc = repack(dev, e);
+    if (rc == 0 && split_applies(C, Kf, R, S)) {  // (6 bytes a weight; without room for them they are split per call)
+        if (hipMalloc(&e.Wsplit, split_filter_bytes(C, R * S, e.Mp)) == hipSuccess) {
+            rc = split_again(dev, e);
+        } else {
+            e.Wsplit = nullptr;
+            (void)hipGetLastError();
+        }
+    }
     if (rc != 0) {
         (void)hipFree(e.Wp);
+        if (e.Wsplit) (void)hipFree(e.Wsplit);
         return rc;
     }
     g_cache[dev].push_back(e);
@@ -3123,10 +3141,11 @@ int conv2d_winograd_fused(bool no_alloc, bool *no_room, const FusedVariant &fv, 
 int conv2d_up2x2(int tile, int slices, int dev, const float *I, const float *K, const float *bias, float *O, int N, int C, int H, int W, int Kf, int P, int Q, const float *bn_g,
                  const float *bn_b, const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu);
 
-// Whose call a launch of the split form is: a convolution's, the same from the fixed scratch array, a dense layer's
-enum class SplitCall { CONV, CONV_NO_ALLOC, PRODUCT };
+// Whose call a launch of the split form is: a convolution's by a plan that names the form, the same by the planner's choice, a convolution's
+// from the fixed scratch array, a dense layer's
+enum class SplitCall { CONV, CONV_CHOICE, CONV_NO_ALLOC, PRODUCT };
 int conv2d_split(SplitCall use, const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room);
-int conv2d_wave_split(bool no_alloc, const WaveSplitVariant &v, int slices, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room);
+int conv2d_wave_split(SplitCall use, const WaveSplitVariant &v, int slices, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room);
 
 // Whether a convolution is the one conv_up2x2_kernel computes: a 2x2 stride-1 filter on ONE tensor upsampled twice in both
 // directions, no padding above or to the left (below and to the right the image is followed by zeros, as many as the
@@ -3551,7 +3570,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     // ... and for few tiles, any channel count
     const bool wave_ok = !gemm && g_algo == 0 && !g_wino_never && wave_applies(C, Kf, R, S);
     if (wave_ok && is_wave_tile(g_force_tile)) {
-        const int rc = conv2d_wave_split(no_alloc, kwave[g_force_tile - WAVE_TILE0], g_force_slices, dev, p, chunk_imgs, &no_room);
+        const int rc = conv2d_wave_split(split_use, kwave[g_force_tile - WAVE_TILE0], g_force_slices, dev, p, chunk_imgs, &no_room);
         if (!no_room) return rc;
     }
     // whether a plan names the direct kernels: forced, found, or the one that a search times as the planner's
@@ -3613,7 +3632,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
             if (!no_room) return rc;
         }
         if (found != nullptr && is_wave_tile(found->tile) && wave_ok) {
-            const int rc = conv2d_wave_split(no_alloc, kwave[found->tile - WAVE_TILE0], found->slices, dev, p, chunk_imgs, &no_room);
+            const int rc = conv2d_wave_split(split_use, kwave[found->tile - WAVE_TILE0], found->slices, dev, p, chunk_imgs, &no_room);
             if (!no_room) return rc;
         }
         if (found != nullptr && found->tile < 4) {
@@ -3631,9 +3650,10 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     }
     if (choice.tile >= 0) {
         no_room = false;
+        const SplitCall choice_use = no_alloc ? SplitCall::CONV_NO_ALLOC : SplitCall::CONV_CHOICE;
         const int rc = is_wave_tile(choice.tile)
-                           ? conv2d_wave_split(no_alloc, kwave[choice.tile - WAVE_TILE0], choice.slices, dev, p, chunk_imgs, &no_room)
-                           : conv2d_split(split_use, split_build(choice.tile - SPLIT_TILE0, R * S, uh, uw),
+                           ? conv2d_wave_split(choice_use, kwave[choice.tile - WAVE_TILE0], choice.slices, dev, p, chunk_imgs, &no_room)
+                           : conv2d_split(choice_use, split_build(choice.tile - SPLIT_TILE0, R * S, uh, uw),
                                           forced_plan(ksplit, choice.tile - SPLIT_TILE0, choice.slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p, chunk_imgs,
                                           &no_room);
         if (!no_room) return rc;
@@ -4151,54 +4171,53 @@ int conv2d_winograd_fused(bool no_alloc, bool *no_room, const FusedVariant &fv, 
     return 0;
 }
 
-// The split copy of a registered filter tensor, made on first use; *Ws stays NULL where there is none.
-int kept_split_filters(bool no_alloc, int dev, const ConvParams &call, size_t w_bytes, const void **Ws) {
+// The split copy of a registered filter tensor, made here where its registration did not; *Ws stays NULL where there is none.
+int kept_split_filters(SplitCall use, int dev, const ConvParams &call, size_t w_bytes, const void **Ws) {
+    if (use == SplitCall::PRODUCT) return 0;  // (the rows that stand for filters are no registered tensor's, wherever they lie)
     std::lock_guard<std::mutex> lock(g_cache_mutex);
-    for (CachedFilters &e : g_cache[dev]) {
-        if (e.K == call.K && e.Kf == call.Kf && e.C == call.C && e.R == call.R && e.S == call.S) {
-            if (e.Wsplit == nullptr && !state(dev).capturing && !no_alloc) {
-                if (hipMalloc(&e.Wsplit, w_bytes) != hipSuccess) {
-                    e.Wsplit = nullptr;
-                    (void)hipGetLastError();
-                    break;  // no room to keep them: split per call
-                }
-                e.stale = true;
-            }
-            if (e.Wsplit != nullptr) {
-                if (e.stale) EH_TRY(repack(dev, e));
-                *Ws = e.Wsplit;
-            }
-            break;
+    CachedFilters *e = registered_filters(dev, call.K, call.Kf, call.C, call.R, call.S);
+    if (e == nullptr) return 0;
+    if (e->Wsplit == nullptr && !state(dev).capturing && use != SplitCall::CONV_NO_ALLOC) {
+        if (hipMalloc(&e->Wsplit, w_bytes) != hipSuccess) {
+            e->Wsplit = nullptr;
+            (void)hipGetLastError();
         }
+        e->split_stale = true;
     }
+    if (e->Wsplit != nullptr && e->split_stale) EH_TRY(split_again(dev, *e));
+    *Ws = e->Wsplit;
     return 0;
 }
 
+// Memory for a launch of the split form.  *no_room: nothing is to be launched, the caller has another form - the fixed scratch array is too
+// small, or the workspace is while a graph is being recorded and the call has not asked for this form (the direct and the fp32 kernels may need less).
+int split_workspace(SplitCall use, int dev, size_t bytes, void **ws, bool *no_room) {
+    if (use == SplitCall::CONV_NO_ALLOC) {
+        *no_room = bytes > (size_t)EDDLHIP_CONV_NOALLOC_SCRATCH_BYTES;
+        *ws = g_scratch_ptr[dev];
+        return 0;
+    }
+    *no_room = use != SplitCall::CONV && state(dev).capturing && bytes > state(dev).workspace_bytes;
+    return bytes > 0 && !*no_room ? get_workspace(dev, bytes, ws) : 0;
+}
+
 // The split form (conv_split.h) of the call that `call` describes, under a plan of split steps.
-// Workspace: [split filters unless kept][partial tiles].  CONV_NO_ALLOC: from the fixed scratch array; nothing is launched and *no_room
-// is set if that is too small.  PRODUCT: the rows that stand for filters are no registered tensor's, wherever they lie, and the launch is
-// none that the convolutions' measuring hooks see (so it is also recorded while they collect).
+// Workspace: [split filters unless kept][partial tiles].  PRODUCT: the launch is none that the convolutions' measuring hooks see (so it is also
+// recorded while they collect).
 int conv2d_split(SplitCall use, const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room) {
     hipStream_t st = state(dev).stream;
-    const bool no_alloc = use == SplitCall::CONV_NO_ALLOC, product = use == SplitCall::PRODUCT;
+    const bool product = use == SplitCall::PRODUCT;
     const int RS = call.R * call.S, N = call.N;
     EH_REQUIRE(plan.tiles <= 0x3fffffffLL, "conv2d: too many tiles");
     const long long leftover = plan.nslices > 1 ? plan.leftover : 0;
     const size_t w_bytes = split_filter_bytes(call.C, RS, call.Mp);
     const size_t partial_bytes = (size_t)plan.nslices * leftover * v.bm * v.bn * sizeof(float);
     const void *Ws = nullptr;
-    if (!product) EH_TRY(kept_split_filters(no_alloc, dev, call, w_bytes, &Ws));
+    EH_TRY(kept_split_filters(use, dev, call, w_bytes, &Ws));
     const size_t ws_filters = Ws ? 0 : ((w_bytes + 255) & ~(size_t)255);
     void *ws = nullptr;
-    if (no_alloc) {
-        if (ws_filters + partial_bytes > (size_t)EDDLHIP_CONV_NOALLOC_SCRATCH_BYTES) {
-            *no_room = true;
-            return 0;
-        }
-        ws = g_scratch_ptr[dev];
-    } else if (ws_filters + partial_bytes > 0) {
-        EH_TRY(get_workspace(dev, ws_filters + partial_bytes, &ws));
-    }
+    EH_TRY(split_workspace(use, dev, ws_filters + partial_bytes, &ws, no_room));
+    if (*no_room) return 0;
     if (Ws == nullptr) {
         EH_TRY(launch_split_filters(dev, call.K, ws, call.Kf, call.C, RS, call.Mp));
         Ws = ws;
@@ -4242,8 +4261,8 @@ int conv2d_split(SplitCall use, const Variant &v, const Plan &plan, int dev, con
     return 0;
 }
 
-// The split form for few tiles (conv_wave_split.h) of the call that `call` describes; workspace and no_alloc as conv2d_split.
-int conv2d_wave_split(bool no_alloc, const WaveSplitVariant &v, int slices, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room) {
+// The split form for few tiles (conv_wave_split.h) of the call that `call` describes; workspace as conv2d_split.
+int conv2d_wave_split(SplitCall use, const WaveSplitVariant &v, int slices, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room) {
     static std::atomic<unsigned> next_count{0};
     hipStream_t st = state(dev).stream;
     const int RS = call.R * call.S, N = call.N;
@@ -4251,18 +4270,11 @@ int conv2d_wave_split(bool no_alloc, const WaveSplitVariant &v, int slices, int 
     const size_t w_bytes = split_filter_bytes(call.C, RS, call.Mp);
     const size_t partial_bytes = nslices > 1 ? (size_t)nslices * wave_tiles(v, call.Kf, chunk_imgs * call.PQ) * v.tm * v.tn * 4096 : 0;
     const void *Ws = nullptr;
-    EH_TRY(kept_split_filters(no_alloc, dev, call, w_bytes, &Ws));
+    EH_TRY(kept_split_filters(use, dev, call, w_bytes, &Ws));
     const size_t ws_filters = Ws ? 0 : ((w_bytes + 255) & ~(size_t)255);
     void *ws = nullptr;
-    if (no_alloc) {
-        if (ws_filters + partial_bytes > (size_t)EDDLHIP_CONV_NOALLOC_SCRATCH_BYTES) {
-            *no_room = true;
-            return 0;
-        }
-        ws = g_scratch_ptr[dev];
-    } else if (ws_filters + partial_bytes > 0) {
-        EH_TRY(get_workspace(dev, ws_filters + partial_bytes, &ws));
-    }
+    EH_TRY(split_workspace(use, dev, ws_filters + partial_bytes, &ws, no_room));
+    if (*no_room) return 0;
     if (Ws == nullptr) {
         EH_TRY(launch_split_filters(dev, call.K, ws, call.Kf, call.C, RS, call.Mp));
         Ws = ws;
@@ -4328,7 +4340,6 @@ int dense_split(int dev, const float *A, const float *B, float *C, int m, int k,
     // output in a launch behind the one that reads, so an output on an operand is theirs)
     auto on_output = [&](const float *operand, size_t floats) { return operand < C + (size_t)m * n && C < operand + floats; };
     if (on_output(A, (size_t)m * k) || on_output(B, (size_t)k * n)) return 0;
-    *taken = true;
     ConvParams p;
     memset(&p, 0, sizeof(p));
     p.I = p.I2 = B;
@@ -4350,7 +4361,9 @@ int dense_split(int dev, const float *A, const float *B, float *C, int m, int k,
     long long slices = (fill * num_cu + tiles - 1) / tiles;
     slices = std::max(1LL, std::min(std::min(slices, 16LL), (long long)steps / 4));
     bool no_room = false;
-    return conv2d_split(SplitCall::PRODUCT, ksplits[ONE_TAP][tile], forced_plan(ksplit, tile, (int)slices, m, k, 1, n, num_cu), dev, p, 1, &no_room);
+    EH_TRY(conv2d_split(SplitCall::PRODUCT, ksplits[ONE_TAP][tile], forced_plan(ksplit, tile, (int)slices, m, k, 1, n, num_cu), dev, p, 1, &no_room));
+    *taken = !no_room;
+    return 0;
 }
 
 }  // namespace eddlhip

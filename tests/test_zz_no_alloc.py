@@ -260,3 +260,85 @@ def test_noalloc_takes_the_planners_plan_where_the_split_winograd_filters_do_not
         assert np.array_equal(O1.numpy(), O2.numpy())
     finally:
         hip.conv_autotune(-1)
+
+
+# the planner takes a tile of the split form for these (the last in slices, where the direct kernels divide nothing)
+CHOSEN = [(2, 128, 28, 30, 128, 3, 3, 1, 1), (8, 256, 28, 28, 256, 1, 1, 1, 0), (1, 48, 8, 18, 256, 3, 3, 1, 1)]
+
+
+@pytest.mark.parametrize("N,C,H,W,Kf,R,S,stride,pad", CHOSEN)
+def test_noalloc_first_call_on_registered_filters_reads_their_copy(hip, N, C, H, W, Kf, R, S, stride, pad):
+    """No call of the other entry point came before: the filters are not split (or repacked) once more.  Seen from a filter tensor that
+    a kernel has written behind the library's back, which is registered again only after that."""
+    rng = np.random.default_rng(74)
+    dx, dw = hip.array(rng.standard_normal((N, C, H, W), dtype=np.float32)), hip.array((rng.standard_normal((Kf, C, R, S)) * 0.05).astype(np.float32))
+    O = hip.full((N, Kf, H, W), float("nan"))
+
+    def run(fn):
+        hip.fill_(O, float("nan"))
+        hip._check(fn(hip.dev, dx.ptr, dw.ptr, None, O.ptr, N, C, H, W, Kf, R, S, stride, stride, pad, pad, H, W, None, None, None, None, 0.0, None, 0))
+        assert "split_kernel" in hip.last_conv_kernel()
+        return O.numpy()
+    before = run(hip.lib.eddlhip_conv2d_fwd)
+    hip.cache_conv_filters(dw)
+    try:
+        hip.relu(dw, dw)
+        assert np.array_equal(run(hip.lib.eddlhip_conv2d_fwd_noalloc), before)
+        hip.cache_conv_filters(dw)
+        after = run(hip.lib.eddlhip_conv2d_fwd_noalloc)
+        assert not np.array_equal(after, before) and np.array_equal(run(hip.lib.eddlhip_conv2d_fwd), after)
+        dw.copy_from(dw.numpy() * 0.5)  # through the library: followed without another registration
+        assert np.array_equal(run(hip.lib.eddlhip_conv2d_fwd_noalloc), after * np.float32(0.5))
+    finally:
+        hip.uncache_conv_filters(dw)
+    assert np.array_equal(run(hip.lib.eddlhip_conv2d_fwd_noalloc), after * np.float32(0.5))
+
+
+@pytest.mark.parametrize("N,C,H,W,Kf,R,S,stride,pad", CHOSEN)
+def test_first_call_recorded_with_registered_filters_and_no_workspace(hip, N, C, H, W, Kf, R, S, stride, pad):
+    """An undivided launch on registered filters takes no workspace in any form, so it is recorded without an eager call before it; where the
+    chosen form is divided and the direct kernels are not, those run."""
+    rng = np.random.default_rng(75)
+    X, K, O = hip.array(rng.standard_normal((N, C, H, W), dtype=np.float32)), hip.array((rng.standard_normal((Kf, C, R, S)) * 0.05).astype(np.float32)), hip.empty((N, Kf, H, W))
+    hip.workspace_trim()
+    hip.cache_conv_filters(K)
+    try:
+        graph = hip.record(lambda: hip.conv2D(X, K, None, O, stride, stride, pad, pad))
+        recorded = hip.last_conv_kernel()
+        got = []
+        for _ in range(3):
+            hip.fill_(O, float("nan"))
+            graph.launch()
+            got.append(O.numpy())
+        divided = "slices" in recorded or "ksplit" in recorded
+        assert not divided and hip.workspace_bytes() == 0
+        hip.conv2D(X, K, None, O, stride, stride, pad, pad)
+        eager = hip.last_conv_kernel()
+        assert "split_kernel" in eager
+        if eager != recorded:
+            assert "split_kernel" not in recorded and "slices" in eager
+            hip.set_conv_algo("winograd_never")
+            hip.conv2D(X, K, None, O, stride, stride, pad, pad)
+            hip.set_conv_algo("winograd_off")
+        assert all(np.array_equal(g, O.numpy()) for g in got)
+    finally:
+        hip.uncache_conv_filters(K)
+
+
+def test_dense_recorded_with_the_workspace_of_the_fp32_product(hip):
+    """Many rows recorded with a workspace that holds what the fp32 product takes and not the rows in three parts: that product is recorded."""
+    rng = np.random.default_rng(76)
+    m, k, n = 64, 25088, 16
+    A, W, C = hip.array(rng.standard_normal((m, k), dtype=np.float32)), hip.array(rng.standard_normal((k, n), dtype=np.float32)), hip.empty((m, n))
+    hip.workspace_trim()
+    hip.set_conv_algo("winograd_never")
+    try:
+        hip.mult2D(A, W, C)
+    finally:
+        hip.set_conv_algo("winograd_off")
+    want = C.numpy()
+    graph = hip.record(lambda: hip.mult2D(A, W, C))
+    for _ in range(3):
+        hip.fill_(C, float("nan"))
+        graph.launch()
+        assert np.array_equal(C.numpy(), want)

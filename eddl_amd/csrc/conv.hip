@@ -2800,13 +2800,13 @@ int repack(int dev, CachedFilters &e) {
     }
     if (e.Wupsplit != nullptr) EH_TRY(launch_up_split_filters(dev, e.K, e.Wupsplit, e.Kf, e.C, e.Mp));
     if (e.Wwsplit != nullptr) EH_TRY(launch_wino_split_filters(dev, e.K, e.Wwsplit, e.Kf, e.C, e.Mp));
-    e.stale = false;
+    e.stale = state(dev).capturing;  // (recorded, the launches have not run: a call before the first replay makes the copies itself)
     return 0;
 }
 
 int split_again(int dev, CachedFilters &e) {
     EH_TRY(launch_split_filters(dev, e.K, e.Wsplit, e.Kf, e.C, e.R * e.S, e.Mp));
-    e.split_stale = false;
+    e.split_stale = state(dev).capturing;
     return 0;
 }
 

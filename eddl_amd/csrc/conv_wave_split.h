@@ -15,8 +15,6 @@
 // Sums: a wavefront's as in conv_split.h (hi hi in one accumulator, the five small products in another), then eight wavefronts
 // in increasing K order, then the slices: a fixed order, shorter chains than one workgroup's.
 
-constexpr int WAVE_SPLIT_WAVES = 8, WAVE_SPLIT_COUNT_WORDS = 16;  // (a count has a cache line to itself)
-
 // Pixels of 16 channels from c0 on for lane half `half`, channels past C zero, two tensors with any division between them.
 // (Channels past the last must not be read: they belong to the next image, and what they hold times a filter's zero need not be zero.)
 __device__ __forceinline__ void wave_split_load_any(const ConvParams &p, __amdgpu_buffer_rsrc_t in1, __amdgpu_buffer_rsrc_t in2, int voff, int c0, int half, int HW4, float (&raw)[8]) {

@@ -2253,3 +2253,29 @@ def test_dense_of_many_rows_is_no_convolution_to_the_measuring_hooks(hip):
         hip.fill_(D, np.nan)
         graph.launch()
         assert np.array_equal(D.numpy(), C.numpy())
+
+
+@pytest.mark.parametrize("plan", [(2, 1), (7, 1), (17, 1), (32, 1)])
+def test_registered_filters_written_before_a_recording_and_read_after_it(hip, plan):
+    """A recording that finds the copy of registered filters out of date holds the launches that renew it and runs none: a call between the
+    recording and its first replay has the new filters all the same."""
+    rng = np.random.default_rng(2890)
+    X, K, O, F = (hip.array(rng.standard_normal(s, dtype=np.float32)) for s in ((2, 32, 12, 20), (64, 32, 3, 3), (2, 64, 12, 20), (2, 64, 12, 20)))
+    new = rng.standard_normal((64, 32, 3, 3), dtype=np.float32)
+    conv = lambda k, o: hip.conv2D(X, k, None, o, 1, 1, 1, 1)
+    hip.force_conv_plan(*plan)
+    hip.cache_conv_filters(K)
+    try:
+        conv(K, O)
+        conv(hip.array(new), F)
+        K.copy_from(new)
+        graph = hip.record(lambda: conv(K, O))
+        conv(K, O)
+        assert np.array_equal(O.numpy(), F.numpy())
+        for _ in range(3):
+            hip.fill_(O, np.nan)
+            graph.launch()
+            assert np.array_equal(O.numpy(), F.numpy())
+    finally:
+        hip.force_conv_plan(-1, 1)
+        hip.uncache_conv_filters(K)

@@ -45,7 +45,6 @@
 #include <string.h>
 
 #include <algorithm>
-#include <atomic>
 #include <mutex>
 #include <type_traits>
 #include <utility>
@@ -62,10 +61,12 @@ using namespace eddlhip;
 // conv_setup_device asks for the device address once per device and everything else uses that pointer.
 static __device__ __align__(256) unsigned char scratch[EDDLHIP_CONV_NOALLOC_SCRATCH_BYTES];
 
-// How many slices of a tile's rows have been written (conv_wave_split.h); who finishes the rows sets their count back to zero.
-// A launch takes the next stretch of the array (conv2d_wave_split), so that launches in flight on two streams never share one.
-constexpr unsigned TILE_COUNTS = 1u << 20;
-static __device__ unsigned tile_counts[TILE_COUNTS];
+// How many slices of a tile's rows have been written (conv_wave_split.h); who finishes the rows sets their count back to zero.  Every launch with
+// slices uses the array from its start, as it uses the partial tiles in the workspace or in `scratch`: launches follow each other on the
+// device's one stream, and two that overlap (two threads, or two streams) race on both.
+constexpr long long WAVE_MAX_TILES = 1024;  // of a launch with slices
+constexpr int WAVE_SPLIT_WAVES = 8, WAVE_SPLIT_COUNT_WORDS = 16;  // of a workgroup, a count for each; a count has a cache line to itself
+static __device__ unsigned tile_counts[WAVE_MAX_TILES * WAVE_SPLIT_WAVES * WAVE_SPLIT_COUNT_WORDS];
 
 namespace {
 
@@ -2479,7 +2480,6 @@ struct WaveSplitVariant {
 const WaveSplitVariant kwave[] = {WAVE_SPLIT(1, 1), WAVE_SPLIT(2, 1)};
 constexpr int NUM_WAVE = (int)(sizeof(kwave) / sizeof(kwave[0]));
 constexpr int WAVE_TILE0 = 40;
-constexpr long long WAVE_MAX_TILES = 1024;  // of a divided launch: its stretch of tile_counts
 bool is_wave_tile(int tile) { return tile >= WAVE_TILE0 && tile < WAVE_TILE0 + NUM_WAVE; }
 // The upsampled-input form in the split arithmetic (conv_up_split.h): plan "tiles" 33 (128 filters x 64 blocks) and 34 (64 x 128, half
 // of a 128-filter tile would idle under 64 filters).  Measured, us, the best of the fp32 and of the direct split plans before -> this
@@ -2862,6 +2862,7 @@ int conv_setup_device(int dev) {
     EH_TRY_HIP(hipGetSymbolAddress(&ptr, HIP_SYMBOL(tile_counts)));
     EH_REQUIRE(ptr != nullptr, "device %d: no address for the convolution's tile counts", dev);
     g_counts_ptr[dev] = (unsigned *)ptr;
+    EH_TRY_HIP(hipMemset(ptr, 0, sizeof(tile_counts)));  // (also after a shutdown that cut launches short)
     for (const Variant(*fam)[4] : {k3x3, k1x1, k2x2, kgen})
         for (int d = 0; d < 2; d++) EH_TRY(family_occupancy(fam[d]));
     return 0;
@@ -4263,7 +4264,6 @@ int conv2d_split(SplitCall use, const Variant &v, const Plan &plan, int dev, con
 
 // The split form for few tiles (conv_wave_split.h) of the call that `call` describes; workspace as conv2d_split.
 int conv2d_wave_split(SplitCall use, const WaveSplitVariant &v, int slices, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room) {
-    static std::atomic<unsigned> next_count{0};
     hipStream_t st = state(dev).stream;
     const int RS = call.R * call.S, N = call.N;
     const int nslices = wave_slices(v, slices, call.Kf, call.C, RS, chunk_imgs * call.PQ);
@@ -4288,6 +4288,7 @@ int conv2d_wave_split(SplitCall use, const WaveSplitVariant &v, int slices, int 
     q.wp_bytes = (unsigned)w_bytes;
     q.partial = (float *)((char *)ws + ws_filters);
     q.nslices = nslices;
+    q.count = g_counts_ptr[dev];
     auto magic = [](int divisor) { return divisor == 1 ? 0u : 0xffffffffu / (unsigned)divisor + 1u; };
     const int units = (call.C + 15) / 16 * RS, parts = nslices * WAVE_SPLIT_WAVES;
     q.units_each = units / parts;
@@ -4307,14 +4308,6 @@ int conv2d_wave_split(SplitCall use, const WaveSplitVariant &v, int slices, int 
         EH_REQUIRE(wgs <= 0x3fffffffLL, "conv2d: too many tiles");
         q.gn = (int)gn;
         q.magic_gn = magic(q.gn), q.magic_gm = magic(q.gm), q.magic_pq = magic(q.PQ), q.magic_q = magic(q.Q), q.magic_rs = magic(RS), q.magic_s = magic(q.S);
-        if (nslices > 1) {
-            // the next stretch of counts that does not run over the end of the array
-            const unsigned need = (unsigned)(gn * q.gm) * (WAVE_SPLIT_WAVES * WAVE_SPLIT_COUNT_WORDS);
-            unsigned at = next_count.load(), first;
-            do first = at + need > TILE_COUNTS ? 0 : at;
-            while (!next_count.compare_exchange_weak(at, first + need));
-            q.count = g_counts_ptr[dev] + first;
-        }
         q.trace = (g_trace != nullptr && wgs <= g_trace_wgs) ? g_trace : nullptr;
         EH_TRY(prof_begin(st));
         hipLaunchKernelGGL(v.kernel[taps], dim3((unsigned)wgs), dim3(64 * WAVE_SPLIT_WAVES), 0, st, q);

@@ -1994,6 +1994,34 @@ def test_conv2d_split_form_for_few_tiles_reads_folded_inputs_and_applies_the_epi
     assert np.array_equal(finite[ok], got[ok])
 
 
+def test_conv2d_split_form_for_few_tiles_divided_launches_in_a_row(hip):
+    """Launches with slices of as many tiles as they may have, and of fewer, queued behind each other: each finds the counts of its slices as
+    the first did."""
+    rng = np.random.default_rng(2480)
+    shapes = [(1, 512, 32, 32, 1024, 4), (1, 256, 7, 9, 96, 2), (1, 512, 31, 33, 1024, 8), (2, 512, 5, 5, 64, 16)]  # (1024 tiles of 32 filters x 32 pixels, 6, 1024, 4)
+    calls = []
+    for N, C, H, W, Kf, slices in shapes:
+        X, K = hip.array(rng.standard_normal((N, C, H, W), dtype=np.float32)), hip.array(rng.standard_normal((Kf, C, 1, 1), dtype=np.float32))
+        calls.append((X, K, slices, [hip.full((N, Kf, H, W), np.nan) for _ in range(7)]))
+    try:
+        for X, K, slices, outs in calls:
+            hip.force_conv_plan(40, slices)
+            hip.conv2D(X, K, None, outs[0], 1, 1, 0, 0)
+            assert hip.last_conv_kernel().endswith("+slices(%d)" % min(slices, X.shape[1] // 128))
+            hip.synchronize()
+        for i in range(1, 7):
+            for X, K, slices, outs in calls:
+                hip.force_conv_plan(40, slices)
+                hip.conv2D(X, K, None, outs[i], 1, 1, 0, 0)
+    finally:
+        hip.force_conv_plan(-1, 1)
+    for X, K, slices, outs in calls:
+        want = outs[0].numpy()
+        ref = np.einsum("nchw,kc->nkhw", X.numpy().astype(np.float64), K.numpy()[:, :, 0, 0].astype(np.float64))
+        assert_conv_close(ref, want, "slices %d" % slices)
+        assert all(np.array_equal(want, o.numpy()) for o in outs[1:])
+
+
 @pytest.mark.parametrize("plan", [(0, 1), (2, 1), (6, 1), (7, 1), (17, 1), (18, 1), (32, 1), (40, 1)])
 @pytest.mark.parametrize("e_pixels,e_deviation", [(0, 0), (-59, 3), (-61, 0), (-75, -20), (59, -3), (62, 0), (70, 20), (-130, 0), (0, -59), (0, -61), (0, 59), (0, 61)])
 def test_conv2d_epilogue_divides_as_the_batch_norm_kernel_does(hip, plan, e_pixels, e_deviation):

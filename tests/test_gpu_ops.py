@@ -2023,7 +2023,8 @@ def test_conv2d_split_form_for_few_tiles_divided_launches_in_a_row(hip):
 
 
 @pytest.mark.parametrize("plan", [(0, 1), (2, 1), (6, 1), (7, 1), (17, 1), (18, 1), (32, 1), (40, 1)])
-@pytest.mark.parametrize("e_pixels,e_deviation", [(0, 0), (-59, 3), (-61, 0), (-75, -20), (59, -3), (62, 0), (70, 20), (-130, 0), (0, -59), (0, -61), (0, 59), (0, 61)])
+@pytest.mark.parametrize("e_pixels,e_deviation", [(0, 0), (-59, 3), (-61, 0), (-75, -20), (59, -3), (62, 0), (70, 20), (-130, 0), (0, -59), (0, -61), (0, 59), (0, 61),
+                                                  (-59, 59), (59, -59), (-59, -59), (59, 59), (-58, 60), (60, -60)])
 def test_conv2d_epilogue_divides_as_the_batch_norm_kernel_does(hip, plan, e_pixels, e_deviation):
     """The quotient by the reciprocal, on either side of the range that it is taken in, bit for bit: numbers and deviations around 2^-60 and
     2^60, zeros of both signs, subnormal numbers, infinities."""

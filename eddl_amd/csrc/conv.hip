@@ -2467,7 +2467,8 @@ bool is_split_tile(int tile) { return tile >= SPLIT_TILE0 && tile < SPLIT_TILE0 
 // 8.8 -> 5.1, 64 3x3 on 56x56 11.2 -> 6.2, 512 -> 128 on 28x28 9.8 -> 5.5, 128 -> 512 8.2 -> 5.4, 256 3x3 on 14x14 12.6 -> 8.3, 256 -> 1024
 // 10.4 -> 5.4, 512 3x3 on 7x7 14.7 -> 8.8, 2048 -> 512 11.5 -> 7.1, 512 3x3 on 14x14 20.1 -> 14.0; 4 images, 512 -> 128 on 28x28 13.1 -> 7.6,
 // 256 3x3 on 14x14 17.3 -> 13.8, 512 3x3 on 7x7 21.2 -> 14.3, 2048 -> 512 13.8 -> 9.7.  No gain where four workgroups per CU do not hold
-// the tiles (4 images, 64 -> 256 on 56x56 10.3 against 21; 12 images, any), so the search tries no more.
+// the tiles (4 images, 64 -> 256 on 56x56 10.3 against 21; 12 images, any), so neither the search nor the planner offers more (the planner with
+// eight: the same time within 0.3 % over eight networks without a search).
 struct WaveSplitVariant {
     const char *name[3];  // by SplitTaps
     int tm, tn;           // 32 tm filters x 32 tn pixels
@@ -2482,6 +2483,7 @@ struct WaveSplitVariant {
 const WaveSplitVariant kwave[] = {WAVE_SPLIT(1, 1), WAVE_SPLIT(2, 1)};
 constexpr int NUM_WAVE = (int)(sizeof(kwave) / sizeof(kwave[0]));
 constexpr int WAVE_TILE0 = 40;
+constexpr long long WAVE_MAX_PER_CU = 4;  // workgroups of a launch that is offered
 bool is_wave_tile(int tile) { return tile >= WAVE_TILE0 && tile < WAVE_TILE0 + NUM_WAVE; }
 // The upsampled-input form in the split arithmetic (conv_up_split.h): plan "tiles" 33 (128 filters x 64 blocks) and 34 (64 x 128, half
 // of a 128-filter tile would idle under 64 filters).  Measured, us, the best of the fp32 and of the direct split plans before -> this
@@ -2510,11 +2512,13 @@ bool split_applies(int C, int Kf, int R, int S) {
 
 bool wave_applies(int C, int Kf, int R, int S) { return split_filter_bytes(C, R * S, (Kf + M_ALIGN - 1) / M_ALIGN * M_ALIGN) < ((size_t)1 << 31); }
 long long wave_tiles(const WaveSplitVariant &v, int Kf, long long npix) { return (long long)((Kf + 32 * v.tm - 1) / (32 * v.tm)) * ((npix + 32 * v.tn - 1) / (32 * v.tn)); }
-// Every tile of 32 pixels reads all filters.  A launch repeated by itself finds them in L2, a network's come from memory and are waited for by
-// every tile again, so neither the search nor the planner offers this form from 64 MB of such reads on (VGG-16, one image, 442 -> 457 us with its
-// 2 ... 14 MB filters in this form for 98 ... 7 tiles, though by itself the last takes 14 us for 20).
+// Every tile of 32 pixels reads all filters.  A launch repeated by itself finds them in L2; a network's come from memory, and the more of them are
+// read the more other data they displace, so neither the search nor the planner offers this form above 256 MB of such reads.  Lines
+// at 64, 110, 210 MB and none, us a pass: ResNet-50 of 7 images of 250 px without a search (198 MB in its last stage) 1176, 1144, 1120, 1119, of 4 images of
+// 200 px with one 772, 740, 726, 726, U-Net of 144 px 545, 532, 509, 509; above the line, 512 3x3 on 28x28 (354 MB; alone as fast as the split form's
+// other tiles) takes 39.7 inside VGG-16 of one image for 33.0, and the dense layer of 411 MB behind it 94 for 81: 457 a pass without a line, 438-455 with any.
 bool wave_filters_fit(int C, int Kf, int RS, long long npix) {
-    return (double)split_filter_bytes(C, RS, (Kf + M_ALIGN - 1) / M_ALIGN * M_ALIGN) * (double)((npix + 31) / 32) <= 64e6;
+    return (double)split_filter_bytes(C, RS, (Kf + M_ALIGN - 1) / M_ALIGN * M_ALIGN) * (double)((npix + 31) / 32) <= 256e6;
 }
 // K slices of a plan that asks for `slices`: no more than there are units of 16 channels under one tap for eight wavefronts each
 int wave_slices(const WaveSplitVariant &v, int slices, int Kf, int C, int RS, long long npix) {
@@ -2648,9 +2652,9 @@ Plan forced_plan(const Variant *family, int tile, int slices, int Kf, int C, int
 // not fit that one's scratch array is none.
 // Time of a workgroup step: `alone` with one workgroup on a CU, at least `shared` for every one that is there; of a workgroup around its
 // steps: `fixed` and `each` for every one there.  Fitted to 6200 timed plans of 281 convolutions (1 - 64 images, 7 - 368 pixels, 16 - 1024
-// channels, filters of 1 - 7, this library's networks among them), rms error 17-20 %; by its choices the 156 of them that have whole groups of
-// 16 channels take 1 / 1.40 of the direct kernels' time together (the best plan of each:
-// 1 / 1.5) and none takes more than 1.02 of it.  Below 7 us of direct kernel nothing is to be gained by this model, and the direct kernel stays.
+// channels, filters of 1 - 7, this library's networks among them), rms error 17-20 %; by its choices the 195 of them that have whole groups of
+// 16 channels take 1 / 1.38 of the direct kernels' time (geometric mean; the best plan of each:
+// 1 / 1.51) and none takes more than 1.02 of it (profiles/split_planner_fit.txt).  Below 7 us of direct kernel nothing is to be gained by this model, and the direct kernel stays.
 struct SplitChoice {
     int tile, slices;
     double cost_us;
@@ -2708,7 +2712,7 @@ SplitChoice plan_split(int Kf, int C, int RS, int Mp, long long npix, int num_cu
         for (int want : kSlices) {
             const int slices = wave_slices(kwave[t], want, Kf, C, RS, npix);
             const long long tiles = wave_tiles(kwave[t], Kf, npix), here = (tiles * slices + num_cu - 1) / num_cu;
-            if (slices == last || tiles * slices > 8LL * num_cu) continue;
+            if (slices == last || tiles * slices > WAVE_MAX_PER_CU * num_cu) continue;
             last = slices;
             const double each = (double)((units + 8 * slices - 1) / (8 * slices)) * k.unit;
             double us = k.launch + (double)(here / k.resident) * (k.group + each * k.resident) + (slices > 1 ? k.slices : 0.0);
@@ -3332,13 +3336,13 @@ int search_plan(const ConvCall &c, const Variant *family, const Plan &planned, l
                 time_plan(5 + v, SPLIT_TILE0 + v, sl);
             }
         }
-    if (wave_ok && wave_filters_fit(c.C, c.Kf, c.R * c.S, chunk_pix))  // the split form for few tiles: up to four workgroups per CU
+    if (wave_ok && wave_filters_fit(c.C, c.Kf, c.R * c.S, chunk_pix))  // the split form for few tiles
         for (int v = 0; v < NUM_WAVE; v++) {
             const long long tiles = wave_tiles(kwave[v], c.Kf, chunk_pix);
             int last_slices = 0;
             for (int sl : kSearchSlices) {
                 const int ns = wave_slices(kwave[v], sl, c.Kf, c.C, c.R * c.S, chunk_pix);
-                if (ns == last_slices || tiles * ns > 4LL * num_cu) continue;
+                if (ns == last_slices || tiles * ns > WAVE_MAX_PER_CU * num_cu) continue;
                 last_slices = ns;
                 time_plan(9, WAVE_TILE0 + v, sl);
             }

@@ -2130,6 +2130,17 @@ def test_conv2d_planner_chooses_alike_for_folded_and_stored_inputs(hip, N, C, Kf
     assert hip.last_conv_kernel() == stored and np.array_equal(A.numpy(), B.numpy())
 
 
+@pytest.mark.parametrize("N,H,W,few", [(7, 8, 8, True), (1, 14, 14, True), (1, 28, 28, False)])
+def test_conv2d_planner_offers_the_form_for_few_tiles_up_to_256_mb_of_filter_reads(hip, N, H, W, few):
+    """512 -> 512 3x3, 14 MB of filters read by 14, 7 and 25 tiles of 32 pixels."""
+    X, K, O = hip.empty((N, 512, H, W)), hip.empty((512, 512, 3, 3)), hip.full((N, 512, H, W), np.nan)
+    hip.rand_normal(X, 0.0, 1.0, 41)
+    hip.rand_normal(K, 0.0, 0.02, 42)
+    hip.conv2D(X, K, None, O, 1, 1, 1, 1)
+    assert hip.last_conv_kernel().startswith("conv_wave_split_kernel") == few
+    assert_conv_close(_conv64(X.numpy(), K.numpy(), (1, 1), (1, 1), H, W), O.numpy(), "%d x %dx%d" % (N, H, W))
+
+
 def test_conv2d_plan_that_names_the_planner_is_its_plan_of_the_direct_kernels(hip, tmp_path):
     """Plan -1 of a table is the launch that it was when it was found, from a search or a file: the fp32 kernels, also where an unsearched
     call takes a tile of the split form."""

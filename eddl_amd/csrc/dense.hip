@@ -182,10 +182,16 @@ bool reads_rows(int m, int k, int n) { return m == 1 || (m <= 32 && (size_t)k * 
 
 // Many rows are bound by the fp32 matrix instruction as much as by the weights, and take the split form of a convolution (dense_split) where that
 // can run it: whole groups of 16 inputs.  us, before -> after: 64 rows 25088 x 4096 159 -> 116, 4096 x 4096 39.3 -> 28.8, 4096 x 1000 26.4
-// -> 18.2; 128 rows 297 -> 171, 63.6 -> 37.2, 37.1 -> 21.6, 512 x 4096 38.5 -> 17.9; error against 64 bits 3.7e-7 -> 2.4e-7 ... 3.3e-7, 1.8e-7 ->
-// 1.0e-7, 1.6e-7 -> 9.7e-8.  33 to 48 rows would gain as much (48 rows 37.7 -> 28.7), but a few rows have the bits that they have
-// among 33, which this would end; up to 32 the weights are streamed no faster by it (25088 x 4096 110 against 112).
-bool split_rows(int m) { return m > 48; }
+// -> 18.2, 512 x 10 22.3 -> 11.3; 128 rows 297 -> 171, 63.6 -> 37.2, 37.1 -> 21.6, 33.6 -> 12.4; error against 64 bits 3.7e-7 -> 2.4e-7 ... 3.3e-7,
+// 1.8e-7 -> 1.0e-7, 1.6e-7 -> 9.7e-8.
+// The line at 48 rows is not where the times cross: 33 to 48 rows would gain as much (48 rows 37.7 -> 28.7; up to 32 the weights are streamed no
+// faster, 25088 x 4096 110 against 112).  It is a choice for calls of varying row counts: up to 48 rows (and, in the fp32 product, up to 128) a row has the
+// same bits in every batch, which the split form's tiles and K slices end.
+// Few columns under a long sum have few tiles, which the K slices do not make enough of, and the rows cost more to split than to multiply: the fp32
+// product from 4 M row elements or 16 K inputs on, up to 256 columns (us, fp32 against split: 256 rows 25088 x 10 60.7 against 66.1, 256 rows 50176 x 64 76
+// against 119, 768 rows 12544 x 100 55 against 68, 1024 rows 16384 x 128 80 against 84; below it 512 rows 8192 x 10 1.26 times as fast in the split form,
+// 256 rows 12544 x 64 1.08, beyond it 384 columns 0.93 ... 1.6, 1000 columns 1.2 ... 1.9).
+bool split_rows(int m, int k, int n) { return m > 48 && (n > 256 || (k <= 16384 && (long long)m * k <= 1LL << 22)); }
 
 int dense_impl(int dev, const float *A, const float *B, float *C, int m, int k, int n, int incC, const float *bias, int relu,
                const char *what) {
@@ -194,7 +200,7 @@ int dense_impl(int dev, const float *A, const float *B, float *C, int m, int k, 
     EH_REQUIRE(A && B && C, "%s: NULL tensor", what);
     EH_TRY(use_device(dev));
     hipStream_t st = state(dev).stream;
-    if (split_rows(m)) {
+    if (split_rows(m, k, n)) {
         bool taken = false;
         EH_TRY(dense_split(dev, A, B, C, m, k, n, incC, bias, relu, &taken));
         if (taken) return 0;

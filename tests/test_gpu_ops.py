@@ -2319,3 +2319,20 @@ def test_registered_filters_written_before_a_recording_and_read_after_it(hip, pl
     finally:
         hip.force_conv_plan(-1, 1)
         hip.uncache_conv_filters(K)
+
+
+@pytest.mark.parametrize("m,k,n,split", [(49, 16384, 256, True), (49, 16400, 256, False), (49, 16400, 257, True), (256, 16384, 16, True), (257, 16384, 16, False),
+                                         (257, 16384, 257, True), (48, 512, 300, False), (49, 512, 1, True)])
+def test_dense_few_columns_under_a_long_sum_take_the_fp32_product(hip, m, k, n, split):
+    """Either side of the lines at 48 rows, 256 columns, 16384 inputs and 4 M row elements, by the bits of the two forms."""
+    A, W, C, D = hip.empty((m, k)), hip.empty((k, n)), hip.full((m, n), np.nan), hip.full((m, n), np.nan)
+    hip.rand_normal(A, 0.0, 1.0, 31)
+    hip.rand_normal(W, 0.0, k ** -0.5, 32)
+    hip.mult2D(A, W, C)
+    hip.set_conv_algo("winograd_never")
+    try:
+        hip.mult2D(A, W, D)
+    finally:
+        hip.set_conv_algo("winograd_off")
+    assert np.array_equal(C.numpy(), D.numpy()) != split
+    assert_conv_close(A.numpy().astype(np.float64) @ W.numpy().astype(np.float64), C.numpy(), "%dx%dx%d" % (m, k, n))

@@ -328,7 +328,7 @@ def test_first_call_recorded_with_registered_filters_and_no_workspace(hip, N, C,
 def test_dense_recorded_with_the_workspace_of_the_fp32_product(hip):
     """Many rows recorded with a workspace that holds what the fp32 product takes and not the rows in three parts: that product is recorded."""
     rng = np.random.default_rng(76)
-    m, k, n = 64, 25088, 16
+    m, k, n = 64, 16384, 16
     A, W, C = hip.array(rng.standard_normal((m, k), dtype=np.float32)), hip.array(rng.standard_normal((k, n), dtype=np.float32)), hip.empty((m, n))
     hip.workspace_trim()
     hip.set_conv_algo("winograd_never")

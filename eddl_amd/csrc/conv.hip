@@ -105,7 +105,6 @@ struct ConvParams {
     const float *bias, *bn_g, *bn_b, *bn_mean, *bn_var, *residual;
     float bn_eps;
     int relu;
-    int residual_row;  // the residual is one plane for all filters (a dense layer's bias, see dense_split)
     // The output is written with the streaming (non-temporal) hint: set by the host for a layer that is bound by its
     // output traffic and whose output is larger than the last-level cache, so that keeping it there helps no reader.
     int stream_out;
@@ -230,8 +229,11 @@ __device__ __forceinline__ float finish_value(const ConvParams &p, const Channel
     if (p.relu) v = v > 0.0f ? v : 0.0f;
     return v;
 }
+// ROW: the residual is one plane for all filters (a dense layer's bias, see dense_split).  Builds of their own: as a flag of the call the
+// address arithmetic alone cost every kernel registers, and the direct 128x128 tile 2.5 % of its time.
+template <bool ROW = false>
 __device__ __forceinline__ float apply_epilogue(const ConvParams &p, const ChannelEpilogue &e, float v, size_t oidx) {
-    return finish_value(p, e, v, p.residual ? p.residual[p.residual_row ? oidx % (size_t)p.PQ : oidx] : 0.0f);
+    return finish_value(p, e, v, p.residual ? p.residual[ROW ? oidx % (size_t)p.PQ : oidx] : 0.0f);
 }
 
 // LDS-direct load: the load unit writes the dword of lane i to LDS address dst + 4*i (out-of-range
@@ -357,7 +359,7 @@ __device__ __forceinline__ void stage_channel_constants(const ConvParams &p, flo
 // the channel constants of four consecutive rows come from LDS in one read; which of batch norm,
 // affine, residual and ReLU apply is decided once per group of four rows (the flags are the same for
 // every lane) instead of once per value.  The arithmetic per value is that of store_tile, step by step.
-template <int TM, int TN, int BM, bool HAS_RES>
+template <int TM, int TN, int BM, bool HAS_RES, bool ROW>
 __device__ __forceinline__ void store_tile_inside(const ConvParams &p, floatx16 (&acc)[TM][TN], const float *epi, int m0, int m_local,
                                                   int n_base, int lane) {
     const int half = lane >> 5;
@@ -371,7 +373,7 @@ __device__ __forceinline__ void store_tile_inside(const ConvParams &p, floatx16 
         const unsigned pq = n - img * (unsigned)p.PQ;
         const size_t idx = ((size_t)img * p.Kf + (size_t)(m0 + m_local + 4 * half)) * plane + pq;
         optr[tn] = p.O + idx;
-        rptr[tn] = p.residual + (p.residual_row ? (size_t)pq : idx);  // not dereferenced without a residual
+        rptr[tn] = p.residual + (ROW ? (size_t)pq : idx);  // not dereferenced without a residual
     }
     const bool has_bias = p.bias != nullptr, has_bn = p.bn_mean != nullptr, affine = p.bn_g != nullptr;
     constexpr bool has_res = HAS_RES;
@@ -382,7 +384,7 @@ __device__ __forceinline__ void store_tile_inside(const ConvParams &p, floatx16 
         for (int q4 = 0; q4 < 4; q4++) {  // rows 8*q4 + 4*half + 0..3 of the block: v = 4*q4 + j
             const int row0 = m_local + tm * 32 + 8 * q4 + 4 * half;
             const size_t roff = (size_t)(tm * 32 + 8 * q4) * plane;
-            const size_t rplane = p.residual_row ? 0 : plane, rroff = p.residual_row ? 0 : roff;
+            const size_t rplane = ROW ? 0 : plane, rroff = ROW ? 0 : roff;
             float res[4][TN];
             if constexpr (has_res) {
 #pragma unroll
@@ -472,23 +474,23 @@ __device__ __forceinline__ void store_tile_inside(const ConvParams &p, floatx16 
 // before the first of them is used, so their latencies overlap.
 // (The residual's presence is a template parameter of the two bodies so that the loads of the residual values and their
 // uses sit in one branch: a kernel that goes on to further work after a tile then carries no load that looks pending.)
-template <int TM, int TN, int BM, bool HAS_RES>
+template <int TM, int TN, int BM, bool HAS_RES, bool ROW>
 __device__ __forceinline__ void store_tile_edge(const ConvParams &p, floatx16 (&acc)[TM][TN], const float *epi, int m0, int m_local, int n_base,
                                                 int lane);
 
-template <int TM, int TN, int BM>
+template <int TM, int TN, int BM, bool ROW = false>
 __device__ __forceinline__ void store_tile(const ConvParams &p, floatx16 (&acc)[TM][TN], const float *epi, int m0, int m_local, int n_base,
                                            int lane) {
     if (m0 + m_local + TM * 32 <= p.Kf && (long long)n_base + TN * 32 <= p.npix) {
-        if (p.residual != nullptr) store_tile_inside<TM, TN, BM, true>(p, acc, epi, m0, m_local, n_base, lane);
-        else store_tile_inside<TM, TN, BM, false>(p, acc, epi, m0, m_local, n_base, lane);
+        if (p.residual != nullptr) store_tile_inside<TM, TN, BM, true, ROW>(p, acc, epi, m0, m_local, n_base, lane);
+        else store_tile_inside<TM, TN, BM, false, ROW>(p, acc, epi, m0, m_local, n_base, lane);
         return;
     }
-    if (p.residual != nullptr) store_tile_edge<TM, TN, BM, true>(p, acc, epi, m0, m_local, n_base, lane);
-    else store_tile_edge<TM, TN, BM, false>(p, acc, epi, m0, m_local, n_base, lane);
+    if (p.residual != nullptr) store_tile_edge<TM, TN, BM, true, ROW>(p, acc, epi, m0, m_local, n_base, lane);
+    else store_tile_edge<TM, TN, BM, false, ROW>(p, acc, epi, m0, m_local, n_base, lane);
 }
 
-template <int TM, int TN, int BM, bool HAS_RES>
+template <int TM, int TN, int BM, bool HAS_RES, bool ROW>
 __device__ __forceinline__ void store_tile_edge(const ConvParams &p, floatx16 (&acc)[TM][TN], const float *epi, int m0, int m_local, int n_base,
                                                 int lane) {
     size_t obase[TN];
@@ -517,7 +519,7 @@ __device__ __forceinline__ void store_tile_edge(const ConvParams &p, floatx16 (&
 #pragma unroll
                     for (int tn = 0; tn < TN; tn++) {
                         const size_t oidx = (mok && nok[tn]) ? obase[tn] + (size_t)(m0 + ml) * p.PQ : 0;
-                        res[vv][tn] = p.residual[p.residual_row ? oidx % (size_t)p.PQ : oidx];
+                        res[vv][tn] = p.residual[ROW ? oidx % (size_t)p.PQ : oidx];
                     }
                 }
             }
@@ -1470,7 +1472,7 @@ __global__ __launch_bounds__(256, (TM * TN >= 4 ? 3 : 4)) void conv_gen_kernel(c
 // wavefront q): adds the slices in increasing K order (a fixed order: results do not depend on scheduling), then
 // applies the fused tail and stores.  A wavefront has few values and therefore all slices' loads in flight at once
 // (fifteen slices at a time): the kernel lasts about one trip to memory.
-template <int WM, int WN, int TM, int TN>
+template <int WM, int WN, int TM, int TN, bool ROW = false>
 __global__ __launch_bounds__(256) void conv_reduce_kernel(const ConvParams p) {
     constexpr int BM = WM * TM * 32, BN = WN * TN * 32, UNITS = 4 * TM * TN;
     const int lane = threadIdx.x & 63, q = threadIdx.x >> 6, half = lane >> 5;
@@ -1524,7 +1526,7 @@ __global__ __launch_bounds__(256) void conv_reduce_kernel(const ConvParams p) {
         const int m = m_first + j;
         if (m < p.Kf) {
             const size_t oidx = ((size_t)img * p.Kf + m) * p.PQ + pq;
-            p.O[oidx] = apply_epilogue(p, chan[j], acc[j], oidx);
+            p.O[oidx] = apply_epilogue<ROW>(p, chan[j], acc[j], oidx);
         }
     }
 }
@@ -2449,14 +2451,15 @@ constexpr int NUM_PLAN_TILES = UP2X2_TILE + 2;
 // 58 -> 42; 3x3 stride 2 of 128 on 56x56: 120 -> 91; 64 -> 256 on 56x56: 70 -> 67, of which 256 MB of traffic are 43; in a
 // ResNet-50 the pipe is busy 28 % of the cycles), 64x128 where there are 64 filters (256 -> 64 on 56x56: 60 -> 52), 64x64 for few
 // tiles.  A 128x64 tile gives every wavefront filters of its own and all the pixels: its filters then cross L1 once, not twice.
-// Each tile comes in three builds, by how a step finds its pixel (SplitTaps).
+// Each tile comes in three builds, by how a step finds its pixel (SplitTaps), the tiles of dense layers in a fourth for their bias.
 #define SPLIT(WM, WN, TM, TN, WGS, TAPS)                                                                       \
     {                                                                                                          \
         "conv_split_kernel<" #WM "," #WN "," #TM "," #TN "," #WGS "," #TAPS ">", WM *TM * 32, WN *TN * 32,     \
-            SPLIT_K, conv_split_kernel<WM, WN, TM, TN, WGS, TAPS>, conv_reduce_kernel<WM, WN, TM, TN>, 0       \
+            SPLIT_K, conv_split_kernel<WM, WN, TM, TN, WGS, TAPS>, conv_reduce_kernel<WM, WN, TM, TN, TAPS == ROW_BIAS>, 0       \
     }
 #define SPLITS(TAPS) {SPLIT(2, 2, 2, 2, 2, TAPS), SPLIT(4, 1, 1, 2, 3, TAPS), SPLIT(2, 2, 1, 2, 3, TAPS), SPLIT(2, 2, 1, 1, 4, TAPS)}
 const Variant ksplits[][4] = {SPLITS(UPSAMPLED), SPLITS(STORED), SPLITS(ONE_TAP)};
+const Variant kproduct[] = {SPLIT(4, 1, 1, 2, 3, ROW_BIAS), SPLIT(2, 2, 1, 2, 3, ROW_BIAS), SPLIT(2, 2, 1, 1, 4, ROW_BIAS)};  // tiles 1 .. 3 (dense_split)
 const Variant *const ksplit = ksplits[UPSAMPLED];  // (the tile shapes, which the plans are made for)
 constexpr int NUM_SPLIT = (int)(sizeof(ksplits[0]) / sizeof(ksplits[0][0]));
 const Variant &split_build(int tile, int RS, int uh, int uw) { return ksplits[RS == 1 ? ONE_TAP : uh * uw == 1 ? STORED : UPSAMPLED][tile]; }
@@ -3464,7 +3467,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     p.uh = uh; p.uw = uw;
     p.K = K; p.O = O; p.Wp = nullptr;
     p.bias = bias; p.bn_g = bn_g; p.bn_b = bn_b; p.bn_mean = bn_mean; p.bn_var = bn_var; p.residual = residual;
-    p.bn_eps = bn_eps; p.relu = relu; p.residual_row = 0;
+    p.bn_eps = bn_eps; p.relu = relu;
     {
         // bound by its output traffic (arithmetic intensity under the ridge of 157.3 TFLOP/s over 8 TB/s) and an output that
         // the 256 MB last-level cache cannot hold for the next layer anyway
@@ -4347,7 +4350,6 @@ int dense_split(int dev, const float *A, const float *B, float *C, int m, int k,
     p.K = A;
     p.O = C;
     p.residual = incC ? C : bias;
-    p.residual_row = incC ? 0 : 1;
     p.relu = relu;
     p.N = 1, p.H = 1, p.W = n, p.Kf = m, p.R = p.S = p.sr = p.sc = 1, p.P = 1, p.Q = n;
     p.CRS = k, p.PQ = n, p.npix = n;
@@ -4360,7 +4362,7 @@ int dense_split(int dev, const float *A, const float *B, float *C, int m, int k,
     long long slices = (fill * num_cu + tiles - 1) / tiles;
     slices = std::max(1LL, std::min(std::min(slices, 16LL), (long long)steps / 4));
     bool no_room = false;
-    EH_TRY(conv2d_split(SplitCall::PRODUCT, ksplits[ONE_TAP][tile], forced_plan(ksplit, tile, (int)slices, m, k, 1, n, num_cu), dev, p, 1, &no_room));
+    EH_TRY(conv2d_split(SplitCall::PRODUCT, bias ? kproduct[tile - 1] : ksplits[ONE_TAP][tile], forced_plan(ksplit, tile, (int)slices, m, k, 1, n, num_cu), dev, p, 1, &no_room));
     *taken = !no_room;
     return 0;
 }

@@ -210,8 +210,8 @@ __device__ __forceinline__ void split_issue_order() {
 // the 52 that split its eight pixels), which slow a kernel that multiplies little per pixel (batch 64, best plans, us, all on one card;
 // UPSAMPLED -> ONE_TAP: 256 -> 64 on 56x56 55.8 -> 52.4, 512 -> 256 on 28x28 78.4 -> 76.5, 128 -> 512 53.1 -> 51.2, 256 -> 1024 on
 // 14x14 46.6 -> 45.2, 1024 -> 256 45.2 -> 43.2, 2048 -> 512 on 7x7 51.8 -> 49.5; UPSAMPLED -> STORED: 128 3x3 stride 2 on 56x56
-// 91.2 -> 89.9, tile 128x128 95.8 -> 94.4).
-enum SplitTaps { UPSAMPLED, STORED, ONE_TAP };
+// 91.2 -> 89.9, tile 128x128 95.8 -> 94.4).  ROW_BIAS: ONE_TAP with a residual of one row for all filters, a dense layer's bias.
+enum SplitTaps { UPSAMPLED, STORED, ONE_TAP, ROW_BIAS };
 template <int WM, int WN, int TM, int TN, int WGS, SplitTaps TAPS>
 __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p) {
     static_assert(WM * WN == 4, "four wavefronts per workgroup");
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
     auto next_load_step = [&]() {
         // (selects: a branch would end the block that the matrix instructions are scheduled in; behind the last step the
         // channels run past the last and the loads bring zeros without touching memory)
-        if constexpr (TAPS == ONE_TAP) {
+        if constexpr (TAPS == ONE_TAP || TAPS == ROW_BIAS) {
             ld_c += SPLIT_K;
             return;
         }
@@ -480,7 +480,7 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
         float *epi = (float *)&Bs[0][0][0][0];  // the K loop ended with a barrier
         put_channel_constants<BM>(epi, chan, tid);
         __syncthreads();
-        store_tile<TM, TN, BM>(p, acc, epi, m0, wm * TM * 32, n_first, lane);
+        store_tile<TM, TN, BM, TAPS == ROW_BIAS>(p, acc, epi, m0, wm * TM * 32, n_first, lane);
     }
     if (p.trace != nullptr) {
         __builtin_amdgcn_s_waitcnt(0x0F70);

@@ -23,7 +23,7 @@ HBM_PEAK_GBS = 8000.0
 FP32_MFMA_PEAK_TFLOPS = 157.3
 BF16_MFMA_PEAK_TFLOPS = 16 * FP32_MFMA_PEAK_TFLOPS
 COPY_PROBE_KIB = 262144.0  # bench.py --copy-probe: one ReLU over 2^26 floats reads 256 MiB and writes 256 MiB
-SPLIT_TAPS = ("UPSAMPLED", "STORED", "ONE_TAP")  # the enumerators of SplitTaps (csrc/conv_split.h), in their order
+SPLIT_TAPS = ("UPSAMPLED", "STORED", "ONE_TAP", "ROW_BIAS")  # the enumerators of SplitTaps (csrc/conv_split.h), in their order
 HOT = ("conv_", "wino_", "maxpool", "avgpool", "dense", "bn_", "add_kernel", "concat", "scale_", "unary_kernel", "pad_", "softmax", "upsample")
 
 

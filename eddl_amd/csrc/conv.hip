@@ -328,16 +328,20 @@ struct TileChannel : ChannelEpilogue {
     Reciprocal k;
 };
 constexpr TileChannel NO_CHANNEL = {{0.0f, 0.0f, 1.0f, 1.0f, 0.0f}, {0.0f, 0.0f}};
-template <int BM>
+// QUOTIENT: whether a kernel's epilogue takes the quotient by the reciprocal.  The kernels of the split form, the split Winograd kernel and the 32-filter
+// tile of the fp32 one do; the direct fp32 kernels, the folded and the 64-filter Winograd kernels and the upsampled fp32 one divide: their K loops hide the
+// divisions, and reciprocals carried through them cost registers and a small launch its start (128x128 tile 3x3 2.5 %, 64-filter Winograd tile
+// 3 %, 3 -> 32 on 32x32 with batch norm 5.7 -> 6.0 us).
+template <int BM, bool QUOTIENT = true>
 __device__ __forceinline__ TileChannel fetch_channel_constants(const ConvParams &p, int m0, int tid) {
     TileChannel e = NO_CHANNEL;
     if (tid < BM && m0 + tid < p.Kf) {
         static_cast<ChannelEpilogue &>(e) = load_channel(p, m0 + tid);
-        if (p.bn_mean) e.k = reciprocal_of(e.sd);
+        if (QUOTIENT && p.bn_mean) e.k = reciprocal_of(e.sd);
     }
     return e;
 }
-template <int BM>
+template <int BM, bool QUOTIENT = true>
 __device__ __forceinline__ void put_channel_constants(float *epi, const TileChannel &e, int tid) {
     if (tid < BM) {
         epi[tid] = e.bias;
@@ -345,13 +349,15 @@ __device__ __forceinline__ void put_channel_constants(float *epi, const TileChan
         epi[2 * BM + tid] = e.sd;
         epi[3 * BM + tid] = e.g;
         epi[4 * BM + tid] = e.b;
-        epi[5 * BM + tid] = e.k.r;
-        epi[6 * BM + tid] = e.k.rl;
+        if constexpr (QUOTIENT) {
+            epi[5 * BM + tid] = e.k.r;
+            epi[6 * BM + tid] = e.k.rl;
+        }
     }
 }
-template <int BM>
+template <int BM, bool QUOTIENT = true>
 __device__ __forceinline__ void stage_channel_constants(const ConvParams &p, float *epi, int m0, int tid) {
-    put_channel_constants<BM>(epi, fetch_channel_constants<BM>(p, m0, tid), tid);
+    put_channel_constants<BM, QUOTIENT>(epi, fetch_channel_constants<BM, QUOTIENT>(p, m0, tid), tid);
 }
 
 // The common case of store_tile below: every row and every pixel of the wavefront's blocks exists.
@@ -359,7 +365,7 @@ __device__ __forceinline__ void stage_channel_constants(const ConvParams &p, flo
 // the channel constants of four consecutive rows come from LDS in one read; which of batch norm,
 // affine, residual and ReLU apply is decided once per group of four rows (the flags are the same for
 // every lane) instead of once per value.  The arithmetic per value is that of store_tile, step by step.
-template <int TM, int TN, int BM, bool HAS_RES, bool ROW>
+template <int TM, int TN, int BM, bool HAS_RES, bool ROW, bool QUOTIENT>
 __device__ __forceinline__ void store_tile_inside(const ConvParams &p, floatx16 (&acc)[TM][TN], const float *epi, int m0, int m_local,
                                                   int n_base, int lane) {
     const int half = lane >> 5;
@@ -407,28 +413,35 @@ __device__ __forceinline__ void store_tile_inside(const ConvParams &p, floatx16 
             if (has_bn) {
                 const floatx4 mean = *reinterpret_cast<const floatx4 *>(epi + BM + row0);
                 const floatx4 sd = *reinterpret_cast<const floatx4 *>(epi + 2 * BM + row0);
-                const floatx4 r = *reinterpret_cast<const floatx4 *>(epi + 5 * BM + row0), rl = *reinterpret_cast<const floatx4 *>(epi + 6 * BM + row0);
-                float least = 1.0f, most = 1.0f;
+                if constexpr (QUOTIENT) {
+                    const floatx4 r = *reinterpret_cast<const floatx4 *>(epi + 5 * BM + row0), rl = *reinterpret_cast<const floatx4 *>(epi + 6 * BM + row0);
+                    float least = 1.0f, most = 1.0f;
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    least = r[j] > 0.0f ? least : 0.0f;
+                    for (int j = 0; j < 4; j++) {
+                        least = r[j] > 0.0f ? least : 0.0f;
 #pragma unroll
-                    for (int tn = 0; tn < TN; tn++) {
-                        x[j][tn] = __fsub_rn(x[j][tn], mean[j]);
-                        least = fminf(least, fabsf(x[j][tn]));
-                        most = fmaxf(most, fabsf(x[j][tn]));
+                        for (int tn = 0; tn < TN; tn++) {
+                            x[j][tn] = __fsub_rn(x[j][tn], mean[j]);
+                            least = fminf(least, fabsf(x[j][tn]));
+                            most = fmaxf(most, fabsf(x[j][tn]));
+                        }
                     }
-                }
-                if (__builtin_expect(out_of_quotient_range(least, most), 0)) {  // (out of line: a jump over it costs a small launch 0.1 us a time)
+                    if (__builtin_expect(out_of_quotient_range(least, most), 0)) {  // (out of line: a jump over it costs a small launch 0.1 us a time)
 #pragma unroll
-                    for (int j = 0; j < 4; j++)
+                        for (int j = 0; j < 4; j++)
 #pragma unroll
-                        for (int tn = 0; tn < TN; tn++) x[j][tn] = __fdiv_rn(x[j][tn], sd[j]);
+                            for (int tn = 0; tn < TN; tn++) x[j][tn] = __fdiv_rn(x[j][tn], sd[j]);
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 4; j++)
+#pragma unroll
+                            for (int tn = 0; tn < TN; tn++) x[j][tn] = quotient(x[j][tn], sd[j], r[j], rl[j]);
+                    }
                 } else {
 #pragma unroll
                     for (int j = 0; j < 4; j++)
 #pragma unroll
-                        for (int tn = 0; tn < TN; tn++) x[j][tn] = quotient(x[j][tn], sd[j], r[j], rl[j]);
+                        for (int tn = 0; tn < TN; tn++) x[j][tn] = __fdiv_rn(__fsub_rn(x[j][tn], mean[j]), sd[j]);
                 }
                 if (affine) {
                     const floatx4 g = *reinterpret_cast<const floatx4 *>(epi + 3 * BM + row0);
@@ -478,12 +491,12 @@ template <int TM, int TN, int BM, bool HAS_RES, bool ROW>
 __device__ __forceinline__ void store_tile_edge(const ConvParams &p, floatx16 (&acc)[TM][TN], const float *epi, int m0, int m_local, int n_base,
                                                 int lane);
 
-template <int TM, int TN, int BM, bool ROW = false>
+template <int TM, int TN, int BM, bool ROW, bool QUOTIENT>
 __device__ __forceinline__ void store_tile(const ConvParams &p, floatx16 (&acc)[TM][TN], const float *epi, int m0, int m_local, int n_base,
                                            int lane) {
     if (m0 + m_local + TM * 32 <= p.Kf && (long long)n_base + TN * 32 <= p.npix) {
-        if (p.residual != nullptr) store_tile_inside<TM, TN, BM, true, ROW>(p, acc, epi, m0, m_local, n_base, lane);
-        else store_tile_inside<TM, TN, BM, false, ROW>(p, acc, epi, m0, m_local, n_base, lane);
+        if (p.residual != nullptr) store_tile_inside<TM, TN, BM, true, ROW, QUOTIENT>(p, acc, epi, m0, m_local, n_base, lane);
+        else store_tile_inside<TM, TN, BM, false, ROW, QUOTIENT>(p, acc, epi, m0, m_local, n_base, lane);
         return;
     }
     if (p.residual != nullptr) store_tile_edge<TM, TN, BM, true, ROW>(p, acc, epi, m0, m_local, n_base, lane);
@@ -679,7 +692,7 @@ __device__ __forceinline__ ChannelEpilogue channel_from_lds(const float *epi, in
 // decided once for the 4 NK values (the flags are the same for every lane), the channel constants of the rows come from
 // LDS in one read each (`epi`: stage_channel_constants' layout, ml = the first row's place in the tile, a multiple of
 // NK), one 64-bit address serves all stores, and the residual's loads are in flight together.
-// QUOTIENT: a kernel with no registers for the reciprocals divides.
+// QUOTIENT: as in fetch_channel_constants.
 template <int BM, int NK, bool QUOTIENT = true>
 __device__ __forceinline__ void wino_store_rows(const ConvParams &p, const float *epi, int ml, int m, int img, int ty, int tx, size_t plane,
                                                 float (&x)[NK][2][2]) {
@@ -872,7 +885,7 @@ __device__ __forceinline__ void conv_tap_body(const ConvParams &p) {
     const int m0 = m_tile * BM;
     const long long n0 = (long long)n_tile * BN;
     TileChannel chan = NO_CHANNEL;
-    if (!split && !UP2) chan = fetch_channel_constants<BM>(p, m0, tid);  // (UP2 has no register to spare in its K loop: fetched after it)
+    if (!split && !UP2) chan = fetch_channel_constants<BM, false>(p, m0, tid);  // (UP2 has no register to spare in its K loop: fetched after it)
 
     const __amdgpu_buffer_rsrc_t rsrc_in = __builtin_amdgcn_make_buffer_rsrc((void *)p.I, 0, p.in_bytes, RSRC_WORD3);
     const __amdgpu_buffer_rsrc_t rsrc_in2 = __builtin_amdgcn_make_buffer_rsrc((void *)p.I2, 0, p.in_bytes, RSRC_WORD3);
@@ -1205,27 +1218,27 @@ __device__ __forceinline__ void conv_tap_body(const ConvParams &p) {
     if constexpr (WINO) {
         // (launched with whole tiles only)
         float *epi = &As[0][0];
-        put_channel_constants<BM>(epi, chan, tid);
+        put_channel_constants<BM, false>(epi, chan, tid);
         __syncthreads();
         wino_store_tile<BM, 4, false>(p, wy, epi, m0, wm * 32, (int)n0 + wn * 32, lane);
     } else if constexpr (UP2) {
         // (launched with whole tiles only; a lane holds the four outputs of a block like the Winograd forms)
         float *epi = &As[0][0];
-        stage_channel_constants<BM>(p, epi, m0, tid);
+        stage_channel_constants<BM, false>(p, epi, m0, tid);
         __syncthreads();
         // (the two blocks written out: the optimizer does not unroll a loop around this much code, and a runtime index
         // would put the accumulators in memory; four rows at a time only in the build whose register budget has room for
         // their values and constants beside the 128 accumulator registers)
         constexpr int NK = MODE == 3 ? 4 : 1;
-        wino_store_tile<BM, NK>(p, uy[0], epi, m0, wm * TM * 32, (int)n0 + wn * 32, lane);
-        wino_store_tile<BM, NK>(p, uy[TM - 1], epi, m0, wm * TM * 32 + 32, (int)n0 + wn * 32, lane);
+        wino_store_tile<BM, NK, false>(p, uy[0], epi, m0, wm * TM * 32, (int)n0 + wn * 32, lane);
+        wino_store_tile<BM, NK, false>(p, uy[TM - 1], epi, m0, wm * TM * 32 + 32, (int)n0 + wn * 32, lane);
     } else if (split) {
         store_partial<TM, TN>(p, acc, local_tile, slice, wave, lane);
     } else {
         float *epi = &As[0][0];  // the K loop ended with a barrier: the filter buffers are free
-        put_channel_constants<BM>(epi, chan, tid);
+        put_channel_constants<BM, false>(epi, chan, tid);
         __syncthreads();
-        store_tile<TM, TN, BM>(p, acc, epi, m0, wm * TM * 32, (int)n0 + wn * TN * 32, lane);
+        store_tile<TM, TN, BM, false, false>(p, acc, epi, m0, wm * TM * 32, (int)n0 + wn * TN * 32, lane);
     }
     if (p.trace != nullptr) {
         __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -1301,7 +1314,7 @@ __global__ __launch_bounds__(256, (TM * TN >= 4 ? 3 : 4)) void conv_gen_kernel(c
     const int m0 = m_tile * BM;
     const long long n0 = (long long)n_tile * BN;
     TileChannel chan = NO_CHANNEL;
-    if (!split) chan = fetch_channel_constants<BM>(p, m0, tid);
+    if (!split) chan = fetch_channel_constants<BM, false>(p, m0, tid);
 
     const __amdgpu_buffer_rsrc_t rsrc_in = __builtin_amdgcn_make_buffer_rsrc((void *)p.I, 0, p.in_bytes, RSRC_WORD3);
 
@@ -1460,9 +1473,9 @@ __global__ __launch_bounds__(256, (TM * TN >= 4 ? 3 : 4)) void conv_gen_kernel(c
         store_partial<TM, TN>(p, acc, local_tile, slice, wave, lane);
     } else {
         float *epi = &As[0][0];  // the K loop ended with a barrier: the filter buffers are free
-        put_channel_constants<BM>(epi, chan, tid);
+        put_channel_constants<BM, false>(epi, chan, tid);
         __syncthreads();
-        store_tile<TM, TN, BM>(p, acc, epi, m0, wm * TM * 32, (int)n0 + wn * TN * 32, lane);
+        store_tile<TM, TN, BM, false, false>(p, acc, epi, m0, wm * TM * 32, (int)n0 + wn * TN * 32, lane);
     }
 }
 
@@ -1996,7 +2009,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
         }
     };
     load_filters(step_lo, (lds_float *)&lds[0]);
-    if (!split) chan = fetch_channel_constants<MF>(p, m0, tid);
+    if (!split) chan = fetch_channel_constants<MF, FM == 1>(p, m0, tid);
 
     // ---- where the tile's pixels go in LDS, and where this lane's patches lie there.  The tile's blocks are a run of
     // consecutive blocks, i.e. a few SEGMENTS of block rows (a segment: cnt neighbouring blocks of one row of blocks of one
@@ -2192,7 +2205,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     const int full_steps = p.C / CK;
     constexpr int WAIT_ALL = 0x0F70;  // vmcnt(0): this wavefront's LDS-direct loads have landed
     load_step(step_lo, us_of(0), rs_of(0), step_lo >= full_steps, false);  // (its filters were requested at the start)
-    if (!split) put_channel_constants<MF>(epi, chan, tid);  // (published by the barrier below)
+    if (!split) put_channel_constants<MF, FM == 1>(epi, chan, tid);  // (published by the barrier below)
     __builtin_amdgcn_s_waitcnt(WAIT_ALL);
     __syncthreads();
     trace_mark(p, 1);

@@ -480,7 +480,7 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
         float *epi = (float *)&Bs[0][0][0][0];  // the K loop ended with a barrier
         put_channel_constants<BM>(epi, chan, tid);
         __syncthreads();
-        store_tile<TM, TN, BM, TAPS == ROW_BIAS>(p, acc, epi, m0, wm * TM * 32, n_first, lane);
+        store_tile<TM, TN, BM, TAPS == ROW_BIAS, true>(p, acc, epi, m0, wm * TM * 32, n_first, lane);
     }
     if (p.trace != nullptr) {
         __builtin_amdgcn_s_waitcnt(0x0F70);

@@ -2753,8 +2753,9 @@ struct CachedFilters {
     float *Wfused;  // 3x3 filters: the transformed filters of the one-launch Winograd form [fused_rows][16][Mp], made on first use
     int fused_rows;
     void *Wwsplit;  // 3x3 filters: the transformed filters as three bf16 parts (wino_split_filter_kernel), made on first use
-    // The filters as three bf16 parts in the operand order of the split form (split_filter_kernel).  Where the planner may choose that form they are
-    // made with the registration, so that no call, allocating or not, recorded or not, splits registered filters; elsewhere on first use.
+    // The filters as three bf16 parts in the operand order of the split form (split_filter_kernel).  Where the planner may choose that form - whole groups
+    // of 16 channels, no plan search - they are made with the registration, so that no call, allocating or not, recorded or not, splits registered
+    // filters; elsewhere on first use (a search keeps other forms for most layers, and the memory costs a small layer's set-up 0.4 ms).
     void *Wsplit;
     bool split_stale;  // K was written since they were made (a state of its own: a tensor that only one form reads is not redone for the other)
     void *Wupsplit;  // 2x2 filters: those rows as three bf16 parts (up2x2_split_filter_kernel), made on first use
@@ -2960,7 +2961,7 @@ int eddlhip_conv2d_cache_filters(int dev, const float *K, int Kf, int C, int R, 
                "conv2d_cache_filters: the repacked filter matrix (%d taps x %d channels) exceeds the 2 GiB a buffer descriptor covers", e.rows, e.Mp);
     EH_TRY_HIP(hipMalloc((void **)&e.Wp, (size_t)e.rows * e.Mp * sizeof(float)));
     int rc = repack(dev, e);
-    if (rc == 0 && split_applies(C, Kf, R, S)) {  // (6 bytes a weight; without room for them they are split per call)
+    if (rc == 0 && !g_autotune && split_applies(C, Kf, R, S)) {  // (6 bytes a weight; without room for them they are split per call)
         if (hipMalloc(&e.Wsplit, split_filter_bytes(C, R * S, e.Mp)) == hipSuccess) {
             rc = split_again(dev, e);
         } else {
@@ -3164,9 +3165,9 @@ int conv2d_winograd_fused(bool no_alloc, bool *no_room, const FusedVariant &fv, 
 int conv2d_up2x2(int tile, int slices, int dev, const float *I, const float *K, const float *bias, float *O, int N, int C, int H, int W, int Kf, int P, int Q, const float *bn_g,
                  const float *bn_b, const float *bn_mean, const float *bn_var, float bn_eps, const float *residual, int relu);
 
-// Whose call a launch of the split form is: a convolution's by a plan that names the form, the same by the planner's choice, a convolution's
-// from the fixed scratch array, a dense layer's
-enum class SplitCall { CONV, CONV_CHOICE, CONV_NO_ALLOC, PRODUCT };
+// Whose call a launch of the split form is: a convolution's by a plan that names the form or by the planner's choice, either from the workspace or
+// from the fixed scratch array; a dense layer's
+enum class SplitCall { PLAN, PLAN_NO_ALLOC, CHOICE, CHOICE_NO_ALLOC, PRODUCT };
 int conv2d_split(SplitCall use, const Variant &v, const Plan &plan, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room);
 int conv2d_wave_split(SplitCall use, const WaveSplitVariant &v, int slices, int dev, const ConvParams &call, long long chunk_imgs, bool *no_room);
 
@@ -3583,7 +3584,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     // the split form: any filter shape, as long as a chunk of the input is addressed like the direct kernels do; from the fixed
     // scratch array where its filters (half as much again as the repacked ones) and partial tiles fit, else the planner's plan
     const bool split_ok = !gemm && g_algo == 0 && !g_wino_never && split_applies(C, Kf, R, S);
-    const SplitCall split_use = no_alloc ? SplitCall::CONV_NO_ALLOC : SplitCall::CONV;
+    const SplitCall split_use = no_alloc ? SplitCall::PLAN_NO_ALLOC : SplitCall::PLAN;
     if (split_ok && is_split_tile(g_force_tile)) {
         const int tile = g_force_tile - SPLIT_TILE0;
         const int rc = conv2d_split(split_use, split_build(tile, R * S, uh, uw), forced_plan(ksplit, tile, g_force_slices, Kf, C, R * S, (long long)chunk_imgs * p.PQ, state(dev).num_cu), dev, p,
@@ -3673,7 +3674,7 @@ int conv2d_fwd_impl(bool no_alloc, int dev, const float *I, const float *I2, int
     }
     if (choice.tile >= 0) {
         no_room = false;
-        const SplitCall choice_use = no_alloc ? SplitCall::CONV_NO_ALLOC : SplitCall::CONV_CHOICE;
+        const SplitCall choice_use = no_alloc ? SplitCall::CHOICE_NO_ALLOC : SplitCall::CHOICE;
         const int rc = is_wave_tile(choice.tile)
                            ? conv2d_wave_split(choice_use, kwave[choice.tile - WAVE_TILE0], choice.slices, dev, p, chunk_imgs, &no_room)
                            : conv2d_split(choice_use, split_build(choice.tile - SPLIT_TILE0, R * S, uh, uw),
@@ -4194,20 +4195,27 @@ int conv2d_winograd_fused(bool no_alloc, bool *no_room, const FusedVariant &fv, 
     return 0;
 }
 
-// The split copy of a registered filter tensor, made here where its registration did not; *Ws stays NULL where there is none.
-int kept_split_filters(SplitCall use, int dev, const ConvParams &call, size_t w_bytes, const void **Ws) {
+// The split copy of a registered filter tensor, made here where its registration did not; *Ws stays NULL where there is none.  *no_room: there is none, none
+// can be made and the call has not asked for this form; the direct kernels have their copy.
+int kept_split_filters(SplitCall use, int dev, const ConvParams &call, size_t w_bytes, const void **Ws, bool *no_room) {
+    *no_room = false;
     if (use == SplitCall::PRODUCT) return 0;  // (the rows that stand for filters are no registered tensor's, wherever they lie)
     std::lock_guard<std::mutex> lock(g_cache_mutex);
     CachedFilters *e = registered_filters(dev, call.K, call.Kf, call.C, call.R, call.S);
     if (e == nullptr) return 0;
-    if (e->Wsplit == nullptr && !state(dev).capturing && use != SplitCall::CONV_NO_ALLOC) {
-        if (hipMalloc(&e->Wsplit, w_bytes) != hipSuccess) {
+    if (e->Wsplit == nullptr) {
+        if (state(dev).capturing || use == SplitCall::PLAN_NO_ALLOC || use == SplitCall::CHOICE_NO_ALLOC) {
+            *no_room = use == SplitCall::CHOICE || use == SplitCall::CHOICE_NO_ALLOC;
+            return 0;
+        }
+        if (hipMalloc(&e->Wsplit, w_bytes) != hipSuccess) {  // (without room for them they are split per call)
             e->Wsplit = nullptr;
             (void)hipGetLastError();
+            return 0;
         }
         e->split_stale = true;
     }
-    if (e->Wsplit != nullptr && e->split_stale) EH_TRY(split_again(dev, *e));
+    if (e->split_stale) EH_TRY(split_again(dev, *e));
     *Ws = e->Wsplit;
     return 0;
 }
@@ -4215,12 +4223,12 @@ int kept_split_filters(SplitCall use, int dev, const ConvParams &call, size_t w_
 // Memory for a launch of the split form.  *no_room: nothing is to be launched, the caller has another form - the fixed scratch array is too
 // small, or the workspace is while a graph is being recorded and the call has not asked for this form (the direct and the fp32 kernels may need less).
 int split_workspace(SplitCall use, int dev, size_t bytes, void **ws, bool *no_room) {
-    if (use == SplitCall::CONV_NO_ALLOC) {
+    if (use == SplitCall::PLAN_NO_ALLOC || use == SplitCall::CHOICE_NO_ALLOC) {
         *no_room = bytes > (size_t)EDDLHIP_CONV_NOALLOC_SCRATCH_BYTES;
         *ws = g_scratch_ptr[dev];
         return 0;
     }
-    *no_room = use != SplitCall::CONV && state(dev).capturing && bytes > state(dev).workspace_bytes;
+    *no_room = use != SplitCall::PLAN && state(dev).capturing && bytes > state(dev).workspace_bytes;
     return bytes > 0 && !*no_room ? get_workspace(dev, bytes, ws) : 0;
 }
 
@@ -4236,7 +4244,8 @@ int conv2d_split(SplitCall use, const Variant &v, const Plan &plan, int dev, con
     const size_t w_bytes = split_filter_bytes(call.C, RS, call.Mp);
     const size_t partial_bytes = (size_t)plan.nslices * leftover * v.bm * v.bn * sizeof(float);
     const void *Ws = nullptr;
-    EH_TRY(kept_split_filters(use, dev, call, w_bytes, &Ws));
+    EH_TRY(kept_split_filters(use, dev, call, w_bytes, &Ws, no_room));
+    if (*no_room) return 0;
     const size_t ws_filters = Ws ? 0 : ((w_bytes + 255) & ~(size_t)255);
     void *ws = nullptr;
     EH_TRY(split_workspace(use, dev, ws_filters + partial_bytes, &ws, no_room));
@@ -4292,7 +4301,8 @@ int conv2d_wave_split(SplitCall use, const WaveSplitVariant &v, int slices, int 
     const size_t w_bytes = split_filter_bytes(call.C, RS, call.Mp);
     const size_t partial_bytes = nslices > 1 ? (size_t)nslices * wave_tiles(v, call.Kf, chunk_imgs * call.PQ) * v.tm * v.tn * 4096 : 0;
     const void *Ws = nullptr;
-    EH_TRY(kept_split_filters(use, dev, call, w_bytes, &Ws));
+    EH_TRY(kept_split_filters(use, dev, call, w_bytes, &Ws, no_room));
+    if (*no_room) return 0;
     const size_t ws_filters = Ws ? 0 : ((w_bytes + 255) & ~(size_t)255);
     void *ws = nullptr;
     EH_TRY(split_workspace(use, dev, ws_filters + partial_bytes, &ws, no_room));

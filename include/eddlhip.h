@@ -267,8 +267,9 @@ int eddlhip_conv2d_fwd_noalloc(int dev, const float *I, const float *K, const fl
  * The planner chooses a tile of this form, or of the one for few tiles below, by itself where its model expects it to be faster than the
  * direct kernels: by the geometry alone (whole groups of 16 channels, filters and partial tiles that fit the fixed scratch array, a
  * direct kernel of 7 us or more), so registered and other filters and all entry points give the same bits.  Not under set_algo(1 .. 5) or (9),
- * and not while a graph is recorded with a workspace that this form does not fit in (one that no call of that size came before): then the
- * direct kernels run, if they do.
+ * and not while a graph is recorded with a workspace that this form does not fit in (one that no call of that size came before), nor, in a
+ * recording and in eddlhip_conv2d_fwd_noalloc, on a tensor that was registered while the plan search was on and that no call has split since:
+ * then the direct kernels run.
  * The one-launch Winograd form in that arithmetic (force_plan(32, .), or the search from 512 blocks of outputs on; channel counts
  * that are multiples of 16): transformed pixels are fp32 numbers as in the third Winograd form, filters are transformed in 64 bits, the
  * products are those of the split form, and the sums of the largest of a patch's positions are rounded once per 16 channels: its error
@@ -335,9 +336,9 @@ int eddlhip_conv2d_force_plan(int tile, int slices);
 /* Filters that stay fixed between calls (inference).  Every eddlhip_conv2d_fwd first repacks its
  * filters into the kernels' tap-major layout (3-10 us per layer).  After
  * eddlhip_conv2d_cache_filters(dev, K, ...) the library keeps that repacked copy in device memory
- * of its own, and calls that pass the same K pointer and shape use it instead; where C is a multiple of 16, the split form's
- * filters as well (6 bytes a weight beside the 4), which the planner's choice may read.  Other forms' filters join them when a
- * plan first asks for that form.  The caller
+ * of its own, and calls that pass the same K pointer and shape use it instead; where C is a multiple of 16 and the plan search
+ * is off, the split form's filters as well (6 bytes a weight beside the 4), which the planner's choice may read.  Other forms' filters
+ * join them when a call first runs that form.  The caller
  * promises that K's contents change only through this library: eddlhip_memcpy_h2d/_d2d, _fill,
  * _add and _inc into a registered tensor mark its copy stale (it is repacked on the next use);
  * a kernel of the caller's own that writes K must be followed by another

@@ -342,3 +342,33 @@ def test_dense_recorded_with_the_workspace_of_the_fp32_product(hip):
         hip.fill_(C, float("nan"))
         graph.launch()
         assert np.array_equal(C.numpy(), want)
+
+
+def test_registered_under_the_search_and_called_without_allocating_first(hip):
+    """A tensor that was registered while the plan search was on has no split copy until a call makes it: a call that cannot runs the direct
+    kernels on the copy that there is, and the planner's choice from then on."""
+    N, C, H, W, Kf, R, S, stride, pad = CHOSEN[1]
+    rng = np.random.default_rng(77)
+    dx, dw = hip.array(rng.standard_normal((N, C, H, W), dtype=np.float32)), hip.array((rng.standard_normal((Kf, C, R, S)) * 0.05).astype(np.float32))
+    O = hip.full((N, Kf, H, W), float("nan"))
+
+    def run(fn):
+        hip.fill_(O, float("nan"))
+        hip._check(fn(hip.dev, dx.ptr, dw.ptr, None, O.ptr, N, C, H, W, Kf, R, S, stride, stride, pad, pad, H, W, None, None, None, None, 0.0, None, 0))
+        return "split_kernel" in hip.last_conv_kernel(), O.numpy()
+    split, want = run(hip.lib.eddlhip_conv2d_fwd)
+    hip.set_conv_algo("winograd_never")
+    direct = run(hip.lib.eddlhip_conv2d_fwd)[1]
+    hip.set_conv_algo("winograd_off")
+    hip.conv_autotune(True)
+    hip.cache_conv_filters(dw)
+    hip.conv_autotune(False)
+    try:
+        first, got = run(hip.lib.eddlhip_conv2d_fwd_noalloc)
+        assert split and not first and np.array_equal(got, direct)
+        for fn in (hip.lib.eddlhip_conv2d_fwd, hip.lib.eddlhip_conv2d_fwd_noalloc):
+            chosen, got = run(fn)
+            assert chosen and np.array_equal(got, want)
+    finally:
+        hip.conv_autotune(-1)
+        hip.uncache_conv_filters(dw)

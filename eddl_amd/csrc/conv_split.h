@@ -363,8 +363,9 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
     trace_mark(p, 1);
     constexpr int T = TM * TN;
     if constexpr (CHUNKS == 1) {
-        // Step t multiplies buffer t % 2, splits the pixels of step t + 1 into the other buffer and loads those of step t + 3.  (In the
-        // last steps nothing is loaded and what is put into the other buffer is not used.)  Two things keep the matrix
+        // Step t multiplies buffer t % 2, splits the pixels of step t + 1 into the other buffer and loads those of step t + 3.  (What the last steps
+        // load - nothing behind the last channel, the next slice's first steps otherwise - is not used; without those loads slices took the
+        // same time.)  Two things keep the matrix
         // pipe from waiting where a CU has one or two workgroups:
         //   * the six products take the parts of the pixels in turn, so the registers of a part take the next 16 channels' as soon as its
         //     last product has started, and the one barrier of a step stands where the first part of the next step is read, half
@@ -372,7 +373,8 @@ __global__ __launch_bounds__(256, WGS) void conv_split_kernel(const ConvParams p
         //   * loads arrive in the order in which they were asked for, so a wait for filters waits for the pixels asked for before
         //     them: pixels are asked for right behind the filters of the next half step, which makes theirs a whole step.
         // 12 images, the loop below -> this: 256 3x3 on 14x14 58.7 -> 53.6 us (64x64 tile 49.9 -> 41.0), 128 3x3 stride 2 on 56x56 34.6 -> 31.0,
-        // 1024 -> 256 on 14x14 26.9 -> 25.3; 64 images 256 3x3 on 14x14 94.8 -> 91.1, 1x1 layers within 1 %.
+        // 1024 -> 256 on 14x14 26.9 -> 25.3; 64 images 256 3x3 on 14x14 94.8 -> 91.1, 1x1 layers within 1 %.  Slices of 5 ... 18 steps with more than one
+        // workgroup on a CU are 1 - 4 % slower (512 3x3 on 28x28 of one image, 8 slices, 33.3 -> 34.0), from 32 steps on all are faster.
 #pragma unroll
         for (int part = 0; part < 3; part++) read_b(part, 0, 0);
         auto whole_step = [&](int step, int s) __attribute__((always_inline)) {  // s: the step's place in the unrolled loop

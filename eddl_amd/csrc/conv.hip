@@ -2886,6 +2886,7 @@ int conv_setup_device(int dev) {
     EH_REQUIRE(ptr != nullptr, "device %d: no address for the convolution's tile counts", dev);
     g_counts_ptr[dev] = (unsigned *)ptr;
     EH_TRY_HIP(hipMemset(ptr, 0, sizeof(tile_counts)));  // (also after a shutdown that cut launches short)
+    EH_TRY_HIP(hipStreamSynchronize(nullptr));  // (a caller's stream need not wait for the null stream)
     for (const Variant(*fam)[4] : {k3x3, k1x1, k2x2, kgen})
         for (int d = 0; d < 2; d++) EH_TRY(family_occupancy(fam[d]));
     return 0;

@@ -2663,8 +2663,9 @@ Plan forced_plan(const Variant *family, int tile, int slices, int Kf, int C, int
 
 // The planner's choice among the tiles of the split form (conv_split.h, conv_wave_split.h) for a convolution that the direct kernels
 // are expected to take `direct_us` for: tile -1 if none is expected to be faster.  It depends on the geometry alone, so that a convolution
-// has the same bits from registered filters, from others (splitting them costs a call what repacking them does: 10 bytes of
-// traffic a weight instead of 8) and from the entry point that allocates nothing - a choice whose filters and partial tiles do
+// has the same bits from registered filters, from others (splitting those costs a call about what repacking them does up to a million weights, 3 - 9 us, and
+// 3 - 5 us more beyond, which the choice does not count: unregistered, 174 chosen layers are 1.29 times as fast, three of more than two million weights 8 - 12 %
+// slower) and from the entry point that allocates nothing - a choice whose filters and partial tiles do
 // not fit that one's scratch array is none.
 // Time of a workgroup step: `alone` with one workgroup on a CU, at least `shared` for every one that is there; of a workgroup around its
 // steps: `fixed` and `each` for every one there.  Fitted to 6200 timed plans of 281 convolutions (1 - 64 images, 7 - 368 pixels, 16 - 1024

@@ -476,8 +476,8 @@ int eddlhip_sum2d_rowwise(int dev, const float *A, const float *B, float *C, int
  * src/hardware/cpu/nn/cpu_activations.cpp:18-33).  Each step is the separate call's fp32 operation,
  * so the result equals eddlhip_mult2d + eddlhip_sum2d_rowwise + eddlhip_relu bit for bit.  Both run products of more than 48 rows and a
  * multiple of 16 inputs in the split form of the convolutions, but for up to 256 columns under sums of more than 16384 inputs (or 4 M row
- * elements), and where C lies on A or B (not under eddlhip_conv2d_set_algo(1 .. 4) or (9)).  Up to 48 rows a row has the same bits
- * in a batch of any size; beyond, its bits may depend on the number of rows. */
+ * elements), and where C lies on A or B (not under eddlhip_conv2d_set_algo(1 .. 4) or (9)).  Among batches of up to 48 rows a
+ * row's bits do not depend on their number; beyond they may. */
 int eddlhip_dense_fwd(int dev, const float *A, const float *W, const float *bias, float *C, int m, int k, int n, int relu);
 
 #ifdef __cplusplus

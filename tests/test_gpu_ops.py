@@ -2336,3 +2336,16 @@ def test_dense_few_columns_under_a_long_sum_take_the_fp32_product(hip, m, k, n, 
         hip.set_conv_algo("winograd_off")
     assert np.array_equal(C.numpy(), D.numpy()) != split
     assert_conv_close(A.numpy().astype(np.float64) @ W.numpy().astype(np.float64), C.numpy(), "%dx%dx%d" % (m, k, n))
+
+
+@pytest.mark.parametrize("k,n", [(512, 300), (2048, 1000), (16400, 10)])
+def test_dense_rows_have_the_same_bits_in_every_batch_of_up_to_48(hip, k, n):
+    A, W, D = hip.empty((48, k)), hip.empty((k, n)), hip.empty((48, n))
+    hip.rand_normal(A, 0.0, 1.0, 51)
+    hip.rand_normal(W, 0.0, k ** -0.5, 52)
+    hip.mult2D(A, W, D)
+    want, rows = D.numpy(), A.numpy()
+    for m in (1, 2, 31, 32, 33, 47):
+        C = hip.full((m, n), np.nan)
+        hip.mult2D(hip.array(rows[48 - m:]), W, C)
+        assert np.array_equal(C.numpy(), want[48 - m:])
